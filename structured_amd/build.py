@@ -18,10 +18,10 @@ SOURCES = ["sg_api.cpp", "sg_kernels.hip", "sg_linalg.hip", "sg_solver.cpp", "sg
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-fopenmp"]
-# Per-source additions.  The chunked-ILU kernels run one work-group per chunk
-# (a few dozen on the whole chip), so their occupancy does not matter and their
-# level loop is a latency chain: the max-ILP scheduler issues a level's LDS
-# reads together and interleaves its FMA chains, where the default
+# Per-source additions.  The chunked-ILU kernels run a few work-groups per
+# chunk (at most some hundred on the whole chip), so their occupancy does not
+# matter and their step loop is a latency chain: the max-ILP scheduler issues a
+# step's LDS reads together and interleaves its FMA chains, where the default
 # occupancy-driven schedule serialises them.
 SOURCE_FLAGS = {"sg_cilu.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]}
 

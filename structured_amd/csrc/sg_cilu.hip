@@ -5,24 +5,21 @@
 // wall-normal line is contiguous and its banded part is factored exactly;
 // couplings between chunks are dropped (block Jacobi over chunks).  In that
 // order the lower neighbours of (i, j) are (-2,0), (-1,-1), (-1,0), (-1,+1),
-// (0,-2), (0,-1) and all of them lie on an earlier level L = j + 2 (i - i0);
-// a chunk has njc + 2W - 2 levels of at most W cells.  One work-group per
-// chunk walks the levels with a barrier between them.
+// (0,-2), (0,-1).  A cell can be solved two rows behind the column before it.
+//
+// The factorisation walks a chunk's levels L = j + 2 (i - i0) with one
+// work-group per chunk.  The apply cuts the chunk once more, into groups of
+// up to 12 (nv 5) or 16 (nv 4) columns with one solving wave each: a column
+// depends on earlier columns only, so the groups run as a pipeline, each on
+// its own CU, and hand the solved values of their edge columns on through
+// memory.
 //
 // Factors are stored in FP32 (the preconditioner only has to approximate
-// A^-1; FGMRES runs in FP64), per chunk in level order, one record per level:
-// rec[(((chunk * nlev + L) * NSLOT + s) * NV + r) * W + c) * NV + m] for entry
-// (r, m) of the block in slot s of the cell in column c of the chunk (row
-// j = L - 2c): slot 0 the inverse of the factored diagonal block, lower slots
-// L_rn (unit lower factor), upper slots U_ru.  A block row is NV contiguous
-// floats and the rows r of a level's cells sit next to each other, so the
-// thread for (r, c) reads its row with two wide loads and a wave's loads are
-// coalesced.  A second copy holds every block transposed, for M^-T: a column
-// of a block is then read like a row, with the same loads.
+// A^-1; FGMRES runs in FP64) in the order the solving waves read them, see
+// Lay below.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 
 #include "sg_linalg.hpp"
 
@@ -37,15 +34,13 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Compile-time stencil tables for the apply kernel (fully unrolled loops
-// fold them away): offsets, the pass's neighbour slots, and the slot of the
-// opposite offset.
+// Compile-time stencil tables (fully unrolled loops fold them away):
+// offsets and the neighbour slots of the factorisation.
 namespace ct {
 constexpr int Di[NSLOT] = {0, 0, 0, -1, 1, -1, 1, -1, 1, 0, 0, -2, 2};
 constexpr int Dj[NSLOT] = {0, -1, 1, 0, 0, -1, -1, 1, 1, -2, 2, 0, 0};
 constexpr int Low[6] = {11, 5, 3, 7, 9, 1};
 constexpr int Up[6] = {2, 10, 6, 4, 8, 12};
-constexpr int Back[NSLOT] = {0, 2, 1, 4, 3, 8, 7, 6, 5, 10, 9, 12, 11};
 // The 3x3-box pattern (slots 0-8; the +-2 slots dropped): four lower and
 // four upper neighbours, in the same order as above.
 constexpr int Low9[4] = {5, 3, 7, 1};
@@ -57,6 +52,13 @@ constexpr int low(int n) { return NINE ? Low9[n] : Low[n]; }
 template <bool NINE>
 constexpr int up(int n) { return NINE ? Up9[n] : Up[n]; }
 constexpr bool in_box(int s) { return s >= 0 && s < 9; }
+// The apply's neighbours, in the order of their records: lower ones for the
+// ascending pass, upper ones for the descending pass, entry n of one being
+// the opposite offset of entry n of the other.  0-2 are the column before
+// (its oldest, middle and newest solved cell in reach), 3 the cell's own
+// column, 4 and 5 the +-2 couplings of the 13-point stencil.
+constexpr int Asc[6] = {5, 3, 7, 1, 9, 11};
+constexpr int Desc[6] = {8, 4, 6, 2, 10, 12};
 constexpr int slot(int di, int dj) {
   for (int s = 0; s < NSLOT; ++s)
     if (Di[s] == di && Dj[s] == dj) return s;
@@ -71,9 +73,78 @@ constexpr int slot(int di, int dj) {
 // loop reads the 13 blocks of its own cells (gathered in level order by
 // cilu_gather_kernel) from memory and nothing else; the elimination exchanges
 // one 5x5 block per cell through LDS per lower neighbour.
-// Record size of one level, in floats.
-template <int NV, int W>
-constexpr int cilu_rs() { return NSLOT * NV * NV * W; }
+
+// Column groups of the apply and the layout of their factor records.
+//
+// Both passes of an apply run through the same steps: the descending one
+// counts columns and rows from the other end (c' = GW - 1 - c and s = njc -
+// 1 - j; c' = c and s = j ascending).  Step t = X + s + 2 c' solves row s of
+// column c'; X steps come first in which only edge columns of the group
+// before arrive (GC of them, none when one group holds the chunk).  Entry k
+// of column c' is on lane c' NV + k.
+//
+// Per step and lane a record holds n1 floats in the pass without the diagonal
+// (row k of the neighbours' blocks, ct::Asc or ct::Desc order), n2 in the
+// pass with it (the diagonal's row last): float4 runs over the lanes, then
+// single floats for the remainder, so a wave reads 16 bytes per lane,
+// contiguous over lanes.  Records of cells or neighbours that do not exist
+// are zero, which makes their values zero without a mask.  Four arrays: M^-1
+// ascending (L) and descending (U, D^-1), then M^-T ascending (U^T, D^-T) and
+// descending (L^T), where a block's column is stored as a row at the cell
+// that multiplies by it.
+template <int NV, int W, bool NINE>
+struct Lay {
+  static constexpr int B = NV * NV, NN = NINE ? 4 : 6;
+  static constexpr int GCX = NINE ? 1 : 2, CAP = 64 / NV;
+  static constexpr int NG = W <= CAP ? 1 : (W + CAP - 1) / CAP;
+  static constexpr int GC = NG == 1 ? 0 : GCX, X = 2 * GC;
+  static constexpr int GW = (W + NG - 1) / NG;  // columns of a group
+  static constexpr int LN = GW * NV;            // lanes with a cell
+  static constexpr int n1 = NN * NV, n2 = (NN + 1) * NV;
+  static constexpr int UN = 8;                  // steps in a block of the solving loop
+  // steps whose records are in flight (they share the registers with the
+  // operands)
+  static constexpr int pd(int n) { return n <= 20 ? 8 : 4; }
+  static constexpr int rs(int n) { return (n * LN + 15) / 16 * 16; }  // floats of a step's record
+  static constexpr int count(int a) { return a == 0 || a == 3 ? n1 : n2; }  // per lane, in array a
+  static_assert(LN <= 64, "a group fits a wave");
+  // steps of a pass, rounded up to the solving loop's blocks, and records
+  // (the loop reads ahead)
+  __host__ __device__ static int steps(int njc) { return (X + njc + 2 * (GW - 1) + UN - 1) / UN * UN; }
+  __host__ __device__ static int nrec(int njc) { return steps(njc) + UN; }
+  // float offset of array a (0-3)
+  __host__ __device__ static size_t array(int a, int nchunk, int njc) {
+    const size_t per = (size_t)nchunk * NG * nrec(njc);
+    return per * (a == 0 ? 0 : a == 1 ? rs(n1) : a == 2 ? rs(n1) + rs(n2) : rs(n1) + 2 * rs(n2));
+  }
+  __host__ __device__ static size_t floats(int nchunk, int njc) {
+    return (size_t)nchunk * NG * nrec(njc) * (2 * rs(n1) + 2 * rs(n2));
+  }
+  // float of entry f on a lane inside a record of n floats per lane
+  __device__ static unsigned in_record(int n, int lane, int f) {
+    const int q = n / 4;
+    return f < 4 * q ? (unsigned)((f / 4 * LN + lane) * 4 + (f & 3)) : (unsigned)(4 * q * LN + (f - 4 * q) * LN + lane);
+  }
+  // words of one link (edge values of one pass, all rows) and of all links
+  __host__ __device__ static size_t link(int njc) { return (size_t)njc * GC * NV; }
+  static size_t links(int nchunk, int njc) { return 2 * (size_t)nchunk * (NG - 1) * link(njc); }
+};
+
+// Zeroes the records that the factorisation does not write, or writes in
+// part: steps at both ends of a pass, and groups with absent columns.  One
+// block per record.
+template <int NV, int W, bool NINE>
+__global__ __launch_bounds__(256) void cilu_zero_kernel(int nic, int njc, int nchunk, float* rec) {
+  using La = Lay<NV, W, NINE>;
+  const int t = blockIdx.x, gg = blockIdx.y, s = t - La::X;
+  const int wk = min(W, nic - gg / La::NG * W) - gg % La::NG * La::GW;
+  if (wk >= La::GW && s >= 2 * (La::GW - 1) && s < njc) return;
+  for (int a = 0; a < 4; ++a) {
+    const int rs = La::rs(La::count(a));
+    float* r = rec + La::array(a, nchunk, njc) + ((size_t)gg * La::nrec(njc) + t) * rs;
+    for (int e = threadIdx.x; e < rs; e += 256) r[e] = 0.0f;
+  }
+}
 
 // Gathers the factorisation's operands into level order: for chunk, level L,
 // slot s, block entry e and column c, entry e of the block of I/dt - J in row
@@ -110,10 +181,18 @@ __global__ __launch_bounds__(256) void cilu_gather_kernel(int nic, int njc, int 
   }
 }
 
-// floats of one record copy (plain or transposed)
-static size_t cilu_copy_floats(int nic, int njc, int nv, int w) {
+// doubles of the gathered factorisation operands
+static size_t cilu_ops_doubles(int nic, int njc, int nv, int w) {
   const int nchunk = (nic + w - 1) / w, nlev = njc + 2 * w - 2;
   return (size_t)nchunk * nlev * NSLOT * nv * nv * w;
+}
+
+// A link word that holds no value: a signalling NaN, which no arithmetic
+// produces.
+constexpr unsigned long long kEmpty = 0x7FF45347454D5054ull;
+__global__ __launch_bounds__(256) void cilu_empty_kernel(unsigned long long* x, size_t n) {
+  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x)
+    x[e] = kEmpty;
 }
 
 // NINE: ILU(0) on the 3x3-box pattern (the +-2 blocks of A and their fill
@@ -121,16 +200,24 @@ static size_t cilu_copy_floats(int nic, int njc, int nv, int w) {
 // fill only), else on the 13-point stencil.
 template <int NV, int W, bool NINE>
 __global__ __launch_bounds__(W * NV * NV) void cilu_factor_kernel(int nic, int njc, int nlev, const double* ops,
-                                                                  float* rec, size_t tcopy) {
-  constexpr int B = NV * NV, RS = cilu_rs<NV, W>(), NR = 4, NN = ct::nn<NINE>();
+                                                                  float* rec) {
+  using La = Lay<NV, W, NINE>;
+  constexpr int B = NV * NV, NR = 4, NN = ct::nn<NINE>();
   __shared__ float ring[NR][7][W][B];  // per level: diagonal inverse, then the six upper blocks (ct::Up order)
   __shared__ double Ab[W][B];
   __shared__ double Lb[W][B];
   __shared__ double cb[2][W][NV];
   const int chunk = blockIdx.x, i0 = chunk * W, wk = min(W, nic - i0);
   const int t = threadIdx.x, c = t / B, e = t % B, r = e / NV, q = e % NV;
-  float* R = rec + (size_t)chunk * nlev * RS;
-  float* RT = R + tcopy;
+  // entry f of component row of cell (cc, jj) in array a
+  const int nchunk = gridDim.x, nrec = La::nrec(njc);
+  auto put = [&](int a, int cc, int jj, int row, int f, float v) {
+    const int n = La::count(a), g = cc / La::GW, cl = cc % La::GW;
+    const bool asc = a == 0 || a == 2;
+    const int c1 = asc ? cl : La::GW - 1 - cl, s = asc ? jj : njc - 1 - jj;
+    rec[La::array(a, nchunk, njc) + ((size_t)(chunk * La::NG + g) * nrec + La::X + s + 2 * c1) * La::rs(n) +
+        La::in_record(n, c1 * NV + row, f)] = v;
+  };
   auto inside = [&](int cc, int jj) { return cc >= 0 && cc < wk && jj >= 0 && jj < njc; };
   for (int L = 0; L < nlev; ++L) {
     const int j = L - 2 * c;
@@ -172,22 +259,24 @@ __global__ __launch_bounds__(W * NV * NV) void cilu_factor_kernel(int nic, int n
         }
       }
     }
-    // the level's L and U blocks are final: store them (record, transposed
-    // record and ring)
-    float* RL = R + (size_t)L * RS;
-    float* RTL = RT + (size_t)L * RS;
+    // the level's L and U blocks are final: store them (records of both
+    // directions and ring).  A block goes to its own row's record and,
+    // transposed, to that of the neighbour it couples to; absent neighbours
+    // leave zeros in this cell's own records.
     const int lr = L & (NR - 1);
-    // one per-thread offset for every slot and a uniform slot stride (offsets
-    // computed per slot were kept live across the level loop and spilled)
-    constexpr int SS = NV * W * NV;
-    const unsigned on = (unsigned)((r * W + c) * NV + q), ot = (unsigned)((q * W + c) * NV + r);
-    auto at_n = [&](int s) { return (size_t)s * SS + on; };
-    auto at_t = [&](int s) { return (size_t)s * SS + ot; };
+    if (valid) {
 #pragma unroll
-    for (int s = 1; s < (NINE ? 9 : NSLOT); ++s) {  // the box pattern never reads the +-2 slots
-      const float v = valid ? (float)a[s] : 0.0f;
-      RL[at_n(s)] = v;
-      RTL[at_t(s)] = v;
+      for (int n = 0; n < NN; ++n) {
+        const int sl = ct::Asc[n], su = ct::Desc[n];
+        put(0, c, j, r, n * NV + q, (float)a[sl]);
+        put(1, c, j, r, n * NV + q, (float)a[su]);
+        const int cl = c + ct::Di[sl], jl = j + ct::Dj[sl], cu = c + ct::Di[su], ju = j + ct::Dj[su];
+        const bool lok = inside(cl, jl), uok = inside(cu, ju);
+        if (lok) put(3, cl, jl, q, n * NV + r, (float)a[sl]);
+        else put(2, c, j, q, n * NV + r, 0.0f);
+        if (uok) put(2, cu, ju, q, n * NV + r, (float)a[su]);
+        else put(3, c, j, q, n * NV + r, 0.0f);
+      }
     }
 #pragma unroll
     for (int ui = 0; ui < NN; ++ui) ring[lr][1 + ui][c][e] = valid ? (float)a[ct::up<NINE>(ui)] : 0.0f;
@@ -238,297 +327,434 @@ __global__ __launch_bounds__(W * NV * NV) void cilu_factor_kernel(int nic, int n
     }
     lds_barrier();
     const float dinv = valid ? (float)Lb[c][e] : 0.0f;
-    RL[at_n(0)] = dinv;
-    RTL[at_t(0)] = dinv;
+    if (valid) {
+      put(1, c, j, r, NN * NV + q, dinv);
+      put(2, c, j, q, NN * NV + r, dinv);
+    }
     ring[lr][0][c][e] = dinv;
   }
 }
 
-// One stored row of a block (NV contiguous floats), widened to double.  The
-// row is read as one unit so that it takes two wide loads (16 + 4 bytes for
-// NV = 5) rather than NV single-float loads: the level loop issues few
-// enough memory instructions that their address processing does not pace it.
-template <int NV>
-struct FRow {
-  float v[NV];
+// LDS of one group's work-group: the solved values of the last kRing steps by
+// step, column and component (edge columns first; idle lanes store to the
+// column after the last), the right-hand sides of the steps to come, and how
+// far each wave has got.
+constexpr int kRing = 64;
+template <int NV, int W, bool NINE>
+struct ApplyLds {
+  using La = Lay<NV, W, NINE>;
+  static constexpr int NVP = (NV + 1) & ~1;  // a cell's values, in 16-byte units
+  static constexpr int NP = La::GCX + La::GW;
+  double ring[kRing][NP + 1][NVP] __attribute__((aligned(16)));
+  double x[kRing][64];
+  double tmp[La::CAP + 1][NVP] __attribute__((aligned(16)));
+  // per pass: steps solved, right-hand-side rows loaded, edge rows received,
+  // rows taken out of the ring, rows whose stores are complete
+  int step[2], loaded[2], edges[2], taken[2], stored[2];
 };
-template <int NV, int W>
-__device__ __forceinline__ void load_row(const float* p, double* out) {
-  const FRow<NV> row = *reinterpret_cast<const FRow<NV>*>(p);
-#pragma unroll
-  for (int m = 0; m < NV; ++m) out[m] = row.v[m];
+__device__ __forceinline__ int lds_read(const int* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void lds_write(int* p, int v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void lds_release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local"); }
+__device__ __forceinline__ void lds_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local"); }
+// Orders this wave's LDS accesses (a wave's LDS operations execute in issue
+// order, so nothing is waited for).
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
 }
 
-// One level's operands of thread (k, c): f[n*NV + m] for the six neighbours n
-// of the pass, d[m] for the diagonal inverse (row k, or column k when
-// transposed; only in the pass that applies it), x the right-hand side.  R is the record copy of the pass: the
-// plain one for M^-1, the transposed one for M^-T, where a column of a block
-// is a stored row.  The factorisation stores exact zeros for neighbours
-// outside the chunk or the grid and for invalid cells (the transposed pass
-// reads the cell's own slot, zero for an absent neighbour), so nothing is
-// masked and all the loads of a level are in flight together.
-template <int NV, int W, bool NINE, bool TR, bool ASC, bool DIAG>
-__device__ __forceinline__ void cilu_fetch(const float* R, int nlev, int njc, int ldi, size_t plane, int i0, int wk,
-                                           int k, int c, int L, const double* src, double* f, double* d, double& x) {
-  constexpr int RS = cilu_rs<NV, W>();
-  const int j = L - 2 * c;
-  const bool lok = L >= 0 && L < nlev;
-  const bool valid = lok && c < wk && j >= 0 && j < njc;
-  const float* RL = R + (size_t)(lok ? L : 0) * RS;
-  auto row = [&](const float* Rlev, int s, int r, int col) { return Rlev + ((size_t)(s * NV + r) * W + col) * NV; };
-#pragma unroll
-  for (int n = 0; n < ct::nn<NINE>(); ++n) {
-    const int s = ASC ? ct::low<NINE>(n) : ct::up<NINE>(n);
-    if (!TR) {
-      load_row<NV, W>(row(RL, s, k, c), f + n * NV);
-    } else {
-      // column k of the neighbour's block that points back to this cell
-      const int cn = c + ct::Di[s], jn = j + ct::Dj[s];
-      const bool nok = valid && cn >= 0 && cn < wk && jn >= 0 && jn < njc;
-      const float* p = nok ? row(R + (size_t)(jn + 2 * cn) * RS, ct::Back[s], k, cn) : row(RL, s, k, c);
-      load_row<NV, W>(p, f + n * NV);
+constexpr int kAll = 1 << 29;  // a count that never holds the solving wave up
+// Polls without a new row before a link gives up (each takes about a
+// microsecond, so several seconds).  The groups of a chunk are dispatched
+// one after another, so the one that fills a link runs or has run, and the
+// wait ends.
+constexpr int kLinkPolls = 1 << 22;
+
+// The receiving wave of one pass: moves the edge rows the group before
+// publishes into the ring.  One poll reads as many rows as fit the wave; a
+// word is read as one 64-bit atomic and holds either a value or kEmpty, so
+// nothing has to be ordered between words.
+template <int NV, int W, bool NINE>
+__device__ void cilu_receive(unsigned long long* in, int njc, ApplyLds<NV, W, NINE>& sh, int pass) {
+  using La = Lay<NV, W, NINE>;
+  constexpr int EN = La::GCX * NV, RP = 64 / EN;
+  const int lane = threadIdx.x & 63, rr = lane / EN, gi = lane % EN / NV, k = lane % NV;
+  int n = 0, polls = 0;
+  while (n < njc) {
+    // edge column gi's row s belongs to step s + X - 2 (1 + gi); its place
+    // holds a value that is read up to three steps after its own
+    const int row = n + rr, free = lds_read(&sh.step[pass]) + kRing - 8 - La::X;
+    unsigned long long v = kEmpty;
+    if (rr < RP && row < njc && row < free)
+      v = __hip_atomic_load(in + (size_t)row * EN + lane % EN, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long missing = ~__ballot(v != kEmpty);
+    const int rows = min(RP, (missing ? __builtin_ctzll(missing) : 64) / EN);
+    if (rows == 0) {
+      if (n < free && ++polls > kLinkPolls) break;  // a full ring is no failure
+      continue;
     }
+    polls = 0;
+    if (rr < rows)
+      sh.ring[(row + La::X - 2 * (1 + gi)) & (kRing - 1)][La::GCX - 1 - gi][k] = __longlong_as_double((long long)v);
+    n += rows;
+    lds_release();
+    if (lane == 0) lds_write(&sh.edges[pass], n < njc ? n : kAll);
   }
-  if (DIAG) load_row<NV, W>(row(RL, 0, k, c), d);
-  x = src[k * plane + (valid ? (size_t)j * ldi + i0 + c : 0)];
+  if (n < njc) {  // never filled: every value that depends on it becomes NaN
+    for (int e = lane; e < kRing * EN; e += 64) sh.ring[e / EN][e % EN / NV][e % NV] = __builtin_nan("");
+    lds_release();
+    if (lane == 0) lds_write(&sh.edges[pass], kAll);
+  }
 }
 
-// One level of a triangular pass with its operands already in registers.
-// Returns the thread's solved value (stored to z by the caller).
+// The storing wave of one pass: takes finished rows out of the ring, stores
+// them to z (a row is contiguous in memory, a step's cells are not) and
+// publishes the edge columns for the next group.  In the solving wave these
+// stores held up the loads, whose waits run in issue order.
+template <int NV, int W, bool NINE, bool ASC>
+__device__ void cilu_store(double* z, int njc, int ldi, size_t plane, int col0, int wk, unsigned long long* out,
+                           ApplyLds<NV, W, NINE>& sh, int pass) {
+  using La = Lay<NV, W, NINE>;
+  constexpr int LAST = La::X + 2 * (La::GW - 1), RB = 4;
+  const int lane = threadIdx.x & 63, k = lane % NV, c1 = lane / NV, c = ASC ? c1 : La::GW - 1 - c1;
+  const int gi = La::GW - 1 - c1;
+  const bool live = c1 < La::GW && c < wk, pub = out && c1 < La::GW && gi < La::GC;
+  double* zl = z + (size_t)k * plane + col0 + (live ? c : 0);
+  for (int n = 0; n < njc;) {
+    const int rows = min(min(lds_read(&sh.step[pass]) - LAST, njc) - n, RB);
+    if (rows <= 0) {
+      __builtin_amdgcn_s_sleep(1);
+      continue;
+    }
+    lds_acquire();
+    double v[RB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+      v[r] = sh.ring[(La::X + n + r + 2 * c1) & (kRing - 1)][min(La::GCX + c1, ApplyLds<NV, W, NINE>::NP)][k];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      if (r >= rows) break;
+      if (pub)
+        __hip_atomic_store(out + ((size_t)(n + r) * La::GCX + gi) * NV + k, (unsigned long long)__double_as_longlong(v[r]),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (live) zl[(size_t)(ASC ? n + r : njc - 1 - n - r) * ldi] = v[r];
+    }
+    n += rows;
+    lds_release();
+    if (lane == 0) lds_write(&sh.taken[pass], n < njc ? n : kAll);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  if (lane == 0) lds_write(&sh.stored[pass], 1);
+}
+
+// The loading wave of one pass: brings the right-hand sides into LDS by step
+// (a row's cells belong to steps two apart), LB rows at a time and one batch
+// ahead, and reads one word of every 128-byte line of the records 16 to 32
+// steps ahead of the solving wave, so that its loads find them in the XCD's
+// L2 instead of memory (much further ahead, the groups of an XCD overflow it).
 template <int NV, int W, bool NINE, bool ASC, bool DIAG>
-__device__ __forceinline__ double cilu_level(int L, int njc, int wk, int k, int c, const double* f, const double* d,
-                                             double x, double (*ring)[NV][W], double (*tmp)[W]) {
-  constexpr int NR = 8;
-  const int j = L - 2 * c;
-  const bool valid = c < wk && j >= 0 && j < njc;
-  double a0 = x, a1 = 0.0;
+__device__ void cilu_load(const float* R, int njc, int ldi, size_t plane, int col0, int wk, const double* src,
+                          ApplyLds<NV, W, NINE>& sh, int pass) {
+  using La = Lay<NV, W, NINE>;
+  constexpr int RS = La::rs(DIAG ? La::n2 : La::n1), LB = 16, TAIL = 2 * (La::GW - 1);
+  // a batch is fetched when the solving wave is at step s0 - (kRing - X - TAIL)
+  constexpr int LEAD = kRing - La::X - TAIL - LB;
+  const int lane = threadIdx.x & 63, k = lane % NV, c1 = lane / NV, c = ASC ? c1 : La::GW - 1 - c1;
+  const int nrec = La::nrec(njc);
+  const bool live = c1 < La::GW && c < wk;
+  const double* sl = src + (size_t)k * plane + col0 + (live ? c : 0);
+  double v[2][LB];
+  float touch[LB];
+  auto fetch = [&](int s0, int b) {
 #pragma unroll
-  for (int n = 0; n < ct::nn<NINE>(); ++n) {
-    const int s = ASC ? ct::low<NINE>(n) : ct::up<NINE>(n);
-    const int cn = c + ct::Di[s], jn = j + ct::Dj[s];
-    // out-of-chunk / out-of-grid neighbours carry f = 0: any in-range ring
-    // entry (all finite) will do
-    const int cc = min(max(cn, 0), W - 1), jr = jn & (NR - 1);
-    double t = 0.0;
+    for (int u = 0; u < LB; ++u) {
+      const int s = min(max(s0 + u, 0), njc - 1);
+      v[b][u] = sl[(size_t)(ASC ? s : njc - 1 - s) * ldi];
+    }
 #pragma unroll
-    for (int m = 0; m < NV; ++m) t += f[n * NV + m] * ring[jr][m][cc];
-    if (n & 1) a1 += t;
-    else a0 -= t;
+    for (int u = 0; u < LB; ++u)
+      touch[u] = R[(size_t)min(max(s0 + u - LEAD, 0), nrec - 1) * RS + min(lane * 32, RS - 1)];
+  };
+  // rows before the first are zero too: every place starts at zero
+  for (int e = lane; e < kRing * 64; e += 64) (&sh.x[0][0])[e] = 0.0;
+  fetch(0, 0);
+  for (int s0 = 0; s0 < njc + TAIL; s0 += 2 * LB) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int s1 = s0 + b * LB;
+#pragma unroll
+      for (int u = 0; u < LB; ++u) asm volatile("" ::"v"(touch[u]));
+      fetch(s1 + LB, b ^ 1);
+      // the last place this batch writes must have been read
+      while (lds_read(&sh.step[pass]) < La::X + s1 + LB - 1 + TAIL + 1 - kRing) __builtin_amdgcn_s_sleep(2);
+#pragma unroll
+      for (int u = 0; u < LB; ++u)
+        sh.x[(La::X + s1 + u + 2 * c1) & (kRing - 1)][lane] = live && s1 + u < njc ? v[b][u] : 0.0;
+      lds_release();
+      if (lane == 0) lds_write(&sh.loaded[pass], s1 + LB);
+    }
   }
-  double acc = a0 - a1;
-  if (DIAG) {
-    if (valid) tmp[k][c] = acc;
-    lds_barrier();
-    double v = 0.0;
-#pragma unroll
-    for (int m = 0; m < NV; ++m) v += d[m] * tmp[m][c];
-    acc = v;
-  }
-  if (valid) ring[j & (NR - 1)][k][c] = acc;
-  lds_barrier();
-  return acc;
+  if (lane == 0) lds_write(&sh.loaded[pass], kAll);
 }
 
-// Operand sets in rotation: the loads of a level are issued NBUF - 1 levels
-// ahead of their use.  Two sets measured best; deeper prefetch does not pay,
-// because a level is paced by how fast the chunk's factor records reach one
-// CU (about 22 KB per level and pass at W = 32), not by the latency of one
-// load.
-constexpr int NBUF = 2;
-
-// Helper work-groups: per chunk, NHELP work-groups on the same XCD (work-groups
-// are dealt to the 8 XCDs round-robin by index) load the factor lines of the
-// levels ahead of the solving work-group, so that its loads hit that XCD's L2
-// instead of HBM.  They only load (nothing they do affects the result), at
-// most HLEAD steps ahead of the progress the solving work-group reports every
-// PROG_EVERY steps, HB of their levels per batch.  Their wait for progress is
-// bounded, so they always finish.  One helper measured best (two or three
-// were no faster, six slower); a report costs the solving work-group about a
-// memory round trip, so reports are sparse and the lead is generous.
-constexpr int NHELP = 1, HB = 4, HLEAD = 32, PROG_EVERY = 16;
-constexpr int HSPIN = 4096, HSPIN_TOTAL = 1 << 16;
-
-// Levels whose solved values are stored to z together.  A store joins the
-// in-order count of outstanding memory operations that every later wait for
-// a load drains, so one burst per ZB levels stalls at most once where a
-// store per level could stall every level.  With the helper in place the
-// measured effect is small (M^-T 603 -> 594 us, M^-1 unchanged at 705x321).
-constexpr int ZB = 8;
-static_assert(ZB % NBUF == 0 && PROG_EVERY % ZB == 0, "batch sizes");
-
-// One triangular pass over the chunk's levels (ascending or descending),
-// applying the diagonal inverse when DIAG.  NBUF operand sets rotate so that
-// the loads of the next NBUF - 1 levels stay in flight while the current
-// level computes.  The level count is rounded up to a multiple of ZB; the
-// extra levels hold no valid cell.  Thread 0 reports the steps done to
-// *prog (tag | steps) for the helpers, right after a level's loads, so that
-// the report's store is not waited for before the next level.
-template <int NV, int W, bool NINE, bool TR, bool ASC, bool DIAG>
-__device__ __forceinline__ void cilu_pass(const float* R, int nlev, int njc, int ldi, size_t plane, int i0, int wk,
-                                          int k, int c, const double* src, double* z, double (*ring)[NV][W],
-                                          double (*tmp)[W], unsigned* prog, unsigned tag) {
-  double f[NBUF][ct::nn<NINE>() * NV], d[NBUF][NV], x[NBUF];
-  auto lev = [&](int step) { return ASC ? step : nlev - 1 - step; };
-#pragma unroll
-  for (int u = 0; u < NBUF - 1; ++u)
-    cilu_fetch<NV, W, NINE, TR, ASC, DIAG>(R, nlev, njc, ldi, plane, i0, wk, k, c, lev(u), src, f[u], d[u], x[u]);
-  for (int step = 0; step < nlev; step += ZB) {
-    double zv[ZB];
-#pragma unroll
-    for (int u = 0; u < ZB; ++u) {
-      const int cur = u % NBUF, nb = (u + NBUF - 1) % NBUF;
-      cilu_fetch<NV, W, NINE, TR, ASC, DIAG>(R, nlev, njc, ldi, plane, i0, wk, k, c, lev(step + u + NBUF - 1), src,
-                                             f[nb], d[nb], x[nb]);
-      if (u == 0 && prog && threadIdx.x == 0 && (step % PROG_EVERY) == 0)
-        __hip_atomic_store(prog, tag + (unsigned)step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      zv[u] = cilu_level<NV, W, NINE, ASC, DIAG>(lev(step + u), njc, wk, k, c, f[cur], d[cur], x[cur], ring, tmp);
-    }
-#pragma unroll
-    for (int u = 0; u < ZB; ++u) {
-      const int j = lev(step + u) - 2 * c;
-      if (c < wk && j >= 0 && j < njc) z[k * plane + (size_t)j * ldi + i0 + c] = zv[u];
-    }
-  }
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
 }
 
-// Helper h of a chunk: loads one word of every 128-byte line of the slots a
-// pass reads, level by level in the pass's order, steps h, h + NHELP, ...
-// Pass p (0 ascending, 1 descending) of M^-1 reads the lower slots, then the
-// upper slots and the diagonal; M^-T reads them the other way round.
-template <int NV, int W, bool NINE, bool TR>
-__device__ void cilu_helper(const float* R, int nlev, const unsigned* prog, unsigned epoch, int h, unsigned* sink) {
-  constexpr int NT = NV * W, SLOTF = NV * NV * W, RS = cilu_rs<NV, W>(), NN = ct::nn<NINE>();
-  constexpr int LPS = (SLOTF + 31) / 32;               // 128-byte lines per slot
-  constexpr int LPT = ((NN + 1) * LPS + NT - 1) / NT;  // lines per thread and level
-  float acc = 0.f;
-  int budget = HSPIN_TOTAL;
-  for (int pass = 0; pass < 2; ++pass) {
-    const bool upper = (pass == 0) == TR;  // upper slots and the diagonal
-    const int nslot = upper ? NN + 1 : NN;
-    int off[LPT];
+// The solving wave of one pass, applying the diagonal inverse when DIAG.  A
+// cell's two critical couplings (its own column and the newest cell of the
+// column before) are read right after the step before is stored; the others
+// were read one and two steps earlier, and their products (`base`) and the
+// conversions of the coming step are formed while an LDS exchange is under
+// way.  The wave issues one instruction every four cycles at best, so its
+// instructions are what a step costs: everything that is not a factor, an FMA
+// or an exchange with its neighbours is done by the other waves, and no step
+// has a branch but the one that waits for them.
+template <int NV, int W, bool NINE, bool DIAG>
+__device__ __forceinline__ void cilu_solve(const float* R, int njc, ApplyLds<NV, W, NINE>& sh, int pass, bool up) {
+  using La = Lay<NV, W, NINE>;
+  using A = ApplyLds<NV, W, NINE>;
+  constexpr int N = DIAG ? La::n2 : La::n1, RS = La::rs(N), NQ = N / 4, NREM = N % 4, PD = La::pd(N), UN = La::UN;
+  static_assert(kRing % UN == 0 && UN % PD == 0, "a block does not wrap around the ring");
+  const int lane = threadIdx.x & 63, k = lane % NV, c1 = lane / NV;
+  const bool real = c1 < La::GW;
+  const int pos = La::GCX + (real ? c1 : 0), wpos = real ? pos : A::NP;
+  const int T = La::steps(njc), rl = min(lane, La::LN - 1);
+  const auto rrec = buffer_of(R, (size_t)La::nrec(njc) * RS * sizeof(float));
+  const unsigned oq = rl * 16, or_ = (4 * NQ * La::LN + rl) * 4;
+  u32x4 fq[PD][NQ > 0 ? NQ : 1];
+  unsigned fr[PD][NREM > 0 ? NREM : 1];
+  auto fetch = [&](int t, int u) {
+    const int so = t * (RS * 4);
 #pragma unroll
-    for (int u = 0; u < LPT; ++u) {
-      const int t = threadIdx.x + u * NT, si = t / LPS, ln = t % LPS;
-      const int s = si >= nslot ? -1 : upper ? (si == NN ? 0 : ct::up<NINE>(si)) : ct::low<NINE>(si);
-      off[u] = (s < 0 || ln * 32 >= SLOTF) ? -1 : s * SLOTF + ln * 32;
+    for (int q = 0; q < NQ; ++q) fq[u][q] = __builtin_amdgcn_raw_buffer_load_b128(rrec, oq + q * La::LN * 16, so, 0);
+#pragma unroll
+    for (int q = 0; q < NREM; ++q) fr[u][q] = __builtin_amdgcn_raw_buffer_load_b32(rrec, or_ + q * La::LN * 4, so, 0);
+  };
+  auto factor = [&](int u, int e) -> double {  // entry e of the record in set u
+    return e < 4 * NQ ? __uint_as_float(fq[u][e / 4 < NQ ? e / 4 : 0][e & 3])
+                      : __uint_as_float(fr[u][e >= 4 * NQ ? e - 4 * NQ : 0]);
+  };
+#pragma unroll
+  for (int u = 0; u < PD; ++u) {
+    fetch(u, u);
+    // in the loop's order: the wait for a load counts what was issued after
+    // it on every path to it
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  int lim = 0;  // steps the other waves allow
+  auto wait = [&](int t) {
+    if (t < lim) return;
+    do {
+      // x is read one step early
+      const int a = lds_read(&sh.loaded[pass]) + La::X - 1, b = up ? lds_read(&sh.edges[pass]) + 1 : kAll;
+      const int c = lds_read(&sh.taken[pass]) + kRing + La::X;
+      lim = __builtin_amdgcn_readfirstlane(min(min(a, b), c));
+    } while (t >= lim);
+    lds_acquire();
+  };
+  // the column before at its newest and middle cell in reach (its oldest is
+  // in base); the own column's last two cells; the column two before; the
+  // coming step's right-hand side, and it without the early couplings
+  double xn[NV], vb[NV], xo[NV], xp[NV], far[NV], fo[NV], fn[NV], fd[NV], x, base;
+#pragma unroll
+  for (int m = 0; m < NV; ++m) xn[m] = vb[m] = xo[m] = xp[m] = far[m] = 0.0;
+  auto early = [&](int u, const double* old, const double* mid, const double* own2) {
+    double p = x, s = 0.0;
+#pragma unroll
+    for (int m = 0; m < NV; ++m) {
+      p -= factor(u, m) * old[m];
+      s += factor(u, NV + m) * mid[m];
     }
-    const unsigned base = (unsigned)(pass * nlev);
-    for (int s0 = h; s0 < nlev; s0 += NHELP * HB) {
-      const unsigned last = base + (unsigned)min(s0 + NHELP * (HB - 1), nlev - 1);
-      for (int spin = 0; spin < HSPIN && budget > 0; ++spin, --budget) {
-        const unsigned v = __hip_atomic_load(prog, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned done = (v >> 16) == epoch ? (v & 0xffffu) : 0u;
-        if (done + HLEAD >= last) break;
-        __builtin_amdgcn_s_sleep(4);
+    if (!NINE) {
+#pragma unroll
+      for (int m = 0; m < NV; ++m) {
+        p -= factor(u, 4 * NV + m) * own2[m];
+        s += factor(u, 5 * NV + m) * far[m];
       }
-      float v[HB][LPT];
+    }
+    base = p - s;
+  };
+  auto widen = [&](int u) {
 #pragma unroll
-      for (int b = 0; b < HB; ++b) {
-        const int step = s0 + NHELP * b, L = pass == 0 ? step : nlev - 1 - step;
+    for (int m = 0; m < NV; ++m) {
+      fo[m] = factor(u, 3 * NV + m);
+      fn[m] = factor(u, 2 * NV + m);
+      if (DIAG) fd[m] = factor(u, La::n1 + m);
+    }
+  };
+  wait(0);
+  x = sh.x[0][lane];
+  early(0, vb, vb, xp);
+  widen(0);
+  x = sh.x[1][lane];
+  for (int t0 = 0; t0 < T; t0 += UN) {
+    const int r0 = t0 & (kRing - 1), r1 = (t0 + UN) & (kRing - 1);
 #pragma unroll
-        for (int u = 0; u < LPT; ++u) v[b][u] = (step < nlev && off[u] >= 0) ? R[(size_t)L * RS + off[u]] : 0.f;
+    for (int u = 0; u < UN; ++u) {
+      const int t = t0 + u, nx = (u + 1) % PD;
+      double p = base, s = 0.0;
+#pragma unroll
+      for (int m = 0; m < NV; ++m) {
+        p -= fo[m] * xo[m];
+        s += fn[m] * xn[m];
       }
+      double r = p - s;
+      if (DIAG) {
+        sh.tmp[c1][k] = r;
+        wave_order();
+        double td[NV];
 #pragma unroll
-      for (int b = 0; b < HB; ++b)
+        for (int m = 0; m < NV; ++m) td[m] = sh.tmp[c1][m];
+        if (NINE) {
+          __builtin_amdgcn_sched_barrier(0);
+          early(nx, vb, xn, xo);
+        }
+        r = 0.0;
 #pragma unroll
-        for (int u = 0; u < LPT; ++u) acc += v[b][u];
+        for (int m = 0; m < NV; ++m) r += fd[m] * td[m];
+      }
+      auto* cur = sh.ring[r0 + u];
+      cur[wpos][k] = r;
+      wave_order();
+      if (u & 1) lds_write(&sh.step[pass], t + 1);
+      wait(t + 1);
+      double own2[NV], old[NV];
+#pragma unroll
+      for (int m = 0; m < NV; ++m) {
+        old[m] = vb[m]; own2[m] = xo[m];
+        vb[m] = xn[m];
+        xo[m] = cur[pos][m];
+        xn[m] = cur[pos - 1][m];
+        if (!NINE) far[m] = sh.ring[(t - 3) & (kRing - 1)][pos - 2][m];
+      }
+      const double x2 = sh.x[u + 2 < UN ? r0 + u + 2 : r1 + u + 2 - UN][lane];
+      __builtin_amdgcn_sched_barrier(0);  // the reads go first: the next step starts with them
+      if (!(DIAG && NINE)) early(nx, old, vb, own2);
+      x = x2;
+      widen(nx);
+      fetch(t + PD, u % PD);
     }
   }
-  // keeps the loads: the sum is used, but it reaches memory only when a factor
-  // is not finite, and then only a word that nothing reads
-  if (acc != acc && threadIdx.x == 0) *sink = 1u;
 }
 
-// z = (LU)^-1 b, or (LU)^-T b when TR.  Thread (k, c): component k of the
-// cell in column c.  Operands are loaded one level ahead of their use.
-// Work-groups [0, nchunk) solve their chunk; with helpers (prog non-null),
-// work-group npad (1 + m) + chunk is helper m of the chunk, npad being the
-// chunk count rounded up to a multiple of 8, so it runs on the chunk's XCD.
+// z = (LU)^-1 b, or (LU)^-T b when TR.  Wave 0 of a work-group solves one
+// column group, wave 1 loads and wave 2 stores for it, and wave 3 receives
+// the edge columns of the group before where a chunk has several.
+// Work-groups are dealt to the XCDs round-robin by index: the groups of a
+// chunk sit on one XCD, consecutive in its order, so a group's neighbours are
+// dispatched with it.
+//
+// What bounds it: a step of the solving wave, about 200 ns of one wave's
+// instructions (a conversion takes 8 cycles, an FMA 4.4, the store and reads
+// that link two steps about 100), times njc + 2 W steps and a pass.  With one
+// work-group of nv W threads per chunk and a barrier per level it was 600 ns.
+// Precond 7, W 32, M^-1 (M^-T alike): 97x65 nv 4 101 -> 56 us, 385x193 315 ->
+// 136, 705x321 455 -> 197, 1409x641 966 -> 450 (there the record loads of one
+// CU, about 18 bytes/ns from memory, hold a step up to 330 ns).
 template <int NV, int W, bool NINE, bool TR>
-__global__ __launch_bounds__(NV * W) void cilu_apply_kernel(int nic, int njc, int ldi, int nlev, const float* rec,
-                                                            size_t tcopy, const double* b, double* z, unsigned* prog,
-                                                            unsigned epoch) {
-  constexpr int RS = cilu_rs<NV, W>();
-  // column index fastest: the lanes of a wave are consecutive columns, so
-  // their LDS reads and writes fall in distinct banks
-  __shared__ double ring[8][NV][W];
-  __shared__ double tmp[NV][W];
-  const int nchunk = (nic + W - 1) / W, npad = (nchunk + 7) & ~7;
-  const int chunk = (int)blockIdx.x % npad, role = (int)blockIdx.x / npad;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void cilu_apply_kernel(
+    int nic, int njc, int ldi, int nchunk, const float* rec, unsigned long long* links, const double* b, double* z) {
+  using La = Lay<NV, W, NINE>;
+  __shared__ ApplyLds<NV, W, NINE> sh;
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int chunk = slot / La::NG * 8 + xcd, g = slot % La::NG;
   if (chunk >= nchunk) return;
-  const float* R = rec + (TR ? tcopy : 0) + (size_t)chunk * nlev * RS;
-  if (role > 0) {
-    cilu_helper<NV, W, NINE, TR>(R, nlev, prog + chunk, epoch, role - 1, prog + npad);
-    return;
+  const int i0 = chunk * W, wk = min(W, nic - i0) - g * La::GW;  // columns from this group on
+  if (wk <= 0) return;
+  const bool left = g > 0, right = wk > La::GW;
+  // values of steps not yet solved meet zero factors: they need to be finite
+  double* zero = &sh.ring[0][0][0];
+  for (int e = threadIdx.x; e < (int)(sizeof(sh.ring) / sizeof(double)); e += blockDim.x) zero[e] = 0.0;
+  if (threadIdx.x < 2) {
+    sh.step[threadIdx.x] = sh.edges[threadIdx.x] = sh.taken[threadIdx.x] = sh.stored[threadIdx.x] = 0;
+    sh.loaded[threadIdx.x] = -La::X;  // not even the steps before the first row may start
   }
-  const int i0 = chunk * W, wk = min(W, nic - i0);
-  const size_t plane = (size_t)njc * ldi;
-  const int k = threadIdx.x / W, c = threadIdx.x % W;
-  unsigned* pc = prog ? prog + chunk : nullptr;
-  const unsigned tag = epoch << 16;
-  // ring cells never written hold zeros (their f is zero too)
-  for (int e = threadIdx.x; e < W * 8 * NV; e += NV * W) (&ring[0][0][0])[e] = 0.0;
   __syncthreads();
+  const size_t plane = (size_t)njc * ldi, gr = (size_t)(chunk * La::NG + g) * La::nrec(njc);
+  const float* R1 = rec + La::array(TR ? 2 : 0, nchunk, njc) + gr * La::rs(TR ? La::n2 : La::n1);
+  const float* R2 = rec + La::array(TR ? 3 : 1, nchunk, njc) + gr * La::rs(TR ? La::n1 : La::n2);
+  const int col0 = i0 + g * La::GW, wg = min(wk, La::GW);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // link l of a pass joins groups l and l + 1
+  const size_t lw = La::link(njc);
+  unsigned long long* la = links + (size_t)chunk * (La::NG - 1) * lw;
+  unsigned long long* ld = la + (size_t)nchunk * (La::NG - 1) * lw;
   // non-transposed: unit-lower L ascending, then D + U descending;
   // transposed: (D + U)^T ascending, then unit-lower L^T descending
-  cilu_pass<NV, W, NINE, TR, true, TR>(R, nlev, njc, ldi, plane, i0, wk, k, c, b, z, ring, tmp, pc, tag);
-  // the second pass reads what the first stored: complete every store first
-  __syncthreads();
-  cilu_pass<NV, W, NINE, TR, false, !TR>(R, nlev, njc, ldi, plane, i0, wk, k, c, z, z, ring, tmp, pc,
-                                         tag + (unsigned)nlev);
+  if (wave == 0) {
+    cilu_solve<NV, W, NINE, TR>(R1, njc, sh, 0, left);
+    cilu_solve<NV, W, NINE, !TR>(R2, njc, sh, 1, right);
+  } else if (wave == 1) {
+    cilu_load<NV, W, NINE, true, TR>(R1, njc, ldi, plane, col0, wg, b, sh, 0);
+    // the second pass loads what the first stored, and reuses its LDS
+    while (!lds_read(&sh.stored[0]) || lds_read(&sh.step[0]) < La::steps(njc)) __builtin_amdgcn_s_sleep(1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    cilu_load<NV, W, NINE, false, !TR>(R2, njc, ldi, plane, col0, wg, z, sh, 1);
+  } else if (wave == 2) {
+    cilu_store<NV, W, NINE, true>(z, njc, ldi, plane, col0, wg, right ? la + g * lw : nullptr, sh, 0);
+    cilu_store<NV, W, NINE, false>(z, njc, ldi, plane, col0, wg, left ? ld + (g - 1) * lw : nullptr, sh, 1);
+  } else {
+    if (left) cilu_receive<NV, W, NINE>(la + (g - 1) * lw, njc, sh, 0);
+    if (right) {
+      // the first pass is done with the edge columns' places
+      while (lds_read(&sh.step[0]) < La::steps(njc)) __builtin_amdgcn_s_sleep(1);
+      cilu_receive<NV, W, NINE>(ld + g * lw, njc, sh, 1);
+    }
+    // the links are empty for the next apply
+    for (size_t e = threadIdx.x & 63; e < lw; e += 64) {
+      if (left) __hip_atomic_store(la + (g - 1) * lw + e, kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (right) __hip_atomic_store(ld + g * lw + e, kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
 }
 
-// progress words of the helpers: one per chunk (padded to a multiple of 8)
-// and one sink, after both copies
-static size_t cilu_prog_words(int nic, int w) { return (size_t)(((nic + w - 1) / w + 7) & ~7) + 1; }
-
-// doubles before the gathered factorisation operands: both copies of FP32
-// factors, then the progress words
-static size_t cilu_ops_offset(int nic, int njc, int nv, int w) {
-  return cilu_copy_floats(nic, njc, nv, w) + (cilu_prog_words(nic, w) + 1) / 2;
-}
-
-// in doubles of storage: the factors, the progress words and the gathered
-// operands (as many doubles as one copy has floats)
-size_t cilu_size(int nic, int njc, int nv, int w) {
-  return cilu_ops_offset(nic, njc, nv, w) + cilu_copy_floats(nic, njc, nv, w);
+template <int NV, int W, bool NINE>
+static size_t cilu_size_t(int nic, int njc) {
+  using La = Lay<NV, W, NINE>;
+  const int nchunk = (nic + W - 1) / W;
+  return (La::floats(nchunk, njc) + 1) / 2 + La::links(nchunk, njc) + cilu_ops_doubles(nic, njc, NV, W);
 }
 
 template <int NV, int W, bool NINE>
 static void cilu_factor_t(int nic, int njc, int ldi, const double* idt, const double* blocks, double* store,
                           hipStream_t s) {
+  using La = Lay<NV, W, NINE>;
   const int nchunk = (nic + W - 1) / W, nlev = njc + 2 * W - 2;
-  const size_t total = cilu_copy_floats(nic, njc, NV, W);
-  double* ops = store + cilu_ops_offset(nic, njc, NV, W);
+  const size_t total = cilu_ops_doubles(nic, njc, NV, W), nl = La::links(nchunk, njc);
+  double* links = store + (La::floats(nchunk, njc) + 1) / 2;
+  double* ops = links + nl;
+  hipLaunchKernelGGL((cilu_zero_kernel<NV, W, NINE>), dim3(La::nrec(njc), nchunk * La::NG), dim3(256), 0, s, nic, njc,
+                     nchunk, reinterpret_cast<float*>(store));
   const size_t nblk = std::min<size_t>((total + 255) / 256, (size_t)1 << 20);
   hipLaunchKernelGGL((cilu_gather_kernel<NV, W>), dim3((unsigned)nblk), dim3(256), 0, s, nic, njc, ldi, nlev, idt,
                      blocks, ops, total);
   hipLaunchKernelGGL((cilu_factor_kernel<NV, W, NINE>), dim3(nchunk), dim3(W * NV * NV), 0, s, nic, njc, nlev, ops,
-                     reinterpret_cast<float*>(store), total);
+                     reinterpret_cast<float*>(store));
+  if (nl)
+    hipLaunchKernelGGL(cilu_empty_kernel, dim3((unsigned)std::min<size_t>((nl + 255) / 256, 1024)), dim3(256), 0, s,
+                       reinterpret_cast<unsigned long long*>(links), nl);
 }
-
-// Launch tag of an apply: helpers only trust progress words that carry it.
-static std::atomic<unsigned> g_apply_epoch{0};
 
 template <int NV, int W, bool NINE>
 static void cilu_apply_t(int nic, int njc, int ldi, double* store, const double* b, double* z, bool tr,
                          hipStream_t s) {
-  const int nchunk = (nic + W - 1) / W, nlev = njc + 2 * W - 2, npad = (nchunk + 7) & ~7;
-  const size_t tcopy = cilu_copy_floats(nic, njc, NV, W);
+  using La = Lay<NV, W, NINE>;
+  const int nchunk = (nic + W - 1) / W;
   const float* rec = reinterpret_cast<const float*>(store);
-  // the progress words follow the two factor copies; the apply writes them
-  unsigned* prog = reinterpret_cast<unsigned*>(reinterpret_cast<float*>(store) + 2 * tcopy);
-  // the progress word holds tag << 16 | steps; without room for 2 nlev steps, no helpers
-  const bool helpers = 2 * nlev < (1 << 16);
-  unsigned epoch = (g_apply_epoch.fetch_add(1) % 0xffffu) + 1;  // never 0, the value of fresh memory
-  const dim3 grid(helpers ? npad * (1 + NHELP) : nchunk);
-  if (!helpers) prog = nullptr, epoch = 0;
+  unsigned long long* links = reinterpret_cast<unsigned long long*>(store + (La::floats(nchunk, njc) + 1) / 2);
+  const dim3 grid((nchunk + 7) / 8 * 8 * La::NG), block(La::NG > 1 ? 256 : 192);
   if (tr)
-    hipLaunchKernelGGL((cilu_apply_kernel<NV, W, NINE, true>), grid, dim3(NV * W), 0, s, nic, njc, ldi, nlev, rec,
-                       tcopy, b, z, prog, epoch);
+    hipLaunchKernelGGL((cilu_apply_kernel<NV, W, NINE, true>), grid, block, 0, s, nic, njc, ldi, nchunk, rec, links, b,
+                       z);
   else
-    hipLaunchKernelGGL((cilu_apply_kernel<NV, W, NINE, false>), grid, dim3(NV * W), 0, s, nic, njc, ldi, nlev, rec,
-                       tcopy, b, z, prog, epoch);
+    hipLaunchKernelGGL((cilu_apply_kernel<NV, W, NINE, false>), grid, block, 0, s, nic, njc, ldi, nchunk, rec, links,
+                       b, z);
 }
 
 bool cilu_width_ok(int w) { return w == 8 || w == 16 || w == 24 || w == 32; }
@@ -563,6 +789,21 @@ static void cilu_apply_n(int nic, int njc, int ldi, int nv, int w, double* store
     else if (w == 24) cilu_apply_t<4, 24, NINE>(nic, njc, ldi, store, b, z, transpose, s);
     else cilu_apply_t<4, 32, NINE>(nic, njc, ldi, store, b, z, transpose, s);
   }
+}
+
+template <bool NINE>
+static size_t cilu_size_n(int nic, int njc, int nv, int w) {
+  if (nv == 5)
+    return w == 8 ? cilu_size_t<5, 8, NINE>(nic, njc)
+                  : w == 16 ? cilu_size_t<5, 16, NINE>(nic, njc)
+                            : w == 24 ? cilu_size_t<5, 24, NINE>(nic, njc) : cilu_size_t<5, 32, NINE>(nic, njc);
+  return w == 8 ? cilu_size_t<4, 8, NINE>(nic, njc)
+                : w == 16 ? cilu_size_t<4, 16, NINE>(nic, njc)
+                          : w == 24 ? cilu_size_t<4, 24, NINE>(nic, njc) : cilu_size_t<4, 32, NINE>(nic, njc);
+}
+
+size_t cilu_size(int nic, int njc, int nv, int w, bool nine) {
+  return nine ? cilu_size_n<true>(nic, njc, nv, w) : cilu_size_n<false>(nic, njc, nv, w);
 }
 
 hipError_t cilu_factor(int nic, int njc, int ldi, int nv, int w, bool nine, const double* idt, const double* blocks,

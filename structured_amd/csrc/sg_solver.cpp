@@ -225,7 +225,7 @@ int factor_preconditioner(sg_ctx* ctx, const double* idt_pc) {
     return SG_OK;
   }
   if (S->precond == 6 || S->precond == 7) {
-    const size_t need = cilu_size(nic, njc, nv, S->pc_width);
+    const size_t need = cilu_size(nic, njc, nv, S->pc_width, S->precond == 7);
     if (S->cilu.n < need && S->cilu.alloc(need) != hipSuccess) return sg_fail(ctx, SG_ERR_HIP, "allocation failed");
     SG_TRY(cilu_factor(nic, njc, ldi, nv, S->pc_width, S->precond == 7, pc_idt, blk, S->cilu.p, ctx->stream),
            "cilu factor");
