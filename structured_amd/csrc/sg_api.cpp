@@ -490,7 +490,7 @@ int sg_set_closure(sg_ctx* ctx, int kind, const double* coef, const float* mlp_p
     SG_TRY(hipMemcpyAsync(ctx->clo_params.p, mlp_params, MLP_NPARAM * sizeof(float), hipMemcpyHostToDevice,
                           ctx->stream), "H2D");
     SG_TRY(mlp_w2_to_bf16(reinterpret_cast<const float*>(ctx->clo_params.p),
-                          reinterpret_cast<__bf16*>(ctx->clo_w2.p), ctx->stream), "w2 bf16");
+                          reinterpret_cast<__bf16*>(ctx->clo_w2.p), nullptr, ctx->stream), "w2 bf16");
     SG_TRY(hipStreamSynchronize(ctx->stream), "closure");
     c.params = reinterpret_cast<const float*>(ctx->clo_params.p);
     c.w2 = ctx->clo_w2.p;

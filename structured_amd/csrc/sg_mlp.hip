@@ -1,256 +1,381 @@
 // Learned closure: a 5 -> 64 -> 64 -> 1 tanh MLP mapping local flow features
 // to the SA production multiplier beta = 1 + MLP(features).
 //
-// The 64 x 64 layer runs on the matrix cores: BF16 operands, FP32
-// accumulation (v_mfma_f32_16x16x32_bf16; fragment layout, lane l of the
-// wave: A[l%16][8(l/16)+t], B[8(l/16)+t][l%16], C[4(l/16)+i][l%16]).  The
-// 5 -> 64 and 64 -> 1 layers, activations, loss, Adam and every reduction
-// are FP32; reductions use fixed orders, so training is bitwise
-// reproducible.  Parameters (FP32 master copy, 4609 floats):
+// One kernel runs the forward pass and, for training, the backward pass and
+// the parameter gradients; everything between the features and the per-block
+// gradient sums stays in registers and LDS.  The three 64 x 64 products run on
+// the matrix cores: BF16 operands, FP32 accumulation
+// (v_mfma_f32_16x16x32_bf16; fragment layout, lane l of the wave:
+// A[l%16][8(l/16)+t], B[8(l/16)+t][l%16], C[4(l/16)+i][l%16]).  The 5 -> 64 and
+// 64 -> 1 layers, activations, loss, Adam and every reduction are FP32;
+// reductions use fixed orders, so training is bitwise reproducible.
+// Parameters (FP32 master copy, 4609 floats):
 //   W1[64][5] | b1[64] | W2[64][64] | b2[64] | W3[64] | b3
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "sg_closure.hpp"
 #include "sg_mlp.hpp"
 
 namespace sg {
 
-// C[m][n] = sum_k A[m][k] B[k][n] (+ epilogue).  A, B bf16 with element
-// strides; C f32.  Block = 4 waves computing a 64 x 64 tile (each wave 32 x
-// 32 = 2 x 2 MFMA tiles); blockIdx.z splits K (partials at C + z * splitc).
-// epi 0: C = acc; 1: C = tanh(acc + bias[n]) and Cb (bf16) = C.
-__global__ __launch_bounds__(256) void gemm_bf16_kernel(int M, int N, int K, int kchunk, const __bf16* A, long sam,
-                                                        long sak, const __bf16* B, long sbk, long sbn, float* C,
-                                                        long scm, long scn, long splitc, int epi, const float* bias,
-                                                        __bf16* Cb) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int m_base = blockIdx.y * 64 + (w >> 1) * 32, n_base = blockIdx.x * 64 + (w & 1) * 32;
-  const int k_begin = blockIdx.z * kchunk, k_end = min(K, k_begin + kchunk);
-  f32x4 acc[2][2];
-  for (int a = 0; a < 2; ++a)
-    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int r16 = lane & 15, kq = 8 * (lane >> 4);
-  for (int k0 = k_begin; k0 < k_end; k0 += 32) {
-    bf16x8 af[2], bf[2];
-    for (int a = 0; a < 2; ++a) {
-      const int m = m_base + 16 * a + r16;
-      for (int t = 0; t < 8; ++t) {
-        const int k = k0 + kq + t;
-        af[a][t] = (m < M && k < k_end) ? A[m * sam + k * sak] : (__bf16)0.0f;
-      }
-    }
-    for (int b = 0; b < 2; ++b) {
-      const int n = n_base + 16 * b + r16;
-      for (int t = 0; t < 8; ++t) {
-        const int k = k0 + kq + t;
-        bf[b][t] = (n < N && k < k_end) ? B[k * sbk + n * sbn] : (__bf16)0.0f;
-      }
-    }
-    for (int a = 0; a < 2; ++a)
-      for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bf[b], acc[a][b], 0, 0, 0);
+// ---- the network on 32 rows per wave ----------------------------------------
+//
+// A wave takes 32 rows as two sub-tiles of 16, row r of a sub-tile on the four
+// lanes l with l % 16 = r.  Those hold the hidden units u = 16 a + 4 q + i
+// (q = l / 16; a, i = 0..3), 16 each: the layout in which the matrix cores
+// return a product whose columns are rows of the batch (C[unit][row]).  With
+// the summation index of the next product enumerated as
+//   slot (s, q, t) -> unit 32 s + 16 (t / 4) + 4 q + t % 4
+// the same registers are its B operand, so layer 1 is computed in place, layer
+// 2 follows from it, and the backward product dH2 W2 from layer 2, without any
+// exchange between lanes; only W2 is read in that order (rows of W2b forward,
+// of its transpose backward).  The weight gradient dH2^T H1 sums over rows:
+// its operands go through LDS once, the two sub-tiles of a lane's row
+// together (4 bytes), which enumerates the rows as 2 (l % 16) + sub-tile for
+// both operands alike.  (Four sub-tiles at a time spilled 105 registers: a lane
+// keeps 192 gradient sums.)
+//
+// What bounds it: a launch of 65,536 rows gives every SIMD one wave with two
+// tiles of 32 rows, 5 us each (its tanh, 4 k cycles, and the latencies of one
+// wave alone), after 14 us for the weights, the gathers and the block's
+// gradient sums.  Against eleven kernels that passed every activation through
+// memory, a training step of 65,536 rows (forward, backward, Adam) takes 24 +
+// 5 us instead of 565.
+constexpr int SUB = 2, MLP_ROWS = 16 * SUB, MLP_WAVES = 4;  // sub-tiles and rows per wave, waves per block
+constexpr int kTld = 40;                     // LDS row stride (BF16) of the row-summed operands
+constexpr int kRld = 68;                     // LDS row stride (float) of the lane-summed values
+
+struct MlpLds {
+  float w1[MLP_H][8];  // W1 row, b1
+  float b2[MLP_H], w3[MLP_H];
+  union {
+    __bf16 t[MLP_WAVES][2][MLP_H][kTld];  // dH2 and H1, [unit][row]
+    float red[MLP_WAVES][MLP_H][kRld];    // gradient sums
+  };
+  float tail[MLP_WAVES][2];  // sums of e^2 and dy
+};
+
+template <bool BWD>
+__global__ __launch_bounds__(64 * MLP_WAVES) __attribute__((amdgpu_waves_per_eu(1, 1))) void mlp_kernel(
+    int n, const float* __restrict__ X, const int* __restrict__ idx, const float* __restrict__ T,
+    const float* __restrict__ P, const __bf16* __restrict__ W2b, const __bf16* __restrict__ W2t, float inv_ntot,
+    float* __restrict__ Y, float* __restrict__ part) {
+  __shared__ MlpLds sh;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, q = lane >> 4, r16 = lane & 15;
+  for (int e = tid; e < MLP_H * 8; e += 64 * MLP_WAVES) {
+    const int u = e >> 3, c = e & 7;
+    sh.w1[u][c] = c < MLP_IN ? P[MLP_W1 + u * MLP_IN + c] : c == MLP_IN ? P[MLP_B1 + u] : 0.f;
   }
-  float* Cz = C + (long)blockIdx.z * splitc;
-  for (int a = 0; a < 2; ++a)
-    for (int b = 0; b < 2; ++b)
-      for (int i = 0; i < 4; ++i) {
-        const int m = m_base + 16 * a + 4 * (lane >> 4) + i, n = n_base + 16 * b + r16;
-        if (m >= M || n >= N) continue;
-        float v = acc[a][b][i];
-        if (epi == 1) {
-          v = tanh_fast(v + bias[n]);
-          Cb[m * scm + n * scn] = (__bf16)v;
+  if (tid < MLP_H) {
+    sh.b2[tid] = P[MLP_B2 + tid];
+    sh.w3[tid] = P[MLP_W3 + tid];
+  }
+  __syncthreads();
+  const float b3 = P[MLP_B3];
+  // fragment of a 64 x 64 matrix M (row-major): rows 16 a + l % 16, slots of s
+  auto frag = [&](const __bf16* M, int a, int s) {
+    const __bf16* p = M + (16 * a + r16) * MLP_H + 32 * s + 4 * q;
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    const bf16x4 lo = *reinterpret_cast<const bf16x4*>(p), hi = *reinterpret_cast<const bf16x4*>(p + 16);
+    bf16x8 f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) { f[t] = lo[t]; f[t + 4] = hi[t]; }
+    return f;
+  };
+  // gradient sums of this lane's units over its rows, and of the wave's dW2
+  float gw1[16][MLP_IN], gb1[16], gb2[16], gw3[16], se = 0.f, sdy = 0.f;
+  f32x4 gw2[4][4];
+  if (BWD) {
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+#pragma unroll
+      for (int c = 0; c < MLP_IN; ++c) gw1[u][c] = 0.f;
+      gb1[u] = gb2[u] = gw3[u] = 0.f;
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) gw2[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const int tiles = (n + MLP_ROWS - 1) / MLP_ROWS, stride = gridDim.x * MLP_WAVES;
+  for (int tile = blockIdx.x * MLP_WAVES + w; tile < tiles; tile += stride) {
+    float x[SUB][MLP_IN], tt[SUB], h1[SUB][16];
+    bool live[SUB];
+    int src[SUB];
+#pragma unroll
+    for (int m = 0; m < SUB; ++m) {
+      const int r = tile * MLP_ROWS + 16 * m + r16;
+      live[m] = r < n;
+      src[m] = live[m] ? (idx ? idx[r] : r) : 0;
+    }
+#pragma unroll
+    for (int m = 0; m < SUB; ++m) {
+#pragma unroll
+      for (int c = 0; c < MLP_IN; ++c) x[m][c] = live[m] ? X[(long)src[m] * MLP_IN + c] : 0.f;
+      if (BWD) tt[m] = live[m] ? T[src[m]] : 0.f;
+    }
+    // layer 1
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const float* w1 = sh.w1[16 * (u >> 2) + 4 * q + (u & 3)];
+      float a[SUB];
+#pragma unroll
+      for (int m = 0; m < SUB; ++m) a[m] = w1[MLP_IN];
+#pragma unroll
+      for (int c = 0; c < MLP_IN; ++c)
+#pragma unroll
+        for (int m = 0; m < SUB; ++m) a[m] = fmaf(w1[c], x[m][c], a[m]);
+#pragma unroll
+      for (int m = 0; m < SUB; ++m) h1[m][u] = tanh_fast(a[m]);
+    }
+    // layer 2, output, loss and dH2, a sub-tile at a time
+    bf16x8 hb[SUB][2], db[SUB][2];
+#pragma unroll
+    for (int m = 0; m < SUB; ++m) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int t = 0; t < 8; ++t) hb[m][s][t] = (__bf16)h1[m][8 * s + t];
+      float h2[16], y = 0.f;
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 2; ++s) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(W2b, a, s), hb[m][s], c, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int u = 16 * a + 4 * q + i;
+          h2[4 * a + i] = tanh_fast(c[i] + sh.b2[u]);
+          y = fmaf(sh.w3[u], h2[4 * a + i], y);
         }
-        Cz[m * scm + n * scn] = v;
       }
-}
-
-hipError_t gemm_bf16(int M, int N, int K, const __bf16* A, long sam, long sak, const __bf16* B, long sbk, long sbn,
-                     float* C, long scm, long scn, int splitk, long splitc, int epi, const float* bias, __bf16* Cb,
-                     hipStream_t s) {
-  const int kchunk = ((K + splitk - 1) / splitk + 31) / 32 * 32;
-  dim3 grid((N + 63) / 64, (M + 63) / 64, splitk);
-  hipLaunchKernelGGL(gemm_bf16_kernel, grid, dim3(256), 0, s, M, N, K, kchunk, A, sam, sak, B, sbk, sbn, C, scm, scn,
-                     splitc, epi, bias, Cb);
-  return hipGetLastError();
-}
-
-// ---- elementwise / reduction kernels -------------------------------------
-// layer 1: a1 = W1 x + b1, h1 = tanh(a1) (f32 and bf16), rows gathered by idx
-__global__ void mlp_layer1_kernel(int n, const float* X, const int* idx, const float* P, float* H1, __bf16* H1b) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  const int src = idx ? idx[r] : r;
-  float x[MLP_IN];
-  for (int c = 0; c < MLP_IN; ++c) x[c] = X[(long)src * MLP_IN + c];
-  const float* W1 = P + MLP_W1;
-  const float* b1 = P + MLP_B1;
-  for (int k = 0; k < MLP_H; ++k) {
-    float a = b1[k];
-    for (int c = 0; c < MLP_IN; ++c) a = fmaf(W1[k * MLP_IN + c], x[c], a);
-    const float h = tanh_fast(a);
-    H1[(long)r * MLP_H + k] = h;
-    H1b[(long)r * MLP_H + k] = (__bf16)h;
-  }
-}
-
-// layer 3, loss and the output-side backward: y = W3 h2 + b3, e = y - t,
-// dy = 2 e / ntot, dH2 = dy W3 (1 - h2^2) (f32 and bf16).  Per-block partial
-// sums of e^2 (one float per block).
-__global__ __launch_bounds__(256) void mlp_layer3_kernel(int n, const float* H2, const float* P, const float* T,
-                                                         const int* idx, float inv_ntot, float* Y, float* dY,
-                                                         float* dH2, __bf16* dH2b, float* loss_partial) {
-  __shared__ float red[256];
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  float e2 = 0.f;
-  if (r < n) {
-    const float* W3 = P + MLP_W3;
-    float y = P[MLP_B3];
-    for (int k = 0; k < MLP_H; ++k) y = fmaf(W3[k], H2[(long)r * MLP_H + k], y);
-    if (Y) Y[r] = y;
-    if (T) {
-      const float e = y - T[idx ? idx[r] : r];
-      e2 = e * e;
-      const float dy = 2.f * e * inv_ntot;
-      dY[r] = dy;
-      for (int k = 0; k < MLP_H; ++k) {
-        const float h = H2[(long)r * MLP_H + k];
-        const float d = dy * W3[k] * (1.f - h * h);
-        dH2[(long)r * MLP_H + k] = d;
-        dH2b[(long)r * MLP_H + k] = (__bf16)d;
+      y += __shfl_xor(y, 16);
+      y += __shfl_xor(y, 32);
+      y += b3;
+      if (Y && live[m] && q == 0) Y[tile * MLP_ROWS + 16 * m + r16] = y;
+      if (BWD) {
+        const float e = live[m] ? y - tt[m] : 0.f, dy = 2.f * e * inv_ntot;
+        if (q == 0) {
+          se = fmaf(e, e, se);
+          sdy += dy;
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+          const float d = dy * sh.w3[16 * (u >> 2) + 4 * q + (u & 3)] * (1.f - h2[u] * h2[u]);
+          gb2[u] += d;
+          gw3[u] = fmaf(dy, h2[u], gw3[u]);
+          db[m][u >> 3][u & 7] = (__bf16)d;
+        }
       }
     }
+    if constexpr (BWD) {
+      // dH1 = (dH2 W2) (1 - h1^2) and the sums it enters
+#pragma unroll
+      for (int m = 0; m < SUB; ++m)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+          f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int s = 0; s < 2; ++s)
+            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(W2t, a, s), db[m][s], c, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int u = 4 * a + i;
+            const float d = c[i] * (1.f - h1[m][u] * h1[m][u]);
+            gb1[u] += d;
+#pragma unroll
+            for (int k = 0; k < MLP_IN; ++k) gw1[u][k] = fmaf(d, x[m][k], gw1[u][k]);
+          }
+        }
+      // dW2[j][k] += sum over rows of dH2[row][j] H1[row][k]
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        bf16x2 d, h;
+#pragma unroll
+        for (int m = 0; m < SUB; ++m) { d[m] = db[m][u >> 3][u & 7]; h[m] = hb[m][u >> 3][u & 7]; }
+        const int row = 16 * (u >> 2) + 4 * q + (u & 3);
+        *reinterpret_cast<bf16x2*>(&sh.t[w][0][row][SUB * r16]) = d;
+        *reinterpret_cast<bf16x2*>(&sh.t[w][1][row][SUB * r16]) = h;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+      __builtin_amdgcn_wave_barrier();
+      {
+        bf16x8 fd[4], fh[4];
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+          fd[a] = *reinterpret_cast<const bf16x8*>(&sh.t[w][0][16 * a + r16][8 * q]);
+          fh[a] = *reinterpret_cast<const bf16x8*>(&sh.t[w][1][16 * a + r16][8 * q]);
+        }
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+          for (int b = 0; b < 4; ++b)
+            gw2[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fd[a], fh[b], gw2[a][b], 0, 0, 0);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+      __builtin_amdgcn_wave_barrier();
+    }
   }
-  if (!loss_partial) return;
-  red[threadIdx.x] = e2;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+  if constexpr (BWD) {
+    float* out = part + (size_t)blockIdx.x * MLP_NPART;
+    // the lanes' sums over rows: 128 values per lane, 64 at a time, each summed
+    // over the 16 lanes of its units and the waves by one thread
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      __syncthreads();
+#pragma unroll
+      for (int v = 0; v < 64; ++v) {
+        const int e = 64 * half + v;  // gw1 (80), gb1, gb2, gw3 (16 each)
+        const float g = e < 80 ? gw1[e / 5][e % 5] : e < 96 ? gb1[e - 80] : e < 112 ? gb2[e - 96] : gw3[e - 112];
+        sh.red[w][v][lane] = g;
+      }
+      __syncthreads();
+      const int v = tid & 63, g4 = tid >> 6;  // thread: value v of the units of lane group g4
+      float s = 0.f;
+#pragma unroll
+      for (int ww = 0; ww < MLP_WAVES; ++ww)
+#pragma unroll
+        for (int l = 0; l < 16; ++l) s += sh.red[ww][v][16 * g4 + l];
+      const int e = 64 * half + v;
+      auto unit = [&](int u) { return 16 * (u >> 2) + 4 * g4 + (u & 3); };
+      if (e < 80) out[MLP_W1 + unit(e / 5) * MLP_IN + e % 5] = s;
+      else if (e < 96) out[MLP_B1 + unit(e - 80)] = s;
+      else if (e < 112) out[MLP_B2 + unit(e - 96)] = s;
+      else out[MLP_W3 + unit(e - 112)] = s;
+    }
+    // the waves' dW2
     __syncthreads();
-  }
-  if (threadIdx.x == 0) loss_partial[blockIdx.x] = red[0];
-}
-
-// dH1 = dH1pre * (1 - h1^2)
-__global__ void mlp_dh1_kernel(long total, const float* dH1pre, const float* H1, float* dH1) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= total) return;
-  const float h = H1[e];
-  dH1[e] = dH1pre[e] * (1.f - h * h);
-}
-
-// Per-block column partial sums for the FP32 parameter gradients:
-//   dW1[k][c] = sum_r dH1[r][k] x[r][c], db1[k] = sum_r dH1[r][k],
-//   db2[k] = sum_r dH2[r][k], dW3[k] = sum_r dY[r] H2[r][k], db3 = sum_r dY[r].
-// One thread per hidden unit k (64 threads), rows [blockIdx.x*rows, +rows).
-__global__ void mlp_colsum_kernel(int n, int rows, const float* X, const int* idx, const float* dH1, const float* dH2,
-                                  const float* H2, const float* dY, float* part) {
-  const int k = threadIdx.x;
-  const int r0 = blockIdx.x * rows, r1 = min(n, r0 + rows);
-  float w1[MLP_IN] = {0, 0, 0, 0, 0};
-  float b1 = 0.f, b2 = 0.f, w3 = 0.f, b3 = 0.f;
-  for (int r = r0; r < r1; ++r) {
-    const int src = idx ? idx[r] : r;
-    const float d1 = dH1[(long)r * MLP_H + k];
-    for (int c = 0; c < MLP_IN; ++c) w1[c] = fmaf(d1, X[(long)src * MLP_IN + c], w1[c]);
-    b1 += d1;
-    b2 += dH2[(long)r * MLP_H + k];
-    w3 = fmaf(dY[r], H2[(long)r * MLP_H + k], w3);
-    if (k == 0) b3 += dY[r];
-  }
-  float* p = part + (long)blockIdx.x * MLP_NPARAM;
-  for (int c = 0; c < MLP_IN; ++c) p[MLP_W1 + k * MLP_IN + c] = w1[c];
-  p[MLP_B1 + k] = b1;
-  p[MLP_B2 + k] = b2;
-  p[MLP_W3 + k] = w3;
-  if (k == 0) p[MLP_B3] = b3;
-}
-
-// grad[p] = sum over partial blocks (fixed order); W2 part from the split-K
-// GEMM partials.
-__global__ void mlp_grad_reduce_kernel(int nblk, const float* part, int nsplit, const float* w2part, float* grad) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= MLP_NPARAM) return;
-  float s = 0.f;
-  if (p >= MLP_W2 && p < MLP_B2) {
-    for (int z = 0; z < nsplit; ++z) s += w2part[(long)z * MLP_H * MLP_H + (p - MLP_W2)];
-  } else {
-    for (int b = 0; b < nblk; ++b) s += part[(long)b * MLP_NPARAM + p];
-  }
-  grad[p] = s;
-}
-
-__global__ void mlp_sum_kernel(int n, const float* v, float scale, float* out) {
-  __shared__ float red[256];
-  float s = 0.f;
-  for (int i = threadIdx.x; i < n; i += 256) s += v[i];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sh.red[w][16 * a + 4 * q + i][16 * b + r16] = gw2[a][b][i];
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) {
+      se += __shfl_xor(se, o);
+      sdy += __shfl_xor(sdy, o);
+    }
+    if (lane == 0) {
+      sh.tail[w][0] = sdy;
+      sh.tail[w][1] = se;
+    }
     __syncthreads();
+    for (int e = tid; e < MLP_H * MLP_H; e += 64 * MLP_WAVES) {
+      float s = 0.f;
+#pragma unroll
+      for (int ww = 0; ww < MLP_WAVES; ++ww) s += sh.red[ww][e >> 6][e & 63];
+      out[MLP_W2 + e] = s;
+    }
+    if (tid < 2) {
+      float s = 0.f;
+#pragma unroll
+      for (int ww = 0; ww < MLP_WAVES; ++ww) s += sh.tail[ww][tid];
+      out[MLP_B3 + tid] = s;  // db3, then the sum of e^2
+    }
   }
-  if (threadIdx.x == 0) *out = red[0] * scale;
 }
 
-// Adam (Kingma & Ba 2015) on the FP32 master parameters, then the BF16 copy of
-// W2 used by the matrix cores.
-__global__ void mlp_adam_kernel(float* P, float* m, float* v, const float* g, float lr, float b1, float b2, float eps,
-                                float c1, float c2, __bf16* W2b) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= MLP_NPARAM) return;
-  const float gp = g[p];
-  const float mp = b1 * m[p] + (1.f - b1) * gp;
-  const float vp = b2 * v[p] + (1.f - b2) * gp * gp;
-  m[p] = mp;
-  v[p] = vp;
-  const float w = P[p] - lr * (mp / c1) / (sqrtf(vp / c2) + eps);
-  P[p] = w;
-  if (p >= MLP_W2 && p < MLP_B2) W2b[p - MLP_W2] = (__bf16)w;
+// grad[p] = sum over the blocks' partials (fixed order: slices of blocks, then
+// the slices), the loss from the entry after the parameters; with ADAM the
+// step (Kingma & Ba 2015) on the FP32 master parameters and the BF16 copies of
+// W2 that the matrix cores read.
+constexpr int RED_P = 32, RED_S = 16;  // parameters per block, slices
+template <bool ADAM>
+__global__ __launch_bounds__(RED_P* RED_S) void mlp_reduce_kernel(int nblk, const float* __restrict__ part,
+                                                                  float* __restrict__ grad, float loss_scale,
+                                                                  float* __restrict__ loss, float* P, float* m,
+                                                                  float* v, float lr, float b1, float b2, float eps,
+                                                                  float c1, float c2, __bf16* W2b, __bf16* W2t) {
+  __shared__ float red[RED_S][RED_P];
+  const int p = blockIdx.x * RED_P + threadIdx.x % RED_P, s = threadIdx.x / RED_P;
+  float a = 0.f;
+  if (p < MLP_NPART) {
+    const int per = (nblk + RED_S - 1) / RED_S, e = min(nblk, (s + 1) * per);
+    int b = s * per;
+    for (; b + 4 <= e; b += 4) {
+      float u[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) u[k] = part[(size_t)(b + k) * MLP_NPART + p];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) a += u[k];
+    }
+    for (; b < e; ++b) a += part[(size_t)b * MLP_NPART + p];
+  }
+  red[s][threadIdx.x % RED_P] = a;
+  __syncthreads();
+  if (s != 0 || p >= MLP_NPART) return;
+  float g = 0.f;
+#pragma unroll
+  for (int k = 0; k < RED_S; ++k) g += red[k][threadIdx.x];
+  if (p == MLP_NPARAM) {
+    *loss = g * loss_scale;
+    return;
+  }
+  if (grad) grad[p] = g;
+  if (ADAM) {
+    const float mp = b1 * m[p] + (1.f - b1) * g;
+    const float vp = b2 * v[p] + (1.f - b2) * g * g;
+    m[p] = mp;
+    v[p] = vp;
+    const float w = P[p] - lr * (mp / c1) / (sqrtf(vp / c2) + eps);
+    P[p] = w;
+    if (p >= MLP_W2 && p < MLP_B2) {
+      const int e = p - MLP_W2;
+      W2b[e] = (__bf16)w;
+      W2t[(e & 63) * MLP_H + (e >> 6)] = (__bf16)w;
+    }
+  }
 }
 
-__global__ void mlp_w2_to_bf16_kernel(const float* P, __bf16* W2b) {
+// BF16 copy of W2, and (if W2t) of its transpose
+__global__ void mlp_w2_to_bf16_kernel(const float* P, __bf16* W2b, __bf16* W2t) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < MLP_H * MLP_H) W2b[e] = (__bf16)P[MLP_W2 + e];
+  if (e >= MLP_H * MLP_H) return;
+  const __bf16 w = (__bf16)P[MLP_W2 + e];
+  W2b[e] = w;
+  if (W2t) W2t[(e & 63) * MLP_H + (e >> 6)] = w;
 }
 
 // ---- host-side drivers ------------------------------------------------------
-hipError_t mlp_w2_to_bf16(const float* P, __bf16* W2b, hipStream_t s) {
-  hipLaunchKernelGGL(mlp_w2_to_bf16_kernel, dim3((MLP_H * MLP_H + 255) / 256), dim3(256), 0, s, P, W2b);
+hipError_t mlp_w2_to_bf16(const float* P, __bf16* W2b, __bf16* W2t, hipStream_t s) {
+  hipLaunchKernelGGL(mlp_w2_to_bf16_kernel, dim3((MLP_H * MLP_H + 255) / 256), dim3(256), 0, s, P, W2b, W2t);
   return hipGetLastError();
 }
 
-// Forward (and, with T, the loss and the full gradient) on n rows.
-hipError_t mlp_forward_backward(const MlpWork& w, int n, const float* X, const int* idx, const float* T, int ntot,
-                                float* Y, float* grad, float* loss, hipStream_t s) {
-  const int nb = (n + 255) / 256;
-  hipLaunchKernelGGL(mlp_layer1_kernel, dim3(nb), dim3(256), 0, s, n, X, idx, w.P, w.H1, w.H1b);
-  // H2 = tanh(H1b W2b^T + b2): A = H1b [n][64], B[k][j] = W2b[j][k]
-  gemm_bf16(n, MLP_H, MLP_H, w.H1b, MLP_H, 1, w.W2b, 1, MLP_H, w.H2, MLP_H, 1, 1, 0, 1, w.P + MLP_B2, w.H2b, s);
-  hipLaunchKernelGGL(mlp_layer3_kernel, dim3(nb), dim3(256), 0, s, n, w.H2, w.P, T, idx, 1.0f / (float)ntot, Y, w.dY,
-                     w.dH2, w.dH2b, T ? w.loss_part : nullptr);
-  if (!T) return hipGetLastError();
-  hipLaunchKernelGGL(mlp_sum_kernel, dim3(1), dim3(256), 0, s, nb, w.loss_part, 1.0f / (float)n, loss);
-  // dW2[j][k] = sum_r dH2[r][j] H1[r][k]  (split-K over rows)
-  const int nsplit = w.nsplit;
-  gemm_bf16(MLP_H, MLP_H, n, w.dH2b, 1, MLP_H, w.H1b, MLP_H, 1, w.w2part, MLP_H, 1, nsplit, (long)MLP_H * MLP_H, 0,
-            nullptr, nullptr, s);
-  // dH1pre[r][k] = sum_j dH2[r][j] W2[j][k]
-  gemm_bf16(n, MLP_H, MLP_H, w.dH2b, MLP_H, 1, w.W2b, MLP_H, 1, w.dH1, MLP_H, 1, 1, 0, 0, nullptr, nullptr, s);
-  const long tot = (long)n * MLP_H;
-  hipLaunchKernelGGL(mlp_dh1_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, tot, w.dH1, w.H1, w.dH1);
-  const int rows = 512, ncb = (n + rows - 1) / rows;
-  hipLaunchKernelGGL(mlp_colsum_kernel, dim3(ncb), dim3(MLP_H), 0, s, n, rows, X, idx, w.dH1, w.dH2, w.H2, w.dY,
-                     w.colpart);
-  hipLaunchKernelGGL(mlp_grad_reduce_kernel, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, s, ncb, w.colpart, nsplit,
-                     w.w2part, grad);
+// blocks of a pass over n rows: one tile per wave while that does not exceed
+// one block per CU, then the waves take several (each block's sums cost 18 KB
+// of partials, which the reduction reads back)
+static int mlp_blocks(int n) {
+  return std::min((n + MLP_ROWS * MLP_WAVES - 1) / (MLP_ROWS * MLP_WAVES), MLP_MAX_BLOCKS);
+}
+
+hipError_t mlp_forward(const MlpWork& w, int n, const float* X, float* Y, hipStream_t s) {
+  hipLaunchKernelGGL(mlp_kernel<false>, dim3(mlp_blocks(n)), dim3(64 * MLP_WAVES), 0, s, n, X, nullptr, nullptr, w.P,
+                     w.W2b, w.W2t, 0.f, Y, nullptr);
   return hipGetLastError();
 }
 
-hipError_t mlp_adam(const MlpWork& w, const float* grad, float lr, int step, hipStream_t s) {
+// Mean squared error over n rows (gathered by idx if given) and its gradient;
+// with step > 0 the Adam step of that number as well.
+hipError_t mlp_train_step(const MlpWork& w, int n, const float* X, const int* idx, const float* T, float* grad,
+                          float* loss, int step, float lr, hipStream_t s) {
+  const int nb = mlp_blocks(n);
+  hipLaunchKernelGGL(mlp_kernel<true>, dim3(nb), dim3(64 * MLP_WAVES), 0, s, n, X, idx, T, w.P, w.W2b, w.W2t,
+                     1.0f / (float)n, nullptr, w.part);
+  const dim3 grid((MLP_NPART + RED_P - 1) / RED_P), block(RED_P * RED_S);
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-  const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
-  hipLaunchKernelGGL(mlp_adam_kernel, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, s, w.P, w.m, w.v, grad, lr, b1,
-                     b2, eps, c1, c2, w.W2b);
+  if (step > 0) {
+    const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
+    hipLaunchKernelGGL(mlp_reduce_kernel<true>, grid, block, 0, s, nb, w.part, grad, 1.0f / (float)n, loss, w.P, w.m,
+                       w.v, lr, b1, b2, eps, c1, c2, w.W2b, w.W2t);
+  } else {
+    hipLaunchKernelGGL(mlp_reduce_kernel<false>, grid, block, 0, s, nb, w.part, grad, 1.0f / (float)n, loss, w.P, w.m,
+                       w.v, lr, b1, b2, eps, 1.f, 1.f, w.W2b, w.W2t);
+  }
   return hipGetLastError();
 }
 

@@ -85,16 +85,11 @@ int sg_mlp_create(sg_mlp** out, int max_rows, unsigned long long seed) {
   };
   if (hipStreamCreate(&net->stream) != hipSuccess) return fail(SG_ERR_HIP);
   MlpWork& w = net->w;
-  const size_t cap = (size_t)max_rows, ch = cap * MLP_H;
+  const size_t cap = (size_t)max_rows;
   w.cap = max_rows;
-  w.nsplit = (int)std::min<size_t>(64, std::max<size_t>(1, cap / 2048));
-  const int ncb = (max_rows + 511) / 512;
   if (dalloc(net, w.P, MLP_NPARAM) || dalloc(net, w.m, MLP_NPARAM) || dalloc(net, w.v, MLP_NPARAM) ||
-      dalloc(net, w.grad, MLP_NPARAM) || dalloc(net, w.W2b, MLP_H * MLP_H) || dalloc(net, w.H1, ch) ||
-      dalloc(net, w.H2, ch) || dalloc(net, w.dH1, ch) || dalloc(net, w.dH2, ch) || dalloc(net, w.dY, cap) ||
-      dalloc(net, w.H1b, ch) || dalloc(net, w.H2b, ch) || dalloc(net, w.dH2b, ch) ||
-      dalloc(net, w.loss_part, (cap + 255) / 256) || dalloc(net, w.colpart, (size_t)ncb * MLP_NPARAM) ||
-      dalloc(net, w.w2part, (size_t)w.nsplit * MLP_H * MLP_H) || dalloc(net, w.loss, 1) || dalloc(net, net->Y, cap) ||
+      dalloc(net, w.grad, MLP_NPARAM) || dalloc(net, w.W2b, MLP_H * MLP_H) || dalloc(net, w.W2t, MLP_H * MLP_H) ||
+      dalloc(net, w.part, (size_t)MLP_MAX_BLOCKS * MLP_NPART) || dalloc(net, w.loss, 1) || dalloc(net, net->Y, cap) ||
       dalloc(net, net->Xd, cap * MLP_IN) || dalloc(net, net->Td, cap))
     return fail(SG_ERR_HIP);
   std::vector<float> p(MLP_NPARAM);
@@ -122,7 +117,7 @@ int sg_mlp_set_params(sg_mlp* net, const float* params) {
   MLP_TRY(hipMemcpyAsync(w.P, params, MLP_NPARAM * sizeof(float), hipMemcpyHostToDevice, net->stream), "H2D");
   MLP_TRY(hipMemsetAsync(w.m, 0, MLP_NPARAM * sizeof(float), net->stream), "memset");
   MLP_TRY(hipMemsetAsync(w.v, 0, MLP_NPARAM * sizeof(float), net->stream), "memset");
-  MLP_TRY(mlp_w2_to_bf16(w.P, w.W2b, net->stream), "w2 bf16");
+  MLP_TRY(mlp_w2_to_bf16(w.P, w.W2b, w.W2t, net->stream), "w2 bf16");
   MLP_TRY(hipStreamSynchronize(net->stream), "set params");
   net->step = 0;
   return SG_OK;
@@ -142,8 +137,7 @@ int sg_mlp_forward(sg_mlp* net, int n, const float* x, float* y) {
     const int m = std::min(cap, n - r0);
     MLP_TRY(hipMemcpyAsync(net->Xd, x + (size_t)r0 * MLP_IN, (size_t)m * MLP_IN * sizeof(float),
                            hipMemcpyHostToDevice, net->stream), "H2D");
-    MLP_TRY(mlp_forward_backward(net->w, m, net->Xd, nullptr, nullptr, m, net->Y, nullptr, nullptr, net->stream),
-            "forward");
+    MLP_TRY(mlp_forward(net->w, m, net->Xd, net->Y, net->stream), "forward");
     MLP_TRY(hipMemcpyAsync(y + r0, net->Y, (size_t)m * sizeof(float), hipMemcpyDeviceToHost, net->stream), "D2H");
   }
   MLP_TRY(hipStreamSynchronize(net->stream), "forward");
@@ -155,8 +149,8 @@ int sg_mlp_loss_grad(sg_mlp* net, int n, const float* x, const float* t, float* 
   if (n > net->w.cap) return mlp_fail(net, SG_ERR_ARG, "more rows than the network was created for");
   MLP_TRY(hipMemcpyAsync(net->Xd, x, (size_t)n * MLP_IN * sizeof(float), hipMemcpyHostToDevice, net->stream), "H2D");
   MLP_TRY(hipMemcpyAsync(net->Td, t, (size_t)n * sizeof(float), hipMemcpyHostToDevice, net->stream), "H2D");
-  MLP_TRY(mlp_forward_backward(net->w, n, net->Xd, nullptr, net->Td, n, nullptr, net->w.grad, net->w.loss,
-                               net->stream), "loss/grad");
+  MLP_TRY(mlp_train_step(net->w, n, net->Xd, nullptr, net->Td, net->w.grad, net->w.loss, 0, 0.f, net->stream),
+          "loss/grad");
   float l = 0.f;
   MLP_TRY(hipMemcpyAsync(&l, net->w.loss, sizeof(float), hipMemcpyDeviceToHost, net->stream), "D2H");
   if (grad)
@@ -205,9 +199,9 @@ int sg_mlp_train(sg_mlp* net, int n, const float* x, const float* t, int epochs,
       MLP_TRY(hipMemcpyAsync(idx, perm.data(), (size_t)n * sizeof(int), hipMemcpyHostToDevice, net->stream), "H2D");
       MLP_TRY(hipStreamSynchronize(net->stream), "epoch");
       for (int b = 0; b < nb; ++b) {
-        MLP_TRY(mlp_forward_backward(net->w, bs, X, idx + (size_t)b * bs, T, bs, nullptr, net->w.grad,
-                                     L + (size_t)e * nb + b, net->stream), "forward/backward");
-        MLP_TRY(mlp_adam(net->w, net->w.grad, lr, ++net->step, net->stream), "adam");
+        ++net->step;
+        MLP_TRY(mlp_train_step(net->w, bs, X, idx + (size_t)b * bs, T, net->w.grad, L + (size_t)e * nb + b, net->step,
+                               lr, net->stream), "training step");
       }
     }
     std::vector<float> lh((size_t)std::max(1, epochs) * nb);
