@@ -33,6 +33,8 @@ struct MlpWork {
 
 hipError_t mlp_w2_to_bf16(const float* P, __bf16* W2b, __bf16* W2t, hipStream_t s);
 hipError_t mlp_forward(const MlpWork& w, int n, const float* X, float* Y, hipStream_t s);
+hipError_t mlp_shuffle_init(int n, int* work, hipStream_t s);
+hipError_t mlp_shuffle(int n, unsigned long long seed, int epoch, int* work, int* perm, hipStream_t s);
 hipError_t mlp_train_step(const MlpWork& w, int n, const float* X, const int* idx, const float* T, float* grad,
                           float* loss, int step, float lr, hipStream_t s);
 

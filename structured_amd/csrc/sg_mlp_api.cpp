@@ -22,6 +22,8 @@ struct sg_mlp {
   float* Y = nullptr;           // forward output staging [cap]
   float* Xd = nullptr;          // staged inputs [cap][5] / targets [cap]
   float* Td = nullptr;
+  float* set = nullptr;         // sg_mlp_train: samples, losses, permutation
+  size_t set_words = 0;
 };
 
 namespace {
@@ -104,6 +106,7 @@ void sg_mlp_destroy(sg_mlp* net) {
   if (!net) return;
   if (net->stream) (void)hipStreamSynchronize(net->stream);
   for (void* p : net->allocs) (void)hipFree(p);
+  if (net->set) (void)hipFree(net->set);
   if (net->stream) (void)hipStreamDestroy(net->stream);
   delete net;
 }
@@ -166,58 +169,45 @@ int sg_mlp_train(sg_mlp* net, int n, const float* x, const float* t, int epochs,
   const int bs = std::min(batch, n);
   if (bs > net->w.cap) return mlp_fail(net, SG_ERR_ARG, "minibatch larger than the network was created for");
   const int nb = n / bs;
-  float *X = nullptr, *T = nullptr, *L = nullptr;
-  int* idx = nullptr;
-  std::vector<void*> tmp;
-  auto cleanup = [&]() {
-    for (void* p : tmp) (void)hipFree(p);
-  };
-  auto alloc = [&](auto*& p, size_t count) {
-    void* v = nullptr;
-    hipError_t e = hipMalloc(&v, std::max<size_t>(count, 1) * sizeof(*p));
-    if (e == hipSuccess) {
-      tmp.push_back(v);
-      p = static_cast<std::remove_reference_t<decltype(p)>>(v);
+  // the training set stays allocated with the network, at its largest so far
+  const size_t rows = (size_t)n, need = rows * (MLP_IN + 1 + 1 + 5) + (size_t)std::max(1, epochs) * nb;
+  if (need > net->set_words) {
+    if (net->set) {
+      MLP_TRY(hipStreamSynchronize(net->stream), "training set");
+      (void)hipFree(net->set);
+      net->set = nullptr;
+      net->set_words = 0;
     }
-    return e;
-  };
-  if (alloc(X, (size_t)n * MLP_IN) || alloc(T, (size_t)n) || alloc(idx, (size_t)n) ||
-      alloc(L, (size_t)std::max(1, epochs) * nb)) {
-    cleanup();
-    return mlp_fail(net, SG_ERR_HIP, "hipMalloc of the training set failed");
+    if (hipMalloc((void**)&net->set, need * sizeof(float)) != hipSuccess) {
+      net->set = nullptr;
+      return mlp_fail(net, SG_ERR_HIP, "hipMalloc of the training set failed");
+    }
+    net->set_words = need;
   }
-  int rc = SG_OK;
-  auto run = [&]() -> int {
-    MLP_TRY(hipMemcpyAsync(X, x, (size_t)n * MLP_IN * sizeof(float), hipMemcpyHostToDevice, net->stream), "H2D");
-    MLP_TRY(hipMemcpyAsync(T, t, (size_t)n * sizeof(float), hipMemcpyHostToDevice, net->stream), "H2D");
-    std::vector<int> perm(n);
-    SplitMix r{seed};
-    for (int e = 0; e < epochs; ++e) {
-      for (int k = 0; k < n; ++k) perm[k] = k;
-      for (int k = n - 1; k > 0; --k) std::swap(perm[k], perm[(int)(r.next() % (unsigned long long)(k + 1))]);
-      // the previous epoch's kernels read idx: order the upload after them
-      MLP_TRY(hipMemcpyAsync(idx, perm.data(), (size_t)n * sizeof(int), hipMemcpyHostToDevice, net->stream), "H2D");
-      MLP_TRY(hipStreamSynchronize(net->stream), "epoch");
-      for (int b = 0; b < nb; ++b) {
-        ++net->step;
-        MLP_TRY(mlp_train_step(net->w, bs, X, idx + (size_t)b * bs, T, net->w.grad, L + (size_t)e * nb + b, net->step,
-                               lr, net->stream), "training step");
-      }
+  float *X = net->set, *T = X + rows * MLP_IN, *L = T + rows;
+  int *perm = reinterpret_cast<int*>(L + (size_t)std::max(1, epochs) * nb), *work = perm + rows;
+  MLP_TRY(hipMemcpyAsync(X, x, rows * MLP_IN * sizeof(float), hipMemcpyHostToDevice, net->stream), "H2D");
+  MLP_TRY(hipMemcpyAsync(T, t, rows * sizeof(float), hipMemcpyHostToDevice, net->stream), "H2D");
+  MLP_TRY(mlp_shuffle_init(n, work, net->stream), "shuffle");
+  for (int e = 0; e < epochs; ++e) {
+    MLP_TRY(mlp_shuffle(n, seed, e, work, perm, net->stream), "shuffle");
+    for (int b = 0; b < nb; ++b) {
+      ++net->step;
+      MLP_TRY(mlp_train_step(net->w, bs, X, perm + (size_t)b * bs, T, net->w.grad, L + (size_t)e * nb + b, net->step,
+                             lr, net->stream), "training step");
     }
-    std::vector<float> lh((size_t)std::max(1, epochs) * nb);
+  }
+  std::vector<float> lh((size_t)std::max(1, epochs) * nb);
+  if (epochs > 0)
     MLP_TRY(hipMemcpyAsync(lh.data(), L, lh.size() * sizeof(float), hipMemcpyDeviceToHost, net->stream), "D2H");
-    MLP_TRY(hipStreamSynchronize(net->stream), "train");
-    if (loss_hist)
-      for (int e = 0; e < epochs; ++e) {
-        double s = 0.0;
-        for (int b = 0; b < nb; ++b) s += lh[(size_t)e * nb + b];
-        loss_hist[e] = (float)(s / nb);
-      }
-    return SG_OK;
-  };
-  rc = run();
-  cleanup();
-  return rc;
+  MLP_TRY(hipStreamSynchronize(net->stream), "train");
+  if (loss_hist)
+    for (int e = 0; e < epochs; ++e) {
+      double s = 0.0;
+      for (int b = 0; b < nb; ++b) s += lh[(size_t)e * nb + b];
+      loss_hist[e] = (float)(s / nb);
+    }
+  return SG_OK;
 }
 
 int sg_set_closure_mlp(sg_ctx* ctx, const sg_mlp* cnet) {
