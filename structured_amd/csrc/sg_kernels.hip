@@ -59,10 +59,11 @@ hipError_t launch_residual(const DevGeom& g, const DevPhys& ph, const DevBc& bc,
 }
 
 hipError_t launch_jv(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool sa, const double* q, const double* v,
-                     double* r, double* jv, hipStream_t s, const double* beta_dot, const DevClosure& clo) {
+                     double* r, double* jv, hipStream_t s, const double* beta_dot, const DevClosure& clo,
+                     const double* idt) {
   dim3 grid = tile_grid(g);
   Field<Dual> fq{q, v};
-  OutField<Dual> fo{r, jv};
+  OutField<Dual> fo{r, jv, idt, v};
   if (sa) launch_cl<Dual, true>(grid, s, g, ph, bc, fq, fo, nullptr, beta_dot, clo);
   else launch_cl<Dual, false>(grid, s, g, ph, bc, fq, fo, nullptr, nullptr, DevClosure());
   return hipGetLastError();

@@ -18,10 +18,11 @@ size_t residual_partial_count(const DevGeom& g);
 hipError_t launch_residual(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool sa, const double* q, double* r,
                            double* partial, unsigned long long* counter, double* l2, hipStream_t s,
                            const DevClosure& clo = DevClosure(), int l2_count = 0, unsigned* parity = nullptr);
-// J.v (+ (dR/dbeta).beta_dot when beta_dot is not null; v may be all zero)
+// J.v (+ (dR/dbeta).beta_dot when beta_dot is not null; v may be all zero);
+// with idt (per cell) jv receives v idt - J.v instead
 hipError_t launch_jv(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool sa, const double* q, const double* v,
                      double* r, double* jv, hipStream_t s, const double* beta_dot = nullptr,
-                     const DevClosure& clo = DevClosure());
+                     const DevClosure& clo = DevClosure(), const double* idt = nullptr);
 hipError_t launch_dt(const DevGeom& g, double mu_inf, int nv, const double* q, const double* dsmin, double cfl,
                      double* dt, hipStream_t s);
 hipError_t launch_aos_to_soa(int nic, int njc, int ldi, int nv, const double* aos, double* soa, hipStream_t s);

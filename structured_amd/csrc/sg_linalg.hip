@@ -15,7 +15,60 @@
 
 namespace sg {
 
-constexpr int DOT_BLOCK = 256;
+// ---- reductions finished inside their kernel --------------------------------
+// Every block stores its partial sums into slots of its own, and one more
+// block (the last of the grid) waits for them, sums them in a fixed order and
+// empties them for the next call.  A slot is one 64-bit atomic that holds
+// either a value or kNoValue, a signalling NaN that no arithmetic produces, so
+// nothing has to be ordered between slots, and no counter is needed: a
+// counter's increments, one after another at some 50 ns, took longer than the
+// second kernel they would have saved.  The other blocks depend on nothing,
+// so the wait ends; past kSlotPolls the result is NaN.
+constexpr unsigned long long kNoValue = 0x7FF4534C4F545321ull;
+constexpr int kSlotPolls = 1 << 22;
+
+__device__ __forceinline__ void slot_store(double* slot, double v) {
+  __hip_atomic_store(slot, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Sum of the slots first, first + stride, ... below n, in that order, U at a
+// time in flight; they are left empty.
+template <int U>
+__device__ double slot_sum(double* slots, int first, int stride, int n) {
+  double sum = 0.0;
+  int polls = 0;
+  for (int b = first; b < n; b += U * stride) {
+    unsigned long long v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      unsigned long long* p = reinterpret_cast<unsigned long long*>(slots + min(b + u * stride, n - 1));
+      v[u] = b + u * stride < n ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (b + u * stride >= n) break;
+      unsigned long long* p = reinterpret_cast<unsigned long long*>(slots + b + u * stride);
+      while (v[u] == kNoValue) {
+        if (++polls > kSlotPolls) {
+          v[u] = (unsigned long long)__double_as_longlong(__builtin_nan(""));
+          break;
+        }
+        v[u] = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __hip_atomic_store(p, kNoValue, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sum += __longlong_as_double((long long)v[u]);
+    }
+  }
+  return sum;
+}
+
+__global__ __launch_bounds__(256) void slots_empty_kernel(unsigned long long* x, size_t n) {
+  for (size_t e = blockIdx.x * (size_t)256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) x[e] = kNoValue;
+}
+hipError_t reduce_slots_init(double* slots, size_t n, hipStream_t s) {
+  hipLaunchKernelGGL(slots_empty_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 1024)), dim3(256), 0, s,
+                     reinterpret_cast<unsigned long long*>(slots), n);
+  return hipGetLastError();
+}
 
 // Gate of the conditional kernels: with ga and gb (device) the kernel runs
 // only when *ga < gf * *gb, else it returns at once (nothing written).
@@ -23,30 +76,42 @@ __device__ __forceinline__ bool gate_open(const double* ga, const double* gb, do
   return !ga || *ga < gf * *gb;
 }
 
-// out_partial[b*k + i] = sum over slice b of V_i . w.  The grid is
-// DOT_SLICES x (groups of DOT_KC vectors): block (b, g) sums vectors
-// g*DOT_KC .. g*DOT_KC + DOT_KC - 1 over the element pairs of slice b (pairs
-// b*DOT_BLOCK + t + m*DOT_SLICES*DOT_BLOCK, read as 16-byte loads; an odd last
-// element goes to slice 0, thread 0), with its accumulators in registers,
-// then over the block in a fixed order (DPP wavefront sums, then the four
-// waves).  All groups run at once, so a launch keeps every vector's loads in
+// out[i] = V_i . w.  The grid is (slices + 1) x (groups of DOT_KC vectors):
+// block (b, g) sums vectors g*DOT_KC .. g*DOT_KC + DOT_KC - 1 over the element
+// pairs of slice b (pairs b*DOT_BLOCK + t + m*slices*DOT_BLOCK, read as
+// 16-byte loads; an odd last element goes to slice 0, thread 0), with its
+// accumulators in registers, then over the block in a fixed order (DPP
+// wavefront sums, then the four waves); the last block of a group sums the
+// slices.  All groups run at once, so a launch keeps every vector's loads in
 // flight together; each group reads w once more, from L2 / MALL after the
 // first.  Vectors start on 16-byte boundaries (the host checks).
+// At 97x65 (24,576 doubles, up to 32 vectors) the sums and their separate
+// finalisation took 4.5 + 4 us and a launch gap, at 385x193 16 + 4.7.
+constexpr int DOT_BLOCK = 256;
 constexpr int DOT_KC = 8;
-constexpr int DOT_SLICES = 512;  // partial sums per dot product
+constexpr int DOT_SLICES = 512;  // at most
 __global__ __launch_bounds__(DOT_BLOCK) void multi_dot_kernel(const double* V, size_t ldv, int k, const double* w,
-                                                              size_t n, double* partial, const double* ga,
+                                                              size_t n, double* slots, double* out, const double* ga,
                                                               const double* gb, double gf) {
   if (!gate_open(ga, gb, gf)) return;
-  __shared__ double red[DOT_BLOCK / 64][DOT_KC];
+  const int slices = (int)gridDim.x - 1;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int i0 = (int)blockIdx.y * DOT_KC, kk = min(DOT_KC, k - i0);
+  if ((int)blockIdx.x == slices) {  // 32 threads per vector
+    const int i = threadIdx.x >> 5, l = threadIdx.x & 31;
+    double s = i < kk ? slot_sum<16>(slots + (size_t)(i0 + i) * slices, l, 32, slices) : 0.0;
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (i < kk && l == 0) out[i0 + i] = s;
+    return;
+  }
+  __shared__ double red[DOT_BLOCK / 64][DOT_KC];
   double acc[DOT_KC];
 #pragma unroll
   for (int i = 0; i < DOT_KC; ++i) acc[i] = 0.0;
   const size_t n2 = n / 2;
   const double2* w2 = reinterpret_cast<const double2*>(w);
-  for (size_t e = (size_t)blockIdx.x * DOT_BLOCK + threadIdx.x; e < n2; e += (size_t)DOT_SLICES * DOT_BLOCK) {
+  for (size_t e = (size_t)blockIdx.x * DOT_BLOCK + threadIdx.x; e < n2; e += (size_t)slices * DOT_BLOCK) {
     const double2 we = w2[e];
 #pragma unroll
     for (int i = 0; i < DOT_KC; ++i)
@@ -71,25 +136,7 @@ __global__ __launch_bounds__(DOT_BLOCK) void multi_dot_kernel(const double* V, s
   if ((int)threadIdx.x < kk) {
     double t = 0.0;
     for (int q = 0; q < DOT_BLOCK / 64; ++q) t += red[q][threadIdx.x];
-    partial[(size_t)blockIdx.x * k + i0 + threadIdx.x] = t;
-  }
-}
-
-// out[i] = sum_b partial[b*k + i]  (+ optional add into out when accumulate)
-__global__ __launch_bounds__(256) void dot_finalize_kernel(const double* partial, int nb, int k, double* out,
-                                                           int accumulate, const double* ga, const double* gb,
-                                                           double gf) {
-  if (!gate_open(ga, gb, gf)) return;
-  const int i = blockIdx.x;
-  __shared__ double red[4];
-  double s = 0.0;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) s += partial[(size_t)b * k + i];
-  s = wave_sum_lane63(s);
-  if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = red[0] + red[1] + red[2] + red[3];
-    out[i] = accumulate ? out[i] + t : t;
+    slot_store(slots + (size_t)(i0 + threadIdx.x) * slices + blockIdx.x, t);
   }
 }
 
@@ -99,60 +146,120 @@ static bool pairs_aligned(const double* V, size_t ldv, int k, const double* w) {
   const uintptr_t a = (uintptr_t)V | (uintptr_t)w;
   return (a & 15) == 0 && (k <= 1 || (ldv & 1) == 0);
 }
+// blocks of 256 threads for n elements taken in pairs, at most `most`
+static int pair_blocks(size_t n, int most) {
+  return (int)std::min<size_t>(std::max<size_t>((n / 2 + 255) / 256, 1), (size_t)most);
+}
 
-hipError_t multi_dot(const double* V, size_t ldv, int k, const double* w, size_t n, double* partial, double* out,
-                     bool accumulate, hipStream_t s, const double* ga, const double* gb, double gf) {
+hipError_t multi_dot(const double* V, size_t ldv, int k, const double* w, size_t n, double* slots, double* out,
+                     hipStream_t s, const double* ga, const double* gb, double gf) {
   if (!pairs_aligned(V, ldv, k, w)) return hipErrorInvalidValue;
-  const dim3 grid(DOT_SLICES, (unsigned)((k + DOT_KC - 1) / DOT_KC));
-  hipLaunchKernelGGL(multi_dot_kernel, grid, dim3(DOT_BLOCK), 0, s, V, ldv, k, w, n, partial, ga, gb, gf);
-  hipLaunchKernelGGL(dot_finalize_kernel, dim3(k), dim3(256), 0, s, partial, DOT_SLICES, k, out, accumulate ? 1 : 0,
-                     ga, gb, gf);
+  const dim3 grid(pair_blocks(n, DOT_SLICES) + 1, (unsigned)((k + DOT_KC - 1) / DOT_KC));
+  hipLaunchKernelGGL(multi_dot_kernel, grid, dim3(DOT_BLOCK), 0, s, V, ldv, k, w, n, slots, out, ga, gb, gf);
   return hipGetLastError();
 }
 
-size_t multi_dot_partial_size(int kmax) { return (size_t)DOT_SLICES * kmax; }
-
-// w -= sum_i c[i] V_i   (c in device memory).  Element pairs (16-byte
-// loads), the vectors taken eight at a time with their loads issued together
-// ahead of the eight updates; the updates keep the order i = 0, 1, ..., so
-// every element gets the arithmetic of a plain loop over i.
+// w -= sum_i c[i] V_i   (c in device memory), and *norm2 = |w|^2 of the
+// result.  Element pairs (16-byte loads), the vectors taken eight at a time
+// with their loads issued together ahead of the eight updates; the updates
+// keep the order i = 0, 1, ..., so every element gets the arithmetic of a
+// plain loop over i.  The norm costs no pass of its own: the blocks sum the
+// squares of what they store, and the last block sums the blocks.
 constexpr int AXPY_KC = 8;
-__global__ void multi_axpy_kernel(const double* V, size_t ldv, int k, const double* c, double* w, size_t n,
-                                  const double* ga, const double* gb, double gf) {
+constexpr int AXPY_BLOCKS = 2048;  // at most
+__global__ __launch_bounds__(256) void multi_axpy_kernel(const double* V, size_t ldv, int k, const double* c, double* w,
+                                                         size_t n, double* slots, double* norm2, const double* ga,
+                                                         const double* gb, double gf) {
   if (!gate_open(ga, gb, gf)) return;
-  const size_t n2 = n / 2;
-  double2* w2 = reinterpret_cast<double2*>(w);
-  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n2; e += (size_t)gridDim.x * blockDim.x) {
-    double2 s = w2[e];
-    int i = 0;
-    for (; i + AXPY_KC <= k; i += AXPY_KC) {
-      double2 v[AXPY_KC];
+  __shared__ double red[4];
+  const int blocks = (int)gridDim.x - 1, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  double sq = 0.0;
+  const bool last = (int)blockIdx.x == blocks;
+  if (last) {
+    sq = slot_sum<8>(slots, threadIdx.x, 256, blocks);
+  } else {
+    const size_t n2 = n / 2;
+    double2* w2 = reinterpret_cast<double2*>(w);
+    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n2; e += (size_t)blocks * 256) {
+      double2 s = w2[e];
+      int i = 0;
+      for (; i + AXPY_KC <= k; i += AXPY_KC) {
+        double2 v[AXPY_KC];
 #pragma unroll
-      for (int u = 0; u < AXPY_KC; ++u) v[u] = reinterpret_cast<const double2*>(V + (size_t)(i + u) * ldv)[e];
+        for (int u = 0; u < AXPY_KC; ++u) v[u] = reinterpret_cast<const double2*>(V + (size_t)(i + u) * ldv)[e];
 #pragma unroll
-      for (int u = 0; u < AXPY_KC; ++u) {
-        s.x -= c[i + u] * v[u].x;
-        s.y -= c[i + u] * v[u].y;
+        for (int u = 0; u < AXPY_KC; ++u) {
+          s.x -= c[i + u] * v[u].x;
+          s.y -= c[i + u] * v[u].y;
+        }
       }
+      for (; i < k; ++i) {
+        const double2 v = reinterpret_cast<const double2*>(V + (size_t)i * ldv)[e];
+        s.x -= c[i] * v.x;
+        s.y -= c[i] * v.y;
+      }
+      w2[e] = s;
+      sq += s.x * s.x;
+      sq += s.y * s.y;
     }
-    for (; i < k; ++i) {
-      const double2 v = reinterpret_cast<const double2*>(V + (size_t)i * ldv)[e];
-      s.x -= c[i] * v.x;
-      s.y -= c[i] * v.y;
+    if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
+      double t = w[n - 1];
+      for (int i = 0; i < k; ++i) t -= c[i] * V[(size_t)i * ldv + n - 1];
+      w[n - 1] = t;
+      sq += t * t;
     }
-    w2[e] = s;
   }
-  if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
-    double t = w[n - 1];
-    for (int i = 0; i < k; ++i) t -= c[i] * V[(size_t)i * ldv + n - 1];
-    w[n - 1] = t;
+  sq = wave_sum_lane63(sq);
+  if (lane == 63) red[wv] = sq;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const double t = red[0] + red[1] + red[2] + red[3];
+    if (last) *norm2 = t;
+    else slot_store(slots + blockIdx.x, t);
   }
 }
 
-hipError_t multi_axpy(const double* V, size_t ldv, int k, const double* c, double* w, size_t n, hipStream_t s,
-                      const double* ga, const double* gb, double gf) {
+hipError_t multi_axpy(const double* V, size_t ldv, int k, const double* c, double* w, size_t n, double* slots,
+                      double* norm2, hipStream_t s, const double* ga, const double* gb, double gf) {
   if (!pairs_aligned(V, ldv, k, w)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(multi_axpy_kernel, dim3(2048), dim3(256), 0, s, V, ldv, k, c, w, n, ga, gb, gf);
+  hipLaunchKernelGGL(multi_axpy_kernel, dim3(pair_blocks(n, AXPY_BLOCKS) + 1), dim3(256), 0, s, V, ldv, k, c, w, n,
+                     slots, norm2, ga, gb, gf);
+  return hipGetLastError();
+}
+
+size_t reduce_slots(int kmax) { return (size_t)std::max(DOT_SLICES * kmax, AXPY_BLOCKS); }
+
+// The end of an Arnoldi step (see sg_linalg.hpp): every block forms the scale
+// from the step's norms; block 0 writes the results.
+__global__ __launch_bounds__(256) void arnoldi_finish_kernel(double* w, size_t n, int j, const double* h,
+                                                             const double* y, const double* norm2b, double gf,
+                                                             double* res) {
+  const bool second = y[j + 1] < gf * h[j + 1];
+  const double hn = sqrt(fmax(0.0, second ? *norm2b : y[j + 1]));
+  if (blockIdx.x == 0) {
+    for (int i = threadIdx.x; i <= j; i += 256) res[i] = h[i] + (second ? y[i] : 0.0);
+    if (threadIdx.x == 0) {
+      res[j + 1] = hn;
+      res[j + 2] = second ? 1.0 : 0.0;
+    }
+  }
+  if (!(hn > 0.0)) return;
+  const double sc = 1.0 / hn;
+  const size_t n2 = n / 2;
+  double2* w2 = reinterpret_cast<double2*>(w);
+  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n2; e += (size_t)gridDim.x * 256) {
+    double2 v = w2[e];
+    v.x *= sc;
+    v.y *= sc;
+    w2[e] = v;
+  }
+  if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) w[n - 1] *= sc;
+}
+
+hipError_t arnoldi_finish(double* w, size_t n, int j, const double* h, const double* y, const double* norm2b, double gf,
+                          double* res, hipStream_t s) {
+  hipLaunchKernelGGL(arnoldi_finish_kernel, dim3(pair_blocks(n, 2048)), dim3(256), 0, s, w, n, j, h, y, norm2b, gf,
+                     res);
   return hipGetLastError();
 }
 
@@ -201,17 +308,6 @@ __global__ void axpby_kernel(double a, const double* x, double b, double* y, siz
 }
 hipError_t axpby(double a, const double* x, double b, double* y, size_t n, hipStream_t s) {
   hipLaunchKernelGGL(axpby_kernel, dim3(1024), dim3(256), 0, s, a, x, b, y, n);
-  return hipGetLastError();
-}
-
-// y = x * scale[k*plane...] style: w = z * idt - jz  (operator I/dt - J)
-__global__ void shift_minus_kernel(const double* z, const double* idt, const double* jz, double* w, size_t plane, int nv) {
-  const size_t n = plane * nv;
-  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x)
-    w[e] = z[e] * idt[e % plane] - jz[e];
-}
-hipError_t shift_minus(const double* z, const double* idt, const double* jz, double* w, size_t plane, int nv, hipStream_t s) {
-  hipLaunchKernelGGL(shift_minus_kernel, dim3(1024), dim3(256), 0, s, z, idt, jz, w, plane, nv);
   return hipGetLastError();
 }
 
@@ -737,9 +833,11 @@ hipError_t lilu_apply(int nic, int njc, int ldi, int nv, const double* ilu, cons
 
 // ---- adjoint products from the Jacobian blocks ----------------------------
 // (J^T psi)_c = sum_s J[c - d_s, c]^T psi_{c - d_s}, with J[r, r + d_s]
-// stored in slot s of row r: a 13-neighbour gather, deterministic.
+// stored in slot s of row r: a 13-neighbour gather, deterministic.  With idt
+// (per cell) the transposed operator psi idt - J^T psi.
 template <int NV>
-__global__ void jt_gather_kernel(int nic, int njc, int ldi, const double* blocks, const double* psi, double* out) {
+__global__ void jt_gather_kernel(int nic, int njc, int ldi, const double* blocks, const double* psi, const double* idt,
+                                 double* out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
   if (i >= nic) return;
   constexpr int B = NV * NV;
@@ -758,18 +856,18 @@ __global__ void jt_gather_kernel(int nic, int njc, int ldi, const double* blocks
       acc[k] += sum;
     }
   }
-  for (int k = 0; k < NV; ++k) out[k * plane + c] = acc[k];
+  const double sh = idt ? idt[c] : 0.0;
+  for (int k = 0; k < NV; ++k) out[k * plane + c] = idt ? psi[k * plane + c] * sh - acc[k] : acc[k];
 }
 
 hipError_t jt_gather(int nic, int njc, int ldi, int nv, const double* blocks, const double* psi, double* out,
-                     hipStream_t s) {
+                     hipStream_t s, const double* idt) {
   dim3 g((nic + 127) / 128, njc), b(128);
-  if (nv == 5) hipLaunchKernelGGL(jt_gather_kernel<5>, g, b, 0, s, nic, njc, ldi, blocks, psi, out);
-  else hipLaunchKernelGGL(jt_gather_kernel<4>, g, b, 0, s, nic, njc, ldi, blocks, psi, out);
+  if (nv == 5) hipLaunchKernelGGL(jt_gather_kernel<5>, g, b, 0, s, nic, njc, ldi, blocks, psi, idt, out);
+  else hipLaunchKernelGGL(jt_gather_kernel<4>, g, b, 0, s, nic, njc, ldi, blocks, psi, idt, out);
   return hipGetLastError();
 }
 
-// w = z * idt - J^T z   (transposed operator I/dt - J^T)
 // dbeta_c = psi_4c * dR4_c/dbeta_c  (dR/dbeta is diagonal: beta_c enters only
 // the SA production of cell c)
 __global__ void dbeta_kernel(int nic, int njc, int ldi, const double* psi, const double* diag, double* out) {

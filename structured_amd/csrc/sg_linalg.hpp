@@ -8,23 +8,31 @@ namespace sg {
 
 constexpr int NSLOT = 13;  // Jacobian stencil blocks kept per cell
 
-size_t multi_dot_partial_size(int kmax);
+// 64-bit slots of the reductions below, which every call finds and leaves
+// empty; reduce_slots_init empties them first.
+size_t reduce_slots(int kmax);
+hipError_t reduce_slots_init(double* slots, size_t n, hipStream_t s);
 // out[i] = V_i . w for i < k (V_i = V + i*ldv); out is device memory.  With
-// ga and gb (device doubles) the kernels run only if *ga < gf * *gb and
-// otherwise write nothing: a conditional pass decided on the device.
-hipError_t multi_dot(const double* V, size_t ldv, int k, const double* w, size_t n, double* partial, double* out,
-                     bool accumulate, hipStream_t s, const double* ga = nullptr, const double* gb = nullptr,
-                     double gf = 0.5);
-// w -= sum_i c[i] V_i, c device memory; gated as multi_dot
-hipError_t multi_axpy(const double* V, size_t ldv, int k, const double* c, double* w, size_t n, hipStream_t s,
-                      const double* ga = nullptr, const double* gb = nullptr, double gf = 0.5);
+// ga and gb (device doubles) the kernel runs only if *ga < gf * *gb and
+// otherwise writes nothing: a conditional pass decided on the device.
+hipError_t multi_dot(const double* V, size_t ldv, int k, const double* w, size_t n, double* slots, double* out,
+                     hipStream_t s, const double* ga = nullptr, const double* gb = nullptr, double gf = 0.5);
+// w -= sum_i c[i] V_i, c device memory, and *norm2 = |w|^2 after it; gated as
+// multi_dot
+hipError_t multi_axpy(const double* V, size_t ldv, int k, const double* c, double* w, size_t n, double* slots,
+                      double* norm2, hipStream_t s, const double* ga = nullptr, const double* gb = nullptr,
+                      double gf = 0.5);
+// The end of an Arnoldi step j: h[0..j+1] = V^T w and |w|^2, y[j+1] = |w'|^2
+// after the projection; if y[j+1] < gf h[j+1] a second one ran, with y[0..j]
+// its projections and *norm2b the norm after it.  Scales w to unit norm (a
+// zero w stays) and leaves in res (host memory the device can write) the
+// column's entries 0..j, then the norm and whether the second pass ran.
+hipError_t arnoldi_finish(double* w, size_t n, int j, const double* h, const double* y, const double* norm2b, double gf,
+                          double* res, hipStream_t s);
 // y (+)= sum_i c[i] X_i, c device memory
 hipError_t lincomb(const double* X, size_t ldx, int k, const double* c_dev, double* y, size_t n, bool accumulate,
                    hipStream_t s);
 hipError_t axpby(double a, const double* x, double b, double* y, size_t n, hipStream_t s);
-// w = z * idt (per cell) - jz
-hipError_t shift_minus(const double* z, const double* idt, const double* jz, double* w, size_t plane, int nv,
-                       hipStream_t s);
 // Coloured Jacobian extraction with colour period per (5: the 13-point
 // stencil; 3: the 3x3 box)
 hipError_t seed_colour(int nic, int njc, int ldi, int nv, int per, int a, int b, int m, double* v, hipStream_t s);
@@ -59,9 +67,9 @@ hipError_t cilu_factor(int nic, int njc, int ldi, int nv, int w, bool nine, cons
                        double* rec, hipStream_t s);
 hipError_t cilu_apply(int nic, int njc, int ldi, int nv, int w, bool nine, double* store, const double* b, double* z,
                       bool transpose, hipStream_t s);
-// adjoint helpers
+// adjoint helpers: J^T psi from the blocks, or with idt psi idt - J^T psi
 hipError_t jt_gather(int nic, int njc, int ldi, int nv, const double* blocks, const double* psi, double* out,
-                     hipStream_t s);
+                     hipStream_t s, const double* idt = nullptr);
 hipError_t dbeta_apply(int nic, int njc, int ldi, const double* psi, const double* diag, double* out, hipStream_t s);
 hipError_t ilu_apply_t(int nic, int njc, int ldi, int nv, const double* ilu, const double* b, double* z, hipStream_t s);
 // per-block minima of the admissible update fraction (see sg_linalg.hip)

@@ -688,7 +688,7 @@ __global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) vo
                                      __HIP_MEMORY_SCOPE_AGENT);
   if (owns) {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) out.put(k * g.plane + oidx, res[k]);
+    for (int k = 0; k < NV; ++k) out.put(k * g.plane, oidx, res[k]);
   }
   // ---- block partial sums of R^2 (fixed order: wavefront DPP sum, then waves)
   if (partial) {

@@ -160,15 +160,18 @@ struct OutField;
 template <>
 struct OutField<double> {
   double* v;
-  __device__ __forceinline__ void put(size_t k, double x) const { v[k] = x; }
+  __device__ __forceinline__ void put(size_t comp, size_t cell, double x) const { v[comp + cell] = x; }
 };
 template <>
 struct OutField<Dual> {
   double* v;  // may be null: value not stored
   double* d;
-  __device__ __forceinline__ void put(size_t k, Dual x) const {
-    if (v) v[k] = x.v;
-    d[k] = x.d;
+  // with idt (per cell), d receives z idt - tangent: the operator z/dt - J z
+  const double* idt = nullptr;
+  const double* z = nullptr;
+  __device__ __forceinline__ void put(size_t comp, size_t cell, Dual x) const {
+    if (v) v[comp + cell] = x.v;
+    d[comp + cell] = idt ? z[comp + cell] * idt[cell] - x.d : x.d;
   }
 };
 

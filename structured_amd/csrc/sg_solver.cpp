@@ -47,7 +47,8 @@ struct SolverState {
   DevBuf V, Z, blocks, fac, ilu, idt, dtv, rhs, x, tmp, jz, qop, seed, hdev, ydev, partial, gst, dbdiag, ones;
   DevBuf blocks_pc;          // preconditioner blocks when lhs_order > 0 (blocks keeps the exact J)
   DevBuf cilu;               // chunked line ILU(0) factors (precond 6)
-  PinnedBuf hpin;            // host copies of hdev and ydev for the Arnoldi step
+  PinnedBuf hpin;            // a dot product, the Krylov coefficients going up
+  PinnedBuf hres;            // results of an Arnoldi step, written by the device
   int pc_width = 16;         // chunk width of precond 6
   // have_lhs: the operator and preconditioner of the caller's last set_lhs are
   // in place.  Every call that changes the preconditioner settings or
@@ -98,18 +99,19 @@ int ensure(sg_ctx* ctx, int restart) {
   if (S->V.alloc((size_t)(restart + 1) * n) || S->Z.alloc((size_t)restart * n) || S->blocks.alloc(nb) ||
       S->fac.alloc(nf) || S->ilu.alloc(nb) || S->gst.alloc(n) || S->dbdiag.alloc(n) || S->ones.alloc(ctx->g.plane) || S->idt.alloc(ctx->g.plane) || S->dtv.alloc(n) || S->rhs.alloc(n) || S->x.alloc(n) ||
       S->tmp.alloc(n) || S->jz.alloc(n) || S->qop.alloc(n) || S->seed.alloc(n) || S->hdev.alloc(restart + 2) ||
-      S->ydev.alloc(restart + 2) || S->partial.alloc(multi_dot_partial_size(restart + 2)) ||
-      S->hpin.alloc(2 * (size_t)(restart + 2)))
+      S->ydev.alloc(restart + 2) || S->partial.alloc(reduce_slots(restart + 2)) ||
+      S->hpin.alloc((size_t)(restart + 2)) || S->hres.alloc((size_t)(restart + 3)))
     return sg_fail(ctx, SG_ERR_HIP, "solver allocation failed");
   for (DevBuf* b : {&S->V, &S->Z, &S->blocks, &S->fac, &S->dtv, &S->rhs, &S->x, &S->tmp, &S->jz, &S->qop, &S->seed})
     if (hipMemset(b->p, 0, b->n * sizeof(double)) != hipSuccess) return sg_fail(ctx, SG_ERR_HIP, "memset");
+  SG_TRY(reduce_slots_init(S->partial.p, S->partial.n, ctx->stream), "reduction slots");
   return SG_OK;
 }
 
 double host_dot(sg_ctx* ctx, const double* a, const double* b, int* rc) {
   SolverState* S = ctx->solver;
   double out = 0.0;
-  hipError_t e = multi_dot(a, 0, 1, b, S->n, S->partial.p, S->hdev.p, false, ctx->stream);
+  hipError_t e = multi_dot(a, 0, 1, b, S->n, S->partial.p, S->hdev.p, ctx->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(S->hpin.p, S->hdev.p, sizeof(double), hipMemcpyDeviceToHost, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e == hipSuccess) out = S->hpin.p[0];
@@ -161,11 +163,11 @@ int precond_apply(sg_ctx* ctx, const double* v, double* z) {
 int apply_operator(sg_ctx* ctx, const double* z, double* w) {
   SolverState* S = ctx->solver;
   if (S->transpose)
-    SG_TRY(jt_gather(ctx->geo.nic, ctx->geo.njc, ctx->g.ldi, ctx->nvar, S->blocks.p, z, S->jz.p, ctx->stream), "jt");
+    SG_TRY(jt_gather(ctx->geo.nic, ctx->geo.njc, ctx->g.ldi, ctx->nvar, S->blocks.p, z, w, ctx->stream, S->idt.p),
+           "jt");
   else
-    SG_TRY(launch_jv(ctx->g, ctx->ph, ctx->bc, ctx->sa, S->qop.p, z, nullptr, S->jz.p, ctx->stream, nullptr, ctx->clo),
-           "jv");
-  SG_TRY(shift_minus(z, S->idt.p, S->jz.p, w, ctx->g.plane, ctx->nvar, ctx->stream), "shift");
+    SG_TRY(launch_jv(ctx->g, ctx->ph, ctx->bc, ctx->sa, S->qop.p, z, nullptr, w, ctx->stream, nullptr, ctx->clo,
+                     S->idt.p), "jv");
   return SG_OK;
 }
 
@@ -309,27 +311,18 @@ int fgmres(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres) {
       double* wn0 = S->hdev.p + j + 1;
       double* wn1 = S->ydev.p + j + 1;
       double* wn2 = S->ydev.p + m + 1;
-      SG_TRY(multi_dot(S->V.p, n, j + 2, W, n, S->partial.p, S->hdev.p, false, ctx->stream), "dot");
-      SG_TRY(multi_axpy(S->V.p, n, j + 1, S->hdev.p, W, n, ctx->stream), "axpy");
-      SG_TRY(multi_dot(W, 0, 1, W, n, S->partial.p, wn1, false, ctx->stream), "dot");
       const double gf = S->dgks;
-      SG_TRY(multi_dot(S->V.p, n, j + 1, W, n, S->partial.p, S->ydev.p, false, ctx->stream, wn1, wn0, gf), "dot");
-      SG_TRY(multi_axpy(S->V.p, n, j + 1, S->ydev.p, W, n, ctx->stream, wn1, wn0, gf), "axpy");
-      SG_TRY(multi_dot(W, 0, 1, W, n, S->partial.p, wn2, false, ctx->stream, wn1, wn0, gf), "dot");
-      const double* h1 = S->hpin.p;          // hdev[0..j+1]
-      const double* h2 = S->hpin.p + m + 2;  // ydev[0..m+1]
-      SG_TRY(hipMemcpyAsync(S->hpin.p, S->hdev.p, (j + 2) * sizeof(double), hipMemcpyDeviceToHost, ctx->stream),
-             "D2H");
-      SG_TRY(hipMemcpyAsync(S->hpin.p + m + 2, S->ydev.p, (m + 2) * sizeof(double), hipMemcpyDeviceToHost,
-                            ctx->stream), "D2H");
+      SG_TRY(multi_dot(S->V.p, n, j + 2, W, n, S->partial.p, S->hdev.p, ctx->stream), "dot");
+      SG_TRY(multi_axpy(S->V.p, n, j + 1, S->hdev.p, W, n, S->partial.p, wn1, ctx->stream), "axpy");
+      SG_TRY(multi_dot(S->V.p, n, j + 1, W, n, S->partial.p, S->ydev.p, ctx->stream, wn1, wn0, gf), "dot");
+      SG_TRY(multi_axpy(S->V.p, n, j + 1, S->ydev.p, W, n, S->partial.p, wn2, ctx->stream, wn1, wn0, gf), "axpy");
+      SG_TRY(arnoldi_finish(W, n, j, S->hdev.p, S->ydev.p, wn2, gf, S->hres.p, ctx->stream), "arnoldi");
       SG_TRY(hipStreamSynchronize(ctx->stream), "sync");
-      const bool reorth = h2[j + 1] < gf * h1[j + 1];  // the device's test on the same doubles
-      for (int i = 0; i <= j; ++i) hcol[i] = h1[i] + (reorth ? h2[i] : 0.0);
-      const double hn = std::sqrt(std::max(0.0, reorth ? h2[m + 1] : h2[j + 1]));
-      S->reorth_count += reorth ? 1 : 0;
+      for (int i = 0; i <= j; ++i) hcol[i] = S->hres.p[i];
+      const double hn = S->hres.p[j + 1];
+      S->reorth_count += S->hres.p[j + 2] != 0.0 ? 1 : 0;
       if (!std::isfinite(hn)) return sg_fail(ctx, SG_ERR_NAN, "non-finite Krylov vector");
       hcol[j + 1] = hn;
-      if (hn > 0.0) SG_TRY(axpby(0.0, W, 1.0 / hn, W, n, ctx->stream), "scale");
       for (int i = 0; i < j; ++i) {  // previous rotations
         const double t = cs[i] * hcol[i] + sn[i] * hcol[i + 1];
         hcol[i + 1] = -sn[i] * hcol[i] + cs[i] * hcol[i + 1];
