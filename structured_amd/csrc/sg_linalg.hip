@@ -24,7 +24,6 @@ namespace sg {
 // counter's increments, one after another at some 50 ns, took longer than the
 // second kernel they would have saved.  The other blocks depend on nothing,
 // so the wait ends; past kSlotPolls the result is NaN.
-constexpr unsigned long long kNoValue = 0x7FF4534C4F545321ull;
 constexpr int kSlotPolls = 1 << 22;
 
 __device__ __forceinline__ void slot_store(double* slot, double v) {
@@ -236,11 +235,12 @@ __global__ __launch_bounds__(256) void arnoldi_finish_kernel(double* w, size_t n
                                                              double* res) {
   const bool second = y[j + 1] < gf * h[j + 1];
   const double hn = sqrt(fmax(0.0, second ? *norm2b : y[j + 1]));
-  if (blockIdx.x == 0) {
-    for (int i = threadIdx.x; i <= j; i += 256) res[i] = h[i] + (second ? y[i] : 0.0);
+  if (blockIdx.x == 0) {  // to the host, word by word: it waits for each
+    auto put = [&](int i, double v) { __hip_atomic_store(res + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
+    for (int i = threadIdx.x; i <= j; i += 256) put(i, h[i] + (second ? y[i] : 0.0));
     if (threadIdx.x == 0) {
-      res[j + 1] = hn;
-      res[j + 2] = second ? 1.0 : 0.0;
+      put(j + 1, hn);
+      put(j + 2, second ? 1.0 : 0.0);
     }
   }
   if (!(hn > 0.0)) return;

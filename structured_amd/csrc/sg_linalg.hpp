@@ -8,6 +8,9 @@ namespace sg {
 
 constexpr int NSLOT = 13;  // Jacobian stencil blocks kept per cell
 
+// What a 64-bit slot holds while it has no value: a signalling NaN, which no
+// arithmetic produces.
+constexpr unsigned long long kNoValue = 0x7FF4534C4F545321ull;
 // 64-bit slots of the reductions below, which every call finds and leaves
 // empty; reduce_slots_init empties them first.
 size_t reduce_slots(int kmax);
@@ -25,8 +28,9 @@ hipError_t multi_axpy(const double* V, size_t ldv, int k, const double* c, doubl
 // The end of an Arnoldi step j: h[0..j+1] = V^T w and |w|^2, y[j+1] = |w'|^2
 // after the projection; if y[j+1] < gf h[j+1] a second one ran, with y[0..j]
 // its projections and *norm2b the norm after it.  Scales w to unit norm (a
-// zero w stays) and leaves in res (host memory the device can write) the
-// column's entries 0..j, then the norm and whether the second pass ran.
+// zero w stays) and leaves in res (host memory the device can write, preset to
+// kNoValue) the column's entries 0..j, then the norm and whether the second
+// pass ran (1 or 0), each as one 64-bit store.
 hipError_t arnoldi_finish(double* w, size_t n, int j, const double* h, const double* y, const double* norm2b, double gf,
                           double* res, hipStream_t s);
 // y (+)= sum_i c[i] X_i, c device memory

@@ -48,7 +48,7 @@ struct SolverState {
   DevBuf blocks_pc;          // preconditioner blocks when lhs_order > 0 (blocks keeps the exact J)
   DevBuf cilu;               // chunked line ILU(0) factors (precond 6)
   PinnedBuf hpin;            // a dot product, the Krylov coefficients going up
-  PinnedBuf hres;            // results of an Arnoldi step, written by the device
+  PinnedBuf hres;            // results of two Arnoldi steps, written by the device
   int pc_width = 16;         // chunk width of precond 6
   // have_lhs: the operator and preconditioner of the caller's last set_lhs are
   // in place.  Every call that changes the preconditioner settings or
@@ -100,7 +100,7 @@ int ensure(sg_ctx* ctx, int restart) {
       S->fac.alloc(nf) || S->ilu.alloc(nb) || S->gst.alloc(n) || S->dbdiag.alloc(n) || S->ones.alloc(ctx->g.plane) || S->idt.alloc(ctx->g.plane) || S->dtv.alloc(n) || S->rhs.alloc(n) || S->x.alloc(n) ||
       S->tmp.alloc(n) || S->jz.alloc(n) || S->qop.alloc(n) || S->seed.alloc(n) || S->hdev.alloc(restart + 2) ||
       S->ydev.alloc(restart + 2) || S->partial.alloc(reduce_slots(restart + 2)) ||
-      S->hpin.alloc((size_t)(restart + 2)) || S->hres.alloc((size_t)(restart + 3)))
+      S->hpin.alloc((size_t)(restart + 2)) || S->hres.alloc(2 * (size_t)(restart + 3)))
     return sg_fail(ctx, SG_ERR_HIP, "solver allocation failed");
   for (DevBuf* b : {&S->V, &S->Z, &S->blocks, &S->fac, &S->dtv, &S->rhs, &S->x, &S->tmp, &S->jz, &S->qop, &S->seed})
     if (hipMemset(b->p, 0, b->n * sizeof(double)) != hipSuccess) return sg_fail(ctx, SG_ERR_HIP, "memset");
@@ -260,8 +260,74 @@ int build_preconditioner(sg_ctx* ctx) {
   return SG_OK;
 }
 
-// Right-preconditioned restarted FGMRES with CGS2.  Solves A x = rhs.
+// Waits until the device has written the n words at p (preset to kNoValue).
+// The stream is asked now and then: a failed launch or a fault ends the wait.
+int wait_words(sg_ctx* ctx, const double* p, int n) {
+  auto missing = [&]() {
+    for (int i = 0; i < n; ++i)
+      if (__atomic_load_n(reinterpret_cast<const unsigned long long*>(p) + i, __ATOMIC_ACQUIRE) == kNoValue) return true;
+    return false;
+  };
+  for (unsigned spins = 1; missing(); ++spins) {
+    if (spins % 8192) continue;
+    const hipError_t e = hipStreamQuery(ctx->stream);
+    if (e == hipErrorNotReady) continue;
+    if (e == hipSuccess && !missing()) break;
+    return e == hipSuccess ? sg_fail(ctx, SG_ERR_HIP, "Krylov step left no result") : sg_hip(ctx, e, "Krylov step");
+  }
+  return SG_OK;
+}
+
+// Enqueues Arnoldi step j: z_j = M^-1 v_j, w = A z_j, its projections and its
+// scaling; the column goes to res.
+int arnoldi_step(sg_ctx* ctx, int j, double* res) {
+  SolverState* S = ctx->solver;
+  const int m = S->m;
+  const size_t n = S->n;
+  double* Vj = S->V.p + (size_t)j * n;
+  double* Zj = S->Z.p + (size_t)j * n;
+  double* W = S->V.p + (size_t)(j + 1) * n;
+  int rc;
+  unsigned long long* words = reinterpret_cast<unsigned long long*>(res);
+  for (int i = 0; i < j + 3; ++i) __atomic_store_n(words + i, kNoValue, __ATOMIC_RELEASE);
+  if ((rc = precond_apply(ctx, Vj, Zj))) return rc;
+  if ((rc = apply_operator(ctx, Zj, W))) return rc;
+  // Classical Gram-Schmidt with selective re-orthogonalisation (the DGKS
+  // criterion): the projection h = V^T w comes with |w|^2 (W is V_{j+1}, so
+  // one more product in the same pass), and the second pass runs only if
+  // |w'|^2 < dgks |w|^2 after the first.  The decision is taken on the device:
+  // the second pass's kernels read the two norms and return at once when it is
+  // not needed, so no host round trip is added.
+  //   hdev[0..j] = h, hdev[j+1] = |w|^2; ydev[j+1] = |w'|^2;
+  //   second pass: ydev[0..j] = V^T w', ydev[m+1] = |w''|^2
+  double* wn0 = S->hdev.p + j + 1;
+  double* wn1 = S->ydev.p + j + 1;
+  double* wn2 = S->ydev.p + m + 1;
+  const double gf = S->dgks;
+  SG_TRY(multi_dot(S->V.p, n, j + 2, W, n, S->partial.p, S->hdev.p, ctx->stream), "dot");
+  SG_TRY(multi_axpy(S->V.p, n, j + 1, S->hdev.p, W, n, S->partial.p, wn1, ctx->stream), "axpy");
+  SG_TRY(multi_dot(S->V.p, n, j + 1, W, n, S->partial.p, S->ydev.p, ctx->stream, wn1, wn0, gf), "dot");
+  SG_TRY(multi_axpy(S->V.p, n, j + 1, S->ydev.p, W, n, S->partial.p, wn2, ctx->stream, wn1, wn0, gf), "axpy");
+  SG_TRY(arnoldi_finish(W, n, j, S->hdev.p, S->ydev.p, wn2, gf, res, ctx->stream), "arnoldi");
+  return SG_OK;
+}
+
+// Right-preconditioned restarted FGMRES with CGS2.  Solves A x = rhs.  Step j +
+// 1 is enqueued before the results of step j are read, so that the device does
+// not wait for the host between steps (some 20 us each); where the residual is
+// about to reach the tolerance, the host looks first.  A step that turns out
+// not to be needed leaves x as it is.  A laminar Newton solve at 97x65:
+// 134 -> 121 ms, 120 adjoint steps at 385x193 48.8 -> 47.4 ms.
+int fgmres_steps(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres);
+
 int fgmres(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres) {
+  const int rc = fgmres_steps(ctx, rtol, maxit, iters, relres);
+  // an early end leaves steps on the stream that still write to hres
+  if (rc) (void)hipStreamSynchronize(ctx->stream);
+  return rc;
+}
+
+int fgmres_steps(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres) {
   SolverState* S = ctx->solver;
   const int m = S->m;
   const size_t n = S->n;
@@ -285,7 +351,7 @@ int fgmres(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres) {
       SG_TRY(hipMemcpyAsync(V0, S->rhs.p, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream), "copy");
       SG_TRY(axpby(-1.0, S->tmp.p, 1.0, V0, n, ctx->stream), "axpby");
     }
-    const double beta = std::sqrt(host_dot(ctx, V0, V0, &rc));
+    const double beta = total == 0 ? bnorm : std::sqrt(host_dot(ctx, V0, V0, &rc));
     if (rc) return rc;
     if (beta == 0.0) { res = 0.0; break; }
     SG_TRY(axpby(0.0, V0, 1.0 / beta, V0, n, ctx->stream), "scale");
@@ -293,34 +359,25 @@ int fgmres(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres) {
     g[0] = beta;
     int jend = -1;
     bool done = false;
+    auto result = [&](int j) { return S->hres.p + (size_t)(j & 1) * (m + 3); };
+    double before = beta;  // the residual one step earlier
+    res = beta;
+    int queued = 0;  // steps on the stream
     for (int j = 0; j < m && total < maxit; ++j) {
-      double* Vj = S->V.p + (size_t)j * n;
-      double* Zj = S->Z.p + (size_t)j * n;
-      double* W = S->V.p + (size_t)(j + 1) * n;
-      if ((rc = precond_apply(ctx, Vj, Zj))) return rc;
-      if ((rc = apply_operator(ctx, Zj, W))) return rc;
-      // Classical Gram-Schmidt with selective re-orthogonalisation (the
-      // DGKS criterion): the projection h = V^T w comes with |w|^2 (W is
-      // V_{j+1}, so one more product in the same pass), and the second pass
-      // runs only if |w'|^2 < dgks |w|^2 after the first.  The decision is
-      // taken on the device: the second pass's kernels read the two norms
-      // and return at once when it is not needed, so no host round trip is
-      // added.
-      //   hdev[0..j] = h, hdev[j+1] = |w|^2; ydev[j+1] = |w'|^2;
-      //   second pass: ydev[0..j] = V^T w', ydev[m+1] = |w''|^2
-      double* wn0 = S->hdev.p + j + 1;
-      double* wn1 = S->ydev.p + j + 1;
-      double* wn2 = S->ydev.p + m + 1;
-      const double gf = S->dgks;
-      SG_TRY(multi_dot(S->V.p, n, j + 2, W, n, S->partial.p, S->hdev.p, ctx->stream), "dot");
-      SG_TRY(multi_axpy(S->V.p, n, j + 1, S->hdev.p, W, n, S->partial.p, wn1, ctx->stream), "axpy");
-      SG_TRY(multi_dot(S->V.p, n, j + 1, W, n, S->partial.p, S->ydev.p, ctx->stream, wn1, wn0, gf), "dot");
-      SG_TRY(multi_axpy(S->V.p, n, j + 1, S->ydev.p, W, n, S->partial.p, wn2, ctx->stream, wn1, wn0, gf), "axpy");
-      SG_TRY(arnoldi_finish(W, n, j, S->hdev.p, S->ydev.p, wn2, gf, S->hres.p, ctx->stream), "arnoldi");
-      SG_TRY(hipStreamSynchronize(ctx->stream), "sync");
-      for (int i = 0; i <= j; ++i) hcol[i] = S->hres.p[i];
-      const double hn = S->hres.p[j + 1];
-      S->reorth_count += S->hres.p[j + 2] != 0.0 ? 1 : 0;
+      if (queued == j) {
+        if ((rc = arnoldi_step(ctx, j, result(j)))) return rc;
+        ++queued;
+      }
+      const bool close = res * (res / before) <= rtol * bnorm;  // this step probably ends the solve
+      if (!close && j + 1 < m && total + 1 < maxit) {
+        if ((rc = arnoldi_step(ctx, j + 1, result(j + 1)))) return rc;
+        ++queued;
+      }
+      const double* col = result(j);
+      if ((rc = wait_words(ctx, col, j + 3))) return rc;
+      for (int i = 0; i <= j; ++i) hcol[i] = col[i];
+      const double hn = col[j + 1];
+      S->reorth_count += col[j + 2] != 0.0 ? 1 : 0;
       if (!std::isfinite(hn)) return sg_fail(ctx, SG_ERR_NAN, "non-finite Krylov vector");
       hcol[j + 1] = hn;
       for (int i = 0; i < j; ++i) {  // previous rotations
@@ -338,6 +395,7 @@ int fgmres(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres) {
       for (int i = 0; i <= j; ++i) H[(size_t)i * m + j] = hcol[i];
       ++total;
       jend = j;
+      before = res;
       res = std::fabs(g[j + 1]);
       if (res <= rtol * bnorm || hn == 0.0) { done = true; break; }
     }
@@ -355,6 +413,7 @@ int fgmres(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres) {
     SG_TRY(lincomb(S->Z.p, n, jend + 1, S->ydev.p, S->x.p, n, true, ctx->stream), "lincomb");
     if (done) break;
   }
+  // also for a step enqueued beyond the last one, which still writes to hres
   SG_TRY(hipStreamSynchronize(ctx->stream), "sync");
   *iters = total;
   *relres = res / bnorm;
