@@ -17,23 +17,22 @@ size_t residual_partial_count(const DevGeom& g) {
   return (size_t)gr.x * gr.y;
 }
 
-template <class S, bool SA>
-static void launch_cl(dim3 grid, hipStream_t s, const DevGeom& g, const DevPhys& ph, const DevBc& bc, Field<S> fq,
-                      OutField<S> fo, double* partial, const double* beta_dot, const DevClosure& clo,
+template <class S, bool SA, class F, class O>
+static void launch_cl(dim3 grid, hipStream_t s, const DevGeom& g, const DevPhys& ph, const DevBc& bc, F fq, O fo, double* partial, const double* beta_dot, const DevClosure& clo,
                       NormOut no = NormOut{nullptr, nullptr, 0, 0u}) {
   if constexpr (SA) {
     if (clo.kind == CLOSURE_ANALYTIC) {
-      hipLaunchKernelGGL((residual_kernel<S, SA, CLOSURE_ANALYTIC>), grid, dim3(NT), 0, s, g, ph, bc, fq, fo, partial,
+      hipLaunchKernelGGL((residual_kernel<S, SA, CLOSURE_ANALYTIC, F, O>), grid, dim3(NT), 0, s, g, ph, bc, fq, fo, partial,
                          beta_dot, clo, no);
       return;
     }
     if (clo.kind == CLOSURE_MLP) {
-      hipLaunchKernelGGL((residual_kernel<S, SA, CLOSURE_MLP>), grid, dim3(NT), 0, s, g, ph, bc, fq, fo, partial,
+      hipLaunchKernelGGL((residual_kernel<S, SA, CLOSURE_MLP, F, O>), grid, dim3(NT), 0, s, g, ph, bc, fq, fo, partial,
                          beta_dot, clo, no);
       return;
     }
   }
-  hipLaunchKernelGGL((residual_kernel<S, SA, CLOSURE_FIELD>), grid, dim3(NT), 0, s, g, ph, bc, fq, fo, partial,
+  hipLaunchKernelGGL((residual_kernel<S, SA, CLOSURE_FIELD, F, O>), grid, dim3(NT), 0, s, g, ph, bc, fq, fo, partial,
                        beta_dot, clo, no);
 }
 
@@ -65,6 +64,26 @@ hipError_t launch_jv(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool 
   Field<Dual> fq{q, v};
   OutField<Dual> fo{r, jv, idt, v};
   if (sa) launch_cl<Dual, true>(grid, s, g, ph, bc, fq, fo, nullptr, beta_dot, clo);
+  else launch_cl<Dual, false>(grid, s, g, ph, bc, fq, fo, nullptr, nullptr, DevClosure());
+  return hipGetLastError();
+}
+
+// Jacobian blocks of the residual at q: one launch takes every coloured
+// direction (per^2 nv of them, 45 or 125 with SA) as the third dimension of
+// its grid, seeds it where the state is loaded and stores its columns where the
+// tangent is formed.  A launch per direction with a seed and an extraction
+// kernel around it took 29 us each at 385x193 (20 of them the sweep, whose 406
+// tiles do not fill the chip), 27 at 97x65, where the sweep is 40 tiles; now
+// 6.2 and 4.1.
+hipError_t launch_blocks(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool sa, const double* q, int per,
+                         double* blocks, hipStream_t s, const DevClosure& clo) {
+  if (per != 3 && per != 5) return hipErrorInvalidValue;
+  const Direction d{per, sa ? 5 : 4};
+  dim3 grid = tile_grid(g);
+  grid.z = (unsigned)d.count();
+  const SeedField fq{q, d};
+  const OutBlocks fo{blocks, d};
+  if (sa) launch_cl<Dual, true>(grid, s, g, ph, bc, fq, fo, nullptr, nullptr, clo);
   else launch_cl<Dual, false>(grid, s, g, ph, bc, fq, fo, nullptr, nullptr, DevClosure());
   return hipGetLastError();
 }

@@ -23,6 +23,10 @@ hipError_t launch_residual(const DevGeom& g, const DevPhys& ph, const DevBc& bc,
 hipError_t launch_jv(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool sa, const double* q, const double* v,
                      double* r, double* jv, hipStream_t s, const double* beta_dot = nullptr,
                      const DevClosure& clo = DevClosure(), const double* idt = nullptr);
+// Jacobian blocks at q by coloured directions (per 5: the 13-point stencil; 3:
+// the 3x3 box, the +-2 slots are not written)
+hipError_t launch_blocks(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool sa, const double* q, int per,
+                         double* blocks, hipStream_t s, const DevClosure& clo);
 hipError_t launch_dt(const DevGeom& g, double mu_inf, int nv, const double* q, const double* dsmin, double cfl,
                      double* dt, hipStream_t s);
 hipError_t launch_aos_to_soa(int nic, int njc, int ldi, int nv, const double* aos, double* soa, hipStream_t s);

@@ -1,8 +1,7 @@
 // Device linear algebra for the matrix-free Newton-Krylov solve:
 // deterministic multi-dot products and multi-axpys for the Gram-Schmidt
 // passes (with device-side gates for the selective second pass), scaling,
-// colour seeding and extraction of Jacobian blocks from J.v products, the
-// block preconditioners other than the chunked line ILU (j-line
+// the block preconditioners other than the chunked line ILU (j-line
 // block-tridiagonal, line Gauss-Seidel, multicolour and natural-order block
 // ILU(0)), and the adjoint products J^T psi and (dR/dbeta)^T psi from the
 // blocks.  All vectors are SoA with zero padding (length nvar*plane).
@@ -311,57 +310,10 @@ hipError_t axpby(double a, const double* x, double b, double* y, size_t n, hipSt
   return hipGetLastError();
 }
 
-// v = e_m on the cells of colour (a, b) = (i mod per, j mod per), 0
-// elsewhere.  per = 5 separates the 13-point stencil (reach 2), per = 3 the
-// 3x3 box (reach 1).
-__global__ void seed_kernel(int nic, int njc, int ldi, int nv, int per, int a, int b, int m, double* v) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
-  if (i >= nic) return;
-  const size_t plane = (size_t)njc * ldi, c = (size_t)j * ldi + i;
-  const bool on = (i % per == a) && (j % per == b);
-  for (int k = 0; k < nv; ++k) v[k * plane + c] = (on && k == m) ? 1.0 : 0.0;
-}
-hipError_t seed_colour(int nic, int njc, int ldi, int nv, int per, int a, int b, int m, double* v, hipStream_t s) {
-  if (per != 3 && per != 5) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(seed_kernel, dim3((nic + 127) / 128, njc), dim3(128), 0, s, nic, njc, ldi, nv, per, a, b, m, v);
-  return hipGetLastError();
-}
-
 // Stencil slots of the exact Jacobian of the residual: the 3x3 box plus
 // (0,+-2) and (+-2,0) (MUSCL reach).  Slot s holds J[r, r + (di,dj)].
 __constant__ int kSlotDi[NSLOT] = {0, 0, 0, -1, 1, -1, 1, -1, 1, 0, 0, -2, 2};
 __constant__ int kSlotDj[NSLOT] = {0, -1, 1, 0, 0, -1, -1, 1, 1, -2, 2, 0, 0};
-
-__device__ __forceinline__ int slot_of(int di, int dj) {
-  for (int s = 0; s < NSLOT; ++s)
-    if (kSlotDi[s] == di && kSlotDj[s] == dj) return s;
-  return -1;
-}
-
-// From J.v of colour (a,b), variable m: row cell r holds column m of the
-// block J[r, c] for the unique colour-(a,b) cell c in r's per x per window.
-// Blocks are struct-of-arrays: blocks[((slot*nv + row)*nv + col)*plane + cell].
-__global__ void extract_kernel(int nic, int njc, int ldi, int nv, int per, int a, int b, int m, const double* jv,
-                               double* blocks) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
-  if (i >= nic) return;
-  const int h = per / 2;
-  int di = ((a - i) % per + per) % per;
-  if (di > h) di -= per;
-  int dj = ((b - j) % per + per) % per;
-  if (dj > h) dj -= per;
-  const int slot = slot_of(di, dj);
-  if (slot < 0) return;
-  const size_t plane = (size_t)njc * ldi, c = (size_t)j * ldi + i;
-  for (int k = 0; k < nv; ++k) blocks[((size_t)(slot * nv + k) * nv + m) * plane + c] = jv[k * plane + c];
-}
-hipError_t extract_blocks(int nic, int njc, int ldi, int nv, int per, int a, int b, int m, const double* jv,
-                          double* blocks, hipStream_t s) {
-  if (per != 3 && per != 5) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(extract_kernel, dim3((nic + 127) / 128, njc), dim3(128), 0, s, nic, njc, ldi, nv, per, a, b, m,
-                     jv, blocks);
-  return hipGetLastError();
-}
 
 // Zeroes n doubles (a kernel rather than a memset, so that the call may be
 // captured into a graph).

@@ -37,11 +37,6 @@ hipError_t arnoldi_finish(double* w, size_t n, int j, const double* h, const dou
 hipError_t lincomb(const double* X, size_t ldx, int k, const double* c_dev, double* y, size_t n, bool accumulate,
                    hipStream_t s);
 hipError_t axpby(double a, const double* x, double b, double* y, size_t n, hipStream_t s);
-// Coloured Jacobian extraction with colour period per (5: the 13-point
-// stencil; 3: the 3x3 box)
-hipError_t seed_colour(int nic, int njc, int ldi, int nv, int per, int a, int b, int m, double* v, hipStream_t s);
-hipError_t extract_blocks(int nic, int njc, int ldi, int nv, int per, int a, int b, int m, const double* jv,
-                          double* blocks, hipStream_t s);
 hipError_t zero_fill(double* x, size_t n, hipStream_t s);
 hipError_t line_factor(int nic, int njc, int ldi, int nv, const double* idt, const double* blocks, double* fac,
                        bool jacobi, hipStream_t s);

@@ -50,12 +50,12 @@ __device__ __forceinline__ Prim<S> prim_from_cons(const S* qc, const DevPhys& ph
   return P;
 }
 
-template <class S, bool SA>
-__device__ __forceinline__ Prim<S> prim_interior(const Field<S>& q, const DevGeom& g, const DevPhys& ph, int ci, int cj) {
+template <class S, bool SA, class F>
+__device__ __forceinline__ Prim<S> prim_interior(const F& q, const DevGeom& g, const DevPhys& ph, int ci, int cj) {
   const size_t idx = (size_t)cj * g.ldi + ci;
   S qc[5];
 #pragma unroll
-  for (int k = 0; k < (SA ? 5 : 4); ++k) qc[k] = q[k * g.plane + idx];
+  for (int k = 0; k < (SA ? 5 : 4); ++k) qc[k] = q.at(k, g.plane, idx, ci, cj);
   return prim_from_cons<S, SA>(qc, ph);
 }
 
@@ -106,14 +106,14 @@ __device__ __forceinline__ Prim<S> apply_op(const BcNode& nd, const Prim<S>& A, 
   return o;
 }
 
-template <class S, bool SA>
-__device__ __forceinline__ Prim<S> ref_leaf(int ref, const Field<S>& q, const DevGeom& g, const DevPhys& ph) {
+template <class S, bool SA, class F>
+__device__ __forceinline__ Prim<S> ref_leaf(int ref, const F& q, const DevGeom& g, const DevPhys& ph) {
   return prim_interior<S, SA>(q, g, ph, ref % g.nic, ref / g.nic);
 }
 
 // Node whose operands are interior cells.
-template <class S, bool SA>
-__device__ Prim<S> eval_leaf_node(const BcNode& nd, const Field<S>& q, const DevGeom& g, const DevPhys& ph) {
+template <class S, bool SA, class F>
+__device__ Prim<S> eval_leaf_node(const BcNode& nd, const F& q, const DevGeom& g, const DevPhys& ph) {
   Prim<S> A, B;
   if (nd.op != OP_FREESTREAM) A = ref_leaf<S, SA>(nd.ra, q, g, ph);
   if (nd.op == OP_SLIP || nd.op == OP_WALL || nd.op == OP_ISO) B = ref_leaf<S, SA>(nd.rb, q, g, ph);
@@ -122,8 +122,8 @@ __device__ Prim<S> eval_leaf_node(const BcNode& nd, const Field<S>& q, const Dev
 
 // Node whose operands are interior cells or leaf nodes (depth <= 2 is
 // guaranteed by the host-side boundary compiler).
-template <class S, bool SA>
-__device__ Prim<S> eval_node(int id, const DevBc& bc, const Field<S>& q, const DevGeom& g, const DevPhys& ph) {
+template <class S, bool SA, class F>
+__device__ Prim<S> eval_node(int id, const DevBc& bc, const F& q, const DevGeom& g, const DevPhys& ph) {
   const BcNode nd = bc.nodes[id];
   Prim<S> A, B;
   if (nd.op != OP_FREESTREAM) {
@@ -366,9 +366,11 @@ struct NormOut {
 constexpr int kNormSpinLimit = 1 << 22;
 
 // CL: closure kind of beta (ClosureKind); CLOSURE_MLP stages the hidden
-// layer of the network (and its tangent) in the same LDS area.
-template <class S, bool SA, int CL>
-__global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) void residual_kernel(DevGeom g, DevPhys ph, DevBc bc, Field<S> q, OutField<S> out,
+// layer of the network (and its tangent) in the same LDS area.  F and O: where
+// the state comes from and the result goes (Field and OutField, or SeedField
+// and OutBlocks for Jacobian blocks).
+template <class S, bool SA, int CL, class F = Field<S>, class O = OutField<S>>
+__global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) void residual_kernel(DevGeom g, DevPhys ph, DevBc bc, F q, O out,
                                                        double* partial, const double* beta_dot, DevClosure clo,
                                                        NormOut nout) {
   constexpr int NL = SA ? L_MAX : (L_K + 1);
@@ -381,6 +383,8 @@ __global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) vo
   S* lds = reinterpret_cast<S*>(lds_raw);
   __shared__ double red[NT / 64][2 * NV];
 
+  q.begin(blockIdx.z);
+  out.begin(blockIdx.z);
   const int tid = threadIdx.x;
   const int tx = tid % TX, ty = tid / TX;
   // XCD-aware tile order: work-groups are handed to the 8 XCDs round-robin in
@@ -414,7 +418,7 @@ __global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) vo
     if (interior) {
       const size_t idx = (size_t)cj * g.ldi + ci;
 #pragma unroll
-      for (int k = 0; k < NQ; ++k) qraw[pass][k] = q[k * g.plane + idx];
+      for (int k = 0; k < NQ; ++k) qraw[pass][k] = q.at(k, g.plane, idx, ci, cj);
     }
   }
 #pragma unroll
@@ -688,7 +692,7 @@ __global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) vo
                                      __HIP_MEMORY_SCOPE_AGENT);
   if (owns) {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) out.put(k * g.plane, oidx, res[k]);
+    for (int k = 0; k < NV; ++k) out.put(k, g.plane, oidx, ci, cj, res[k]);
   }
   // ---- block partial sums of R^2 (fixed order: wavefront DPP sum, then waves)
   if (partial) {

@@ -139,20 +139,49 @@ __device__ __forceinline__ Dual spow16(Dual z) {
 __device__ __forceinline__ double smin(double a, double b) { return a < b ? a : b; }
 __device__ __forceinline__ Dual smin(Dual a, double b) { return a.v < b ? a : Dual(b); }
 
-// Loads of a state component for scalar type S: the dual reads the tangent
-// from a second array of the same layout.
+// Loads of a state component for scalar type S: component k of the cell with
+// index idx (column ci, row cj).  The dual reads the tangent from a second
+// array of the same layout.
 template <class S>
 struct Field;
 template <>
 struct Field<double> {
   const double* v;
-  __device__ __forceinline__ double operator[](size_t k) const { return v[k]; }
+  __device__ __forceinline__ void begin(int) {}
+  __device__ __forceinline__ double at(int k, size_t plane, size_t idx, int, int) const { return v[k * plane + idx]; }
 };
 template <>
 struct Field<Dual> {
   const double* v;
   const double* d;
-  __device__ __forceinline__ Dual operator[](size_t k) const { return Dual(v[k], d[k]); }
+  __device__ __forceinline__ void begin(int) {}
+  __device__ __forceinline__ Dual at(int k, size_t plane, size_t idx, int, int) const {
+    return Dual(v[k * plane + idx], d[k * plane + idx]);
+  }
+};
+
+// One coloured direction: tangent 1 in component m of the cells of colour
+// (a, b) = (column, row) mod per, 0 elsewhere.  A launch takes every
+// direction in its grid's third dimension.  per = 5 separates the 13-point
+// stencil (reach 2), per = 3 the 3x3 box (reach 1).
+struct Direction {
+  int per, nv;
+  int a = 0, b = 0, m = 0;
+  __host__ __device__ int count() const { return per * per * nv; }
+  __device__ __forceinline__ void begin(int z) {
+    m = z % nv;
+    b = z / nv % per;
+    a = z / nv / per;
+  }
+};
+struct SeedField {
+  const double* v;
+  Direction dir;
+  __device__ __forceinline__ void begin(int z) { dir.begin(z); }
+  __device__ __forceinline__ Dual at(int k, size_t plane, size_t idx, int ci, int cj) const {
+    const bool on = k == dir.m && ci % dir.per == dir.a && cj % dir.per == dir.b;
+    return Dual(v[k * plane + idx], on ? 1.0 : 0.0);
+  }
 };
 
 template <class S>
@@ -160,7 +189,10 @@ struct OutField;
 template <>
 struct OutField<double> {
   double* v;
-  __device__ __forceinline__ void put(size_t comp, size_t cell, double x) const { v[comp + cell] = x; }
+  __device__ __forceinline__ void begin(int) {}
+  __device__ __forceinline__ void put(int k, size_t plane, size_t idx, int, int, double x) const {
+    v[k * plane + idx] = x;
+  }
 };
 template <>
 struct OutField<Dual> {
@@ -169,9 +201,35 @@ struct OutField<Dual> {
   // with idt (per cell), d receives z idt - tangent: the operator z/dt - J z
   const double* idt = nullptr;
   const double* z = nullptr;
-  __device__ __forceinline__ void put(size_t comp, size_t cell, Dual x) const {
-    if (v) v[comp + cell] = x.v;
-    d[comp + cell] = idt ? z[comp + cell] * idt[cell] - x.d : x.d;
+  __device__ __forceinline__ void begin(int) {}
+  __device__ __forceinline__ void put(int k, size_t plane, size_t idx, int, int, Dual x) const {
+    if (v) v[k * plane + idx] = x.v;
+    d[k * plane + idx] = idt ? z[k * plane + idx] * idt[idx] - x.d : x.d;
+  }
+};
+
+// Jacobian blocks from coloured directions: the tangent at row cell r is
+// column m of the block J[r, c] for the one cell c of the direction's colour
+// in r's per x per window.  blocks[((slot nv + row) nv + col) plane + cell];
+// slots are the 3x3 box, then (0,-+2) and (-+2,0).
+struct OutBlocks {
+  double* blocks;
+  Direction dir;
+  __device__ __forceinline__ void begin(int z) { dir.begin(z); }
+  __device__ __forceinline__ void put(int k, size_t plane, size_t idx, int ci, int cj, Dual x) const {
+    const int h = dir.per / 2;
+    int di = (dir.a - ci) % dir.per, dj = (dir.b - cj) % dir.per;
+    di += di < -h ? dir.per : 0;
+    di -= di > h ? dir.per : 0;
+    dj += dj < -h ? dir.per : 0;
+    dj -= dj > h ? dir.per : 0;
+    const bool box = di >= -1 && di <= 1 && dj >= -1 && dj <= 1;
+    // (dj, di) of the box in rows -1, 0, 1, four bits each
+    constexpr unsigned long long kBox = 0x827403615ull;  // (1,1)8 (0,1)2 (-1,1)7 (1,0)4 (0,0)0 (-1,0)3 (1,-1)6 (0,-1)1 (-1,-1)5
+    int slot = box ? (int)(kBox >> (4 * (3 * (dj + 1) + di + 1))) & 15 : -1;
+    if (!box && di == 0) slot = dj < 0 ? 9 : 10;
+    if (!box && dj == 0) slot = di < 0 ? 11 : 12;
+    if (slot >= 0) blocks[(size_t)((slot * dir.nv + k) * dir.nv + dir.m) * plane + idx] = x.d;
   }
 };
 

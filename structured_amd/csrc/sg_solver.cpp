@@ -104,6 +104,9 @@ int ensure(sg_ctx* ctx, int restart) {
     return sg_fail(ctx, SG_ERR_HIP, "solver allocation failed");
   for (DevBuf* b : {&S->V, &S->Z, &S->blocks, &S->fac, &S->dtv, &S->rhs, &S->x, &S->tmp, &S->jz, &S->qop, &S->seed})
     if (hipMemset(b->p, 0, b->n * sizeof(double)) != hipSuccess) return sg_fail(ctx, SG_ERR_HIP, "memset");
+  // seed stays zero and ones one: the directions of dR/dbeta
+  const std::vector<double> one(ctx->g.plane, 1.0);
+  SG_TRY(hipMemcpy(S->ones.p, one.data(), one.size() * sizeof(double), hipMemcpyHostToDevice), "H2D");
   SG_TRY(reduce_slots_init(S->partial.p, S->partial.n, ctx->stream), "reduction slots");
   return SG_OK;
 }
@@ -184,20 +187,13 @@ int extract_jacobian(sg_ctx* ctx, int order = 0, double* dst = nullptr) {
   if (order > 0) ph.order = order;
   if (!dst) dst = ctx->solver->blocks.p;
   SolverState* S = ctx->solver;
-  const int nic = ctx->geo.nic, njc = ctx->geo.njc, ldi = ctx->g.ldi, nv = ctx->nvar;
+  const int nv = ctx->nvar;
   const int per = (ph.order == 1 && ctx->bcc.local_box) ? 3 : 5;
   if (per == 3) {  // slots 9-12 hold the (0,+-2) and (+-2,0) blocks
     const size_t slot = (size_t)nv * nv * ctx->g.plane;
     SG_TRY(zero_fill(dst + 9 * slot, 4 * slot, ctx->stream), "zero");
   }
-  for (int a = 0; a < per; ++a)
-    for (int b = 0; b < per; ++b)
-      for (int m = 0; m < nv; ++m) {
-        SG_TRY(seed_colour(nic, njc, ldi, nv, per, a, b, m, S->seed.p, ctx->stream), "seed");
-        SG_TRY(launch_jv(ctx->g, ph, ctx->bc, ctx->sa, S->qop.p, S->seed.p, nullptr, S->jz.p, ctx->stream, nullptr,
-                         ctx->clo), "jv");
-        SG_TRY(extract_blocks(nic, njc, ldi, nv, per, a, b, m, S->jz.p, dst, ctx->stream), "extract");
-      }
+  SG_TRY(launch_blocks(ctx->g, ph, ctx->bc, ctx->sa, S->qop.p, per, dst, ctx->stream, ctx->clo), "blocks");
   return SG_OK;
 }
 
@@ -712,12 +708,8 @@ int adjoint_prepare(sg_ctx* ctx, const double* q_dev) {
   SG_TRY(hipMemcpyAsync(S->qop.p, q_dev, S->n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream), "copy");
   if ((rc = extract_jacobian(ctx))) return rc;
   if (ctx->sa) {
-    SG_TRY(hipMemsetAsync(S->seed.p, 0, S->n * sizeof(double), ctx->stream), "memset");
-    std::vector<double> one(ctx->g.plane, 1.0);
-    SG_TRY(hipMemcpyAsync(S->ones.p, one.data(), one.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream), "H2D");
     SG_TRY(launch_jv(ctx->g, ctx->ph, ctx->bc, true, S->qop.p, S->seed.p, nullptr, S->dbdiag.p, ctx->stream, S->ones.p),
            "dbeta");
-    SG_TRY(hipStreamSynchronize(ctx->stream), "sync");
   }
   return SG_OK;
 }
