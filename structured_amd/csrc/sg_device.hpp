@@ -5,11 +5,9 @@
 #include <cstddef>
 
 namespace sg {
-// Arrival counters of the fused norm: one per group of residual tiles
-// (kNormGroups, tile index modulo kNormGroups: the XCD the tile runs on) and
-// one for the groups, each on its own 128-byte line; 64-bit words.
-constexpr int kNormGroups = 8, kNormLineWords = 16;
-constexpr int kNormStateWords = (kNormGroups + 1) * kNormLineWords;
+// An empty slot of a reduction across work-groups: a signalling NaN, which no
+// arithmetic produces.
+constexpr unsigned long long kNoValue = 0x7FF4534C4F545321ull;
 }  // namespace sg
 
 namespace sg {
@@ -29,6 +27,13 @@ struct DevGeom {
   const double* wd;          // wall distance (SA)
   const double* beta;        // SA production multiplier
 };
+
+// Tiles of the residual kernel: TX x TY faces, (TX - 1) x (TY - 1) cells.
+constexpr int TX = 32, OX = TX - 1;
+constexpr int kTileSmall = 8, kTileLarge = 16;  // TY
+inline __host__ __device__ int residual_tiles(const DevGeom& g, int ty) {
+  return ((g.nic + OX - 1) / OX) * ((g.njc + ty - 2) / (ty - 1));
+}
 
 struct DevPhys {
   double rho_inf, u_inf, v_inf, p_inf, T_inf, mu_inf, pr, nut_inf;
@@ -108,11 +113,16 @@ __device__ __forceinline__ double dpp_move(double v) {
   const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROW_MASK, 0xF, false);
   return __hiloint2double(hi, lo);
 }
-__device__ __forceinline__ double wave_sum_lane63(double v) {
+// Sum over each row of 16 lanes, in all of them.
+__device__ __forceinline__ double row_sum(double v) {
   v += dpp_move<0xB1>(v);        // quad_perm [1,0,3,2]
   v += dpp_move<0x4E>(v);        // quad_perm [2,3,0,1]
   v += dpp_move<0x141>(v);       // row_half_mirror
   v += dpp_move<0x140>(v);       // row_mirror
+  return v;
+}
+__device__ __forceinline__ double wave_sum_lane63(double v) {
+  v = row_sum(v);
   v += dpp_move<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
   v += dpp_move<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
   return v;

@@ -3,68 +3,90 @@
 // layout conversion, wall quantities).  Everything is FP64.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "sg_kernels.hpp"
 #include "sg_residual.hpp"
 
 namespace sg {
 
-namespace {
-inline dim3 tile_grid(const DevGeom& g) { return dim3((g.nic + OX - 1) / OX, (g.njc + OY - 1) / OY); }
-}  // namespace
-
-size_t residual_partial_count(const DevGeom& g) {
-  dim3 gr = tile_grid(g);
-  return (size_t)gr.x * gr.y;
+// Rows so long (some 27 million columns) that the rows a tile reads span more
+// than 32-bit byte offsets can.
+static bool wide_rows(const DevGeom& g) {
+  return (size_t)(kTileLarge + 4) * (size_t)std::max(g.ldi, g.ldf) * sizeof(double) > 0xFFFFFFFFull;
 }
 
-template <class S, bool SA, class F, class O>
-static void launch_cl(dim3 grid, hipStream_t s, const DevGeom& g, const DevPhys& ph, const DevBc& bc, F fq, O fo, double* partial, const double* beta_dot, const DevClosure& clo,
-                      NormOut no = NormOut{nullptr, nullptr, 0, 0u}) {
+// Tile height by the size of the grid.  Tiles of 16 rows of faces (512
+// threads) recompute 10% of the faces and stage 43% more cells than they own;
+// tiles of 8 rows 18% and 77%.  But the launch takes as long as the CU with
+// the most work-groups, and a work-group of 16 rows takes twice as long as one
+// of 8 (dual numbers 2.2 times: one of 16 rows or two of 8 fill the CU's
+// registers, and the one has nothing to run at its barriers).  Measured, 16
+// against 8 rows, SA residual: 67 / 75 us at 1409x641, 22 / 25 at 705x321,
+// equal at 545x385, 20.5 / 18 at 481x257, 15.7 / 14.7 at 449x225; J.v: 32 / 36
+// at 705x321, 32 / 30 at 545x385, 76 / 68 at 1001x501.
+// With a coloured direction per z-layer the chip is full and the larger tile is
+// 4% faster (J^T psi at 385x193: 1.91 / 1.99 ms).
+template <class S>
+static int tile_rows(const DevGeom& g) {
+  constexpr int kCUs = 256, kRatio = sizeof(S) == sizeof(double) ? 20 : 22;  // tenths
+  const int small = (residual_tiles(g, kTileSmall) + kCUs - 1) / kCUs;
+  const int large = (residual_tiles(g, kTileLarge) + kCUs - 1) / kCUs;
+  return !wide_rows(g) && kRatio * large < 10 * small ? kTileLarge : kTileSmall;
+}
+
+size_t residual_partial_count(const DevGeom& g) { return (size_t)residual_tiles(g, tile_rows<double>(g)); }
+
+template <int TY, class I, class S, bool SA, class F, class O>
+static void launch_tiles(unsigned extra, unsigned nz, hipStream_t s, const DevGeom& g, const DevPhys& ph, const DevBc& bc, F fq, O fo,
+                         const double* beta_dot, const DevClosure& clo, NormOut no) {
+  const dim3 grid((unsigned)residual_tiles(g, TY) + extra, 1, nz), block(TX * TY);
   if constexpr (SA) {
     if (clo.kind == CLOSURE_ANALYTIC) {
-      hipLaunchKernelGGL((residual_kernel<S, SA, CLOSURE_ANALYTIC, F, O>), grid, dim3(NT), 0, s, g, ph, bc, fq, fo, partial,
+      hipLaunchKernelGGL((residual_kernel<TY, I, S, SA, CLOSURE_ANALYTIC, F, O>), grid, block, 0, s, g, ph, bc, fq, fo,
                          beta_dot, clo, no);
       return;
     }
     if (clo.kind == CLOSURE_MLP) {
-      hipLaunchKernelGGL((residual_kernel<S, SA, CLOSURE_MLP, F, O>), grid, dim3(NT), 0, s, g, ph, bc, fq, fo, partial,
-                         beta_dot, clo, no);
+      hipLaunchKernelGGL((residual_kernel<TY, I, S, SA, CLOSURE_MLP, F, O>), grid, block, 0, s, g, ph, bc, fq, fo, beta_dot,
+                         clo, no);
       return;
     }
   }
-  hipLaunchKernelGGL((residual_kernel<S, SA, CLOSURE_FIELD, F, O>), grid, dim3(NT), 0, s, g, ph, bc, fq, fo, partial,
-                       beta_dot, clo, no);
+  hipLaunchKernelGGL((residual_kernel<TY, I, S, SA, CLOSURE_FIELD, F, O>), grid, block, 0, s, g, ph, bc, fq, fo, beta_dot,
+                     clo, no);
+}
+template <class S, bool SA, class F, class O>
+static void launch_cl(hipStream_t s, const DevGeom& g, const DevPhys& ph, const DevBc& bc, F fq, O fo,
+                      const double* beta_dot, const DevClosure& clo, NormOut no = NormOut{nullptr, nullptr, 0},
+                      unsigned nz = 1) {
+  const unsigned extra = no.slots ? 1 : 0;  // the work-group that sums the norms
+  if (wide_rows(g)) launch_tiles<kTileSmall, size_t, S, SA>(extra, nz, s, g, ph, bc, fq, fo, beta_dot, clo, no);
+  else if (nz > 1 || tile_rows<S>(g) == kTileLarge)
+    launch_tiles<kTileLarge, unsigned, S, SA>(extra, nz, s, g, ph, bc, fq, fo, beta_dot, clo, no);
+  else launch_tiles<kTileSmall, unsigned, S, SA>(extra, nz, s, g, ph, bc, fq, fo, beta_dot, clo, no);
 }
 
 hipError_t launch_residual(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool sa, const double* q, double* r,
-                           double* partial, unsigned long long* counter, double* l2, hipStream_t s, const DevClosure& clo,
-                           int l2_count, unsigned* parity) {
-  dim3 grid = tile_grid(g);
-  Field<double> fq{q};
-  OutField<double> fo{r};
+                           double* slots, double* l2, hipStream_t s, const DevClosure& clo, int l2_count) {
+  if ((l2 != nullptr) != (slots != nullptr)) return hipErrorInvalidValue;
   const int nv2 = 2 * (sa ? 5 : 4);
   if (l2_count <= 0 || l2_count > nv2) l2_count = nv2;
-  // the norms are finalised inside the residual kernel; partials without a
-  // state pair and a norm buffer are not a supported combination
-  if ((l2 != nullptr) != (partial != nullptr && counter != nullptr && parity != nullptr) || (partial && !l2))
-    return hipErrorInvalidValue;
-  const NormOut no{counter, l2, l2_count, parity ? *parity : 0u};
-  if (sa) launch_cl<double, true>(grid, s, g, ph, bc, fq, fo, partial, nullptr, clo, no);
-  else launch_cl<double, false>(grid, s, g, ph, bc, fq, fo, partial, nullptr, DevClosure(), no);
-  const hipError_t e = hipGetLastError();
-  // the next fused launch on these partials uses the other parity
-  if (e == hipSuccess && l2) *parity ^= 1u;
-  return e;
+  Field<double> fq{q};
+  OutField<double> fo{r};
+  const NormOut no{reinterpret_cast<unsigned long long*>(slots), l2, l2_count};
+  if (sa) launch_cl<double, true>(s, g, ph, bc, fq, fo, nullptr, clo, no);
+  else launch_cl<double, false>(s, g, ph, bc, fq, fo, nullptr, DevClosure(), no);
+  return hipGetLastError();
 }
 
 hipError_t launch_jv(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool sa, const double* q, const double* v,
                      double* r, double* jv, hipStream_t s, const double* beta_dot, const DevClosure& clo,
                      const double* idt) {
-  dim3 grid = tile_grid(g);
   Field<Dual> fq{q, v};
   OutField<Dual> fo{r, jv, idt, v};
-  if (sa) launch_cl<Dual, true>(grid, s, g, ph, bc, fq, fo, nullptr, beta_dot, clo);
-  else launch_cl<Dual, false>(grid, s, g, ph, bc, fq, fo, nullptr, nullptr, DevClosure());
+  if (sa) launch_cl<Dual, true>(s, g, ph, bc, fq, fo, beta_dot, clo);
+  else launch_cl<Dual, false>(s, g, ph, bc, fq, fo, nullptr, DevClosure());
   return hipGetLastError();
 }
 
@@ -79,12 +101,12 @@ hipError_t launch_blocks(const DevGeom& g, const DevPhys& ph, const DevBc& bc, b
                          double* blocks, hipStream_t s, const DevClosure& clo) {
   if (per != 3 && per != 5) return hipErrorInvalidValue;
   const Direction d{per, sa ? 5 : 4};
-  dim3 grid = tile_grid(g);
-  grid.z = (unsigned)d.count();
   const SeedField fq{q, d};
   const OutBlocks fo{blocks, d};
-  if (sa) launch_cl<Dual, true>(grid, s, g, ph, bc, fq, fo, nullptr, nullptr, clo);
-  else launch_cl<Dual, false>(grid, s, g, ph, bc, fq, fo, nullptr, nullptr, DevClosure());
+  const unsigned nz = (unsigned)d.count();
+  const NormOut no{nullptr, nullptr, 0};
+  if (sa) launch_cl<Dual, true>(s, g, ph, bc, fq, fo, nullptr, clo, no, nz);
+  else launch_cl<Dual, false>(s, g, ph, bc, fq, fo, nullptr, DevClosure(), no, nz);
   return hipGetLastError();
 }
 

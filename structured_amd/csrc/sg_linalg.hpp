@@ -4,13 +4,12 @@
 
 #include <cstddef>
 
+#include "sg_device.hpp"
+
 namespace sg {
 
 constexpr int NSLOT = 13;  // Jacobian stencil blocks kept per cell
 
-// What a 64-bit slot holds while it has no value: a signalling NaN, which no
-// arithmetic produces.
-constexpr unsigned long long kNoValue = 0x7FF4534C4F545321ull;
 // 64-bit slots of the reductions below, which every call finds and leaves
 // empty; reduce_slots_init empties them first.
 size_t reduce_slots(int kmax);

@@ -11,14 +11,24 @@
 // ConvectiveFluxAUSM (:149-224), Mesh::calc_gradient / calc_face
 // (src/utils/mesh.cpp:8-131) and DiffusiveFluxGreenGauss (src/model/flux.cpp:12-48).
 //
-// Tiling.  A 256-thread block is a 32 x 8 grid of face owners: thread
-// (tx, ty) computes the chi face i0+tx on row j0+ty and the eta face j0+ty on
-// column i0+tx, so every thread evaluates exactly two faces.  The block then
-// assembles the 31 x 7 cells whose four faces it owns; tiles advance by
-// (31, 7), so one column and one row of faces per tile are computed twice.
-// The cell data of the tile plus its halo (two cells along each face normal
-// for MUSCL, one cell around for the viscous stencil) is staged once in LDS
-// as primitives and transport properties.
+// Tiling.  A block of TX x TY threads (32 x 8 or 32 x 16) is a grid of face
+// owners: thread (tx, ty) computes the chi face i0+tx on row j0+ty and the eta
+// face j0+ty on column i0+tx, so every thread evaluates exactly two faces.
+// The block then assembles the (TX - 1) x (TY - 1) cells whose four faces it
+// owns, so one column and one row of faces per tile are computed twice.  The
+// cell data of the tile plus its halo (two cells along each face normal for
+// MUSCL, one cell around for the viscous stencil) is staged once in LDS as
+// primitives and transport properties.
+//
+// Bound.  FP64 issue on large grids (two thirds of the vector instructions are
+// FP64, the rest address, select and move), the chain load - stage - barrier -
+// faces - barrier - cell - norms on small ones.  Both want few branches: the
+// ends of grid lines are handled by clamped indices and selects, where a
+// branch per variable and per kind of face kept the loads of a face behind one
+// another and cost a third of the instructions that are not FP64; ghost cells
+// are evaluated once, by threads of their own.  With it and a finaliser that
+// waits on slots instead of counting arrivals, SA at 545x385 24.0 -> 21.6 us,
+// 1409x641 76 -> 68, laminar 97x65 16.4 -> 9.0; J.v at 705x321 41.5 -> 32.7.
 #pragma once
 #include "sg_closure.hpp"
 #include "sg_device.hpp"
@@ -26,10 +36,7 @@
 
 namespace sg {
 
-constexpr int TX = 32, TY = 8, NT = TX * TY;
-constexpr int RW = TX + 3, RH = TY + 3, NPOS = RW * RH;  // LDS region, origin (i0-2, j0-2)
-constexpr int OX = TX - 1, OY = TY - 1;                    // output cells per tile
-
+constexpr int RW = TX + 3;           // LDS region, origin (i0-2, j0-2)
 template <class S>
 struct Prim {
   S r, u, v, p, T, n;
@@ -350,32 +357,70 @@ __device__ __forceinline__ SaTerms<S> sa_terms(S r, S n, S ml, const S* gu, cons
   return t;
 }
 
-// Fused norm output: with l2 set, the block that finishes last finalises the
-// norms.  state holds the arrival counters (kNormStateWords words: one per
-// tile group, then the count of groups done; all 0 between launches); parity
-// alternates between consecutive fused launches on the same partials.
+// Fused norm output.  With slots set the launch has one more block, the last,
+// which waits for every tile's partial sums, adds them in a fixed order and
+// empties the slots for the next launch.  A slot is one 64-bit atomic that
+// holds either a partial sum or kNoValue (a signalling NaN that no arithmetic
+// produces), so nothing has to be ordered between slots.  The tiles depend on
+// nothing, so the wait ends; past kNormPolls the norms are NaN.
 struct NormOut {
-  unsigned long long* state;
-  double* l2;         // ||R_k||_2 (k < NV), then ||V R_k||_2 (NV <= k < 2 NV)
-  int count;          // entries of l2 written: NV (caller's buffer) or 2 NV
-  unsigned parity;
+  unsigned long long* slots;  // 2 NV per tile, component-major; all empty between launches
+  double* l2;                 // ||R_k||_2 (k < NV), then ||V R_k||_2 (NV <= k < 2 NV)
+  int count;                  // entries of l2 written: NV (caller's buffer) or 2 NV
 };
+constexpr int kNormPolls = 1 << 22;
 
-// Spin budget of the finalising block per thread (polls beyond the first
-// load of each partial); past it the norms are written as NaN.
-constexpr int kNormSpinLimit = 1 << 22;
+template <int NT, int NV2>
+__device__ __forceinline__ void finalise_norms(const NormOut& no, int ntile, double (*red)[NV2]) {
+  const int tid = threadIdx.x;
+  double acc[NV2];
+#pragma unroll
+  for (int k = 0; k < NV2; ++k) acc[k] = 0.0;
+  int polls = 0;
+  for (int b = tid; b < ntile; b += NT) {
+    unsigned long long v[NV2];
+    bool wait = true;
+    while (wait) {  // every sum of the tile again, all loads in flight together
+#pragma unroll
+      for (int k = 0; k < NV2; ++k)
+        v[k] = k < no.count ? __hip_atomic_load(no.slots + (size_t)k * ntile + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                            : 0ull;
+      wait = false;
+#pragma unroll
+      for (int k = 0; k < NV2; ++k) wait = wait || v[k] == kNoValue;
+      if (wait && ++polls > kNormPolls) break;
+    }
+#pragma unroll
+    for (int k = 0; k < NV2; ++k) {
+      if (k < no.count) __hip_atomic_store(no.slots + (size_t)k * ntile + b, kNoValue, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      acc[k] += wait ? __builtin_nan("") : __longlong_as_double((long long)v[k]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < NV2; ++k) acc[k] = wave_sum_lane63(acc[k]);
+  if ((tid & 63) == 63) {
+#pragma unroll
+    for (int k = 0; k < NV2; ++k) red[tid >> 6][k] = acc[k];
+  }
+  __syncthreads();
+  if (tid < no.count) {
+    double s = 0.0;
+    for (int w = 0; w < NT / 64; ++w) s += red[w][tid];
+    no.l2[tid] = sqrt(s);
+  }
+}
 
 // CL: closure kind of beta (ClosureKind); CLOSURE_MLP stages the hidden
 // layer of the network (and its tangent) in the same LDS area.  F and O: where
 // the state comes from and the result goes (Field and OutField, or SeedField
 // and OutBlocks for Jacobian blocks).
-template <class S, bool SA, int CL, class F = Field<S>, class O = OutField<S>>
-__global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) void residual_kernel(DevGeom g, DevPhys ph, DevBc bc, F q, O out,
-                                                       double* partial, const double* beta_dot, DevClosure clo,
-                                                       NormOut nout) {
+template <int TY, class I, class S, bool SA, int CL, class F, class O>
+__global__ __launch_bounds__(TX * TY, sizeof(S) == sizeof(double) ? 4 : 2) void residual_kernel(
+    DevGeom g, DevPhys ph, DevBc bc, F q, O out, const double* beta_dot, DevClosure clo, NormOut nout) {
+  constexpr int NT = TX * TY, OY = TY - 1, RH = TY + 3, NPOS = RW * RH;
   constexpr int NL = SA ? L_MAX : (L_K + 1);
   constexpr int NV = SA ? 5 : 4;
-  constexpr int NLDS0 = NL * NPOS > 2 * NV * NT ? NL * NPOS : 2 * NV * NT;
+  constexpr int NLDS0 = NL * NPOS > 2 * NV * (NT + 16) ? NL * NPOS : 2 * NV * (NT + 16);  // cells, then fluxes, then sums
   constexpr int NLDS_D = NLDS0 * (int)(sizeof(S) / sizeof(double));
   constexpr bool TAN = sizeof(S) > sizeof(double);
   constexpr int NMLP_D = (CL == CLOSURE_MLP) ? (TAN ? 2 : 1) * (NT / 64) * 64 * kHld / 4 : 0;
@@ -383,6 +428,13 @@ __global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) vo
   S* lds = reinterpret_cast<S*>(lds_raw);
   __shared__ double red[NT / 64][2 * NV];
 
+  const int ncol = (g.nic + OX - 1) / OX, ntile = residual_tiles(g, TY);
+  int tile = blockIdx.x;
+  if (tile == ntile) {
+    finalise_norms<NT, 2 * NV>(nout, ntile, red);
+    return;
+  }
+  const int bid = tile;
   q.begin(blockIdx.z);
   out.begin(blockIdx.z);
   const int tid = threadIdx.x;
@@ -391,15 +443,35 @@ __global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) vo
   // linear order, so XCD x's k-th group takes the k-th tile of the x-th
   // contiguous run of tiles; neighbouring tiles then share their halo rows in
   // the same L2.  The map is a bijection on the tiles for any tile count.
-  int tile = blockIdx.y * gridDim.x + blockIdx.x;
   {
-    const int N = gridDim.x * gridDim.y, x = tile & 7, k = tile >> 3, qn = N >> 3, rn = N & 7;
+    const int x = tile & 7, k = tile >> 3, qn = ntile >> 3, rn = ntile & 7;
     tile = (x < rn) ? x * (qn + 1) + k : rn * (qn + 1) + (x - rn) * qn + k;
   }
-  const int i0 = (tile % gridDim.x) * OX, j0 = (tile / gridDim.x) * OY;
+  const int trow = tile / ncol, i0 = (tile - trow * ncol) * OX, j0 = trow * OY;
   const int nic = g.nic, njc = g.njc;
-  const double nan = __builtin_nan("");
-  const bool fused = partial && nout.l2;
+
+  const int jo = max(j0 - 2, 0), io = max(i0 - 2, 0);
+
+  // ---- ghost cells of the ring around the grid that lie in this tile's
+  // region: at most RW on a row and RH on a column, one thread each.  The
+  // threads counted from the end take them, since the first waves have the
+  // second pass of the staging.  The boundary node is asked for first; what it
+  // reads is two dependent loads away.
+  static_assert(2 * (RW + RH) <= NT, "a thread per ghost cell");
+  int gp = -1, node = -1;
+  {
+    const int t = NT - 1 - tid;
+    int lx, ly;
+    if (t < 2 * RW) { lx = t < RW ? t : t - RW; ly = t < RW ? 1 - j0 : njc - j0 + 2; }
+    else { const int u = t - 2 * RW; ly = u < RH ? u : u - RH; lx = u < RH ? 1 - i0 : nic - i0 + 2; }
+    const int ci = i0 - 2 + lx, cj = j0 - 2 + ly;
+    // a corner belongs to the row
+    if (t < 2 * (RW + RH) && lx >= 0 && lx < RW && ly >= 0 && ly < RH && ci >= -1 && ci <= nic && cj >= -1 && cj <= njc &&
+        (t < 2 * RW || (cj >= 0 && cj < njc))) {
+      gp = ly * RW + lx;
+      node = bc.ghost_map[ghost_index(ci, cj, nic, njc)];
+    }
+  }
 
   // ---- stage primitives (+ transport properties) of tile + halo in LDS.
   // A thread stages at most NPASS positions; the conservative values of its
@@ -407,19 +479,26 @@ __global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) vo
   // then converted.
   constexpr int NPASS = (NPOS + NT - 1) / NT;
   constexpr int NQ = SA ? 5 : 4;
+  auto stage = [&](int p, int lx, int ly, const Prim<S>& P) {
+    lds[L_R * NPOS + p] = P.r; lds[L_U * NPOS + p] = P.u; lds[L_V * NPOS + p] = P.v; lds[L_P * NPOS + p] = P.p;
+    lds[L_T * NPOS + p] = P.T;
+    if (SA) lds[L_N * NPOS + p] = P.n;
+    // the viscous stencil reads transport properties one cell around only
+    if (ph.viscous && lx >= 1 && lx < RW - 1 && ly >= 1 && ly < RH - 1) {
+      S slot[L_MAX];
+      transport<S, SA>(P, ph, slot);
+      lds[L_MU * NPOS + p] = slot[L_MU]; lds[L_K * NPOS + p] = slot[L_K];
+      if (SA) { lds[L_ETA * NPOS + p] = slot[L_ETA]; lds[L_ML * NPOS + p] = slot[L_ML]; }
+    }
+  };
   S qraw[NPASS][NQ];
 #pragma unroll
   for (int pass = 0; pass < NPASS; ++pass) {
     const int p = tid + pass * NT;
     const int ci = i0 - 2 + p % RW, cj = j0 - 2 + p / RW;
-    const bool interior = p < NPOS && ci >= 0 && ci < nic && cj >= 0 && cj < njc;
-#pragma unroll
-    for (int k = 0; k < NQ; ++k) qraw[pass][k] = S(0.0);
-    if (interior) {
-      const size_t idx = (size_t)cj * g.ldi + ci;
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) qraw[pass][k] = q.at(k, g.plane, idx, ci, cj);
-    }
+    // positions outside the grid load the nearest cell and do not use it
+    const int cc = min(max(ci, 0), nic - 1), cr = min(max(cj, 0), njc - 1);
+    if (p < NPOS) q.template load<NQ, I>(qraw[pass], g.plane, g.ldi, jo, io, cc, cr);
   }
 #pragma unroll
   for (int pass = 0; pass < NPASS; ++pass) {
@@ -427,164 +506,143 @@ __global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) vo
     if (p >= NPOS) break;
     const int lx = p % RW, ly = p / RW;
     const int ci = i0 - 2 + lx, cj = j0 - 2 + ly;
-    S slot[L_MAX];
-    const bool interior = ci >= 0 && ci < nic && cj >= 0 && cj < njc;
-    const bool ring = !interior && ci >= -1 && ci <= nic && cj >= -1 && cj <= njc;
-    int node = -1;
-    if (ring) node = bc.ghost_map[ghost_index(ci, cj, nic, njc)];
-    if (interior || node >= 0) {
-      Prim<S> P = interior ? prim_from_cons<S, SA>(qraw[pass], ph) : eval_node<S, SA>(node, bc, q, g, ph);
-      slot[L_R] = P.r; slot[L_U] = P.u; slot[L_V] = P.v; slot[L_P] = P.p; slot[L_T] = P.T;
-      if (SA) slot[L_N] = P.n;
-      const bool box = lx >= 1 && lx < RW - 1 && ly >= 1 && ly < RH - 1;
-      if (ph.viscous && box) transport<S, SA>(P, ph, slot);
-      else { slot[L_MU] = S(nan); slot[L_K] = S(nan); if (SA) { slot[L_ETA] = S(nan); slot[L_ML] = S(nan); } }
-    } else {
-#pragma unroll
-      for (int k = 0; k < L_MAX; ++k) slot[k] = S(nan);
-    }
-#pragma unroll
-    for (int k = 0; k < NL; ++k) lds[k * NPOS + p] = slot[k];
+    if (ci < 0 || ci >= nic || cj < 0 || cj >= njc) continue;
+    stage(p, lx, ly, prim_from_cons<S, SA>(qraw[pass], ph));
   }
+  if (gp >= 0) {
+    const S nan(__builtin_nan(""));
+    Prim<S> P{nan, nan, nan, nan, nan, nan};
+    if (node >= 0) P = eval_node<S, SA>(node, bc, q, g, ph);
+    stage(gp, gp % RW, gp / RW, P);
+  }
+  // ---- metrics of this thread's two faces and cell, in flight over the barrier and
+  // the reconstruction.  At the ends of a grid
+  // line the neighbour index is clamped: the mean of a face's normal (a
+  // cell's volume) with itself is the one-sided value that belongs there,
+  // and a thread without a face computes one that nothing reads.
+  const int fi = i0 + tx, cj = j0 + ty;  // the chi face's row is the eta face's upper cell
+  double2 C0, CL_, CR, Cb, CRb, E0, EL, Et, ELt, Eb;
+  double V0, VL, VB;
+  const int f0 = min(fi, nic), fr = min(f0 + 1, nic), c0 = min(fi, nic - 1);
+  const int e0 = min(cj, njc), eb = max(e0 - 1, 0);
+  auto nc = [&](int f, int r) { return double2{tile_at<I>(g.ncx, g.ldf, jo, io, f, r), tile_at<I>(g.ncy, g.ldf, jo, io, f, r)}; };
+  auto ne = [&](int c, int r) { return double2{tile_at<I>(g.nex, g.ldi, jo, io, c, r), tile_at<I>(g.ney, g.ldi, jo, io, c, r)}; };
+  auto vol = [&](int c, int r) { return tile_at<I>(g.vol, g.ldi, jo, io, c, r); };
+  {
+    const int fl = max(f0 - 1, 0), cl = min(fl, c0), r0 = min(cj, njc - 1), et = min(e0 + 1, njc);
+    C0 = nc(f0, r0); CL_ = nc(fl, r0); CR = nc(fr, r0);
+    E0 = ne(c0, e0); EL = ne(cl, e0); Et = ne(c0, et); ELt = ne(cl, et);
+    V0 = vol(c0, r0); VL = vol(cl, r0);
+  }
+
   __syncthreads();
 
   auto at = [&](int k, int lx, int ly) -> S { return lds[k * NPOS + ly * RW + lx]; };
-  auto ncx = [&](int fi, int cj) { return g.ncx[(size_t)cj * g.ldf + fi]; };
-  auto ncy = [&](int fi, int cj) { return g.ncy[(size_t)cj * g.ldf + fi]; };
-  auto nex = [&](int ci, int fj) { return g.nex[(size_t)fj * g.ldi + ci]; };
-  auto ney = [&](int ci, int fj) { return g.ney[(size_t)fj * g.ldi + ci]; };
-  auto vol = [&](int ci, int cj) { return g.vol[(size_t)cj * g.ldi + ci]; };
+
 
   S hc[NV], he[NV];
-#pragma unroll
-  for (int k = 0; k < NV; ++k) { hc[k] = S(0.0); he[k] = S(0.0); }
 
-  // ---- chi face fi = i0+tx on row cj = j0+ty (between cells fi-1 and fi)
+  // ---- chi face fi on row cj (between cells fi-1 and fi)
   {
-    const int fi = i0 + tx, cj = j0 + ty;
-    if (fi <= nic && cj < njc) {
-      const int xl = tx + 1, xr = tx + 2, y = ty + 2;  // LDS coords of the left/right cells
-      S st[2][5];
+    const int xl = tx + 1, xr = tx + 2, y = ty + 2;  // LDS coords of the left/right cells
+    S st[2][4];
+    const bool sl = fi >= 1, sr = fi <= nic - 1;  // first order from a ghost cell
+    if (ph.order == 2) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        S cl = at(L_R + k, xl, y), cr = at(L_R + k, xr, y);
-        if (ph.order == 2) {
-          st[0][k] = (fi >= 1) ? muscl_left(at(L_R + k, xl - 1, y), cl, cr, ph.eps_chi) : cl;
-          st[1][k] = (fi <= nic - 1) ? muscl_right(cl, cr, at(L_R + k, xr + 1, y), ph.eps_chi) : cr;
-        } else {
-          st[0][k] = cl; st[1][k] = cr;
-        }
+        const S cl = at(L_R + k, xl, y), cr = at(L_R + k, xr, y);
+        st[0][k] = ssel(sl, muscl_left(at(L_R + k, xl - 1, y), cl, cr, ph.eps_chi), cl);
+        st[1][k] = ssel(sr, muscl_right(cl, cr, at(L_R + k, xr + 1, y), ph.eps_chi), cr);
       }
-      S ntl(0.0), ntr(0.0);
-      if (SA) { ntl = at(L_N, xl, y); ntr = at(L_N, xr, y); }
-      const double nx = ncx(fi, cj), ny = ncy(fi, cj);
-      conv_flux<S, SA>(ph.flux, nx, ny, st[0][0], st[0][1], st[0][2], st[0][3], st[1][0], st[1][1], st[1][2], st[1][3],
-                       ntl, ntr, hc);
-      if (ph.viscous) {
-        FaceGeo<S> G;
-        if (fi == 0) {
-          G.tx = nex(0, cj + 1); G.ty = ney(0, cj + 1); G.bx = nex(0, cj); G.by = ney(0, cj);
-          G.rx = 0.5 * (ncx(0, cj) + ncx(1, cj)); G.ry = 0.5 * (ncy(0, cj) + ncy(1, cj));
-          G.lx = ncx(0, cj); G.ly = ncy(0, cj); G.ivol = frcp(vol(0, cj));
-        } else if (fi == nic) {
-          G.tx = nex(nic - 1, cj + 1); G.ty = ney(nic - 1, cj + 1); G.bx = nex(nic - 1, cj); G.by = ney(nic - 1, cj);
-          G.rx = ncx(nic, cj); G.ry = ncy(nic, cj);
-          G.lx = 0.5 * (ncx(nic, cj) + ncx(nic - 1, cj)); G.ly = 0.5 * (ncy(nic, cj) + ncy(nic - 1, cj));
-          G.ivol = frcp(vol(nic - 1, cj));
-        } else {
-          G.tx = 0.5 * (nex(fi, cj + 1) + nex(fi - 1, cj + 1)); G.ty = 0.5 * (ney(fi, cj + 1) + ney(fi - 1, cj + 1));
-          G.bx = 0.5 * (nex(fi, cj) + nex(fi - 1, cj)); G.by = 0.5 * (ney(fi, cj) + ney(fi - 1, cj));
-          G.rx = 0.5 * (ncx(fi, cj) + ncx(fi + 1, cj)); G.ry = 0.5 * (ncy(fi, cj) + ncy(fi + 1, cj));
-          G.lx = 0.5 * (ncx(fi, cj) + ncx(fi - 1, cj)); G.ly = 0.5 * (ncy(fi, cj) + ncy(fi - 1, cj));
-          G.ivol = frcp(0.5 * (vol(fi, cj) + vol(fi - 1, cj)));
-        }
-        // left/right cells and their north/south neighbours
-        auto grad_avg = [&](int k, S* gr, S* avg) {
-          S a = at(k, xl, y), b = at(k, xr, y);
-          S qt = 0.25 * (a + b + at(k, xl, y + 1) + at(k, xr, y + 1));
-          S qb = 0.25 * (a + b + at(k, xl, y - 1) + at(k, xr, y - 1));
-          if (gr) gg_grad(G, qt, qb, a, b, gr);
-          if (avg) *avg = 0.25 * (a + b + qt + qb);
-        };
-        S gu[2], gv[2], gT[2], gn[2] = {S(0.0), S(0.0)}, ub, vb, mb, kb, eb(0.0);
-        grad_avg(L_U, gu, &ub);
-        grad_avg(L_V, gv, &vb);
-        grad_avg(L_T, gT, nullptr);
-        grad_avg(L_MU, nullptr, &mb);
-        grad_avg(L_K, nullptr, &kb);
-        if (SA) { grad_avg(L_N, gn, nullptr); grad_avg(L_ETA, nullptr, &eb); }
-        S fv[5];
-        visc_flux<S, SA>(nx, ny, gu, gv, gT, ub, vb, mb, kb, gn, eb, fv);
+    } else {
 #pragma unroll
-        for (int k = 1; k < NV; ++k) hc[k] = hc[k] - fv[k];
-      }
+      for (int k = 0; k < 4; ++k) { st[0][k] = at(L_R + k, xl, y); st[1][k] = at(L_R + k, xr, y); }
+    }
+    S ntl(0.0), ntr(0.0);
+    if (SA) { ntl = at(L_N, xl, y); ntr = at(L_N, xr, y); }
+    conv_flux<S, SA>(ph.flux, C0.x, C0.y, st[0][0], st[0][1], st[0][2], st[0][3], st[1][0], st[1][1], st[1][2], st[1][3],
+                     ntl, ntr, hc);
+    if (ph.viscous) {
+      FaceGeo<S> G;
+      G.tx = 0.5 * (Et.x + ELt.x); G.ty = 0.5 * (Et.y + ELt.y);
+      G.bx = 0.5 * (E0.x + EL.x); G.by = 0.5 * (E0.y + EL.y);
+      G.rx = 0.5 * (C0.x + CR.x); G.ry = 0.5 * (C0.y + CR.y);
+      G.lx = 0.5 * (C0.x + CL_.x); G.ly = 0.5 * (C0.y + CL_.y);
+      G.ivol = frcp(0.5 * (V0 + VL));
+      // left/right cells and their north/south neighbours
+      auto grad_avg = [&](int k, S* gr, S* avg) {
+        S a = at(k, xl, y), b = at(k, xr, y);
+        S qt = 0.25 * (a + b + at(k, xl, y + 1) + at(k, xr, y + 1));
+        S qb = 0.25 * (a + b + at(k, xl, y - 1) + at(k, xr, y - 1));
+        if (gr) gg_grad(G, qt, qb, a, b, gr);
+        if (avg) *avg = 0.25 * (a + b + qt + qb);
+      };
+      S gu[2], gv[2], gT[2], gn[2] = {S(0.0), S(0.0)}, ub, vb, mb, kb, eb(0.0);
+      grad_avg(L_U, gu, &ub);
+      grad_avg(L_V, gv, &vb);
+      grad_avg(L_T, gT, nullptr);
+      grad_avg(L_MU, nullptr, &mb);
+      grad_avg(L_K, nullptr, &kb);
+      if (SA) { grad_avg(L_N, gn, nullptr); grad_avg(L_ETA, nullptr, &eb); }
+      S fv[5];
+      visc_flux<S, SA>(C0.x, C0.y, gu, gv, gT, ub, vb, mb, kb, gn, eb, fv);
+#pragma unroll
+      for (int k = 1; k < NV; ++k) hc[k] = hc[k] - fv[k];
     }
   }
 
-  // ---- eta face fj = j0+ty on column ci = i0+tx (between cells fj-1 and fj)
+  Cb = nc(f0, eb); CRb = nc(fr, eb); Eb = ne(c0, eb); VB = vol(c0, eb);
+
+  // ---- eta face fj on column ci (between cells fj-1 and fj)
   {
-    const int fj = j0 + ty, ci = i0 + tx;
-    if (fj <= njc && ci < nic) {
-      const int x = tx + 2, ys = ty + 1, yn = ty + 2;
-      S st[2][5];
+    const int x = tx + 2, ys = ty + 1, yn = ty + 2;
+    S st[2][4];
+    const bool sl = cj >= 1, sr = cj <= njc - 1;  // first order from a ghost cell
+    if (ph.order == 2) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        S cs = at(L_R + k, x, ys), cn = at(L_R + k, x, yn);
-        if (ph.order == 2) {
-          st[0][k] = (fj >= 1) ? muscl_left(at(L_R + k, x, ys - 1), cs, cn, ph.eps_eta) : cs;
-          st[1][k] = (fj <= njc - 1) ? muscl_right(cs, cn, at(L_R + k, x, yn + 1), ph.eps_eta) : cn;
-        } else {
-          st[0][k] = cs; st[1][k] = cn;
-        }
+        const S cl = at(L_R + k, x, ys), cr = at(L_R + k, x, yn);
+        st[0][k] = ssel(sl, muscl_left(at(L_R + k, x, ys - 1), cl, cr, ph.eps_eta), cl);
+        st[1][k] = ssel(sr, muscl_right(cl, cr, at(L_R + k, x, yn + 1), ph.eps_eta), cr);
       }
-      S nts(0.0), ntn(0.0);
-      if (SA) { nts = at(L_N, x, ys); ntn = at(L_N, x, yn); }
-      const double nx = nex(ci, fj), ny = ney(ci, fj);
-      conv_flux<S, SA>(ph.flux, nx, ny, st[0][0], st[0][1], st[0][2], st[0][3], st[1][0], st[1][1], st[1][2], st[1][3],
-                       nts, ntn, he);
-      if (ph.viscous) {
-        FaceGeo<S> G;
-        if (fj == 0) {
-          G.tx = 0.5 * (nex(ci, 0) + nex(ci, 1)); G.ty = 0.5 * (ney(ci, 0) + ney(ci, 1));
-          G.bx = nex(ci, 0); G.by = ney(ci, 0);
-          G.lx = ncx(ci, 0); G.ly = ncy(ci, 0); G.rx = ncx(ci + 1, 0); G.ry = ncy(ci + 1, 0);
-          G.ivol = frcp(vol(ci, 0));
-        } else if (fj == njc) {
-          G.tx = nex(ci, njc); G.ty = ney(ci, njc);
-          G.bx = 0.5 * (nex(ci, njc) + nex(ci, njc - 1)); G.by = 0.5 * (ney(ci, njc) + ney(ci, njc - 1));
-          G.lx = ncx(ci, njc - 1); G.ly = ncy(ci, njc - 1); G.rx = ncx(ci + 1, njc - 1); G.ry = ncy(ci + 1, njc - 1);
-          G.ivol = frcp(vol(ci, njc - 1));
-        } else {
-          G.tx = 0.5 * (nex(ci, fj) + nex(ci, fj + 1)); G.ty = 0.5 * (ney(ci, fj) + ney(ci, fj + 1));
-          G.bx = 0.5 * (nex(ci, fj) + nex(ci, fj - 1)); G.by = 0.5 * (ney(ci, fj) + ney(ci, fj - 1));
-          G.lx = 0.5 * (ncx(ci, fj) + ncx(ci, fj - 1)); G.ly = 0.5 * (ncy(ci, fj) + ncy(ci, fj - 1));
-          G.rx = 0.5 * (ncx(ci + 1, fj) + ncx(ci + 1, fj - 1)); G.ry = 0.5 * (ncy(ci + 1, fj) + ncy(ci + 1, fj - 1));
-          G.ivol = frcp(0.5 * (vol(ci, fj) + vol(ci, fj - 1)));
-        }
-        auto grad_avg = [&](int k, S* gr, S* avg) {
-          S t = at(k, x, yn), b = at(k, x, ys);
-          S l = 0.25 * (t + b + at(k, x - 1, yn) + at(k, x - 1, ys));
-          S r = 0.25 * (t + b + at(k, x + 1, yn) + at(k, x + 1, ys));
-          if (gr) gg_grad(G, t, b, l, r, gr);
-          if (avg) *avg = 0.25 * (l + r + t + b);
-        };
-        S gu[2], gv[2], gT[2], gn[2] = {S(0.0), S(0.0)}, ub, vb, mb, kb, eb(0.0);
-        grad_avg(L_U, gu, &ub);
-        grad_avg(L_V, gv, &vb);
-        grad_avg(L_T, gT, nullptr);
-        grad_avg(L_MU, nullptr, &mb);
-        grad_avg(L_K, nullptr, &kb);
-        if (SA) { grad_avg(L_N, gn, nullptr); grad_avg(L_ETA, nullptr, &eb); }
-        S fv[5];
-        visc_flux<S, SA>(nx, ny, gu, gv, gT, ub, vb, mb, kb, gn, eb, fv);
+    } else {
 #pragma unroll
-        for (int k = 1; k < NV; ++k) he[k] = he[k] - fv[k];
-      }
+      for (int k = 0; k < 4; ++k) { st[0][k] = at(L_R + k, x, ys); st[1][k] = at(L_R + k, x, yn); }
+    }
+    S nts(0.0), ntn(0.0);
+    if (SA) { nts = at(L_N, x, ys); ntn = at(L_N, x, yn); }
+    conv_flux<S, SA>(ph.flux, E0.x, E0.y, st[0][0], st[0][1], st[0][2], st[0][3], st[1][0], st[1][1], st[1][2], st[1][3],
+                     nts, ntn, he);
+    if (ph.viscous) {
+      FaceGeo<S> G;
+      G.tx = 0.5 * (E0.x + Et.x); G.ty = 0.5 * (E0.y + Et.y);
+      G.bx = 0.5 * (E0.x + Eb.x); G.by = 0.5 * (E0.y + Eb.y);
+      G.lx = 0.5 * (C0.x + Cb.x); G.ly = 0.5 * (C0.y + Cb.y);
+      G.rx = 0.5 * (CR.x + CRb.x); G.ry = 0.5 * (CR.y + CRb.y);
+      G.ivol = frcp(0.5 * (V0 + VB));
+      auto grad_avg = [&](int k, S* gr, S* avg) {
+        S t = at(k, x, yn), b = at(k, x, ys);
+        S l = 0.25 * (t + b + at(k, x - 1, yn) + at(k, x - 1, ys));
+        S r = 0.25 * (t + b + at(k, x + 1, yn) + at(k, x + 1, ys));
+        if (gr) gg_grad(G, t, b, l, r, gr);
+        if (avg) *avg = 0.25 * (l + r + t + b);
+      };
+      S gu[2], gv[2], gT[2], gn[2] = {S(0.0), S(0.0)}, ub, vb, mb, kb, eb(0.0);
+      grad_avg(L_U, gu, &ub);
+      grad_avg(L_V, gv, &vb);
+      grad_avg(L_T, gT, nullptr);
+      grad_avg(L_MU, nullptr, &mb);
+      grad_avg(L_K, nullptr, &kb);
+      if (SA) { grad_avg(L_N, gn, nullptr); grad_avg(L_ETA, nullptr, &eb); }
+      S fv[5];
+      visc_flux<S, SA>(E0.x, E0.y, gu, gv, gT, ub, vb, mb, kb, gn, eb, fv);
+#pragma unroll
+      for (int k = 1; k < NV; ++k) he[k] = he[k] - fv[k];
     }
   }
 
   // ---- SA source of the owned output cell (needs the staged cells)
-  const int ci = i0 + tx, cj = j0 + ty;
+  const int ci = i0 + tx;
   const bool owns = tx < OX && ty < OY && ci < nic && cj < njc;
   S src(0.0);
   if (SA && ph.viscous) {  // uniform over the block
@@ -593,15 +651,13 @@ __global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) vo
     S feat[kNFeat];
     if (owns) {
       const int x = tx + 2, y = ty + 2;
-      const double ex = ncx(ci + 1, cj), ey = ncy(ci + 1, cj), wx = ncx(ci, cj), wy = ncy(ci, cj);
-      const double nx_ = nex(ci, cj + 1), ny_ = ney(ci, cj + 1), sx = nex(ci, cj), sy = ney(ci, cj);
-      const double iV = frcp(vol(ci, cj));
+      const double iV = frcp(V0);
       auto cgrad = [&](int k, S* o) {
         S c = at(k, x, y);
         S fe = 0.5 * (c + at(k, x + 1, y)), fw = 0.5 * (c + at(k, x - 1, y));
         S fn = 0.5 * (c + at(k, x, y + 1)), fs = 0.5 * (c + at(k, x, y - 1));
-        o[0] = (fe * ex - fw * wx + fn * nx_ - fs * sx) * iV;
-        o[1] = (fe * ey - fw * wy + fn * ny_ - fs * sy) * iV;
+        o[0] = (fe * CR.x - fw * C0.x + fn * Et.x - fs * E0.x) * iV;
+        o[1] = (fe * CR.y - fw * C0.y + fn * Et.y - fs * E0.y) * iV;
       };
       S gu[2], gv[2], gn[2], gr[2];
       cgrad(L_U, gu); cgrad(L_V, gv); cgrad(L_N, gn); cgrad(L_R, gr);
@@ -661,7 +717,7 @@ __global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) vo
 #pragma unroll
   for (int k = 0; k < 2 * NV; ++k) sq[k] = 0.0;
   if (owns) {
-    const double V = vol(ci, cj), iV = frcp(V);
+    const double V = V0, iV = frcp(V);
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       S hw = lds[k * NT + tid], hE = lds[k * NT + tid + 1];
@@ -677,133 +733,30 @@ __global__ __launch_bounds__(NT, sizeof(S) == sizeof(double) ? 1024 / NT : 1) vo
       sq[NV + k] = sq[k] * V * V;
     }
   }
-  // Fused norm: count this block's arrival before its stores.  Vector memory
-  // operations complete in issue order, so a wait for the count's return
-  // issued after the stores would also wait for them to be acknowledged; the
-  // parity protocol below makes the order of arrival and stores irrelevant.
-  // Blocks count on the counter of their group (tile index modulo
-  // kNormGroups, one 128-byte line each), so that arrivals on one word come
-  // from one XCD's blocks only; the last of a group counts on the group
-  // counter, and the last group's last block finalises.
-  const int grp = (int)(blockIdx.y * gridDim.x + blockIdx.x) % kNormGroups;
-  unsigned long long arrival = 0;
-  if (fused && tid == 0)
-    arrival = __hip_atomic_fetch_add(nout.state + grp * kNormLineWords, 1ull, __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT);
   if (owns) {
 #pragma unroll
     for (int k = 0; k < NV; ++k) out.put(k, g.plane, oidx, ci, cj, res[k]);
   }
-  // ---- block partial sums of R^2 (fixed order: wavefront DPP sum, then waves)
-  if (partial) {
-    const int lane = tid & 63, wv = tid >> 6;
-    const int nb = gridDim.x * gridDim.y, bid = blockIdx.y * gridDim.x + blockIdx.x;
-    // only the norms the caller asked for (the first nout.count of R^2 then
-    // (V R)^2) are reduced and summed
+  // ---- the tile's sums of R^2, in a fixed order: 16 threads per norm add 16
+  // values each from LDS, then one another's by DPP (a wavefront sum per norm,
+  // 18 instructions each, was 5% of the kernel's)
+  if (nout.slots) {
+    constexpr int LD = NT + 16;  // a norm's row: 16 doubles on, so that four rows read different banks
+    double* sums = lds_raw;
     const int nsum = nout.count;
+    __syncthreads();
 #pragma unroll
     for (int k = 0; k < 2 * NV; ++k)
-      if (k < nsum) sq[k] = wave_sum_lane63(sq[k]);
-    if (lane == 63) {
-#pragma unroll
-      for (int k = 0; k < 2 * NV; ++k) red[wv][k] = sq[k];
-    }
+      if (k < nsum) sums[k * LD + tid] = sq[k];
     __syncthreads();
-    // Fused: the sign bit of each stored partial (a sum of squares, >= 0)
-    // carries the launch parity -- set on launches of parity 0 -- so the
-    // finalising block recognises this launch's value in every slot from
-    // that slot alone.  A block therefore counts its arrival without waiting
-    // for its partial stores, and no ordering between slots, or between a
-    // slot and the counter, is needed: each slot is one 64-bit atomic store,
-    // read by atomic loads of the same location, and launches on a stream
-    // are ordered by the kernel boundary.  Slots start at +0.0 (parity 1), so
-    // a slot never written in this context never passes for parity 0.
-    const bool want_neg = fused && (nout.parity & 1u) == 0u;
-    __shared__ bool last;
-    // every slot is stored on every fused launch (zero beyond nsum), so that
-    // a slot always holds this launch's parity or the previous launch's
-    if (tid < 2 * NV) {
-      double s = 0.0;
-      if (tid < nsum)
-        for (int w = 0; w < NT / 64; ++w) s += red[w][tid];
-      if (want_neg) s = -s;
-      __hip_atomic_store(&partial[(size_t)tid * nb + bid], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (fused && tid == 0) {
-      // blocks of group grp: grp, grp + G, ... < nb; groups with a block: min(nb, G)
-      const unsigned long long gsize = (unsigned long long)((nb - grp + kNormGroups - 1) / kNormGroups);
-      bool l = false;
-      if (arrival == gsize - 1) {
-        const unsigned long long gdone = __hip_atomic_fetch_add(nout.state + kNormGroups * kNormLineWords, 1ull,
-                                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        l = gdone == (unsigned long long)(min(nb, kNormGroups) - 1);
-      }
-      last = l;
-    }
-    if (fused) __syncthreads();
-    if (fused && last) {
-      // The block that arrives last sums the partials of all blocks in a
-      // fixed order (so the norm does not depend on which block it is),
-      // polling each slot until it holds this launch's value.  Every other
-      // block has arrived (each group counter reached its group's size before
-      // the group count reached the number of groups: single-location
-      // read-modify-write order), so it is running and stores its partials,
-      // and the wait ends.
-      int spins = 0;
-      double acc[2 * NV];
+    const int k = tid >> 4, l = tid & 15;
+    if (k < nsum) {
+      double a = 0.0;
 #pragma unroll
-      for (int k = 0; k < 2 * NV; ++k) acc[k] = 0.0;
-      // the plain norms, then (if asked for) the weighted ones; four rows of
-      // blocks per round (one round up to 1,024 blocks), all loads of a round
-      // in flight together
-      constexpr int NR = 4;
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        if (half * NV >= nsum) break;
-        for (int b0 = 0; b0 < nb; b0 += NR * NT) {
-          double v[NR][NV];
-#pragma unroll
-          for (int u = 0; u < NR; ++u) {
-            const int b = b0 + u * NT + tid;
-#pragma unroll
-            for (int kk = 0; kk < NV; ++kk) {
-              const int k = half * NV + kk;
-              v[u][kk] = (b < nb && k < nsum) ? __hip_atomic_load(&partial[(size_t)k * nb + b], __ATOMIC_RELAXED,
-                                                                  __HIP_MEMORY_SCOPE_AGENT)
-                                              : (want_neg ? -0.0 : 0.0);
-            }
-          }
-#pragma unroll
-          for (int u = 0; u < NR; ++u) {
-            const int b = b0 + u * NT + tid;
-#pragma unroll
-            for (int kk = 0; kk < NV; ++kk) {
-              const int k = half * NV + kk;
-              while (__builtin_signbit(v[u][kk]) != want_neg) {
-                if (++spins > kNormSpinLimit) { v[u][kk] = nan; break; }
-                v[u][kk] = __hip_atomic_load(&partial[(size_t)k * nb + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-              }
-              acc[k] += fabs(v[u][kk]);
-            }
-          }
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < 2 * NV; ++k) acc[k] = wave_sum_lane63(acc[k]);
-      __syncthreads();  // red[] is reused below; every wave of this block reached here
-      if (lane == 63) {
-#pragma unroll
-        for (int k = 0; k < 2 * NV; ++k) red[wv][k] = acc[k];
-      }
-      __syncthreads();
-      if (tid < 2 * NV && tid < nout.count) {
-        double s = 0.0;
-        for (int w = 0; w < NT / 64; ++w) s += red[w][tid];
-        nout.l2[tid] = sqrt(s);
-      }
-      // every arrival of this launch is in: reset the counters
-      if (tid <= kNormGroups)
-        __hip_atomic_store(nout.state + tid * kNormLineWords, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int m = 0; m < NT / 16; ++m) a += sums[k * LD + m * 16 + l];
+      a = row_sum(a);
+      if (l == 0)
+        __hip_atomic_store(nout.slots + (size_t)k * ntile + bid, (unsigned long long)__double_as_longlong(a), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
 }

@@ -136,8 +136,20 @@ __device__ __forceinline__ Dual spow16(Dual z) {
   const double y = pow16(z.v);
   return Dual(y, (1.0 / 6.0) * y * frcp(z.v) * z.d);
 }
+__device__ __forceinline__ double ssel(bool c, double a, double b) { return c ? a : b; }
+__device__ __forceinline__ Dual ssel(bool c, Dual a, Dual b) { return Dual(c ? a.v : b.v, c ? a.d : b.d); }
 __device__ __forceinline__ double smin(double a, double b) { return a < b ? a : b; }
 __device__ __forceinline__ Dual smin(Dual a, double b) { return a.v < b ? a : Dual(b); }
+
+// Element (r, c) of a row-major array, for the cells of one tile: the tile's
+// origin (jo, io) goes into the scalar base, so that a lane needs one byte
+// offset for all arrays of the same row length.  I: 32 bits, or 64 where a
+// tile's rows span more than 4 GiB.
+template <class I>
+__device__ __forceinline__ double tile_at(const double* a, int ld, int jo, int io, int c, int r) {
+  const char* base = reinterpret_cast<const char*>(a + (size_t)jo * ld + io);
+  return *reinterpret_cast<const double*>(base + ((I)(r - jo) * (I)ld + (I)(c - io)) * 8u);
+}
 
 // Loads of a state component for scalar type S: component k of the cell with
 // index idx (column ci, row cj).  The dual reads the tangent from a second
@@ -149,6 +161,11 @@ struct Field<double> {
   const double* v;
   __device__ __forceinline__ void begin(int) {}
   __device__ __forceinline__ double at(int k, size_t plane, size_t idx, int, int) const { return v[k * plane + idx]; }
+  template <int NQ, class I>
+  __device__ __forceinline__ void load(double* o, size_t plane, int ld, int jo, int io, int c, int r) const {
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) o[k] = tile_at<I>(v + k * plane, ld, jo, io, c, r);
+  }
 };
 template <>
 struct Field<Dual> {
@@ -157,6 +174,12 @@ struct Field<Dual> {
   __device__ __forceinline__ void begin(int) {}
   __device__ __forceinline__ Dual at(int k, size_t plane, size_t idx, int, int) const {
     return Dual(v[k * plane + idx], d[k * plane + idx]);
+  }
+  template <int NQ, class I>
+  __device__ __forceinline__ void load(Dual* o, size_t plane, int ld, int jo, int io, int c, int r) const {
+#pragma unroll
+    for (int k = 0; k < NQ; ++k)
+      o[k] = Dual(tile_at<I>(v + k * plane, ld, jo, io, c, r), tile_at<I>(d + k * plane, ld, jo, io, c, r));
   }
 };
 
@@ -181,6 +204,12 @@ struct SeedField {
   __device__ __forceinline__ Dual at(int k, size_t plane, size_t idx, int ci, int cj) const {
     const bool on = k == dir.m && ci % dir.per == dir.a && cj % dir.per == dir.b;
     return Dual(v[k * plane + idx], on ? 1.0 : 0.0);
+  }
+  template <int NQ, class I>
+  __device__ __forceinline__ void load(Dual* o, size_t plane, int ld, int jo, int io, int c, int r) const {
+    const bool colour = c % dir.per == dir.a && r % dir.per == dir.b;
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) o[k] = Dual(tile_at<I>(v + k * plane, ld, jo, io, c, r), colour && k == dir.m ? 1.0 : 0.0);
   }
 };
 
