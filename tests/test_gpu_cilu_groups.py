@@ -42,6 +42,10 @@ def oracle_blocks(case, q, wd):
     (24, 9, False, 24),   # two groups of 12
     (30, 67, False, 32),  # nv = 4, last group not full, the ring wraps
     (17, 66, False, 16),  # nv = 4: one group of 16, then one column
+    (6, 65, True, 32),    # the widths that two lanes a row allow: 6 columns, nv 5
+    (13, 12, True, 16),
+    (8, 64, False, 8),    # and 8, nv 4
+    (25, 5, False, 32),
 ])
 @pytest.mark.parametrize("precond", [6, 7])
 def test_groups_match_model(cols, rows, sa, width, precond):
