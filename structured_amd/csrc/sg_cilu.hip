@@ -20,6 +20,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 #include "sg_linalg.hpp"
 
@@ -52,6 +54,15 @@ constexpr int low(int n) { return NINE ? Low9[n] : Low[n]; }
 template <bool NINE>
 constexpr int up(int n) { return NINE ? Up9[n] : Up[n]; }
 constexpr bool in_box(int s) { return s >= 0 && s < 9; }
+// offsets of a slot known at run time, four bits each, plus 2
+constexpr unsigned long long pack(const int* d) {
+  unsigned long long v = 0;
+  for (int s = 0; s < NSLOT; ++s) v |= (unsigned long long)(d[s] + 2) << (4 * s);
+  return v;
+}
+constexpr unsigned long long kDi = pack(Di), kDj = pack(Dj);
+__device__ __forceinline__ int di(int s) { return (int)(kDi >> (4 * s) & 15) - 2; }
+__device__ __forceinline__ int dj(int s) { return (int)(kDj >> (4 * s) & 15) - 2; }
 // The apply's neighbours, in the order of their records: lower ones for the
 // ascending pass, upper ones for the descending pass, entry n of one being
 // the opposite offset of entry n of the other.  0-2 are the column before
@@ -59,20 +70,50 @@ constexpr bool in_box(int s) { return s >= 0 && s < 9; }
 // column, 4 and 5 the +-2 couplings of the 13-point stencil.
 constexpr int Asc[6] = {5, 3, 7, 1, 9, 11};
 constexpr int Desc[6] = {8, 4, 6, 2, 10, 12};
+__device__ __forceinline__ int asc(int n) { return (int)(0xB91735ull >> (4 * n)) & 15; }
+__device__ __forceinline__ int desc(int n) { return (int)(0xCA2648ull >> (4 * n)) & 15; }
+static_assert(Asc[0] == 5 && Asc[1] == 3 && Asc[2] == 7 && Asc[3] == 1 && Asc[4] == 9 && Asc[5] == 11, "asc");
+static_assert(Desc[0] == 8 && Desc[1] == 4 && Desc[2] == 6 && Desc[3] == 2 && Desc[4] == 10 && Desc[5] == 12, "desc");
+// place of an upper neighbour's slot among them
+template <bool NINE>
+constexpr int up_index(int s) {
+  for (int u = 0; u < nn<NINE>(); ++u)
+    if (up<NINE>(u) == s) return u;
+  return -1;
+}
 constexpr int slot(int di, int dj) {
   for (int s = 0; s < NSLOT; ++s)
     if (Di[s] == di && Dj[s] == dj) return s;
   return -1;
 }
+// The products of a row's elimination, in order: with lower neighbour n's
+// diagonal inverse (u = -1), then with those of its upper blocks u that meet a
+// block `target` of the row.
+struct Product {
+  int n, u, target;
+};
+template <bool NINE>
+struct Plan {
+  Product p[6 * 7] = {};
+  int count = 0;
+  constexpr Plan() {
+    for (int n = 0; n < nn<NINE>(); ++n) {
+      p[count++] = {n, -1, low<NINE>(n)};
+      for (int u = 0; u < nn<NINE>(); ++u) {
+        const int t = slot(Di[low<NINE>(n)] + Di[up<NINE>(u)], Dj[low<NINE>(n)] + Dj[up<NINE>(u)]);
+        if (t >= 0 && (!NINE || in_box(t))) p[count++] = {n, u, t};
+      }
+    }
+  }
+};
+template <bool NINE>
+constexpr Plan<NINE> plan;
+// f(integral_constant) for 0 .. N - 1
+template <class F, int... I>
+__device__ __forceinline__ void each(F f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>()), ...);
+}
 }  // namespace ct
-
-// Factorisation, one level after another.  Thread (c, e) holds entry e of
-// every stencil block of its cell's row in registers.  A row's lower
-// neighbours lie on the four previous levels (L-1 .. L-4), whose factored
-// diagonal inverses and upper blocks are kept in an LDS ring, so the level
-// loop reads the 13 blocks of its own cells (gathered in level order by
-// cilu_gather_kernel) from memory and nothing else; the elimination exchanges
-// one 5x5 block per cell through LDS per lower neighbour.
 
 // Column groups of the apply and the layout of their factor records.
 //
@@ -116,6 +157,9 @@ struct Lay {
   // place there
   static constexpr int half(int n) { return P == 2 && (n == 1 || n == 2 || n == 5); }
   static constexpr int place(int n) { return P == 1 ? n : n == 2 || n == 3 ? 0 : n < 2 ? 1 : 2; }
+  __host__ __device__ static int neighbour(int h, int place) {
+    return P == 1 ? place : place == 0 ? (h ? 2 : 3) : place == 1 ? h : 4 + h;
+  }
   static constexpr int rs(int n) { return (n * LN + 15) / 16 * 16; }  // floats of a step's record
   static constexpr int count(int a) { return a == 0 || a == 3 ? n1 : n2; }  // per lane, in array a
   static_assert(LN <= 64, "a group fits a wave");
@@ -141,8 +185,8 @@ struct Lay {
   static size_t links(int nchunk, int njc) { return 2 * (size_t)nchunk * (NG - 1) * link(njc); }
 };
 
-// Zeroes the records that the factorisation does not write, or writes in
-// part: steps at both ends of a pass, and groups with absent columns.  One
+// Zeroes the records of M^-1 that the factorisation does not write, or writes
+// in part: steps at both ends of a pass, and groups with absent columns.  One
 // block per record.
 template <int NV, int W, bool NINE, int P>
 __global__ __launch_bounds__(256) void cilu_zero_kernel(int nic, int njc, int nchunk, float* rec) {
@@ -150,52 +194,123 @@ __global__ __launch_bounds__(256) void cilu_zero_kernel(int nic, int njc, int nc
   const int t = blockIdx.x, gg = blockIdx.y, s = t - La::X;
   const int wk = min(W, nic - gg / La::NG * W) - gg % La::NG * La::GW;
   if (wk >= La::GW && s >= 2 * (La::GW - 1) && s < njc) return;
-  for (int a = 0; a < 4; ++a) {
+  for (int a = 0; a < 2; ++a) {
     const int rs = La::rs(La::count(a));
     float* r = rec + La::array(a, nchunk, njc) + ((size_t)gg * La::nrec(njc) + t) * rs;
     for (int e = threadIdx.x; e < rs; e += 256) r[e] = 0.0f;
   }
 }
 
+// The records of M^-T from those of M^-1: row r of a cell's U^T and D^-T from
+// the U blocks of its lower neighbours and its own D^-1, row r of L^T from the
+// L blocks of its upper neighbours, zeros elsewhere.  One block per record.
+// Written by the factorisation, they were half of the bytes that one CU per
+// chunk had to move; here the whole chip does.
+template <int NV, int W, bool NINE, int P>
+__global__ __launch_bounds__(256) void cilu_transpose_kernel(int nic, int njc, int nchunk, float* rec) {
+  using La = Lay<NV, W, NINE, P>;
+  const int t = blockIdx.x, gg = blockIdx.y, chunk = gg / La::NG, c0 = gg % La::NG * La::GW, wk = min(W, nic - chunk * W);
+  const int nrec = La::nrec(njc);
+  // float of row `row`, half h, place f of cell (c, j) in array a
+  auto from = [&](int a, int c, int j, int row, int h, int f) {
+    const int n = La::count(a), g = c / La::GW, cl = c % La::GW;
+    const bool asc = a == 0 || a == 2;
+    const int c1 = asc ? cl : La::GW - 1 - cl, s = asc ? j : njc - 1 - j;
+    return rec[La::array(a, nchunk, njc) + ((size_t)(chunk * La::NG + g) * nrec + La::X + s + 2 * c1) * La::rs(n) +
+               La::in_record(n, P * (c1 * NV + row) + h, f)];
+  };
+#pragma unroll
+  for (int a = 2; a < 4; ++a) {
+    constexpr int N[2] = {La::n2, La::n1};
+    const int n = N[a - 2], rs = La::rs(n);
+    float* out = rec + La::array(a, nchunk, njc) + ((size_t)gg * nrec + t) * rs;
+    for (int e = threadIdx.x; e < rs; e += 256) {
+      // lane and float of the lane, as in Lay::in_record
+      const int q4 = n / 4 * 4 * La::LN;
+      const int lane = e < q4 ? e / 4 % La::LN : (e - q4) % La::LN;
+      const int f = e < q4 ? e / 4 / La::LN * 4 + e % 4 : n / 4 * 4 + (e - q4) / La::LN;
+      const int h = lane % P, row = lane / P % NV, c1 = lane / P / NV;
+      const int s = t - La::X - 2 * c1, c = c0 + (a == 2 ? c1 : La::GW - 1 - c1), j = a == 2 ? s : njc - 1 - s;
+      float v = 0.0f;
+      if (f < n && c < wk && s >= 0 && s < njc) {
+        if (f < La::n1) {
+          const int place = f / NV, k = f % NV, nb = La::neighbour(h, place);
+          const int slot = a == 2 ? ct::asc(nb) : ct::desc(nb);
+          const int cn = c + ct::di(slot), jn = j + ct::dj(slot);
+          if (cn >= 0 && cn < wk && jn >= 0 && jn < njc) v = from(a == 2 ? 1 : 0, cn, jn, k, h, place * NV + row);
+        } else {
+          const int q = h * La::ND + f - La::n1;
+          if (q < NV) v = from(1, c, j, q, row / La::ND, La::n1 + row % La::ND);
+        }
+      }
+      out[e] = v;
+    }
+  }
+}
+
+// Shape of the factorisation: a thread holds one row of a cell, CW cells to a
+// wave.
+template <int NV, int W, bool NINE>
+struct Fac {
+  static constexpr int NN = NINE ? 4 : 6, NS = NINE ? 9 : NSLOT;  // blocks of a row
+  static constexpr int CW = 64 / NV, NW = (W + CW - 1) / CW;      // cells of a wave, waves
+  static constexpr int N2 = (NS * NV + 1) / 2;                    // 16-byte words of a row
+  // levels kept: a cell's lower neighbours lie on the three (13-point: four)
+  // levels before its own
+  static constexpr int NR = NINE ? 4 : 5;
+  // the kept blocks hold FP32 values; where they fit as doubles nothing has to
+  // be converted when they are read
+  using R = std::conditional_t<NINE, double, float>;
+  // block and cell strides: the cells of a wave read different banks
+  static constexpr int BP = NINE ? (NV == 5 ? 26 : 18) : (NV == 5 ? 28 : 20);
+  static constexpr int GP = 2 * NV * NV + (NV == 4 ? 2 : 0);
+};
+
 // Gathers the factorisation's operands into level order: for chunk, level L,
-// slot s, block entry e and column c, entry e of the block of I/dt - J in row
-// (i0 + c, L - 2c) and neighbour slot s, or zero where the cell or the
-// neighbour lies outside the chunk or the grid.  Consecutive columns are
-// contiguous, so the factorisation reads a level's operands in runs of W
-// doubles.  Read in place, a level's W cells lie on a diagonal of rows 2 ldi
+// 16-byte word e and row (c, r) of the level, entries 2 e and 2 e + 1 of row r
+// of the blocks of I/dt - J at cell (i0 + c, L - 2c), slot after slot, or zero
+// where the cell or the neighbour lies outside the chunk or the grid.  The rows
+// of a level are contiguous, so the factorisation reads 16 bytes a thread, all
+// used.  Read in place, a level's W cells lie on a diagonal of rows 2 ldi
 // apart: every 8-byte read took its own line, used again only ~W levels later
 // after L2 had evicted it.  Here all levels are gathered at once and the
-// levels that share a line are read together.
-template <int NV, int W>
+// levels that share a line are read together.  Only the pattern's blocks: at
+// 545x385 the box 0.44 ms, all 13 blocks 0.73.
+template <int NV, int W, bool NINE>
 __global__ __launch_bounds__(256) void cilu_gather_kernel(int nic, int njc, int ldi, int nlev, const double* idt,
-                                                          const double* blocks, double* ops, size_t total) {
+                                                          const double* blocks, double2* ops, size_t total) {
+  using Fa = Fac<NV, W, NINE>;
   constexpr int B = NV * NV;
   const size_t plane = (size_t)njc * ldi;
   for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
     size_t u = t;
-    const int c = (int)(u % W);
-    u /= W;
-    const int e = (int)(u % B);
-    u /= B;
-    const int s = (int)(u % NSLOT);
-    u /= NSLOT;
+    const int row = (int)(u % (W * NV)), c = row / NV, r = row % NV;
+    u /= W * NV;
+    const int e = (int)(u % Fa::N2);
+    u /= Fa::N2;
     const int L = (int)(u % (size_t)nlev), chunk = (int)(u / (size_t)nlev);
     const int i0 = chunk * W, wk = min(W, nic - i0), j = L - 2 * c;
-    const int cn = c + ct::Di[s], jn = j + ct::Dj[s];
-    double v = 0.0;
-    if (c < wk && j >= 0 && j < njc && cn >= 0 && cn < wk && jn >= 0 && jn < njc) {
-      const size_t cell = (size_t)j * ldi + i0 + c;
-      v = -blocks[(size_t)(s * B + e) * plane + cell];
-      if (s == 0 && e / NV == e % NV) v += idt[cell];
+    const size_t cell = (size_t)j * ldi + i0 + c;
+    double v[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const int f = 2 * e + x, s = f / NV, q = f % NV;
+      const int cn = c + ct::di(s), jn = j + ct::dj(s);
+      v[x] = 0.0;
+      if (s < Fa::NS && c < wk && j >= 0 && j < njc && cn >= 0 && cn < wk && jn >= 0 && jn < njc) {
+        v[x] = -blocks[(size_t)(s * B + r * NV + q) * plane + cell];
+        if (s == 0 && r == q) v[x] += idt[cell];
+      }
     }
-    ops[t] = v;
+    ops[t] = double2{v[0], v[1]};
   }
 }
 
-// doubles of the gathered factorisation operands
-static size_t cilu_ops_doubles(int nic, int njc, int nv, int w) {
-  const int nchunk = (nic + w - 1) / w, nlev = njc + 2 * w - 2;
-  return (size_t)nchunk * nlev * NSLOT * nv * nv * w;
+// 16-byte words of the gathered factorisation operands
+template <int NV, int W, bool NINE>
+static size_t cilu_ops(int nic, int njc) {
+  const int nchunk = (nic + W - 1) / W, nlev = njc + 2 * W - 2;
+  return (size_t)nchunk * nlev * Fac<NV, W, NINE>::N2 * W * NV;
 }
 
 // A link word that holds no value: a signalling NaN, which no arithmetic
@@ -206,151 +321,240 @@ __global__ __launch_bounds__(256) void cilu_empty_kernel(unsigned long long* x, 
     x[e] = kEmpty;
 }
 
-// NINE: ILU(0) on the 3x3-box pattern (the +-2 blocks of A and their fill
-// dropped; with the first-order Jacobian of lhs_order 1 those slots hold
-// fill only), else on the 13-point stencil.
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
+}
+
+constexpr unsigned kNowhere = 0xFFFFFF00u;  // beyond every buffer: such a store is dropped
+// A record's n floats of a lane, in the layout of Lay::in_record, at byte
+// offset `at` of the buffer.
+template <int N, int LN>
+__device__ __forceinline__ void put_record(__amdgpu_buffer_rsrc_t rec, unsigned at, int lane, bool on, const float* v) {
+#pragma unroll
+  for (int q = 0; q < N / 4; ++q) {
+    const u32x4 w = {__float_as_uint(v[4 * q]), __float_as_uint(v[4 * q + 1]), __float_as_uint(v[4 * q + 2]),
+                     __float_as_uint(v[4 * q + 3])};
+    __builtin_amdgcn_raw_buffer_store_b128(w, rec, on ? at + (q * LN + lane) * 16 : kNowhere, 0, 0);
+  }
+#pragma unroll
+  for (int f = N / 4 * 4; f < N; ++f)
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[f]), rec,
+                                          on ? at + (4 * (N / 4) * LN + (f - 4 * (N / 4)) * LN + lane) * 4 : kNowhere, 0, 0);
+}
+
+// Orders this wave's LDS accesses (a wave's LDS operations execute in issue
+// order, so nothing is waited for).
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Factorisation, one level after another, one work-group per chunk.  NINE:
+// ILU(0) on the 3x3-box pattern (the +-2 blocks of A and their fill dropped;
+// with the first-order Jacobian of lhs_order 1 those slots hold fill only),
+// else on the 13-point stencil.
+//
+// Thread (c, r) holds row r of the blocks of its level's cell in column c.  A
+// row is eliminated without the cell's other rows: it is multiplied by the
+// lower neighbours' diagonal inverses and upper blocks, which an LDS ring keeps
+// and the threads of a cell read together (a broadcast).  The diagonal block is
+// inverted by Gauss-Jordan with partial pivoting on [D | I], a row a thread:
+// rows stay where they are and carry the position that swapping would have
+// given them.  The next level's operands are in flight meanwhile.  One barrier a
+// level: the ring has room for the level that is written.
+//
+// What bounds it: a level, njc + 2 W - 2 times.  A wave issues some 1,600
+// instructions for it (about 430 FP64 FMAs, the LDS reads that feed them, the
+// pivots' exchanges), some 3 us, and one CU moves 59 KB of operands and 29 KB
+// of records (nv 5, W 32), about 20 bytes/ns.  A level takes 5.3 us (nv 4:
+// 3.3).  With a thread per block entry, two barriers per neighbour and one per
+// pivot, every product read ten LDS words for five FMAs and a level took 14 us
+// (6.0).  545x385 nv 5 6.35 -> 2.36 ms, and 0.15 for M^-T, which the whole chip
+// writes afterwards; 97x65 nv 4 0.76 -> 0.42.
 template <int NV, int W, bool NINE, int P>
-__global__ __launch_bounds__(W * NV * NV) void cilu_factor_kernel(int nic, int njc, int nlev, const double* ops,
-                                                                  float* rec) {
+__global__ __launch_bounds__((64 * Fac<NV, W, NINE>::NW)) __attribute__((amdgpu_waves_per_eu(1, 1))) void
+cilu_factor_kernel(int nic, int njc, int nlev, const double2* ops, float* rec) {
   using La = Lay<NV, W, NINE, P>;
-  constexpr int B = NV * NV, NR = 4, NN = ct::nn<NINE>();
-  __shared__ float ring[NR][7][W][B];  // per level: diagonal inverse, then the six upper blocks (ct::Up order)
-  __shared__ double Ab[W][B];
-  __shared__ double Lb[W][B];
-  __shared__ double cb[2][W][NV];
-  const int chunk = blockIdx.x, i0 = chunk * W, wk = min(W, nic - i0);
-  const int t = threadIdx.x, c = t / B, e = t % B, r = e / NV, q = e % NV;
-  // float f of half h of row `row` of cell (cc, jj) in array a
-  const int nchunk = gridDim.x, nrec = La::nrec(njc);
-  auto put_at = [&](int a, int cc, int jj, int row, int h, int f, float v) {
-    const int n = La::count(a), g = cc / La::GW, cl = cc % La::GW;
+  using Fa = Fac<NV, W, NINE>;
+  using R = typename Fa::R;
+  constexpr int B = NV * NV, NR = Fa::NR, NN = Fa::NN, NS = Fa::NS, N2 = Fa::N2, CW = Fa::CW, ND = La::ND;
+  // per level: diagonal inverse, then the upper blocks (ct::up order)
+  __shared__ R ring[(NR * (1 + NN) * W + 1) * Fa::BP] __attribute__((aligned(16)));
+  constexpr int kNone = NR * (1 + NN) * W;  // the block of an absent neighbour: zero
+  // block b of column ci at the level `back` levels before level L
+  auto block = [&](int L, int back, int b, int ci) {
+    return (int)((((unsigned)(L + NR - back) % NR) * (1 + NN) + b) * W) + ci;
+  };
+  auto block_or_none = [&](bool there, int at) -> const R* {
+    asm volatile("" : "+v"(at));  // a select, not a branch around the index
+    return ring + (there ? at : kNone) * Fa::BP;
+  };
+  __shared__ double gj[Fa::NW * CW + 1][Fa::GP] __attribute__((aligned(16)));  // [D | I] by position; the last: idle lanes
+  const int chunk = blockIdx.x, nchunk = gridDim.x, i0 = chunk * W, wk = min(W, nic - i0);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cw = lane / NV, r = lane % NV;
+  const int c = cw < CW ? wave * CW + cw : W, cc = min(c, W - 1);
+  double* mat = gj[cw < CW ? wave * CW + cw : Fa::NW * CW];
+  const int nrec = La::nrec(njc);
+  // the chunk's records in array a, and the record of cell (ci, jj) there
+  auto records = [&](int a) {
+    const size_t n = (size_t)La::NG * nrec * La::rs(La::count(a));
+    return buffer_of(rec + La::array(a, nchunk, njc) + chunk * n, n * sizeof(float));
+  };
+  const auto rec0 = records(0), rec1 = records(1);
+  auto record = [&](int a, int ci, int jj) {
+    const int g = ci / La::GW, cl = ci % La::GW;
     const bool asc = a == 0 || a == 2;
     const int c1 = asc ? cl : La::GW - 1 - cl, s = asc ? jj : njc - 1 - jj;
-    rec[La::array(a, nchunk, njc) + ((size_t)(chunk * La::NG + g) * nrec + La::X + s + 2 * c1) * La::rs(n) +
-        La::in_record(n, P * (c1 * NV + row) + h, f)] = v;
+    return (unsigned)(g * nrec + La::X + s + 2 * c1) * (unsigned)(La::rs(La::count(a)) * sizeof(float));
   };
-  auto put = [&](int a, int cc, int jj, int row, int n, int qq, float v) {  // neighbour n's entry qq
-    put_at(a, cc, jj, row, La::half(n), La::place(n) * NV + qq, v);
+  // lane of half h of row `row` of column ci
+  auto lane_of = [&](bool asc, int ci, int row, int h) {
+    const int cl = ci % La::GW;
+    return P * ((asc ? cl : La::GW - 1 - cl) * NV + row) + h;
   };
-  auto put_diag = [&](int a, int cc, int jj, int row, int qq, float v) {
-    put_at(a, cc, jj, row, qq / La::ND, La::n1 + qq % La::ND, v);
-    // the second half of an odd row ends in a zero
-    if (NV % P && qq == NV - 1) put_at(a, cc, jj, row, 1, La::n1 + La::ND - 1, 0.0f);
+  // (without a branch: a level is one block of code, or its products are not
+  // scheduled as written)
+  auto inside = [&](int ci, int jj) { return ((unsigned)ci < (unsigned)wk) & ((unsigned)jj < (unsigned)njc); };
+  for (int e = threadIdx.x; e < (int)(sizeof(ring) / sizeof(R)); e += blockDim.x) ring[e] = R(0);
+
+  const double2* op = ops + (size_t)chunk * nlev * N2 * (W * NV) + (cc * NV + r);
+  double2 next[N2];  // the coming level's operands
+  auto fetch = [&](int L) {
+    const double2* from = op + (size_t)min(L, nlev - 1) * N2 * (W * NV);
+#pragma unroll
+    for (int e = 0; e < N2; ++e) next[e] = from[(size_t)e * (W * NV)];
   };
-  auto inside = [&](int cc, int jj) { return cc >= 0 && cc < wk && jj >= 0 && jj < njc; };
+  fetch(0);
+  // arrived before the loop: its wait for a level's operands then counts the
+  // stores that follow them in the loop, and waits for none of those
+#pragma unroll
+  for (int e = N2 - 1; e >= 0; --e) asm volatile("" : "+v"(next[e].x), "+v"(next[e].y));
+  lds_barrier();
   for (int L = 0; L < nlev; ++L) {
     const int j = L - 2 * c;
-    const bool valid = inside(c, j);
-    // this row's 13 blocks of I/dt - J, gathered in level order (zero where
-    // the cell or the neighbour is outside)
-    const double* opl = ops + ((size_t)(chunk * nlev + L) * NSLOT * B + e) * W + c;
-    double a[NSLOT];
+    const bool valid = inside(c, j);  // (the idle lanes' c = W is outside)
+    double a[NS][NV];
 #pragma unroll
-    for (int s = 0; s < NSLOT; ++s) a[s] = opl[(size_t)s * B * W];
+    for (int f = 0; f < NS * NV; ++f) a[f / NV][f % NV] = f & 1 ? next[f / 2].y : next[f / 2].x;
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(L + 1);
+
+    // ---- elimination of the lower neighbours; a product's block is read while
+    // the one before is formed.  An absent neighbour's blocks, and its block in
+    // this row, are zero; so are the blocks that couple a neighbour to a cell
+    // outside.
+    R blk[2][B];
+    double l[NV];
+    constexpr int NP = ct::plan<NINE>.count;
+    auto read = [&](auto at) {
+      constexpr int i = decltype(at)::value;
+      constexpr ct::Product pr = ct::plan<NINE>.p[i];
+      constexpr int s = ct::low<NINE>(pr.n), di = ct::Di[s], dj = ct::Dj[s];
+      const R* m = block_or_none(valid & inside(c + di, j + dj), block(L, -dj - 2 * di, 1 + pr.u, c + di));
 #pragma unroll
-    for (int qi = 0; qi < NN; ++qi) {
-      const int s = ct::low<NINE>(qi), di = ct::Di[s], dj = ct::Dj[s];
-      const int cn = c + di, jn = j + dj;
-      const bool nok = valid && inside(cn, jn);
-      const int ln = (L + dj + 2 * di) & (NR - 1);  // the neighbour's level in the ring
-      const int cs = nok ? cn : c;
-      Ab[c][e] = a[s];
-      lds_barrier();
-      double l = 0.0;
-      if (nok) {
+      for (int k = 0; k < B; ++k) blk[i & 1][k] = m[k];
+    };
+    read(std::integral_constant<int, 0>());
+    ct::each([&](auto at) {
+      constexpr int i = decltype(at)::value;
+      constexpr ct::Product pr = ct::plan<NINE>.p[i];
+      // one wait for the whole block, before the next one's reads
 #pragma unroll
-        for (int k = 0; k < NV; ++k) l += Ab[c][r * NV + k] * (double)ring[ln][0][cs][k * NV + q];
+      for (int k = B - 1; k >= 0; --k) asm volatile("" : "+v"(blk[i & 1][k]));
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (i + 1 < NP) read(std::integral_constant<int, i + 1>());
+      double sum[NV];
+#pragma unroll
+      for (int q = 0; q < NV; ++q) sum[q] = 0.0;
+#pragma unroll
+      for (int k = 0; k < NV; ++k)
+#pragma unroll
+        for (int q = 0; q < NV; ++q) sum[q] += (pr.u < 0 ? a[pr.target][k] : l[k]) * (double)blk[i & 1][k * NV + q];
+#pragma unroll
+      for (int q = 0; q < NV; ++q) {
+        if (pr.u < 0) a[pr.target][q] = l[q] = sum[q];
+        else a[pr.target][q] -= sum[q];
+        asm volatile("" : "+v"(a[pr.target][q]));  // formed here, not where it is used
       }
-      a[s] = l;
-      Lb[c][e] = l;
-      lds_barrier();
-      if (nok) {
+    }, std::make_integer_sequence<int, NP>());
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- the level's L and U rows are final: the upper blocks into the ring,
+    // both into this cell's records of M^-1
+    float r0[P][La::n1], r1[P][La::n2];
 #pragma unroll
-        for (int ui = 0; ui < NN; ++ui) {
-          const int ts = ct::up<NINE>(ui);
-          const int ri = di + ct::Di[ts], rj = dj + ct::Dj[ts];
-          const int su = ct::slot(ri, rj);
-          if (su < 0 || (NINE && !ct::in_box(su)) || !inside(c + ri, j + rj)) continue;
-          double sum = 0.0;
+    for (int n = 0; n < NN; ++n)
 #pragma unroll
-          for (int k = 0; k < NV; ++k) sum += Lb[c][r * NV + k] * (double)ring[ln][1 + ui][cs][k * NV + q];
-          a[su] -= sum;
-        }
+      for (int q = 0; q < NV; ++q) {
+        r0[La::half(n)][La::place(n) * NV + q] = (float)a[ct::Asc[n]][q];
+        r1[La::half(n)][La::place(n) * NV + q] = (float)a[ct::Desc[n]][q];
       }
+    R* const cell = ring + block(L, 0, 0, cc) * Fa::BP;
+    constexpr int kStep = W * Fa::BP;  // from one of a cell's blocks to the next
+    if (c < W) {
+#pragma unroll
+      for (int n = 0; n < NN; ++n)
+#pragma unroll
+        for (int q = 0; q < NV; ++q)
+          cell[(1 + ct::up_index<NINE>(ct::Desc[n])) * kStep + r * NV + q] =
+              valid ? (R)r1[La::half(n)][La::place(n) * NV + q] : R(0);
     }
-    // the level's L and U blocks are final: store them (records of both
-    // directions and ring).  A block goes to its own row's record and,
-    // transposed, to that of the neighbour it couples to; absent neighbours
-    // leave zeros in this cell's own records.
-    const int lr = L & (NR - 1);
-    if (valid) {
+    double d[NV], id[NV];
 #pragma unroll
-      for (int n = 0; n < NN; ++n) {
-        const int sl = ct::Asc[n], su = ct::Desc[n];
-        put(0, c, j, r, n, q, (float)a[sl]);
-        put(1, c, j, r, n, q, (float)a[su]);
-        const int cl = c + ct::Di[sl], jl = j + ct::Dj[sl], cu = c + ct::Di[su], ju = j + ct::Dj[su];
-        const bool lok = inside(cl, jl), uok = inside(cu, ju);
-        if (lok) put(3, cl, jl, q, n, r, (float)a[sl]);
-        else put(2, c, j, q, n, r, 0.0f);
-        if (uok) put(2, cu, ju, q, n, r, (float)a[su]);
-        else put(3, c, j, q, n, r, 0.0f);
-      }
-    }
+    for (int q = 0; q < NV; ++q) { d[q] = a[0][q]; id[q] = q == r ? 1.0 : 0.0; }
+    // Stores without a branch around them: where one may be skipped, the next
+    // wait for a load waits for all of them.
 #pragma unroll
-    for (int ui = 0; ui < NN; ++ui) ring[lr][1 + ui][c][e] = valid ? (float)a[ct::up<NINE>(ui)] : 0.0f;
-    // inverse of the factored diagonal block: Gauss-Jordan with partial
-    // pivoting on [D | I], column-parallel (thread e < 2 NV of a cell owns
-    // column e; the pivot column is broadcast through LDS each step)
-    Ab[c][e] = a[0];
-    lds_barrier();
-    double col[NV];
-#pragma unroll
-    for (int rr = 0; rr < NV; ++rr) col[rr] = (e < NV) ? Ab[c][rr * NV + e] : ((e - NV == rr) ? 1.0 : 0.0);
+    for (int h = 0; h < P; ++h)
+      put_record<La::n1, La::LN>(rec0, record(0, cc, j), lane_of(true, cc, r, h), valid, r0[h]);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- inverse of the factored diagonal block
+    int pos = r;
 #pragma unroll
     for (int p = 0; p < NV; ++p) {
-      if (e == p) {
 #pragma unroll
-        for (int rr = 0; rr < NV; ++rr) cb[p & 1][c][rr] = col[rr];
-      }
-      lds_barrier();
-      double cp[NV];
+      for (int q = p; q < NV; ++q) mat[pos * 2 * NV + q] = d[q];
 #pragma unroll
-      for (int rr = 0; rr < NV; ++rr) cp[rr] = cb[p & 1][c][rr];
+      for (int q = 0; q < NV; ++q) mat[pos * 2 * NV + NV + q] = id[q];
+      wave_order();
+      double cp = mat[p * 2 * NV + p], best = fabs(cp);
       int piv = p;
-      double best = fabs(cp[p]);
 #pragma unroll
       for (int rr = p + 1; rr < NV; ++rr) {
-        const double v = fabs(cp[rr]);
-        if (v > best) { best = v; piv = rr; }
+        const double x = mat[rr * 2 * NV + p], v = fabs(x);
+        if (v > best) { best = v; piv = rr; cp = x; }
+      }
+      const double ip = 1.0 / cp, f = d[p];
+      const double* prow = mat + piv * 2 * NV;
+      const bool mine = pos == piv;
+#pragma unroll
+      for (int q = p + 1; q < NV; ++q) {
+        const double x = prow[q] * ip;
+        d[q] = mine ? x : f != 0.0 ? d[q] - f * x : d[q];
       }
 #pragma unroll
-      for (int rr = p + 1; rr < NV; ++rr) {
-        const bool sw = piv == rr;
-        const double x = cp[p], y = cp[rr], u = col[p], w = col[rr];
-        cp[p] = sw ? y : x; cp[rr] = sw ? x : y;
-        col[p] = sw ? w : u; col[rr] = sw ? u : w;
+      for (int q = 0; q < NV; ++q) {
+        const double x = prow[NV + q] * ip;
+        id[q] = mine ? x : f != 0.0 ? id[q] - f * x : id[q];
       }
-      const double ip = 1.0 / cp[p];
-      col[p] *= ip;
-#pragma unroll
-      for (int rr = 0; rr < NV; ++rr) {
-        if (rr == p) continue;
-        const double f = cp[rr];
-        col[rr] = (f != 0.0) ? col[rr] - f * col[p] : col[rr];
-      }
+      pos = mine ? p : pos == p ? piv : pos;
+      wave_order();
     }
-    if (e >= NV && e < 2 * NV) {
+    if (c < W) {
 #pragma unroll
-      for (int rr = 0; rr < NV; ++rr) Lb[c][rr * NV + e - NV] = col[rr];
+      for (int q = 0; q < NV; ++q) cell[pos * NV + q] = valid ? (R)(float)id[q] : R(0);
     }
+    wave_order();
+#pragma unroll
+    for (int q = 0; q < P * ND; ++q) {  // an odd row's second half ends in a zero
+      r1[q / ND][La::n1 + q % ND] = q < NV ? (float)cell[r * NV + min(q, NV - 1)] : 0.0f;
+    }
+#pragma unroll
+    for (int h = 0; h < P; ++h)
+      put_record<La::n2, La::LN>(rec1, record(1, cc, j), lane_of(false, cc, r, h), valid, r1[h]);
     lds_barrier();
-    const float dinv = valid ? (float)Lb[c][e] : 0.0f;
-    if (valid) {
-      put_diag(1, c, j, r, q, dinv);
-      put_diag(2, c, j, q, r, dinv);
-    }
-    ring[lr][0][c][e] = dinv;
   }
 }
 
@@ -379,12 +583,6 @@ __device__ __forceinline__ void lds_write(int* p, int v) {
 }
 __device__ __forceinline__ void lds_release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local"); }
 __device__ __forceinline__ void lds_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local"); }
-// Orders this wave's LDS accesses (a wave's LDS operations execute in issue
-// order, so nothing is waited for).
-__device__ __forceinline__ void wave_order() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-  __builtin_amdgcn_wave_barrier();
-}
 
 constexpr int kAll = 1 << 29;  // a count that never holds the solving wave up
 // Polls without a new row before a link gives up (each takes about a
@@ -520,10 +718,6 @@ __device__ void cilu_load(const float* R, int njc, int ldi, size_t plane, int co
   if (lane == 0) lds_write(&sh.loaded[pass], kAll);
 }
 
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, size_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
-}
 
 // The value of the other lane of the pair.
 __device__ __forceinline__ double pair_sum(double v) {
@@ -886,7 +1080,7 @@ template <int NV, int W, bool NINE, int P>
 static size_t cilu_size_t(int nic, int njc) {
   using La = Lay<NV, W, NINE, P>;
   const int nchunk = (nic + W - 1) / W;
-  return (La::floats(nchunk, njc) + 1) / 2 + La::links(nchunk, njc) + cilu_ops_doubles(nic, njc, NV, W);
+  return (La::floats(nchunk, njc) + 3) / 4 * 2 + La::links(nchunk, njc) + 2 * cilu_ops<NV, W, NINE>(nic, njc) + 1;
 }
 
 template <int NV, int W, bool NINE, int P>
@@ -894,16 +1088,18 @@ static void cilu_factor_t(int nic, int njc, int ldi, const double* idt, const do
                           hipStream_t s) {
   using La = Lay<NV, W, NINE, P>;
   const int nchunk = (nic + W - 1) / W, nlev = njc + 2 * W - 2;
-  const size_t total = cilu_ops_doubles(nic, njc, NV, W), nl = La::links(nchunk, njc);
-  double* links = store + (La::floats(nchunk, njc) + 1) / 2;
-  double* ops = links + nl;
+  const size_t total = cilu_ops<NV, W, NINE>(nic, njc), nl = La::links(nchunk, njc);
+  double* links = store + (La::floats(nchunk, njc) + 3) / 4 * 2;
+  double2* ops = reinterpret_cast<double2*>(links + (nl + 1) / 2 * 2);
   hipLaunchKernelGGL((cilu_zero_kernel<NV, W, NINE, P>), dim3(La::nrec(njc), nchunk * La::NG), dim3(256), 0, s, nic, njc,
                      nchunk, reinterpret_cast<float*>(store));
   const size_t nblk = std::min<size_t>((total + 255) / 256, (size_t)1 << 20);
-  hipLaunchKernelGGL((cilu_gather_kernel<NV, W>), dim3((unsigned)nblk), dim3(256), 0, s, nic, njc, ldi, nlev, idt,
+  hipLaunchKernelGGL((cilu_gather_kernel<NV, W, NINE>), dim3((unsigned)nblk), dim3(256), 0, s, nic, njc, ldi, nlev, idt,
                      blocks, ops, total);
-  hipLaunchKernelGGL((cilu_factor_kernel<NV, W, NINE, P>), dim3(nchunk), dim3(W * NV * NV), 0, s, nic, njc, nlev, ops,
+  hipLaunchKernelGGL((cilu_factor_kernel<NV, W, NINE, P>), dim3(nchunk), dim3(64 * Fac<NV, W, NINE>::NW), 0, s, nic, njc, nlev, ops,
                      reinterpret_cast<float*>(store));
+  hipLaunchKernelGGL((cilu_transpose_kernel<NV, W, NINE, P>), dim3(La::nrec(njc), nchunk * La::NG), dim3(256), 0, s, nic,
+                     njc, nchunk, reinterpret_cast<float*>(store));
   if (nl)
     hipLaunchKernelGGL(cilu_empty_kernel, dim3((unsigned)std::min<size_t>((nl + 255) / 256, 1024)), dim3(256), 0, s,
                        reinterpret_cast<unsigned long long*>(links), nl);
@@ -915,7 +1111,7 @@ static void cilu_apply_t(int nic, int njc, int ldi, double* store, const double*
   using La = Lay<NV, W, NINE, P>;
   const int nchunk = (nic + W - 1) / W;
   const float* rec = reinterpret_cast<const float*>(store);
-  unsigned long long* links = reinterpret_cast<unsigned long long*>(store + (La::floats(nchunk, njc) + 1) / 2);
+  unsigned long long* links = reinterpret_cast<unsigned long long*>(store + (La::floats(nchunk, njc) + 3) / 4 * 2);
   const dim3 grid((nchunk + 7) / 8 * 8 * La::NG), block(La::NG > 1 ? 256 : 192);
   if (tr)
     hipLaunchKernelGGL((cilu_apply_kernel<NV, W, NINE, P, true>), grid, block, 0, s, nic, njc, ldi, nchunk, rec, links, b,
