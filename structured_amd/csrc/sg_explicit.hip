@@ -2,12 +2,12 @@
 // without ADOL-C (src/solver/solver.cpp:103-121) and the loop of
 // Solver::solve (:197-236).
 //
-// Each stage is one residual launch (norms fused into it) and one
-// bandwidth-bound update kernel.  The update recomputes the cell's local time
-// step from the step's base state instead of storing a dt array: the
-// reference computes dt once per step from q (calc_dt, before the stages), and
-// every stage reads that q anyway, so the dt field never reaches HBM.  Per
-// cell and stage the update moves q (nv) + R (nv) + the shorter face length
+// A Runge-Kutta stage is one launch: the residual kernel writes the stage's
+// state instead of R, with the cell's local time step recomputed from the
+// step's base state (the reference computes dt once per step from q, calc_dt,
+// before the stages).  Only the last stage's norms are formed, the others are
+// never seen.  Forward Euler updates the residual's own input, so its update
+// is a kernel of its own, which moves q (nv) + R (nv) + the shorter face length
 // in and nv values out.
 #include <hip/hip_runtime.h>
 
@@ -29,35 +29,26 @@ using namespace sg;
 
 namespace {
 
-// out = q0 + (R dt) / denom with dt = calc_dt(q0) of the cell: update_forward_euler
-// (denom 1) and update_rk4 (denom 4 - stage), src/solver/solver.cpp:12-26.
-// out may alias q0 (each thread reads its cell before writing it).
-__global__ __launch_bounds__(256) void explicit_stage_kernel(DevGeom g, int nv, const double* q0, const double* R,
-                                                             const double* dsmin, double mu_inf, double cfl,
-                                                             double denom, double* out) {
+// q += R dt with dt = calc_dt(q) of the cell: update_forward_euler,
+// src/solver/solver.cpp:12-18.
+__global__ __launch_bounds__(256) void forward_euler_kernel(DevGeom g, int nv, double* q, const double* R,
+                                                            const double* dsmin, double mu_inf, double cfl) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
   if (i >= g.nic) return;
   const size_t c = (size_t)j * g.ldi + i;
   double qv[5], rv[5];
 #pragma unroll
   for (int k = 0; k < 5; ++k) {
-    if (k < nv) { qv[k] = q0[k * g.plane + c]; rv[k] = R[k * g.plane + c]; }
+    if (k < nv) { qv[k] = q[k * g.plane + c]; rv[k] = R[k * g.plane + c]; }
   }
   const double dt = cell_dt(qv[0], qv[1], qv[2], qv[3], dsmin[c], mu_inf, cfl);
 #pragma unroll
   for (int k = 0; k < 5; ++k) {
     if (k < nv) {
 #pragma clang fp contract(off)
-      out[k * g.plane + c] = qv[k] + (rv[k] * dt) / denom;
+      q[k * g.plane + c] = qv[k] + rv[k] * dt;
     }
   }
-}
-
-hipError_t launch_stage(sg_ctx* ctx, const double* q0, const double* R, double cfl, double denom, double* out) {
-  const DevGeom& g = ctx->g;
-  hipLaunchKernelGGL(explicit_stage_kernel, dim3((g.nic + 255) / 256, g.njc), dim3(256), 0, ctx->stream, g, ctx->nvar,
-                     q0, R, ctx->dsmin.p, ctx->ph.mu_inf, cfl, denom, out);
-  return hipGetLastError();
 }
 
 int ensure_buffers(sg_ctx* ctx) {
@@ -69,26 +60,29 @@ int ensure_buffers(sg_ctx* ctx) {
 
 // Enqueues one step; the norms of the last stage's residual land in ctx->l2.
 int enqueue_step(sg_ctx* ctx, double* q, int scheme, double cfl) {
-  double* R = ctx->ex_r.p;
-  auto residual = [&](const double* in) {
-    return launch_residual(ctx->g, ctx->ph, ctx->bc, ctx->sa, in, R, ctx->partial.p, ctx->l2.p, ctx->stream,
-                           ctx->clo);
-  };
+  const DevGeom& g = ctx->g;
   if (scheme == SG_SCHEME_FORWARD_EULER) {
-    SG_TRY(residual(q), "residual");
-    SG_TRY(launch_stage(ctx, q, R, cfl, 1.0, q), "update");
+    double* R = ctx->ex_r.p;
+    SG_TRY(launch_residual(g, ctx->ph, ctx->bc, ctx->sa, q, R, ctx->partial.p, ctx->l2.p, ctx->stream, ctx->clo,
+                           ctx->nvar),
+           "residual");
+    hipLaunchKernelGGL(forward_euler_kernel, dim3((g.nic + 255) / 256, g.njc), dim3(256), 0, ctx->stream, g, ctx->nvar, q,
+                       R, ctx->dsmin.p, ctx->ph.mu_inf, cfl);
+    SG_TRY(hipGetLastError(), "update");
     return SG_OK;
   }
-  // RK4-Jameson: the stage input starts at q (q_tmp = q at the start of
-  // every step of the reference), stages ping-pong between two buffers and
-  // the last one writes q itself.
+  // RK4-Jameson (update_rk4, src/solver/solver.cpp:20-26): the stage input
+  // starts at q (q_tmp = q at the start of every step of the reference),
+  // stages ping-pong between two buffers and the last one writes q itself.
   const double* in = q;
   double* stage_buf[2] = {ctx->ex_a.p, ctx->ex_b.p};
   for (int s = 0; s < 4; ++s) {
-    SG_TRY(residual(in), "residual");
-    double* out = (s == 3) ? q : stage_buf[s & 1];
-    SG_TRY(launch_stage(ctx, q, R, cfl, 4.0 - s, out), "update");
-    in = out;
+    const bool last = s == 3;
+    const ExplicitStage st{q, ctx->dsmin.p, ctx->ph.mu_inf, cfl, 4.0 - s, last ? q : stage_buf[s & 1]};
+    SG_TRY(launch_stage(g, ctx->ph, ctx->bc, ctx->sa, in, st, last ? ctx->partial.p : nullptr, last ? ctx->l2.p : nullptr,
+                        ctx->stream, ctx->clo),
+           "stage");
+    in = st.out;
   }
   return SG_OK;
 }

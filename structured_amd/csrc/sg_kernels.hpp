@@ -15,6 +15,15 @@ size_t residual_partial_count(const DevGeom& g);
 hipError_t launch_residual(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool sa, const double* q, double* r,
                            double* slots, double* l2, hipStream_t s, const DevClosure& clo = DevClosure(),
                            int l2_count = 0);
+// out = q0 + (R(q) dt(q0)) / denom, the stages of an explicit step; with slots
+// the norms of R (nv entries of l2).  out may be q0, but not q.
+struct ExplicitStage {
+  const double *q0, *dsmin;
+  double mu_inf, cfl, denom;
+  double* out;
+};
+hipError_t launch_stage(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool sa, const double* q,
+                        const ExplicitStage& st, double* slots, double* l2, hipStream_t s, const DevClosure& clo);
 // J.v (+ (dR/dbeta).beta_dot when beta_dot is not null; v may be all zero);
 // with idt (per cell) jv receives v idt - J.v instead
 hipError_t launch_jv(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool sa, const double* q, const double* v,

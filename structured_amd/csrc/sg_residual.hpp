@@ -734,8 +734,7 @@ __global__ __launch_bounds__(TX * TY, sizeof(S) == sizeof(double) ? 4 : 2) void 
     }
   }
   if (owns) {
-#pragma unroll
-    for (int k = 0; k < NV; ++k) out.put(k, g.plane, oidx, ci, cj, res[k]);
+    out.template put<NV>(g.plane, oidx, ci, cj, res);
   }
   // ---- the tile's sums of R^2, in a fixed order: 16 threads per norm add 16
   // values each from LDS, then one another's by DPP (a wavefront sum per norm,

@@ -219,8 +219,10 @@ template <>
 struct OutField<double> {
   double* v;
   __device__ __forceinline__ void begin(int) {}
-  __device__ __forceinline__ void put(int k, size_t plane, size_t idx, int, int, double x) const {
-    v[k * plane + idx] = x;
+  template <int NV>
+  __device__ __forceinline__ void put(size_t plane, size_t idx, int, int, const double* x) const {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v[k * plane + idx] = x[k];
   }
 };
 template <>
@@ -231,9 +233,13 @@ struct OutField<Dual> {
   const double* idt = nullptr;
   const double* z = nullptr;
   __device__ __forceinline__ void begin(int) {}
-  __device__ __forceinline__ void put(int k, size_t plane, size_t idx, int, int, Dual x) const {
-    if (v) v[k * plane + idx] = x.v;
-    d[k * plane + idx] = idt ? z[k * plane + idx] * idt[idx] - x.d : x.d;
+  template <int NV>
+  __device__ __forceinline__ void put(size_t plane, size_t idx, int, int, const Dual* x) const {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      if (v) v[k * plane + idx] = x[k].v;
+      d[k * plane + idx] = idt ? z[k * plane + idx] * idt[idx] - x[k].d : x[k].d;
+    }
   }
 };
 
@@ -245,7 +251,8 @@ struct OutBlocks {
   double* blocks;
   Direction dir;
   __device__ __forceinline__ void begin(int z) { dir.begin(z); }
-  __device__ __forceinline__ void put(int k, size_t plane, size_t idx, int ci, int cj, Dual x) const {
+  template <int NV>
+  __device__ __forceinline__ void put(size_t plane, size_t idx, int ci, int cj, const Dual* x) const {
     const int h = dir.per / 2;
     int di = (dir.a - ci) % dir.per, dj = (dir.b - cj) % dir.per;
     di += di < -h ? dir.per : 0;
@@ -258,7 +265,9 @@ struct OutBlocks {
     int slot = box ? (int)(kBox >> (4 * (3 * (dj + 1) + di + 1))) & 15 : -1;
     if (!box && di == 0) slot = dj < 0 ? 9 : 10;
     if (!box && dj == 0) slot = di < 0 ? 11 : 12;
-    if (slot >= 0) blocks[(size_t)((slot * dir.nv + k) * dir.nv + dir.m) * plane + idx] = x.d;
+    if (slot < 0) return;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) blocks[(size_t)((slot * NV + k) * NV + dir.m) * plane + idx] = x[k].d;
   }
 };
 

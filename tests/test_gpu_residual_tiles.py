@@ -35,3 +35,33 @@ def test_tiles_vs_oracle(cols, rows, sa, flux, order):
         np.testing.assert_allclose(l2, np.sqrt((r ** 2).sum(axis=(0, 1))), rtol=1e-12)
     assert rel(eq.jv(q, v), of.jv(case, q, v, wd=wd)[1]) <= 1e-10
     eq.close()
+
+
+@pytest.mark.parametrize("cols,rows", [(3, 3), (31, 7), (32, 8), (495, 239)])
+@pytest.mark.parametrize("sa", [False, True])
+def test_stages_written_by_the_residual(cols, rows, sa):
+    """A Runge-Kutta step, whose stages are the residual kernel's output,
+    against its residuals and time steps taken one by one."""
+    import torch
+    case = cases.sa_bump(cols + 1, rows + 1, dy1=1e-3) if sa else cases.laminar_plate(cols + 1, rows + 1, dy1=1e-3)
+    q0 = case.perturbed_state(seed=3, amp=0.01)
+    eq = lib.Equation(case)
+    dev = torch.device("cuda:0")
+    aos = torch.from_numpy(np.ascontiguousarray(q0).reshape(-1)).to(dev)
+    qd = torch.zeros(eq.nvar * eq.plane, dtype=torch.float64, device=dev)
+    eq.aos_to_soa_dev(aos.data_ptr(), qd.data_ptr())
+    eq.synchronize()
+    l2 = eq.step_explicit_dev(qd.data_ptr(), "rk4_jameson", 0.5)
+    eq.soa_to_aos_dev(qd.data_ptr(), aos.data_ptr())
+    eq.synchronize()
+    got = aos.cpu().numpy().reshape(q0.shape)
+    dt, q = eq.calc_dt(q0, 0.5), q0
+    for s in range(4):
+        r, norms = eq.calc_residual(q)
+        q = q0 + (r * dt) / (4.0 - s)
+    # the same operations on the same residuals; the host's and the device's
+    # square root and divisions may differ in the last place
+    for m in range(eq.nvar):
+        assert rel(got[..., m], q[..., m]) <= 1e-13
+    np.testing.assert_allclose(l2, norms, rtol=1e-10)
+    eq.close()
