@@ -24,7 +24,8 @@ static bool wide_rows(const DevGeom& g) {
 // registers, and the one has nothing to run at its barriers).  Measured, 16
 // against 8 rows, SA residual: 67 / 75 us at 1409x641, 22 / 25 at 705x321,
 // equal at 545x385, 20.5 / 18 at 481x257, 15.7 / 14.7 at 449x225; J.v: 32 / 36
-// at 705x321, 32 / 30 at 545x385, 76 / 68 at 1001x501.
+// at 705x321, 32 / 30 at 545x385, 76 / 68 at 1001x501 (both sides while the
+// kernels still spilled, which cost either 4 to 8%).
 // With a coloured direction per z-layer the chip is full and the larger tile is
 // 4% faster (J^T psi at 385x193: 1.91 / 1.99 ms).
 template <class S>

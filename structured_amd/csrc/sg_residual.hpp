@@ -26,9 +26,10 @@
 // ends of grid lines are handled by clamped indices and selects, where a
 // branch per variable and per kind of face kept the loads of a face behind one
 // another and cost a third of the instructions that are not FP64; ghost cells
-// are evaluated once, by threads of their own.  With it and a finaliser that
-// waits on slots instead of counting arrivals, SA at 545x385 24.0 -> 21.6 us,
-// 1409x641 76 -> 68, laminar 97x65 16.4 -> 9.0; J.v at 705x321 41.5 -> 32.7.
+// are evaluated once, by threads of their own.  With it, a finaliser that waits
+// on slots instead of counting arrivals, and metrics loaded just ahead of their
+// use so that nothing spills, SA at 545x385 24.0 -> 20.8 us, 1409x641 77 -> 62.5,
+// laminar 97x65 16.4 -> 9.0; J.v at 705x321 41.5 -> 32.6.
 #pragma once
 #include "sg_closure.hpp"
 #include "sg_device.hpp"
@@ -515,11 +516,13 @@ __global__ __launch_bounds__(TX * TY, sizeof(S) == sizeof(double) ? 4 : 2) void 
     if (node >= 0) P = eval_node<S, SA>(node, bc, q, g, ph);
     stage(gp, gp % RW, gp / RW, P);
   }
-  // ---- metrics of this thread's two faces and cell, in flight over the barrier and
-  // the reconstruction.  At the ends of a grid
-  // line the neighbour index is clamped: the mean of a face's normal (a
-  // cell's volume) with itself is the one-sided value that belongs there,
-  // and a thread without a face computes one that nothing reads.
+  // ---- metrics of this thread's two faces and cell, loaded where they are used.
+  // Loaded together ahead of the reconstruction, the 128 registers did not hold
+  // them: the spills were 10 of 40 MB that a launch moved at 545x385, and cost 1 us
+  // there, 6 at 1409x641.  The other waves cover the wait.  At the ends of a grid
+  // line the neighbour index is clamped: the mean of a face's normal (a cell's
+  // volume) with itself is the one-sided value that belongs there, and a thread
+  // without a face computes one that nothing reads.
   const int fi = i0 + tx, cj = j0 + ty;  // the chi face's row is the eta face's upper cell
   double2 C0, CL_, CR, Cb, CRb, E0, EL, Et, ELt, Eb;
   double V0, VL, VB;
@@ -528,17 +531,11 @@ __global__ __launch_bounds__(TX * TY, sizeof(S) == sizeof(double) ? 4 : 2) void 
   auto nc = [&](int f, int r) { return double2{tile_at<I>(g.ncx, g.ldf, jo, io, f, r), tile_at<I>(g.ncy, g.ldf, jo, io, f, r)}; };
   auto ne = [&](int c, int r) { return double2{tile_at<I>(g.nex, g.ldi, jo, io, c, r), tile_at<I>(g.ney, g.ldi, jo, io, c, r)}; };
   auto vol = [&](int c, int r) { return tile_at<I>(g.vol, g.ldi, jo, io, c, r); };
-  {
-    const int fl = max(f0 - 1, 0), cl = min(fl, c0), r0 = min(cj, njc - 1), et = min(e0 + 1, njc);
-    C0 = nc(f0, r0); CL_ = nc(fl, r0); CR = nc(fr, r0);
-    E0 = ne(c0, e0); EL = ne(cl, e0); Et = ne(c0, et); ELt = ne(cl, et);
-    V0 = vol(c0, r0); VL = vol(cl, r0);
-  }
-
+  const int fl = max(f0 - 1, 0), cl = min(fl, c0), r0 = min(cj, njc - 1), et = min(e0 + 1, njc);
+  C0 = nc(f0, r0);
   __syncthreads();
 
   auto at = [&](int k, int lx, int ly) -> S { return lds[k * NPOS + ly * RW + lx]; };
-
 
   S hc[NV], he[NV];
 
@@ -550,9 +547,9 @@ __global__ __launch_bounds__(TX * TY, sizeof(S) == sizeof(double) ? 4 : 2) void 
     if (ph.order == 2) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const S cl = at(L_R + k, xl, y), cr = at(L_R + k, xr, y);
-        st[0][k] = ssel(sl, muscl_left(at(L_R + k, xl - 1, y), cl, cr, ph.eps_chi), cl);
-        st[1][k] = ssel(sr, muscl_right(cl, cr, at(L_R + k, xr + 1, y), ph.eps_chi), cr);
+        const S a = at(L_R + k, xl, y), b = at(L_R + k, xr, y);
+        st[0][k] = ssel(sl, muscl_left(at(L_R + k, xl - 1, y), a, b, ph.eps_chi), a);
+        st[1][k] = ssel(sr, muscl_right(a, b, at(L_R + k, xr + 1, y), ph.eps_chi), b);
       }
     } else {
 #pragma unroll
@@ -562,6 +559,9 @@ __global__ __launch_bounds__(TX * TY, sizeof(S) == sizeof(double) ? 4 : 2) void 
     if (SA) { ntl = at(L_N, xl, y); ntr = at(L_N, xr, y); }
     conv_flux<S, SA>(ph.flux, C0.x, C0.y, st[0][0], st[0][1], st[0][2], st[0][3], st[1][0], st[1][1], st[1][2], st[1][3],
                      ntl, ntr, hc);
+    CL_ = nc(fl, r0); CR = nc(fr, r0);
+    E0 = ne(c0, e0); EL = ne(cl, e0); Et = ne(c0, et); ELt = ne(cl, et);
+    V0 = vol(c0, r0); VL = vol(cl, r0);
     if (ph.viscous) {
       FaceGeo<S> G;
       G.tx = 0.5 * (Et.x + ELt.x); G.ty = 0.5 * (Et.y + ELt.y);
@@ -591,8 +591,6 @@ __global__ __launch_bounds__(TX * TY, sizeof(S) == sizeof(double) ? 4 : 2) void 
     }
   }
 
-  Cb = nc(f0, eb); CRb = nc(fr, eb); Eb = ne(c0, eb); VB = vol(c0, eb);
-
   // ---- eta face fj on column ci (between cells fj-1 and fj)
   {
     const int x = tx + 2, ys = ty + 1, yn = ty + 2;
@@ -613,6 +611,7 @@ __global__ __launch_bounds__(TX * TY, sizeof(S) == sizeof(double) ? 4 : 2) void 
     if (SA) { nts = at(L_N, x, ys); ntn = at(L_N, x, yn); }
     conv_flux<S, SA>(ph.flux, E0.x, E0.y, st[0][0], st[0][1], st[0][2], st[0][3], st[1][0], st[1][1], st[1][2], st[1][3],
                      nts, ntn, he);
+    Cb = nc(f0, eb); CRb = nc(fr, eb); Eb = ne(c0, eb); VB = vol(c0, eb);
     if (ph.viscous) {
       FaceGeo<S> G;
       G.tx = 0.5 * (E0.x + Et.x); G.ty = 0.5 * (E0.y + Et.y);
