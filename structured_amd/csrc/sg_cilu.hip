@@ -24,6 +24,7 @@
 #include <utility>
 
 #include "sg_linalg.hpp"
+#include "sg_pass_order.hpp"
 
 namespace sg {
 
@@ -180,9 +181,9 @@ struct Lay {
     const int q = n / 4;
     return f < 4 * q ? (unsigned)((f / 4 * LN + lane) * 4 + (f & 3)) : (unsigned)(4 * q * LN + (f - 4 * q) * LN + lane);
   }
-  // words of one link (edge values of one pass, all rows) and of all links
+  // words of one link (edge values, all rows) and of all links
   __host__ __device__ static size_t link(int njc) { return (size_t)njc * GC * NV; }
-  static size_t links(int nchunk, int njc) { return 2 * (size_t)nchunk * (NG - 1) * link(njc); }
+  static size_t links(int nchunk, int njc) { return (size_t)nchunk * (NG - 1) * link(njc); }
 };
 
 // Zeroes the records of M^-1 that the factorisation does not write, or writes
@@ -571,9 +572,9 @@ struct ApplyLds {
   double ring[kRing][NP + 1][NVP] __attribute__((aligned(16)));
   double x[kRing][La::ROWS + 1];  // the last place is always zero
   double tmp[La::GW + 1][8] __attribute__((aligned(16)));  // a row's halves at 0 and 4
-  // per pass: steps solved, right-hand-side rows loaded, edge rows received,
-  // rows taken out of the ring, rows whose stores are complete
-  int step[2], loaded[2], edges[2], taken[2], stored[2];
+  // steps solved, right-hand-side rows loaded, edge rows received, rows taken
+  // out of the ring
+  int step, loaded, edges, taken;
 };
 __device__ __forceinline__ int lds_read(const int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -586,9 +587,8 @@ __device__ __forceinline__ void lds_acquire() { __builtin_amdgcn_fence(__ATOMIC_
 
 constexpr int kAll = 1 << 29;  // a count that never holds the solving wave up
 // Polls without a new row before a link gives up (each takes about a
-// microsecond, so several seconds).  The groups of a chunk are dispatched
-// one after another, so the one that fills a link runs or has run, and the
-// wait ends.
+// microsecond, so several seconds).  The one that fills a link runs or has run
+// (sg_pass_order.hpp), so the wait ends.
 constexpr int kLinkPolls = 1 << 22;
 
 // The receiving wave of one pass: moves the edge rows the group before
@@ -596,7 +596,7 @@ constexpr int kLinkPolls = 1 << 22;
 // word is read as one 64-bit atomic and holds either a value or kEmpty, so
 // nothing has to be ordered between words.
 template <int NV, int W, bool NINE, int P>
-__device__ void cilu_receive(unsigned long long* in, int njc, ApplyLds<NV, W, NINE, P>& sh, int pass) {
+__device__ void cilu_receive(unsigned long long* in, int njc, ApplyLds<NV, W, NINE, P>& sh) {
   using La = Lay<NV, W, NINE, P>;
   constexpr int EN = La::GCX * NV, RP = 64 / EN;
   const int lane = threadIdx.x & 63, rr = lane / EN, gi = lane % EN / NV, k = lane % NV;
@@ -604,7 +604,7 @@ __device__ void cilu_receive(unsigned long long* in, int njc, ApplyLds<NV, W, NI
   while (n < njc) {
     // edge column gi's row s belongs to step s + X - 2 (1 + gi); its place
     // holds a value that is read up to three steps after its own
-    const int row = n + rr, free = lds_read(&sh.step[pass]) + kRing - 8 - La::X;
+    const int row = n + rr, free = lds_read(&sh.step) + kRing - 8 - La::X;
     unsigned long long v = kEmpty;
     if (rr < RP && row < njc && row < free)
       v = __hip_atomic_load(in + (size_t)row * EN + lane % EN, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -619,12 +619,12 @@ __device__ void cilu_receive(unsigned long long* in, int njc, ApplyLds<NV, W, NI
       sh.ring[(row + La::X - 2 * (1 + gi)) & (kRing - 1)][La::GCX - 1 - gi][k] = __longlong_as_double((long long)v);
     n += rows;
     lds_release();
-    if (lane == 0) lds_write(&sh.edges[pass], n < njc ? n : kAll);
+    if (lane == 0) lds_write(&sh.edges, n < njc ? n : kAll);
   }
   if (n < njc) {  // never filled: every value that depends on it becomes NaN
     for (int e = lane; e < kRing * EN; e += 64) sh.ring[e / EN][e % EN / NV][e % NV] = __builtin_nan("");
     lds_release();
-    if (lane == 0) lds_write(&sh.edges[pass], kAll);
+    if (lane == 0) lds_write(&sh.edges, kAll);
   }
 }
 
@@ -634,7 +634,7 @@ __device__ void cilu_receive(unsigned long long* in, int njc, ApplyLds<NV, W, NI
 // stores held up the loads, whose waits run in issue order.
 template <int NV, int W, bool NINE, int P, bool ASC>
 __device__ void cilu_store(double* z, int njc, int ldi, size_t plane, int col0, int wk, unsigned long long* out,
-                           ApplyLds<NV, W, NINE, P>& sh, int pass) {
+                           ApplyLds<NV, W, NINE, P>& sh) {
   using La = Lay<NV, W, NINE, P>;
   constexpr int LAST = La::X + 2 * (La::GW - 1), RB = 4;
   const int lane = threadIdx.x & 63, k = lane % NV, c1 = lane / NV, c = ASC ? c1 : La::GW - 1 - c1;
@@ -642,7 +642,7 @@ __device__ void cilu_store(double* z, int njc, int ldi, size_t plane, int col0, 
   const bool live = c1 < La::GW && c < wk, pub = out && c1 < La::GW && gi < La::GC;
   double* zl = z + (size_t)k * plane + col0 + (live ? c : 0);
   for (int n = 0; n < njc;) {
-    const int rows = min(min(lds_read(&sh.step[pass]) - LAST, njc) - n, RB);
+    const int rows = min(min(lds_read(&sh.step) - LAST, njc) - n, RB);
     if (rows <= 0) {
       __builtin_amdgcn_s_sleep(1);
       continue;
@@ -662,10 +662,8 @@ __device__ void cilu_store(double* z, int njc, int ldi, size_t plane, int col0, 
     }
     n += rows;
     lds_release();
-    if (lane == 0) lds_write(&sh.taken[pass], n < njc ? n : kAll);
+    if (lane == 0) lds_write(&sh.taken, n < njc ? n : kAll);
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  if (lane == 0) lds_write(&sh.stored[pass], 1);
 }
 
 // The loading wave of one pass: brings the right-hand sides into LDS by step
@@ -675,7 +673,7 @@ __device__ void cilu_store(double* z, int njc, int ldi, size_t plane, int col0, 
 // L2 instead of memory (much further ahead, the groups of an XCD overflow it).
 template <int NV, int W, bool NINE, int P, bool ASC, bool DIAG>
 __device__ void cilu_load(const float* R, int njc, int ldi, size_t plane, int col0, int wk, const double* src,
-                          ApplyLds<NV, W, NINE, P>& sh, int pass) {
+                          ApplyLds<NV, W, NINE, P>& sh) {
   using La = Lay<NV, W, NINE, P>;
   constexpr int RS = La::rs(DIAG ? La::n2 : La::n1), LB = 16, TAIL = 2 * (La::GW - 1);
   // a batch is fetched when the solving wave is at step s0 - (kRing - X - TAIL)
@@ -707,15 +705,15 @@ __device__ void cilu_load(const float* R, int njc, int ldi, size_t plane, int co
       for (int u = 0; u < LB; ++u) asm volatile("" ::"v"(touch[u]));
       fetch(s1 + LB, b ^ 1);
       // the last place this batch writes must have been read
-      while (lds_read(&sh.step[pass]) < La::X + s1 + LB - 1 + TAIL + 1 - kRing) __builtin_amdgcn_s_sleep(2);
+      while (lds_read(&sh.step) < La::X + s1 + LB - 1 + TAIL + 1 - kRing) __builtin_amdgcn_s_sleep(2);
 #pragma unroll
       for (int u = 0; u < LB; ++u)
         if (lane < La::ROWS) sh.x[(La::X + s1 + u + 2 * c1) & (kRing - 1)][lane] = live && s1 + u < njc ? v[b][u] : 0.0;
       lds_release();
-      if (lane == 0) lds_write(&sh.loaded[pass], s1 + LB);
+      if (lane == 0) lds_write(&sh.loaded, s1 + LB);
     }
   }
-  if (lane == 0) lds_write(&sh.loaded[pass], kAll);
+  if (lane == 0) lds_write(&sh.loaded, kAll);
 }
 
 
@@ -736,7 +734,7 @@ __device__ __forceinline__ double pair_sum(double v) {
 // neighbours is done by the other waves, and no step has a branch but the one
 // that waits for them.
 template <int NV, int W, bool NINE, bool DIAG>
-__device__ __forceinline__ void cilu_solve_pairs(const float* R, int njc, ApplyLds<NV, W, NINE, 2>& sh, int pass, bool up) {
+__device__ __forceinline__ void cilu_solve_pairs(const float* R, int njc, ApplyLds<NV, W, NINE, 2>& sh, bool up) {
   using La = Lay<NV, W, NINE, 2>;
   using A = ApplyLds<NV, W, NINE, 2>;
   constexpr int N = DIAG ? La::n2 : La::n1, RS = La::rs(N), NQ = N / 4, NREM = N % 4, PD = La::pd(N), UN = La::UN, ND = La::ND;
@@ -778,8 +776,8 @@ __device__ __forceinline__ void cilu_solve_pairs(const float* R, int njc, ApplyL
     if (__builtin_expect(t < lim, 1)) return;
     do {
       // x is read one step early
-      const int a = lds_read(&sh.loaded[pass]) + La::X - 1, b = up ? lds_read(&sh.edges[pass]) + 1 : kAll;
-      const int c = lds_read(&sh.taken[pass]) + kRing + La::X;
+      const int a = lds_read(&sh.loaded) + La::X - 1, b = up ? lds_read(&sh.edges) + 1 : kAll;
+      const int c = lds_read(&sh.taken) + kRing + La::X;
       lim = __builtin_amdgcn_readfirstlane(min(min(a, b), c));
     } while (t >= lim);
     lds_acquire();
@@ -846,7 +844,7 @@ __device__ __forceinline__ void cilu_solve_pairs(const float* R, int njc, ApplyL
       auto* cur = sh.ring[r0 + u];
       cur[wpos][k] = r;
       wave_order();
-      if (u & 1) lds_write(&sh.step[pass], t + 1);
+      if (u & 1) lds_write(&sh.step, t + 1);
       if (u & 1) wait(t + 2);  // for the next two steps
       const double* yn = u == 0 ? y0 : sh.ring[r0 + u - 1 + h][pos - 1];
 #pragma unroll
@@ -867,7 +865,7 @@ __device__ __forceinline__ void cilu_solve_pairs(const float* R, int njc, ApplyL
 
 // The same with one lane a row, which takes both operands of either kind.
 template <int NV, int W, bool NINE, bool DIAG>
-__device__ __forceinline__ void cilu_solve_rows(const float* R, int njc, ApplyLds<NV, W, NINE, 1>& sh, int pass, bool up) {
+__device__ __forceinline__ void cilu_solve_rows(const float* R, int njc, ApplyLds<NV, W, NINE, 1>& sh, bool up) {
   using La = Lay<NV, W, NINE, 1>;
   using A = ApplyLds<NV, W, NINE, 1>;
   constexpr int N = DIAG ? La::n2 : La::n1, RS = La::rs(N), NQ = N / 4, NREM = N % 4, PD = La::pd(N), UN = La::UN;
@@ -904,8 +902,8 @@ __device__ __forceinline__ void cilu_solve_rows(const float* R, int njc, ApplyLd
     if (__builtin_expect(t < lim, 1)) return;
     do {
       // x is read one step early
-      const int a = lds_read(&sh.loaded[pass]) + La::X - 1, b = up ? lds_read(&sh.edges[pass]) + 1 : kAll;
-      const int c = lds_read(&sh.taken[pass]) + kRing + La::X;
+      const int a = lds_read(&sh.loaded) + La::X - 1, b = up ? lds_read(&sh.edges) + 1 : kAll;
+      const int c = lds_read(&sh.taken) + kRing + La::X;
       lim = __builtin_amdgcn_readfirstlane(min(min(a, b), c));
     } while (t >= lim);
     lds_acquire();
@@ -974,7 +972,7 @@ __device__ __forceinline__ void cilu_solve_rows(const float* R, int njc, ApplyLd
       auto* cur = sh.ring[r0 + u];
       cur[wpos][k] = r;
       wave_order();
-      if (u & 1) lds_write(&sh.step[pass], t + 1);
+      if (u & 1) lds_write(&sh.step, t + 1);
       if (u & 1) wait(t + 2);  // for the next two steps
       double own2[NV], old[NV];
 #pragma unroll
@@ -996,17 +994,19 @@ __device__ __forceinline__ void cilu_solve_rows(const float* R, int njc, ApplyLd
 }
 
 template <int NV, int W, bool NINE, int P, bool DIAG>
-__device__ __forceinline__ void cilu_solve(const float* R, int njc, ApplyLds<NV, W, NINE, P>& sh, int pass, bool up) {
-  if constexpr (P == 2) cilu_solve_pairs<NV, W, NINE, DIAG>(R, njc, sh, pass, up);
-  else cilu_solve_rows<NV, W, NINE, DIAG>(R, njc, sh, pass, up);
+__device__ __forceinline__ void cilu_solve(const float* R, int njc, ApplyLds<NV, W, NINE, P>& sh, bool up) {
+  if constexpr (P == 2) cilu_solve_pairs<NV, W, NINE, DIAG>(R, njc, sh, up);
+  else cilu_solve_rows<NV, W, NINE, DIAG>(R, njc, sh, up);
 }
 
-// z = (LU)^-1 b, or (LU)^-T b when TR.  Wave 0 of a work-group solves one
-// column group, wave 1 loads and wave 2 stores for it, and wave 3 receives
-// the edge columns of the group before where a chunk has several.
-// Work-groups are dealt to the XCDs round-robin by index: the groups of a
-// chunk sit on one XCD, consecutive in its order, so a group's neighbours are
-// dispatched with it.
+// One pass of z = (LU)^-1 b, or of (LU)^-T b when TR: the ascending one, or
+// the descending one, in place.  Wave 0 of a work-group solves one column
+// group, wave 1 loads and wave 2 stores for it, and wave 3 receives the edge
+// columns of the group before where a chunk has several.  A launch per pass:
+// with both in one, a group waited in the second for groups started after it,
+// which needs room for all groups of a chunk on its XCD.  The second launch
+// costs 2% of an apply at 1409x641 (450 us against 442), 1% of a Newton solve
+// at 97x65.
 //
 // What bounds it: a step of the solving wave, some 57 instructions of one wave
 // and the LDS exchanges that link two steps, times njc + 2 W steps and a pass,
@@ -1014,65 +1014,54 @@ __device__ __forceinline__ void cilu_solve(const float* R, int njc, ApplyLds<NV,
 // a step (nv 4: 120-150), one lane 200-215 (155-185; with its records beyond
 // L2 290, as one CU takes about 18 bytes/ns from memory); with one work-group
 // of nv W threads per chunk and a barrier per level it was 600.  Precond 7,
-// W 32, M^-1 (M^-T alike), at first / one lane / two lanes: 97x65 nv 4 101 / 54
-// / 51 us, 97x257 nv 5 - / 156 / 135, 705x257 - / 160 / 141, 1409x641 966 / 442
-// / 576 (more groups than CUs).
-template <int NV, int W, bool NINE, int P, bool TR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void cilu_apply_kernel(
-    int nic, int njc, int ldi, int nchunk, const float* rec, unsigned long long* links, const double* b, double* z) {
+// W 32, M^-1 (M^-T alike), at first / one lane / two lanes (the first two of a
+// row with both passes in one launch): 97x65 nv 4 101 / 54 / 52 us, 97x257 nv 5
+// - / 156 / 136, 705x257 - / 160 / 143; 1409x641 (more groups than CUs with two
+// lanes) 966 / 448 / 576, the last with both passes in one launch.
+template <int NV, int W, bool NINE, int P, bool TR, bool ASC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void cilu_pass_kernel(
+    int nic, int njc, int ldi, int nchunk, const float* rec, unsigned long long* links, const double* src, double* z) {
   using La = Lay<NV, W, NINE, P>;
+  // non-transposed: unit-lower L ascending, then D + U descending;
+  // transposed: (D + U)^T ascending, then unit-lower L^T descending
+  constexpr bool DIAG = TR == ASC;
+  constexpr int A = (TR ? 2 : 0) + (ASC ? 0 : 1);
   __shared__ ApplyLds<NV, W, NINE, P> sh;
-  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int chunk = slot / La::NG * 8 + xcd, g = slot % La::NG;
+  const PassGroup at = pass_group((int)blockIdx.x, La::NG, ASC);
+  const int chunk = at.chunk, g = at.group;
   if (chunk >= nchunk) return;
   const int i0 = chunk * W, wk = min(W, nic - i0) - g * La::GW;  // columns from this group on
   if (wk <= 0) return;
-  const bool left = g > 0, right = wk > La::GW;
+  const bool left = g > 0, right = wk > La::GW, from = ASC ? left : right, to = ASC ? right : left;
   // values of steps not yet solved, and the place after an odd row's last
   // entry, meet zero factors: they need to be finite
   double* zero = &sh.ring[0][0][0];
   for (int e = threadIdx.x; e < (int)(sizeof(sh.ring) / sizeof(double)); e += blockDim.x) zero[e] = 0.0;
   for (int e = threadIdx.x; e < (int)(sizeof(sh.tmp) / sizeof(double)); e += blockDim.x) (&sh.tmp[0][0])[e] = 0.0;
-  if (threadIdx.x < 2) {
-    sh.step[threadIdx.x] = sh.edges[threadIdx.x] = sh.taken[threadIdx.x] = sh.stored[threadIdx.x] = 0;
-    sh.loaded[threadIdx.x] = -La::X;  // not even the steps before the first row may start
+  if (threadIdx.x == 0) {
+    sh.step = sh.edges = sh.taken = 0;
+    sh.loaded = -La::X;  // not even the steps before the first row may start
   }
   __syncthreads();
   const size_t plane = (size_t)njc * ldi, gr = (size_t)(chunk * La::NG + g) * La::nrec(njc);
-  const float* R1 = rec + La::array(TR ? 2 : 0, nchunk, njc) + gr * La::rs(TR ? La::n2 : La::n1);
-  const float* R2 = rec + La::array(TR ? 3 : 1, nchunk, njc) + gr * La::rs(TR ? La::n1 : La::n2);
+  const float* R = rec + La::array(A, nchunk, njc) + gr * La::rs(La::count(A));
   const int col0 = i0 + g * La::GW, wg = min(wk, La::GW);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // link l of a pass joins groups l and l + 1
+  // link l joins groups l and l + 1
   const size_t lw = La::link(njc);
-  unsigned long long* la = links + (size_t)chunk * (La::NG - 1) * lw;
-  unsigned long long* ld = la + (size_t)nchunk * (La::NG - 1) * lw;
-  // non-transposed: unit-lower L ascending, then D + U descending;
-  // transposed: (D + U)^T ascending, then unit-lower L^T descending
+  unsigned long long* link = links + (size_t)chunk * (La::NG - 1) * lw;
+  unsigned long long *in = link + (ASC ? g - 1 : g) * lw, *out = link + (ASC ? g : g - 1) * lw;
   if (wave == 0) {
-    cilu_solve<NV, W, NINE, P, TR>(R1, njc, sh, 0, left);
-    cilu_solve<NV, W, NINE, P, !TR>(R2, njc, sh, 1, right);
+    cilu_solve<NV, W, NINE, P, DIAG>(R, njc, sh, from);
   } else if (wave == 1) {
-    cilu_load<NV, W, NINE, P, true, TR>(R1, njc, ldi, plane, col0, wg, b, sh, 0);
-    // the second pass loads what the first stored, and reuses its LDS
-    while (!lds_read(&sh.stored[0]) || lds_read(&sh.step[0]) < La::steps(njc)) __builtin_amdgcn_s_sleep(1);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    cilu_load<NV, W, NINE, P, false, !TR>(R2, njc, ldi, plane, col0, wg, z, sh, 1);
+    cilu_load<NV, W, NINE, P, ASC, DIAG>(R, njc, ldi, plane, col0, wg, src, sh);
   } else if (wave == 2) {
-    cilu_store<NV, W, NINE, P, true>(z, njc, ldi, plane, col0, wg, right ? la + g * lw : nullptr, sh, 0);
-    cilu_store<NV, W, NINE, P, false>(z, njc, ldi, plane, col0, wg, left ? ld + (g - 1) * lw : nullptr, sh, 1);
-  } else {
-    if (left) cilu_receive<NV, W, NINE, P>(la + (g - 1) * lw, njc, sh, 0);
-    if (right) {
-      // the first pass is done with the edge columns' places
-      while (lds_read(&sh.step[0]) < La::steps(njc)) __builtin_amdgcn_s_sleep(1);
-      cilu_receive<NV, W, NINE, P>(ld + g * lw, njc, sh, 1);
-    }
-    // the links are empty for the next apply
-    for (size_t e = threadIdx.x & 63; e < lw; e += 64) {
-      if (left) __hip_atomic_store(la + (g - 1) * lw + e, kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (right) __hip_atomic_store(ld + g * lw + e, kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    cilu_store<NV, W, NINE, P, ASC>(z, njc, ldi, plane, col0, wg, to ? out : nullptr, sh);
+  } else if (from) {
+    cilu_receive<NV, W, NINE, P>(in, njc, sh);
+    // empty for the next pass
+    for (size_t e = threadIdx.x & 63; e < lw; e += 64)
+      __hip_atomic_store(in + e, kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -1112,13 +1101,17 @@ static void cilu_apply_t(int nic, int njc, int ldi, double* store, const double*
   const int nchunk = (nic + W - 1) / W;
   const float* rec = reinterpret_cast<const float*>(store);
   unsigned long long* links = reinterpret_cast<unsigned long long*>(store + (La::floats(nchunk, njc) + 3) / 4 * 2);
-  const dim3 grid((nchunk + 7) / 8 * 8 * La::NG), block(La::NG > 1 ? 256 : 192);
-  if (tr)
-    hipLaunchKernelGGL((cilu_apply_kernel<NV, W, NINE, P, true>), grid, block, 0, s, nic, njc, ldi, nchunk, rec, links, b,
-                       z);
-  else
-    hipLaunchKernelGGL((cilu_apply_kernel<NV, W, NINE, P, false>), grid, block, 0, s, nic, njc, ldi, nchunk, rec, links,
-                       b, z);
+  const dim3 grid(pass_blocks(nchunk, La::NG)), block(La::NG > 1 ? 256 : 192);
+  auto pass = [&](auto kernel, const double* src) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, nic, njc, ldi, nchunk, rec, links, src, z);
+  };
+  if (tr) {
+    pass(cilu_pass_kernel<NV, W, NINE, P, true, true>, b);
+    pass(cilu_pass_kernel<NV, W, NINE, P, true, false>, z);
+  } else {
+    pass(cilu_pass_kernel<NV, W, NINE, P, false, true>, b);
+    pass(cilu_pass_kernel<NV, W, NINE, P, false, false>, z);
+  }
 }
 
 bool cilu_width_ok(int w) { return w == 8 || w == 16 || w == 24 || w == 32; }
