@@ -173,9 +173,11 @@ struct Lay {
     const size_t per = (size_t)nchunk * NG * nrec(njc);
     return per * (a == 0 ? 0 : a == 1 ? rs(n1) : a == 2 ? rs(n1) + rs(n2) : rs(n1) + 2 * rs(n2));
   }
-  __host__ __device__ static size_t floats(int nchunk, int njc) {
-    return (size_t)nchunk * NG * nrec(njc) * (2 * rs(n1) + 2 * rs(n2));
+  // one more record per chunk, for what the factorisation's idle lanes store
+  __host__ __device__ static size_t spare(int chunk, int nchunk, int njc) {
+    return (size_t)nchunk * NG * nrec(njc) * (2 * rs(n1) + 2 * rs(n2)) + (size_t)chunk * rs(n2);
   }
+  __host__ __device__ static size_t floats(int nchunk, int njc) { return spare(nchunk, nchunk, njc); }
   // float of entry f on a lane inside a record of n floats per lane
   __device__ static unsigned in_record(int n, int lane, int f) {
     const int q = n / 4;
@@ -327,21 +329,16 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, size_
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
 }
 
-constexpr unsigned kNowhere = 0xFFFFFF00u;  // beyond every buffer: such a store is dropped
-// A record's n floats of a lane, in the layout of Lay::in_record, at byte
-// offset `at` of the buffer.
+// A record's n floats of a lane, in the layout of Lay::in_record.
 template <int N, int LN>
-__device__ __forceinline__ void put_record(__amdgpu_buffer_rsrc_t rec, unsigned at, int lane, bool on, const float* v) {
+__device__ __forceinline__ void put_record(float* rec, int lane, const float* v) {
+  float* quads = rec + 4 * lane;
 #pragma unroll
-  for (int q = 0; q < N / 4; ++q) {
-    const u32x4 w = {__float_as_uint(v[4 * q]), __float_as_uint(v[4 * q + 1]), __float_as_uint(v[4 * q + 2]),
-                     __float_as_uint(v[4 * q + 3])};
-    __builtin_amdgcn_raw_buffer_store_b128(w, rec, on ? at + (q * LN + lane) * 16 : kNowhere, 0, 0);
-  }
+  for (int q = 0; q < N / 4; ++q)
+    *reinterpret_cast<float4*>(quads + q * LN * 4) = float4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+  float* rest = rec + 4 * (N / 4) * LN + lane;
 #pragma unroll
-  for (int f = N / 4 * 4; f < N; ++f)
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[f]), rec,
-                                          on ? at + (4 * (N / 4) * LN + (f - 4 * (N / 4)) * LN + lane) * 4 : kNowhere, 0, 0);
+  for (int f = N / 4 * 4; f < N; ++f) rest[(f - 4 * (N / 4)) * LN] = v[f];
 }
 
 // Orders this wave's LDS accesses (a wave's LDS operations execute in issue
@@ -397,17 +394,14 @@ cilu_factor_kernel(int nic, int njc, int nlev, const double2* ops, float* rec) {
   const int c = cw < CW ? wave * CW + cw : W, cc = min(c, W - 1);
   double* mat = gj[cw < CW ? wave * CW + cw : Fa::NW * CW];
   const int nrec = La::nrec(njc);
-  // the chunk's records in array a, and the record of cell (ci, jj) there
-  auto records = [&](int a) {
-    const size_t n = (size_t)La::NG * nrec * La::rs(La::count(a));
-    return buffer_of(rec + La::array(a, nchunk, njc) + chunk * n, n * sizeof(float));
-  };
-  const auto rec0 = records(0), rec1 = records(1);
-  auto record = [&](int a, int ci, int jj) {
+  // the record of cell (ci, jj) in array a, or the spare one
+  auto record = [&](bool there, int a, int ci, int jj) {
     const int g = ci / La::GW, cl = ci % La::GW;
     const bool asc = a == 0 || a == 2;
     const int c1 = asc ? cl : La::GW - 1 - cl, s = asc ? jj : njc - 1 - jj;
-    return (unsigned)(g * nrec + La::X + s + 2 * c1) * (unsigned)(La::rs(La::count(a)) * sizeof(float));
+    const size_t at = La::array(a, nchunk, njc) +
+                      ((size_t)(chunk * La::NG + g) * nrec + La::X + s + 2 * c1) * La::rs(La::count(a));
+    return rec + (there ? at : La::spare(chunk, nchunk, njc));
   };
   // lane of half h of row `row` of column ci
   auto lane_of = [&](bool asc, int ci, int row, int h) {
@@ -506,9 +500,9 @@ cilu_factor_kernel(int nic, int njc, int nlev, const double2* ops, float* rec) {
     for (int q = 0; q < NV; ++q) { d[q] = a[0][q]; id[q] = q == r ? 1.0 : 0.0; }
     // Stores without a branch around them: where one may be skipped, the next
     // wait for a load waits for all of them.
+    float* const to0 = record(valid, 0, cc, j);
 #pragma unroll
-    for (int h = 0; h < P; ++h)
-      put_record<La::n1, La::LN>(rec0, record(0, cc, j), lane_of(true, cc, r, h), valid, r0[h]);
+    for (int h = 0; h < P; ++h) put_record<La::n1, La::LN>(to0, lane_of(true, cc, r, h), r0[h]);
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- inverse of the factored diagonal block
@@ -552,9 +546,9 @@ cilu_factor_kernel(int nic, int njc, int nlev, const double2* ops, float* rec) {
     for (int q = 0; q < P * ND; ++q) {  // an odd row's second half ends in a zero
       r1[q / ND][La::n1 + q % ND] = q < NV ? (float)cell[r * NV + min(q, NV - 1)] : 0.0f;
     }
+    float* const to1 = record(valid, 1, cc, j);
 #pragma unroll
-    for (int h = 0; h < P; ++h)
-      put_record<La::n2, La::LN>(rec1, record(1, cc, j), lane_of(false, cc, r, h), valid, r1[h]);
+    for (int h = 0; h < P; ++h) put_record<La::n2, La::LN>(to1, lane_of(false, cc, r, h), r1[h]);
     lds_barrier();
   }
 }
@@ -744,13 +738,16 @@ __device__ __forceinline__ void cilu_solve_pairs(const float* R, int njc, ApplyL
   const int pos = La::GCX + (real ? c1 : 0), wpos = real ? pos : A::NP;
   const int xrow = h ? La::ROWS : row, tk = k / ND * 4 + k % ND;  // the right-hand side is taken once
   const int T = La::steps(njc), rl = min(lane, La::LN - 1);
-  const auto rrec = buffer_of(R, (size_t)La::nrec(njc) * RS * sizeof(float));
+  // the records of a block of steps and of those that are loaded in it: a pass's
+  // whole array may be beyond a buffer's 32-bit offsets
+  auto block_of = [&](int t0) { return buffer_of(R + (size_t)t0 * RS, 2 * UN * RS * sizeof(float)); };
+  auto rrec = block_of(0);
   const unsigned oq = rl * 16, or_ = (4 * NQ * La::LN + rl) * 4;
   u32x4 fq[PD][NQ > 0 ? NQ : 1];
   unsigned fr[PD][NREM > 0 ? NREM : 1];
   // the record's part that is used first is loaded last, so that one wait
   // covers the record
-  int so = 0;
+  int so = 0;  // the record that is loaded next, in the buffer
   auto fetch = [&](int u) {
 #pragma unroll
     for (int q = 0; q < NREM; ++q) fr[u][q] = __builtin_amdgcn_raw_buffer_load_b32(rrec, or_ + q * La::LN * 4, so, 0);
@@ -811,6 +808,9 @@ __device__ __forceinline__ void cilu_solve_pairs(const float* R, int njc, ApplyL
   widen(0);
   x = sh.x[1][xrow];
   for (int t0 = 0; t0 < T; t0 += UN) {
+    rrec = block_of(t0);
+    so = PD * RS * 4;
+    asm volatile("" : "+s"(so));  // a running scalar, not a constant per step
     const int r0 = t0 & (kRing - 1), r1 = (t0 + UN) & (kRing - 1);
     // cell of the column before that is ynext at the block's first step
     const double* y0 = sh.ring[h ? r0 : (r0 - 1) & (kRing - 1)][pos - 1];
@@ -874,11 +874,14 @@ __device__ __forceinline__ void cilu_solve_rows(const float* R, int njc, ApplyLd
   const bool real = row < La::ROWS;
   const int pos = La::GCX + (real ? c1 : 0), wpos = real ? pos : A::NP;
   const int T = La::steps(njc), rl = min(lane, La::LN - 1);
-  const auto rrec = buffer_of(R, (size_t)La::nrec(njc) * RS * sizeof(float));
+  // the records of a block of steps and of those that are loaded in it: a pass's
+  // whole array may be beyond a buffer's 32-bit offsets
+  auto block_of = [&](int t0) { return buffer_of(R + (size_t)t0 * RS, 2 * UN * RS * sizeof(float)); };
+  auto rrec = block_of(0);
   const unsigned oq = rl * 16, or_ = (4 * NQ * La::LN + rl) * 4;
   u32x4 fq[PD][NQ > 0 ? NQ : 1];
   unsigned fr[PD][NREM > 0 ? NREM : 1];
-  int so = 0;
+  int so = 0;  // the record that is loaded next, in the buffer
   auto fetch = [&](int u) {
 #pragma unroll
     for (int q = 0; q < NQ; ++q) fq[u][q] = __builtin_amdgcn_raw_buffer_load_b128(rrec, oq + q * La::LN * 16, so, 0);
@@ -944,6 +947,9 @@ __device__ __forceinline__ void cilu_solve_rows(const float* R, int njc, ApplyLd
   widen(0);
   x = sh.x[1][row];
   for (int t0 = 0; t0 < T; t0 += UN) {
+    rrec = block_of(t0);
+    so = PD * RS * 4;
+    asm volatile("" : "+s"(so));  // a running scalar, not a constant per step
     const int r0 = t0 & (kRing - 1), r1 = (t0 + UN) & (kRing - 1);
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
