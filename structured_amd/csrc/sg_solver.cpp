@@ -29,6 +29,7 @@
 #include <cstdio>
 #include <vector>
 
+#include "sg_ahead.hpp"
 #include "sg_context.hpp"
 #include "sg_kernels.hpp"
 #include "sg_linalg.hpp"
@@ -309,10 +310,9 @@ int arnoldi_step(sg_ctx* ctx, int j, double* res) {
 }
 
 // Right-preconditioned restarted FGMRES with CGS2.  Solves A x = rhs.  Step j +
-// 1 is enqueued before the results of step j are read, so that the device does
-// not wait for the host between steps (some 20 us each); where the residual is
-// about to reach the tolerance, the host looks first.  A step that turns out
-// not to be needed leaves x as it is.  A laminar Newton solve at 97x65:
+// 1 is enqueued before the results of step j are read (where enqueue_ahead says
+// so), so that the device does not wait for the host between steps.  A step that
+// turns out not to be needed leaves x as it is.  A laminar Newton solve at 97x65:
 // 134 -> 121 ms, 120 adjoint steps at 385x193 48.8 -> 47.4 ms.
 int fgmres_steps(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres);
 
@@ -337,7 +337,7 @@ int fgmres_steps(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres
   if (!std::isfinite(bnorm)) return sg_fail(ctx, SG_ERR_NAN, "non-finite right-hand side");
   std::vector<double> H((size_t)(m + 1) * m, 0.0), cs(m), sn(m), g(m + 1), y(m), hcol(m + 2);
   int total = 0;
-  double res = bnorm;
+  double res = bnorm, rate = 0.0;
   while (total < maxit) {
     double* V0 = S->V.p;
     if (total == 0) {
@@ -356,7 +356,6 @@ int fgmres_steps(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres
     int jend = -1;
     bool done = false;
     auto result = [&](int j) { return S->hres.p + (size_t)(j & 1) * (m + 3); };
-    double before = beta;  // the residual one step earlier
     res = beta;
     int queued = 0;  // steps on the stream
     for (int j = 0; j < m && total < maxit; ++j) {
@@ -364,8 +363,7 @@ int fgmres_steps(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres
         if ((rc = arnoldi_step(ctx, j, result(j)))) return rc;
         ++queued;
       }
-      const bool close = res * (res / before) <= rtol * bnorm;  // this step probably ends the solve
-      if (!close && j + 1 < m && total + 1 < maxit) {
+      if (j + 1 < m && total + 1 < maxit && enqueue_ahead(S->precond, res, rate, rtol * bnorm)) {
         if ((rc = arnoldi_step(ctx, j + 1, result(j + 1)))) return rc;
         ++queued;
       }
@@ -391,7 +389,7 @@ int fgmres_steps(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres
       for (int i = 0; i <= j; ++i) H[(size_t)i * m + j] = hcol[i];
       ++total;
       jend = j;
-      before = res;
+      rate = std::fabs(g[j + 1]) / res;
       res = std::fabs(g[j + 1]);
       if (res <= rtol * bnorm || hn == 0.0) { done = true; break; }
     }
