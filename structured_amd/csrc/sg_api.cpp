@@ -23,6 +23,13 @@ int sg_fail(sg_ctx* ctx, int code, const std::string& msg) {
   return code;
 }
 
+void sg_norms_returned(sg_ctx* ctx, const double* l2, int n) {
+  // NaN from the state, or from a wait that gave up: empty the slots for the
+  // next launch
+  if (std::any_of(l2, l2 + n, [](double v) { return v != v; }))
+    (void)reduce_slots_init(ctx->partial.p, ctx->partial.n, ctx->stream, ctx->wait_polls);
+}
+
 int sg_hip(sg_ctx* ctx, hipError_t e, const char* what) {
   if (e == hipSuccess) return SG_OK;
   return sg_fail(ctx, SG_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
@@ -434,7 +441,7 @@ int sg_create(int ni, int nj, const double* xv, const double* yv, const sg_frees
   }
   // work buffers
   const size_t naos = ctx->ncell() * ctx->nvar, nsoa = ctx->nsoa();
-  const size_t npart = residual_partial_count(g) * 2 * ctx->nvar;
+  const size_t npart = norm_slots(g, 2 * ctx->nvar);
   if (ctx->aos_a.alloc(naos) || ctx->aos_b.alloc(naos) || ctx->q.alloc(nsoa) || ctx->r.alloc(nsoa) ||
       ctx->v.alloc(nsoa) || ctx->w.alloc(nsoa) || ctx->partial.alloc(npart) || ctx->l2.alloc(16) ||
       ctx->wall_cp.alloc(G.ni) || ctx->wall_cf.alloc(G.ni) || ctx->wall_f.alloc(4))
@@ -558,9 +565,23 @@ int sg_get_metrics(sg_ctx* ctx, double* nchi, double* neta, double* volume, doub
 int sg_residual_dev_async(sg_ctx* ctx, const double* q_dev, double* r_dev, double* l2_dev) {
   if (!ctx || !q_dev || !r_dev) return SG_ERR_ARG;
   // the caller's l2_dev holds nvar norms (||R_k||_2): only those are written
-  SG_TRY(launch_residual(ctx->g, ctx->ph, ctx->bc, ctx->sa, q_dev, r_dev, l2_dev ? ctx->partial.p : nullptr, l2_dev, ctx->stream,
-                         ctx->clo, ctx->nvar),
+  SG_TRY(launch_residual(ctx->g, ctx->ph, ctx->bc, ctx->sa, q_dev, r_dev, l2_dev ? ctx->partial.p : nullptr, l2_dev,
+                         ctx->stream, ctx->clo, ctx->nvar),
          "residual launch");
+  return SG_OK;
+}
+
+// The bound of the kernels' waits for one another, in polls (negative: the
+// usual one).  Not part of the interface: the tests reach what follows a wait
+// that gave up with it.
+int sg_test_wait_polls(sg_ctx* ctx, int polls) {
+  if (!ctx) return SG_ERR_ARG;
+  ctx->wait_polls = polls < 0 ? kWaitPolls : polls;
+  const unsigned long long bound = (unsigned long long)ctx->wait_polls;
+  char* head = reinterpret_cast<char*>(ctx->partial.p);
+  SG_TRY(hipMemcpyAsync(head + offsetof(SlotHead, polls), &bound, sizeof(bound), hipMemcpyHostToDevice, ctx->stream),
+         "H2D");
+  SG_TRY(hipStreamSynchronize(ctx->stream), "sync");
   return SG_OK;
 }
 
@@ -574,6 +595,7 @@ int sg_residual_dev(sg_ctx* ctx, const double* q_dev, double* r_dev, double* l2_
   double l2[8];
   SG_TRY(hipMemcpyAsync(l2, ctx->l2.p, ctx->nvar * sizeof(double), hipMemcpyDeviceToHost, ctx->stream), "D2H");
   SG_TRY(hipStreamSynchronize(ctx->stream), "residual");
+  sg_norms_returned(ctx, l2, ctx->nvar);
   if (l2_host) std::copy(l2, l2 + ctx->nvar, l2_host);
   return check_finite(ctx, l2);
 }
@@ -583,12 +605,13 @@ int sg_residual(sg_ctx* ctx, const double* q_aos, double* r_aos, double* l2) {
   int rc;
   if ((rc = upload_aos(ctx, q_aos, ctx->q.p))) return rc;
   double l2h[8];
-  SG_TRY(launch_residual(ctx->g, ctx->ph, ctx->bc, ctx->sa, ctx->q.p, ctx->r.p, ctx->partial.p, ctx->l2.p, ctx->stream,
-                         ctx->clo, 0),
+  SG_TRY(launch_residual(ctx->g, ctx->ph, ctx->bc, ctx->sa, ctx->q.p, ctx->r.p, ctx->partial.p, ctx->l2.p,
+                         ctx->stream, ctx->clo, 0),
          "residual launch");
   SG_TRY(hipMemcpyAsync(l2h, ctx->l2.p, ctx->nvar * sizeof(double), hipMemcpyDeviceToHost, ctx->stream), "D2H");
   if ((rc = download_aos(ctx, ctx->r.p, r_aos))) return rc;
   SG_TRY(hipStreamSynchronize(ctx->stream), "residual");
+  sg_norms_returned(ctx, l2h, ctx->nvar);
   if (l2) std::copy(l2h, l2h + ctx->nvar, l2);
   return check_finite(ctx, l2h);
 }

@@ -107,6 +107,7 @@ struct sg_ctx {
   sg::DevBuf aos_a, aos_b;         // AoS staging (nvar * ncell)
   sg::DevBuf q, r, v, w;           // SoA work vectors (nvar * plane)
   sg::DevBuf partial, l2;  // slots of the norm's partial sums (empty between launches), the norms
+  int wait_polls = sg::kWaitPolls;  // bound of the waits on slots
   sg::DevBuf wall_cp, wall_cf, wall_f;
   sg::DevClosure clo;              // beta closure applied by every residual / J.v launch
   sg::DevBuf clo_params, clo_w2;   // MLP parameters (FP32) and W2 (BF16), raw storage
@@ -122,3 +123,5 @@ int sg_fail(sg_ctx* ctx, int code, const std::string& msg);
 int sg_noalloc_setup(sg_ctx* ctx);
 void sg_solver_free(sg_ctx* ctx);
 int sg_hip(sg_ctx* ctx, hipError_t e, const char* what);
+// to be called with the norms that came back from a launch on ctx->partial
+void sg_norms_returned(sg_ctx* ctx, const double* l2, int n);

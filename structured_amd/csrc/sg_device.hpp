@@ -8,6 +8,23 @@ namespace sg {
 // An empty slot of a reduction across work-groups: a signalling NaN, which no
 // arithmetic produces.
 constexpr unsigned long long kNoValue = 0x7FF4534C4F545321ull;
+
+// Polls before a wait for another work-group's value gives up (each takes about
+// a microsecond, so several seconds).  Such waits are for work-groups started
+// earlier, so they end.
+constexpr int kWaitPolls = 1 << 22;
+
+// Slots of a reduction across work-groups (device memory): a head, then the
+// values, which are empty between launches.  A wait that gave up makes its result
+// NaN and fills the head's state: values that came late may then lie in the
+// slots, where the next reduction would take them for its own.  So later results
+// are not used until reduce_slots_init: the residual's norms are NaN then, and
+// the Krylov solver, which looks at every result, ends.
+struct SlotHead {
+  unsigned long long state;  // empty, or a wait gave up
+  unsigned long long polls;  // bound of the norms' waits
+};
+constexpr int kSlotHead = 16;  // words: a line of its own
 }  // namespace sg
 
 namespace sg {
@@ -113,6 +130,18 @@ __device__ __forceinline__ double dpp_move(double v) {
   const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROW_MASK, 0xF, false);
   return __hiloint2double(hi, lo);
 }
+__device__ __forceinline__ unsigned long long slot_load(const unsigned long long* slot) {
+  return __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void slot_store(unsigned long long* slot, unsigned long long v) {
+  __hip_atomic_store(slot, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The head as it was when the launch began; slots: the first value.
+__device__ __forceinline__ SlotHead slot_head(const unsigned long long* slots) {
+  return *reinterpret_cast<const SlotHead*>(slots - kSlotHead);
+}
+__device__ __forceinline__ void slots_lost(unsigned long long* slots) { slot_store(slots - kSlotHead, 0); }
+
 // Sum over each row of 16 lanes, in all of them.
 __device__ __forceinline__ double row_sum(double v) {
   v += dpp_move<0xB1>(v);        // quad_perm [1,0,3,2]

@@ -111,6 +111,7 @@ int sg_step_explicit_dev(sg_ctx* ctx, double* q_dev, int scheme, double cfl, dou
   double h[10];
   SG_TRY(hipMemcpyAsync(h, ctx->l2.p, ctx->nvar * sizeof(double), hipMemcpyDeviceToHost, ctx->stream), "D2H");
   SG_TRY(hipStreamSynchronize(ctx->stream), "explicit step");
+  sg_norms_returned(ctx, h, ctx->nvar);
   if (l2) std::copy(h, h + ctx->nvar, l2);
   for (int k = 0; k < ctx->nvar; ++k)
     if (!std::isfinite(h[k])) return sg_fail(ctx, SG_ERR_NAN, "non-finite residual norm in an explicit step");
@@ -137,6 +138,7 @@ int sg_solve_explicit(sg_ctx* ctx, double* q_aos, const sg_explicit_opts* o, sg_
     if ((rc = enqueue_step(ctx, q, o->scheme, cfl))) return rc;
     SG_TRY(hipMemcpyAsync(l2, ctx->l2.p, nv * sizeof(double), hipMemcpyDeviceToHost, ctx->stream), "D2H");
     SG_TRY(hipStreamSynchronize(ctx->stream), "explicit step");
+    sg_norms_returned(ctx, l2, nv);
     if (counter == 0) std::copy(l2, l2 + nv, R.l2_initial);
     if (l2_hist) std::copy(l2, l2 + nv, l2_hist + (size_t)counter * nv);
     if (o->verbose && counter % o->verbose == 0)

@@ -36,7 +36,10 @@ static int tile_rows(const DevGeom& g) {
   return !wide_rows(g) && kRatio * large < 10 * small ? kTileLarge : kTileSmall;
 }
 
-size_t residual_partial_count(const DevGeom& g) { return (size_t)residual_tiles(g, tile_rows<double>(g)); }
+size_t norm_slots(const DevGeom& g, int norms) { return kSlotHead + (size_t)residual_tiles(g, tile_rows<double>(g)) * norms; }
+static unsigned long long* norm_words(double* slots) {
+  return slots ? reinterpret_cast<unsigned long long*>(slots) + kSlotHead : nullptr;
+}
 
 template <int TY, class I, class S, bool SA, class F, class O>
 static void launch_tiles(unsigned extra, unsigned nz, hipStream_t s, const DevGeom& g, const DevPhys& ph, const DevBc& bc, F fq, O fo,
@@ -59,7 +62,7 @@ static void launch_tiles(unsigned extra, unsigned nz, hipStream_t s, const DevGe
 }
 template <class S, bool SA, class F, class O>
 static void launch_cl(hipStream_t s, const DevGeom& g, const DevPhys& ph, const DevBc& bc, F fq, O fo,
-                      const double* beta_dot, const DevClosure& clo, NormOut no = NormOut{nullptr, nullptr, 0},
+                      const double* beta_dot, const DevClosure& clo, NormOut no = NormOut(),
                       unsigned nz = 1) {
   const unsigned extra = no.slots ? 1 : 0;  // the work-group that sums the norms
   if (wide_rows(g)) launch_tiles<kTileSmall, size_t, S, SA>(extra, nz, s, g, ph, bc, fq, fo, beta_dot, clo, no);
@@ -75,7 +78,7 @@ hipError_t launch_residual(const DevGeom& g, const DevPhys& ph, const DevBc& bc,
   if (l2_count <= 0 || l2_count > nv2) l2_count = nv2;
   Field<double> fq{q};
   OutField<double> fo{r};
-  const NormOut no{reinterpret_cast<unsigned long long*>(slots), l2, l2_count};
+  const NormOut no{norm_words(slots), l2, l2_count};
   if (sa) launch_cl<double, true>(s, g, ph, bc, fq, fo, nullptr, clo, no);
   else launch_cl<double, false>(s, g, ph, bc, fq, fo, nullptr, DevClosure(), no);
   return hipGetLastError();
@@ -104,7 +107,7 @@ struct StageField {
 hipError_t launch_stage(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool sa, const double* q,
                         const ExplicitStage& st, double* slots, double* l2, hipStream_t s, const DevClosure& clo) {
   if ((l2 != nullptr) != (slots != nullptr)) return hipErrorInvalidValue;
-  const NormOut no{reinterpret_cast<unsigned long long*>(slots), l2, sa ? 5 : 4};
+  const NormOut no{norm_words(slots), l2, sa ? 5 : 4};
   if (sa) launch_cl<double, true>(s, g, ph, bc, Field<double>{q}, StageField{st}, nullptr, clo, no);
   else launch_cl<double, false>(s, g, ph, bc, Field<double>{q}, StageField{st}, nullptr, DevClosure(), no);
   return hipGetLastError();
@@ -134,7 +137,7 @@ hipError_t launch_blocks(const DevGeom& g, const DevPhys& ph, const DevBc& bc, b
   const SeedField fq{q, d};
   const OutBlocks fo{blocks, d};
   const unsigned nz = (unsigned)d.count();
-  const NormOut no{nullptr, nullptr, 0};
+  const NormOut no;
   if (sa) launch_cl<Dual, true>(s, g, ph, bc, fq, fo, nullptr, clo, no, nz);
   else launch_cl<Dual, false>(s, g, ph, bc, fq, fo, nullptr, DevClosure(), no, nz);
   return hipGetLastError();

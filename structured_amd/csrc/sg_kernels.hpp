@@ -6,12 +6,12 @@
 
 namespace sg {
 
-size_t residual_partial_count(const DevGeom& g);
-// Norms (optional: both of slots and l2, or neither): slots holds 2 nv partial
-// sums per tile, all empty (kNoValue) before the first launch and after every
-// launch.  The launch's last block adds them and writes the L2 norms of R,
-// then of V R, to l2 (device): l2_count entries (0: all 2 nv; nv: the norms
-// of R only).
+size_t norm_slots(const DevGeom& g, int norms);
+// Norms (optional: both of slots and l2, or neither): slots holds nv or 2 nv
+// partial sums per tile (norm_slots words with the head), all empty before
+// the first launch and after every launch.  The launch's last block adds them
+// and writes the L2 norms of R, then of V R, to l2 (device): l2_count entries
+// (0: all 2 nv; nv: the norms of R only).
 hipError_t launch_residual(const DevGeom& g, const DevPhys& ph, const DevBc& bc, bool sa, const double* q, double* r,
                            double* slots, double* l2, hipStream_t s, const DevClosure& clo = DevClosure(),
                            int l2_count = 0);

@@ -18,53 +18,60 @@ namespace sg {
 // Every block stores its partial sums into slots of its own, and one more
 // block (the last of the grid) waits for them, sums them in a fixed order and
 // empties them for the next call.  A slot is one 64-bit atomic that holds
-// either a value or kNoValue, a signalling NaN that no arithmetic produces, so
-// nothing has to be ordered between slots, and no counter is needed: a
-// counter's increments, one after another at some 50 ns, took longer than the
-// second kernel they would have saved.  The other blocks depend on nothing,
-// so the wait ends; past kSlotPolls the result is NaN.
-constexpr int kSlotPolls = 1 << 22;
+// either a value or kNoValue, so nothing has to be ordered between slots, and no
+// counter is needed: a counter's increments, one after another at some 50 ns,
+// took longer than the second kernel they would have saved.  The other blocks
+// depend on nothing, so the wait ends; see SlotHead for one that gives up.
 
-__device__ __forceinline__ void slot_store(double* slot, double v) {
-  __hip_atomic_store(slot, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+struct SlotSet {
+  unsigned long long* w;  // the first value
+  int polls;
+};
+static SlotSet slot_set(Slots s) { return {reinterpret_cast<unsigned long long*>(s.p) + kSlotHead, s.polls}; }
+__device__ __forceinline__ void put_sum(unsigned long long* slot, double v) {
+  slot_store(slot, (unsigned long long)__double_as_longlong(v));
 }
-// Sum of the slots first, first + stride, ... below n, in that order, U at a
-// time in flight; they are left empty.
+// Sum of the values from `from` on at first, first + stride, ... below n, in that
+// order, U at a time in flight; they are left empty.
 template <int U>
-__device__ double slot_sum(double* slots, int first, int stride, int n) {
+__device__ double slot_sum(SlotSet set, size_t from, int first, int stride, int n) {
+  unsigned long long* const sums = set.w + from;
   double sum = 0.0;
   int polls = 0;
   for (int b = first; b < n; b += U * stride) {
     unsigned long long v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      unsigned long long* p = reinterpret_cast<unsigned long long*>(slots + min(b + u * stride, n - 1));
-      v[u] = b + u * stride < n ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+      const unsigned long long* p = sums + min(b + u * stride, n - 1);
+      v[u] = b + u * stride < n ? slot_load(p) : 0ull;
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (b + u * stride >= n) break;
-      unsigned long long* p = reinterpret_cast<unsigned long long*>(slots + b + u * stride);
+      unsigned long long* p = sums + b + u * stride;
       while (v[u] == kNoValue) {
-        if (++polls > kSlotPolls) {
+        if (++polls > set.polls) {
           v[u] = (unsigned long long)__double_as_longlong(__builtin_nan(""));
           break;
         }
-        v[u] = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        v[u] = slot_load(p);
       }
-      __hip_atomic_store(p, kNoValue, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      slot_store(p, kNoValue);
       sum += __longlong_as_double((long long)v[u]);
     }
   }
+  if (polls > set.polls) slots_lost(set.w);
   return sum;
 }
 
-__global__ __launch_bounds__(256) void slots_empty_kernel(unsigned long long* x, size_t n) {
-  for (size_t e = blockIdx.x * (size_t)256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) x[e] = kNoValue;
+__global__ __launch_bounds__(256) void slots_empty_kernel(unsigned long long* x, size_t n, int polls) {
+  for (size_t e = blockIdx.x * (size_t)256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256)
+    x[e] = e == 1 ? (unsigned long long)polls : kNoValue;
 }
-hipError_t reduce_slots_init(double* slots, size_t n, hipStream_t s) {
+hipError_t reduce_slots_init(double* slots, size_t n, hipStream_t s, int polls) {
+  static_assert(offsetof(SlotHead, state) == 0 && offsetof(SlotHead, polls) == 8, "the head's words");
   hipLaunchKernelGGL(slots_empty_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 1024)), dim3(256), 0, s,
-                     reinterpret_cast<unsigned long long*>(slots), n);
+                     reinterpret_cast<unsigned long long*>(slots), n, polls);
   return hipGetLastError();
 }
 
@@ -89,7 +96,7 @@ constexpr int DOT_BLOCK = 256;
 constexpr int DOT_KC = 8;
 constexpr int DOT_SLICES = 512;  // at most
 __global__ __launch_bounds__(DOT_BLOCK) void multi_dot_kernel(const double* V, size_t ldv, int k, const double* w,
-                                                              size_t n, double* slots, double* out, const double* ga,
+                                                              size_t n, SlotSet slots, double* out, const double* ga,
                                                               const double* gb, double gf) {
   if (!gate_open(ga, gb, gf)) return;
   const int slices = (int)gridDim.x - 1;
@@ -97,7 +104,7 @@ __global__ __launch_bounds__(DOT_BLOCK) void multi_dot_kernel(const double* V, s
   const int i0 = (int)blockIdx.y * DOT_KC, kk = min(DOT_KC, k - i0);
   if ((int)blockIdx.x == slices) {  // 32 threads per vector
     const int i = threadIdx.x >> 5, l = threadIdx.x & 31;
-    double s = i < kk ? slot_sum<16>(slots + (size_t)(i0 + i) * slices, l, 32, slices) : 0.0;
+    double s = i < kk ? slot_sum<16>(slots, (size_t)(i0 + i) * slices, l, 32, slices) : 0.0;
 #pragma unroll
     for (int o = 16; o > 0; o >>= 1) s += __shfl_xor(s, o);
     if (i < kk && l == 0) out[i0 + i] = s;
@@ -134,7 +141,7 @@ __global__ __launch_bounds__(DOT_BLOCK) void multi_dot_kernel(const double* V, s
   if ((int)threadIdx.x < kk) {
     double t = 0.0;
     for (int q = 0; q < DOT_BLOCK / 64; ++q) t += red[q][threadIdx.x];
-    slot_store(slots + (size_t)(i0 + threadIdx.x) * slices + blockIdx.x, t);
+    put_sum(slots.w + (size_t)(i0 + threadIdx.x) * slices + blockIdx.x, t);
   }
 }
 
@@ -149,11 +156,12 @@ static int pair_blocks(size_t n, int most) {
   return (int)std::min<size_t>(std::max<size_t>((n / 2 + 255) / 256, 1), (size_t)most);
 }
 
-hipError_t multi_dot(const double* V, size_t ldv, int k, const double* w, size_t n, double* slots, double* out,
+hipError_t multi_dot(const double* V, size_t ldv, int k, const double* w, size_t n, Slots slots, double* out,
                      hipStream_t s, const double* ga, const double* gb, double gf) {
   if (!pairs_aligned(V, ldv, k, w)) return hipErrorInvalidValue;
   const dim3 grid(pair_blocks(n, DOT_SLICES) + 1, (unsigned)((k + DOT_KC - 1) / DOT_KC));
-  hipLaunchKernelGGL(multi_dot_kernel, grid, dim3(DOT_BLOCK), 0, s, V, ldv, k, w, n, slots, out, ga, gb, gf);
+  hipLaunchKernelGGL(multi_dot_kernel, grid, dim3(DOT_BLOCK), 0, s, V, ldv, k, w, n, slot_set(slots), out, ga, gb,
+                     gf);
   return hipGetLastError();
 }
 
@@ -166,7 +174,7 @@ hipError_t multi_dot(const double* V, size_t ldv, int k, const double* w, size_t
 constexpr int AXPY_KC = 8;
 constexpr int AXPY_BLOCKS = 2048;  // at most
 __global__ __launch_bounds__(256) void multi_axpy_kernel(const double* V, size_t ldv, int k, const double* c, double* w,
-                                                         size_t n, double* slots, double* norm2, const double* ga,
+                                                         size_t n, SlotSet slots, double* norm2, const double* ga,
                                                          const double* gb, double gf) {
   if (!gate_open(ga, gb, gf)) return;
   __shared__ double red[4];
@@ -174,7 +182,7 @@ __global__ __launch_bounds__(256) void multi_axpy_kernel(const double* V, size_t
   double sq = 0.0;
   const bool last = (int)blockIdx.x == blocks;
   if (last) {
-    sq = slot_sum<8>(slots, threadIdx.x, 256, blocks);
+    sq = slot_sum<8>(slots, 0, threadIdx.x, 256, blocks);
   } else {
     const size_t n2 = n / 2;
     double2* w2 = reinterpret_cast<double2*>(w);
@@ -213,19 +221,19 @@ __global__ __launch_bounds__(256) void multi_axpy_kernel(const double* V, size_t
   if (threadIdx.x == 0) {
     const double t = red[0] + red[1] + red[2] + red[3];
     if (last) *norm2 = t;
-    else slot_store(slots + blockIdx.x, t);
+    else put_sum(slots.w + blockIdx.x, t);
   }
 }
 
-hipError_t multi_axpy(const double* V, size_t ldv, int k, const double* c, double* w, size_t n, double* slots,
+hipError_t multi_axpy(const double* V, size_t ldv, int k, const double* c, double* w, size_t n, Slots slots,
                       double* norm2, hipStream_t s, const double* ga, const double* gb, double gf) {
   if (!pairs_aligned(V, ldv, k, w)) return hipErrorInvalidValue;
   hipLaunchKernelGGL(multi_axpy_kernel, dim3(pair_blocks(n, AXPY_BLOCKS) + 1), dim3(256), 0, s, V, ldv, k, c, w, n,
-                     slots, norm2, ga, gb, gf);
+                     slot_set(slots), norm2, ga, gb, gf);
   return hipGetLastError();
 }
 
-size_t reduce_slots(int kmax) { return (size_t)std::max(DOT_SLICES * kmax, AXPY_BLOCKS); }
+size_t reduce_slots(int kmax) { return kSlotHead + (size_t)std::max(DOT_SLICES * kmax, AXPY_BLOCKS); }
 
 // The end of an Arnoldi step (see sg_linalg.hpp): every block forms the scale
 // from the step's norms; block 0 writes the results.
@@ -239,7 +247,7 @@ __global__ __launch_bounds__(256) void arnoldi_finish_kernel(double* w, size_t n
     for (int i = threadIdx.x; i <= j; i += 256) put(i, h[i] + (second ? y[i] : 0.0));
     if (threadIdx.x == 0) {
       put(j + 1, hn);
-      put(j + 2, second ? 1.0 : 0.0);
+      put(j + 2, second ? 1.0 : h[j + 1] == h[j + 1] ? 0.0 : h[j + 1]);
     }
   }
   if (!(hn > 0.0)) return;

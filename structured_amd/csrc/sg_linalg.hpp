@@ -10,18 +10,22 @@ namespace sg {
 
 constexpr int NSLOT = 13;  // Jacobian stencil blocks kept per cell
 
-// 64-bit slots of the reductions below, which every call finds and leaves
-// empty; reduce_slots_init empties them first.
+// 64-bit words of the slots of the reductions below, which every call finds and
+// leaves empty; reduce_slots_init writes their head and empties them first.
 size_t reduce_slots(int kmax);
-hipError_t reduce_slots_init(double* slots, size_t n, hipStream_t s);
+struct Slots {
+  double* p;
+  int polls;  // bound of a wait on them
+};
+hipError_t reduce_slots_init(double* slots, size_t n, hipStream_t s, int polls = kWaitPolls);
 // out[i] = V_i . w for i < k (V_i = V + i*ldv); out is device memory.  With
 // ga and gb (device doubles) the kernel runs only if *ga < gf * *gb and
 // otherwise writes nothing: a conditional pass decided on the device.
-hipError_t multi_dot(const double* V, size_t ldv, int k, const double* w, size_t n, double* slots, double* out,
+hipError_t multi_dot(const double* V, size_t ldv, int k, const double* w, size_t n, Slots slots, double* out,
                      hipStream_t s, const double* ga = nullptr, const double* gb = nullptr, double gf = 0.5);
 // w -= sum_i c[i] V_i, c device memory, and *norm2 = |w|^2 after it; gated as
 // multi_dot
-hipError_t multi_axpy(const double* V, size_t ldv, int k, const double* c, double* w, size_t n, double* slots,
+hipError_t multi_axpy(const double* V, size_t ldv, int k, const double* c, double* w, size_t n, Slots slots,
                       double* norm2, hipStream_t s, const double* ga = nullptr, const double* gb = nullptr,
                       double gf = 0.5);
 // The end of an Arnoldi step j: h[0..j+1] = V^T w and |w|^2, y[j+1] = |w'|^2
@@ -29,7 +33,7 @@ hipError_t multi_axpy(const double* V, size_t ldv, int k, const double* c, doubl
 // its projections and *norm2b the norm after it.  Scales w to unit norm (a
 // zero w stays) and leaves in res (host memory the device can write, preset to
 // kNoValue) the column's entries 0..j, then the norm and whether the second
-// pass ran (1 or 0), each as one 64-bit store.
+// pass ran (1 or 0; NaN if |w|^2 is), each as one 64-bit store.
 hipError_t arnoldi_finish(double* w, size_t n, int j, const double* h, const double* y, const double* norm2b, double gf,
                           double* res, hipStream_t s);
 // y (+)= sum_i c[i] X_i, c device memory

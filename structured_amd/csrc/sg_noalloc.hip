@@ -17,8 +17,8 @@
 
 namespace {
 
-// 2 nvar slots per residual tile, component-major.
-constexpr size_t kScratchDoubles = (size_t)SG_NOALLOC_MAX_TILES * 10;
+// The head, then up to 10 slots per residual tile, component-major.
+constexpr size_t kScratchDoubles = sg::kSlotHead + (size_t)SG_NOALLOC_MAX_TILES * 10;
 
 static __device__ __align__(256) double scratch[kScratchDoubles];
 
@@ -57,7 +57,7 @@ extern "C" int sg_residual_dev_async_noalloc(sg_ctx* ctx, const double* q_dev, d
     slots = ctx->noalloc_scratch;
     // emptied by each call: the array starts as zeros and is shared by contexts;
     // a kernel, not a memset, so that the call can be captured into a graph
-    if (sg::reduce_slots_init(slots, sg::residual_partial_count(ctx->g) * (size_t)ctx->nvar, ctx->stream) != hipSuccess)
+    if (sg::reduce_slots_init(slots, sg::norm_slots(ctx->g, ctx->nvar), ctx->stream, ctx->wait_polls) != hipSuccess)
       return sg_fail(ctx, SG_ERR_HIP, "scratch clear launch");
   }
   const hipError_t e = sg::launch_residual(ctx->g, ctx->ph, ctx->bc, ctx->sa, q_dev, r_dev, slots, l2_dev, ctx->stream,

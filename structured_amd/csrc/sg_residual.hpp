@@ -361,41 +361,44 @@ __device__ __forceinline__ SaTerms<S> sa_terms(S r, S n, S ml, const S* gu, cons
 // Fused norm output.  With slots set the launch has one more block, the last,
 // which waits for every tile's partial sums, adds them in a fixed order and
 // empties the slots for the next launch.  A slot is one 64-bit atomic that
-// holds either a partial sum or kNoValue (a signalling NaN that no arithmetic
-// produces), so nothing has to be ordered between slots.  The tiles depend on
-// nothing, so the wait ends; past kNormPolls the norms are NaN.
+// holds either a partial sum or kNoValue, so nothing has to be ordered between
+// slots.  The tiles depend on nothing, so the wait ends; see SlotHead for one that
+// gives up.
 struct NormOut {
-  unsigned long long* slots;  // 2 NV per tile, component-major; all empty between launches
-  double* l2;                 // ||R_k||_2 (k < NV), then ||V R_k||_2 (NV <= k < 2 NV)
-  int count;                  // entries of l2 written: NV (caller's buffer) or 2 NV
+  unsigned long long* slots = nullptr;  // 2 NV per tile, component-major, after their head
+  double* l2 = nullptr;                 // ||R_k||_2 (k < NV), then ||V R_k||_2 (NV <= k < 2 NV)
+  int count = 0;                        // entries of l2 written: NV (caller's buffer) or 2 NV
 };
-constexpr int kNormPolls = 1 << 22;
 
 template <int NT, int NV2>
 __device__ __forceinline__ void finalise_norms(const NormOut& no, int ntile, double (*red)[NV2]) {
   const int tid = threadIdx.x;
+  const SlotHead head = slot_head(no.slots);
   double acc[NV2];
 #pragma unroll
   for (int k = 0; k < NV2; ++k) acc[k] = 0.0;
-  int polls = 0;
+  unsigned long long polls = 0;
   for (int b = tid; b < ntile; b += NT) {
     unsigned long long v[NV2];
     bool wait = true;
     while (wait) {  // every sum of the tile again, all loads in flight together
 #pragma unroll
-      for (int k = 0; k < NV2; ++k)
-        v[k] = k < no.count ? __hip_atomic_load(no.slots + (size_t)k * ntile + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                            : 0ull;
+      for (int k = 0; k < NV2; ++k) v[k] = k < no.count ? slot_load(no.slots + (size_t)k * ntile + b) : 0ull;
       wait = false;
 #pragma unroll
       for (int k = 0; k < NV2; ++k) wait = wait || v[k] == kNoValue;
-      if (wait && ++polls > kNormPolls) break;
+      if (wait && ++polls > head.polls) break;
     }
 #pragma unroll
     for (int k = 0; k < NV2; ++k) {
-      if (k < no.count) __hip_atomic_store(no.slots + (size_t)k * ntile + b, kNoValue, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (k < no.count) slot_store(no.slots + (size_t)k * ntile + b, kNoValue);
       acc[k] += wait ? __builtin_nan("") : __longlong_as_double((long long)v[k]);
     }
+  }
+  if (polls > head.polls) slots_lost(no.slots);
+  if (head.state != kNoValue) {
+#pragma unroll
+    for (int k = 0; k < NV2; ++k) acc[k] = __builtin_nan("");
   }
 #pragma unroll
   for (int k = 0; k < NV2; ++k) acc[k] = wave_sum_lane63(acc[k]);
@@ -754,7 +757,7 @@ __global__ __launch_bounds__(TX * TY, sizeof(S) == sizeof(double) ? 4 : 2) void 
       for (int m = 0; m < NT / 16; ++m) a += sums[k * LD + m * 16 + l];
       a = row_sum(a);
       if (l == 0)
-        __hip_atomic_store(nout.slots + (size_t)k * ntile + bid, (unsigned long long)__double_as_longlong(a), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        slot_store(nout.slots + (size_t)k * ntile + bid, (unsigned long long)__double_as_longlong(a));
     }
   }
 }

@@ -112,10 +112,22 @@ int ensure(sg_ctx* ctx, int restart) {
   return SG_OK;
 }
 
+Slots slots(sg_ctx* ctx) { return {ctx->solver->partial.p, ctx->wait_polls}; }
+
+// An error if a reduction of this solve gave up waiting.  Asked only where a
+// result is NaN or a norm 0: such a reduction leaves one or the other.
+int reductions_ended(sg_ctx* ctx) {
+  unsigned long long state = 0;
+  static_assert(offsetof(SlotHead, state) == 0, "the head's first word");
+  SG_TRY(hipMemcpyAsync(&state, ctx->solver->partial.p, sizeof(state), hipMemcpyDeviceToHost, ctx->stream), "D2H");
+  SG_TRY(hipStreamSynchronize(ctx->stream), "sync");
+  return state == kNoValue ? SG_OK : sg_fail(ctx, SG_ERR_HIP, "a reduction gave up waiting for its partial sums");
+}
+
 double host_dot(sg_ctx* ctx, const double* a, const double* b, int* rc) {
   SolverState* S = ctx->solver;
   double out = 0.0;
-  hipError_t e = multi_dot(a, 0, 1, b, S->n, S->partial.p, S->hdev.p, ctx->stream);
+  hipError_t e = multi_dot(a, 0, 1, b, S->n, slots(ctx), S->hdev.p, ctx->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(S->hpin.p, S->hdev.p, sizeof(double), hipMemcpyDeviceToHost, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e == hipSuccess) out = S->hpin.p[0];
@@ -301,10 +313,10 @@ int arnoldi_step(sg_ctx* ctx, int j, double* res) {
   double* wn1 = S->ydev.p + j + 1;
   double* wn2 = S->ydev.p + m + 1;
   const double gf = S->dgks;
-  SG_TRY(multi_dot(S->V.p, n, j + 2, W, n, S->partial.p, S->hdev.p, ctx->stream), "dot");
-  SG_TRY(multi_axpy(S->V.p, n, j + 1, S->hdev.p, W, n, S->partial.p, wn1, ctx->stream), "axpy");
-  SG_TRY(multi_dot(S->V.p, n, j + 1, W, n, S->partial.p, S->ydev.p, ctx->stream, wn1, wn0, gf), "dot");
-  SG_TRY(multi_axpy(S->V.p, n, j + 1, S->ydev.p, W, n, S->partial.p, wn2, ctx->stream, wn1, wn0, gf), "axpy");
+  SG_TRY(multi_dot(S->V.p, n, j + 2, W, n, slots(ctx), S->hdev.p, ctx->stream), "dot");
+  SG_TRY(multi_axpy(S->V.p, n, j + 1, S->hdev.p, W, n, slots(ctx), wn1, ctx->stream), "axpy");
+  SG_TRY(multi_dot(S->V.p, n, j + 1, W, n, slots(ctx), S->ydev.p, ctx->stream, wn1, wn0, gf), "dot");
+  SG_TRY(multi_axpy(S->V.p, n, j + 1, S->ydev.p, W, n, slots(ctx), wn2, ctx->stream, wn1, wn0, gf), "axpy");
   SG_TRY(arnoldi_finish(W, n, j, S->hdev.p, S->ydev.p, wn2, gf, res, ctx->stream), "arnoldi");
   return SG_OK;
 }
@@ -329,6 +341,8 @@ int fgmres_steps(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres
   const size_t n = S->n;
   int rc = SG_OK;
   SG_TRY(hipMemsetAsync(S->x.p, 0, n * sizeof(double), ctx->stream), "memset");
+  // empty also after a wait that gave up in an earlier solve
+  SG_TRY(reduce_slots_init(S->partial.p, S->partial.n, ctx->stream, ctx->wait_polls), "reduction slots");
   const double bnorm = std::sqrt(host_dot(ctx, S->rhs.p, S->rhs.p, &rc));
   if (rc) return rc;
   *iters = 0;
@@ -349,6 +363,7 @@ int fgmres_steps(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres
     }
     const double beta = total == 0 ? bnorm : std::sqrt(host_dot(ctx, V0, V0, &rc));
     if (rc) return rc;
+    if (std::isnan(beta) && (rc = reductions_ended(ctx))) return rc;
     if (beta == 0.0) { res = 0.0; break; }
     SG_TRY(axpby(0.0, V0, 1.0 / beta, V0, n, ctx->stream), "scale");
     std::fill(g.begin(), g.end(), 0.0);
@@ -371,7 +386,9 @@ int fgmres_steps(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres
       if ((rc = wait_words(ctx, col, j + 3))) return rc;
       for (int i = 0; i <= j; ++i) hcol[i] = col[i];
       const double hn = col[j + 1];
-      S->reorth_count += col[j + 2] != 0.0 ? 1 : 0;
+      if (hn == 0.0 || std::any_of(col, col + j + 3, [](double v) { return std::isnan(v); }))
+        if ((rc = reductions_ended(ctx))) return rc;
+      S->reorth_count += col[j + 2] == 1.0 ? 1 : 0;
       if (!std::isfinite(hn)) return sg_fail(ctx, SG_ERR_NAN, "non-finite Krylov vector");
       hcol[j + 1] = hn;
       for (int i = 0; i < j; ++i) {  // previous rotations
@@ -546,6 +563,7 @@ int sg_solve(sg_ctx* ctx, double* q_aos, const sg_newton_opts* o, sg_solve_repor
            "residual");
     SG_TRY(hipMemcpyAsync(l2, ctx->l2.p, 2 * nv * sizeof(double), hipMemcpyDeviceToHost, ctx->stream), "D2H");
     SG_TRY(hipStreamSynchronize(ctx->stream), "sync");
+    sg_norms_returned(ctx, l2, 2 * nv);
     t_res += tr.s();
     if (it == 0) std::copy(l2, l2 + nv, l2_0);
     for (int k = 0; k < nv; ++k) S->l2_hist.push_back(l2[k]);

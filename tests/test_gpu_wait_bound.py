@@ -1,0 +1,95 @@
+"""What follows a wait between work-groups that gave up: with no polls allowed, a
+launch's reducing block gives up while the other blocks still run, and their
+values stay behind in the slots that it emptied.  Later results may not be made
+of them: each is NaN or right, and right again after a call that returned to the
+host."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from structured_amd import cases, lib
+
+pytestmark = pytest.mark.gpu
+
+
+def set_polls(eq, polls):
+    assert lib.load().sg_test_wait_polls(eq.h, C.c_int(polls)) == 0
+
+
+@pytest.fixture
+def eq():
+    case = cases.laminar_plate(97, 65)
+    e = lib.Equation(case)
+    yield e
+    set_polls(e, -1)
+    e.close()
+
+
+def states(eq):
+    return [eq.case.perturbed_state(seed=s, amp=0.01) for s in (1, 2)]
+
+
+def on_device(eq, q):
+    torch = pytest.importorskip("torch")
+    aos = torch.from_numpy(np.ascontiguousarray(q).reshape(-1)).to("cuda:0")
+    d = torch.zeros(eq.nvar * eq.plane, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    eq.aos_to_soa_dev(aos.data_ptr(), d.data_ptr())
+    eq.synchronize()
+    return d
+
+
+def test_norms_after_a_wait_that_gave_up(eq):
+    torch = pytest.importorskip("torch")
+    qd = [on_device(eq, q) for q in states(eq)]
+    rd = torch.zeros_like(qd[0])
+    l2 = torch.zeros(eq.nvar, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+
+    def norms(k):
+        eq.residual_dev_async(qd[k].data_ptr(), rd.data_ptr(), l2.data_ptr())
+        eq.synchronize()
+        return l2.cpu().numpy()
+    ref = norms(1)
+    assert np.isfinite(ref).all()
+    set_polls(eq, 0)
+    assert np.isnan(norms(0)).any()
+    set_polls(eq, -1)
+    for _ in range(2):
+        after = norms(1)
+        print("after", after, "right", ref)
+        assert np.array_equal(after, ref) or np.isnan(after).all()
+    eq.residual_dev(qd[1].data_ptr(), rd.data_ptr())
+    assert np.array_equal(norms(1), ref)
+
+
+def test_explicit_step_after_a_wait_that_gave_up(eq):
+    q1, q2 = states(eq)
+    d1, d2, d3 = on_device(eq, q1), on_device(eq, q2), on_device(eq, q2)
+    ref = eq.step_explicit_dev(d2.data_ptr(), "rk4_jameson", 0.5)
+    assert np.isfinite(ref).all()
+    set_polls(eq, 0)
+    with pytest.raises(lib.SgError):
+        eq.step_explicit_dev(d1.data_ptr(), "rk4_jameson", 0.5)
+    set_polls(eq, -1)
+    assert np.array_equal(eq.step_explicit_dev(d3.data_ptr(), "rk4_jameson", 0.5), ref)
+
+
+def test_linear_solve_after_a_wait_that_gave_up(eq):
+    q1, q2 = states(eq)
+    dt = eq.calc_dt(q1, 20.0)
+    r1, _ = eq.calc_residual(q1)
+    r2, _ = eq.calc_residual(q2)
+    eq.ls_preallocate(restart=12, precond=4, maxit=12, rtol=1e-6)
+    eq.ls_set_lhs(q1, dt)
+    eq.ls_set_rhs(r2)
+    ref = eq.ls_solve()
+    eq.ls_set_rhs(r1)
+    set_polls(eq, 0)
+    with pytest.raises(lib.SgError):
+        eq.ls_solve()
+    set_polls(eq, -1)
+    eq.ls_set_rhs(r2)
+    got = eq.ls_solve()
+    assert got[1:] == ref[1:] and np.array_equal(got[0], ref[0])
