@@ -183,9 +183,12 @@ struct Lay {
     const int q = n / 4;
     return f < 4 * q ? (unsigned)((f / 4 * LN + lane) * 4 + (f & 3)) : (unsigned)(4 * q * LN + (f - 4 * q) * LN + lane);
   }
-  // words of one link (edge values, all rows) and of all links
+  // words of one link (edge values, all rows), and of the links with their head
+  // (on whole lines)
   __host__ __device__ static size_t link(int njc) { return (size_t)njc * GC * NV; }
-  static size_t links(int nchunk, int njc) { return (size_t)nchunk * (NG - 1) * link(njc); }
+  static size_t links(int nchunk, int njc) {
+    return kSlotHead + ((size_t)nchunk * (NG - 1) * link(njc) + 15) / 16 * 16;
+  }
 };
 
 // Zeroes the records of M^-1 that the factorisation does not write, or writes
@@ -314,14 +317,6 @@ template <int NV, int W, bool NINE>
 static size_t cilu_ops(int nic, int njc) {
   const int nchunk = (nic + W - 1) / W, nlev = njc + 2 * W - 2;
   return (size_t)nchunk * nlev * Fac<NV, W, NINE>::N2 * W * NV;
-}
-
-// A link word that holds no value: a signalling NaN, which no arithmetic
-// produces.
-constexpr unsigned long long kEmpty = 0x7FF45347454D5054ull;
-__global__ __launch_bounds__(256) void cilu_empty_kernel(unsigned long long* x, size_t n) {
-  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x)
-    x[e] = kEmpty;
 }
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -580,17 +575,15 @@ __device__ __forceinline__ void lds_release() { __builtin_amdgcn_fence(__ATOMIC_
 __device__ __forceinline__ void lds_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local"); }
 
 constexpr int kAll = 1 << 29;  // a count that never holds the solving wave up
-// Polls without a new row before a link gives up (each takes about a
-// microsecond, so several seconds).  The one that fills a link runs or has run
-// (sg_pass_order.hpp), so the wait ends.
-constexpr int kLinkPolls = 1 << 22;
-
 // The receiving wave of one pass: moves the edge rows the group before
 // publishes into the ring.  One poll reads as many rows as fit the wave; a
-// word is read as one 64-bit atomic and holds either a value or kEmpty, so
-// nothing has to be ordered between words.
+// word is read as one 64-bit atomic and holds either a value or kNoValue, so
+// nothing has to be ordered between words.  The one that fills a link runs or has
+// run (sg_pass_order.hpp), so the wait ends.  One that gives up, after `most`
+// polls without a new row, fills the state of the links' head (see SlotHead).
 template <int NV, int W, bool NINE, int P>
-__device__ void cilu_receive(unsigned long long* in, int njc, ApplyLds<NV, W, NINE, P>& sh) {
+__device__ void cilu_receive(unsigned long long* links, unsigned long long* in, int njc, int most,
+                             ApplyLds<NV, W, NINE, P>& sh) {
   using La = Lay<NV, W, NINE, P>;
   constexpr int EN = La::GCX * NV, RP = 64 / EN;
   const int lane = threadIdx.x & 63, rr = lane / EN, gi = lane % EN / NV, k = lane % NV;
@@ -599,13 +592,12 @@ __device__ void cilu_receive(unsigned long long* in, int njc, ApplyLds<NV, W, NI
     // edge column gi's row s belongs to step s + X - 2 (1 + gi); its place
     // holds a value that is read up to three steps after its own
     const int row = n + rr, free = lds_read(&sh.step) + kRing - 8 - La::X;
-    unsigned long long v = kEmpty;
-    if (rr < RP && row < njc && row < free)
-      v = __hip_atomic_load(in + (size_t)row * EN + lane % EN, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned long long missing = ~__ballot(v != kEmpty);
+    unsigned long long v = kNoValue;
+    if (rr < RP && row < njc && row < free) v = slot_load(in + (size_t)row * EN + lane % EN);
+    const unsigned long long missing = ~__ballot(v != kNoValue);
     const int rows = min(RP, (missing ? __builtin_ctzll(missing) : 64) / EN);
     if (rows == 0) {
-      if (n < free && ++polls > kLinkPolls) break;  // a full ring is no failure
+      if (n < free && ++polls > most) break;  // a full ring is no failure
       continue;
     }
     polls = 0;
@@ -616,6 +608,7 @@ __device__ void cilu_receive(unsigned long long* in, int njc, ApplyLds<NV, W, NI
     if (lane == 0) lds_write(&sh.edges, n < njc ? n : kAll);
   }
   if (n < njc) {  // never filled: every value that depends on it becomes NaN
+    if (lane == 0) slots_lost(links);
     for (int e = lane; e < kRing * EN; e += 64) sh.ring[e / EN][e % EN / NV][e % NV] = __builtin_nan("");
     lds_release();
     if (lane == 0) lds_write(&sh.edges, kAll);
@@ -625,16 +618,19 @@ __device__ void cilu_receive(unsigned long long* in, int njc, ApplyLds<NV, W, NI
 // The storing wave of one pass: takes finished rows out of the ring, stores
 // them to z (a row is contiguous in memory, a step's cells are not) and
 // publishes the edge columns for the next group.  In the solving wave these
-// stores held up the loads, whose waits run in issue order.
+// stores held up the loads, whose waits run in issue order.  After a wait on a
+// link that gave up in an earlier launch it stores NaN instead, until the next
+// factorisation: values that came late may lie in the links.
 template <int NV, int W, bool NINE, int P, bool ASC>
 __device__ void cilu_store(double* z, int njc, int ldi, size_t plane, int col0, int wk, unsigned long long* out,
-                           ApplyLds<NV, W, NINE, P>& sh) {
+                           const unsigned long long* links, ApplyLds<NV, W, NINE, P>& sh) {
   using La = Lay<NV, W, NINE, P>;
   constexpr int LAST = La::X + 2 * (La::GW - 1), RB = 4;
   const int lane = threadIdx.x & 63, k = lane % NV, c1 = lane / NV, c = ASC ? c1 : La::GW - 1 - c1;
   const int gi = La::GW - 1 - c1;
   const bool live = c1 < La::GW && c < wk, pub = out && c1 < La::GW && gi < La::GC;
   double* zl = z + (size_t)k * plane + col0 + (live ? c : 0);
+  const bool lost = La::NG > 1 && slot_head(links).state != kNoValue;
   for (int n = 0; n < njc;) {
     const int rows = min(min(lds_read(&sh.step) - LAST, njc) - n, RB);
     if (rows <= 0) {
@@ -647,11 +643,12 @@ __device__ void cilu_store(double* z, int njc, int ldi, size_t plane, int col0, 
     for (int r = 0; r < RB; ++r)
       v[r] = sh.ring[(La::X + n + r + 2 * c1) & (kRing - 1)][min(La::GCX + c1, ApplyLds<NV, W, NINE, P>::NP)][k];
 #pragma unroll
+    for (int r = 0; r < RB; ++r) v[r] = lost ? __builtin_nan("") : v[r];
+#pragma unroll
     for (int r = 0; r < RB; ++r) {
       if (r >= rows) break;
       if (pub)
-        __hip_atomic_store(out + ((size_t)(n + r) * La::GCX + gi) * NV + k, (unsigned long long)__double_as_longlong(v[r]),
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        slot_store(out + ((size_t)(n + r) * La::GCX + gi) * NV + k, (unsigned long long)__double_as_longlong(v[r]));
       if (live) zl[(size_t)(ASC ? n + r : njc - 1 - n - r) * ldi] = v[r];
     }
     n += rows;
@@ -1026,7 +1023,8 @@ __device__ __forceinline__ void cilu_solve(const float* R, int njc, ApplyLds<NV,
 // lanes) 966 / 448 / 576, the last with both passes in one launch.
 template <int NV, int W, bool NINE, int P, bool TR, bool ASC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void cilu_pass_kernel(
-    int nic, int njc, int ldi, int nchunk, const float* rec, unsigned long long* links, const double* src, double* z) {
+    int nic, int njc, int ldi, int nchunk, const float* rec, unsigned long long* links, int most,
+    const double* src, double* z) {
   using La = Lay<NV, W, NINE, P>;
   // non-transposed: unit-lower L ascending, then D + U descending;
   // transposed: (D + U)^T ascending, then unit-lower L^T descending
@@ -1062,54 +1060,53 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   } else if (wave == 1) {
     cilu_load<NV, W, NINE, P, ASC, DIAG>(R, njc, ldi, plane, col0, wg, src, sh);
   } else if (wave == 2) {
-    cilu_store<NV, W, NINE, P, ASC>(z, njc, ldi, plane, col0, wg, to ? out : nullptr, sh);
+    cilu_store<NV, W, NINE, P, ASC>(z, njc, ldi, plane, col0, wg, to ? out : nullptr, links, sh);
   } else if (from) {
-    cilu_receive<NV, W, NINE, P>(in, njc, sh);
+    cilu_receive<NV, W, NINE, P>(links, in, njc, most, sh);
     // empty for the next pass
-    for (size_t e = threadIdx.x & 63; e < lw; e += 64)
-      __hip_atomic_store(in + e, kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (size_t e = threadIdx.x & 63; e < lw; e += 64) slot_store(in + e, kNoValue);
   }
 }
 
+// The store of a factorisation: the links with their head, the records, the
+// factorisation's operands.
 template <int NV, int W, bool NINE, int P>
 static size_t cilu_size_t(int nic, int njc) {
   using La = Lay<NV, W, NINE, P>;
   const int nchunk = (nic + W - 1) / W;
-  return (La::floats(nchunk, njc) + 3) / 4 * 2 + La::links(nchunk, njc) + 2 * cilu_ops<NV, W, NINE>(nic, njc) + 1;
+  return La::links(nchunk, njc) + La::floats(nchunk, njc) / 2 + 2 * cilu_ops<NV, W, NINE>(nic, njc);
 }
 
 template <int NV, int W, bool NINE, int P>
-static void cilu_factor_t(int nic, int njc, int ldi, const double* idt, const double* blocks, double* store,
-                          hipStream_t s) {
+static hipError_t cilu_factor_t(int nic, int njc, int ldi, const double* idt, const double* blocks, double* store,
+                                hipStream_t s) {
   using La = Lay<NV, W, NINE, P>;
   const int nchunk = (nic + W - 1) / W, nlev = njc + 2 * W - 2;
   const size_t total = cilu_ops<NV, W, NINE>(nic, njc), nl = La::links(nchunk, njc);
-  double* links = store + (La::floats(nchunk, njc) + 3) / 4 * 2;
-  double2* ops = reinterpret_cast<double2*>(links + (nl + 1) / 2 * 2);
+  float* rec = reinterpret_cast<float*>(store + nl);
+  double2* ops = reinterpret_cast<double2*>(rec + La::floats(nchunk, njc));
   hipLaunchKernelGGL((cilu_zero_kernel<NV, W, NINE, P>), dim3(La::nrec(njc), nchunk * La::NG), dim3(256), 0, s, nic, njc,
-                     nchunk, reinterpret_cast<float*>(store));
+                     nchunk, rec);
   const size_t nblk = std::min<size_t>((total + 255) / 256, (size_t)1 << 20);
   hipLaunchKernelGGL((cilu_gather_kernel<NV, W, NINE>), dim3((unsigned)nblk), dim3(256), 0, s, nic, njc, ldi, nlev, idt,
                      blocks, ops, total);
   hipLaunchKernelGGL((cilu_factor_kernel<NV, W, NINE, P>), dim3(nchunk), dim3(64 * Fac<NV, W, NINE>::NW), 0, s, nic, njc, nlev, ops,
-                     reinterpret_cast<float*>(store));
+                     rec);
   hipLaunchKernelGGL((cilu_transpose_kernel<NV, W, NINE, P>), dim3(La::nrec(njc), nchunk * La::NG), dim3(256), 0, s, nic,
-                     njc, nchunk, reinterpret_cast<float*>(store));
-  if (nl)
-    hipLaunchKernelGGL(cilu_empty_kernel, dim3((unsigned)std::min<size_t>((nl + 255) / 256, 1024)), dim3(256), 0, s,
-                       reinterpret_cast<unsigned long long*>(links), nl);
+                     njc, nchunk, rec);
+  return reduce_slots_init(store, nl, s);
 }
 
 template <int NV, int W, bool NINE, int P>
-static void cilu_apply_t(int nic, int njc, int ldi, double* store, const double* b, double* z, bool tr,
+static void cilu_apply_t(int nic, int njc, int ldi, double* store, const double* b, double* z, bool tr, int most,
                          hipStream_t s) {
   using La = Lay<NV, W, NINE, P>;
   const int nchunk = (nic + W - 1) / W;
-  const float* rec = reinterpret_cast<const float*>(store);
-  unsigned long long* links = reinterpret_cast<unsigned long long*>(store + (La::floats(nchunk, njc) + 3) / 4 * 2);
+  const float* rec = reinterpret_cast<const float*>(store + La::links(nchunk, njc));
+  unsigned long long* links = reinterpret_cast<unsigned long long*>(store) + kSlotHead;
   const dim3 grid(pass_blocks(nchunk, La::NG)), block(La::NG > 1 ? 256 : 192);
   auto pass = [&](auto kernel, const double* src) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, s, nic, njc, ldi, nchunk, rec, links, src, z);
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, nic, njc, ldi, nchunk, rec, links, most, src, z);
   };
   if (tr) {
     pass(cilu_pass_kernel<NV, W, NINE, P, true, true>, b);
@@ -1134,9 +1131,9 @@ static size_t cilu_size_w(int nic, int njc) {
   return cilu_lanes<NV, W, NINE>(nic) == 2 ? cilu_size_t<NV, W, NINE, 2>(nic, njc) : cilu_size_t<NV, W, NINE, 1>(nic, njc);
 }
 template <int NV, int W, bool NINE, class... T>
-static void cilu_factor_w(int nic, T... a) {
-  if (cilu_lanes<NV, W, NINE>(nic) == 2) cilu_factor_t<NV, W, NINE, 2>(nic, a...);
-  else cilu_factor_t<NV, W, NINE, 1>(nic, a...);
+static hipError_t cilu_factor_w(int nic, T... a) {
+  if (cilu_lanes<NV, W, NINE>(nic) == 2) return cilu_factor_t<NV, W, NINE, 2>(nic, a...);
+  return cilu_factor_t<NV, W, NINE, 1>(nic, a...);
 }
 template <int NV, int W, bool NINE, class... T>
 static void cilu_apply_w(int nic, T... a) {
@@ -1145,34 +1142,33 @@ static void cilu_apply_w(int nic, T... a) {
 }
 
 template <bool NINE>
-static void cilu_factor_n(int nic, int njc, int ldi, int nv, int w, const double* idt, const double* blocks,
-                          double* store, hipStream_t s) {
+static hipError_t cilu_factor_n(int nic, int njc, int ldi, int nv, int w, const double* idt, const double* blocks,
+                                double* store, hipStream_t s) {
   if (nv == 5) {
-    if (w == 8) cilu_factor_w<5, 8, NINE>(nic, njc, ldi, idt, blocks, store, s);
-    else if (w == 16) cilu_factor_w<5, 16, NINE>(nic, njc, ldi, idt, blocks, store, s);
-    else if (w == 24) cilu_factor_w<5, 24, NINE>(nic, njc, ldi, idt, blocks, store, s);
-    else cilu_factor_w<5, 32, NINE>(nic, njc, ldi, idt, blocks, store, s);
-  } else {
-    if (w == 8) cilu_factor_w<4, 8, NINE>(nic, njc, ldi, idt, blocks, store, s);
-    else if (w == 16) cilu_factor_w<4, 16, NINE>(nic, njc, ldi, idt, blocks, store, s);
-    else if (w == 24) cilu_factor_w<4, 24, NINE>(nic, njc, ldi, idt, blocks, store, s);
-    else cilu_factor_w<4, 32, NINE>(nic, njc, ldi, idt, blocks, store, s);
+    if (w == 8) return cilu_factor_w<5, 8, NINE>(nic, njc, ldi, idt, blocks, store, s);
+    if (w == 16) return cilu_factor_w<5, 16, NINE>(nic, njc, ldi, idt, blocks, store, s);
+    if (w == 24) return cilu_factor_w<5, 24, NINE>(nic, njc, ldi, idt, blocks, store, s);
+    return cilu_factor_w<5, 32, NINE>(nic, njc, ldi, idt, blocks, store, s);
   }
+  if (w == 8) return cilu_factor_w<4, 8, NINE>(nic, njc, ldi, idt, blocks, store, s);
+  if (w == 16) return cilu_factor_w<4, 16, NINE>(nic, njc, ldi, idt, blocks, store, s);
+  if (w == 24) return cilu_factor_w<4, 24, NINE>(nic, njc, ldi, idt, blocks, store, s);
+  return cilu_factor_w<4, 32, NINE>(nic, njc, ldi, idt, blocks, store, s);
 }
 
 template <bool NINE>
 static void cilu_apply_n(int nic, int njc, int ldi, int nv, int w, double* store, const double* b, double* z,
-                         bool transpose, hipStream_t s) {
+                         bool transpose, int most, hipStream_t s) {
   if (nv == 5) {
-    if (w == 8) cilu_apply_w<5, 8, NINE>(nic, njc, ldi, store, b, z, transpose, s);
-    else if (w == 16) cilu_apply_w<5, 16, NINE>(nic, njc, ldi, store, b, z, transpose, s);
-    else if (w == 24) cilu_apply_w<5, 24, NINE>(nic, njc, ldi, store, b, z, transpose, s);
-    else cilu_apply_w<5, 32, NINE>(nic, njc, ldi, store, b, z, transpose, s);
+    if (w == 8) cilu_apply_w<5, 8, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
+    else if (w == 16) cilu_apply_w<5, 16, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
+    else if (w == 24) cilu_apply_w<5, 24, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
+    else cilu_apply_w<5, 32, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
   } else {
-    if (w == 8) cilu_apply_w<4, 8, NINE>(nic, njc, ldi, store, b, z, transpose, s);
-    else if (w == 16) cilu_apply_w<4, 16, NINE>(nic, njc, ldi, store, b, z, transpose, s);
-    else if (w == 24) cilu_apply_w<4, 24, NINE>(nic, njc, ldi, store, b, z, transpose, s);
-    else cilu_apply_w<4, 32, NINE>(nic, njc, ldi, store, b, z, transpose, s);
+    if (w == 8) cilu_apply_w<4, 8, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
+    else if (w == 16) cilu_apply_w<4, 16, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
+    else if (w == 24) cilu_apply_w<4, 24, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
+    else cilu_apply_w<4, 32, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
   }
 }
 
@@ -1193,15 +1189,14 @@ size_t cilu_size(int nic, int njc, int nv, int w, bool nine) {
 
 hipError_t cilu_factor(int nic, int njc, int ldi, int nv, int w, bool nine, const double* idt, const double* blocks,
                        double* store, hipStream_t s) {
-  if (nine) cilu_factor_n<true>(nic, njc, ldi, nv, w, idt, blocks, store, s);
-  else cilu_factor_n<false>(nic, njc, ldi, nv, w, idt, blocks, store, s);
-  return hipGetLastError();
+  return nine ? cilu_factor_n<true>(nic, njc, ldi, nv, w, idt, blocks, store, s)
+              : cilu_factor_n<false>(nic, njc, ldi, nv, w, idt, blocks, store, s);
 }
 
 hipError_t cilu_apply(int nic, int njc, int ldi, int nv, int w, bool nine, double* store, const double* b, double* z,
-                      bool transpose, hipStream_t s) {
-  if (nine) cilu_apply_n<true>(nic, njc, ldi, nv, w, store, b, z, transpose, s);
-  else cilu_apply_n<false>(nic, njc, ldi, nv, w, store, b, z, transpose, s);
+                      bool transpose, int polls, hipStream_t s) {
+  if (nine) cilu_apply_n<true>(nic, njc, ldi, nv, w, store, b, z, transpose, polls, s);
+  else cilu_apply_n<false>(nic, njc, ldi, nv, w, store, b, z, transpose, polls, s);
   return hipGetLastError();
 }
 

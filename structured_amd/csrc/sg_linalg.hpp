@@ -60,15 +60,15 @@ hipError_t lilu_apply(int nic, int njc, int ldi, int nv, const double* ilu, cons
 // chunked line block ILU(0) (sg_cilu.hip): chunks of w in {8, 16, 24, 32}
 // columns, on the 13-point stencil or (nine) the 3x3-box pattern; cilu_size
 // is the storage in doubles that cilu_factor writes and cilu_apply reads: the
-// FP32 factors in the order of M^-1 and of M^-T, the links between column
-// groups (empty between applies), and the factorisation's operands gathered
-// in level order
+// links between column groups with their SlotHead (empty between applies), the
+// FP32 factors in the order of M^-1 and of M^-T, and the factorisation's operands
+// gathered in level order.  polls bounds the apply's waits on the links
 bool cilu_width_ok(int w);
 size_t cilu_size(int nic, int njc, int nv, int w, bool nine);
 hipError_t cilu_factor(int nic, int njc, int ldi, int nv, int w, bool nine, const double* idt, const double* blocks,
                        double* rec, hipStream_t s);
 hipError_t cilu_apply(int nic, int njc, int ldi, int nv, int w, bool nine, double* store, const double* b, double* z,
-                      bool transpose, hipStream_t s);
+                      bool transpose, int polls, hipStream_t s);
 // adjoint helpers: J^T psi from the blocks, or with idt psi idt - J^T psi
 hipError_t jt_gather(int nic, int njc, int ldi, int nv, const double* blocks, const double* psi, double* out,
                      hipStream_t s, const double* idt = nullptr);

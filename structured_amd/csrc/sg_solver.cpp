@@ -114,14 +114,19 @@ int ensure(sg_ctx* ctx, int restart) {
 
 Slots slots(sg_ctx* ctx) { return {ctx->solver->partial.p, ctx->wait_polls}; }
 
-// An error if a reduction of this solve gave up waiting.  Asked only where a
-// result is NaN or a norm 0: such a reduction leaves one or the other.
-int reductions_ended(sg_ctx* ctx) {
-  unsigned long long state = 0;
+// An error if a wait inside a kernel of this solve gave up.  Asked only where a
+// result is NaN or a norm 0: such a wait leaves one or the other.
+int waits_ended(sg_ctx* ctx) {
+  SolverState* S = ctx->solver;
+  unsigned long long state[2] = {kNoValue, kNoValue};
   static_assert(offsetof(SlotHead, state) == 0, "the head's first word");
-  SG_TRY(hipMemcpyAsync(&state, ctx->solver->partial.p, sizeof(state), hipMemcpyDeviceToHost, ctx->stream), "D2H");
+  SG_TRY(hipMemcpyAsync(&state[0], S->partial.p, sizeof(state[0]), hipMemcpyDeviceToHost, ctx->stream), "D2H");
+  if (S->precond >= 6)
+    SG_TRY(hipMemcpyAsync(&state[1], S->cilu.p, sizeof(state[1]), hipMemcpyDeviceToHost, ctx->stream), "D2H");
   SG_TRY(hipStreamSynchronize(ctx->stream), "sync");
-  return state == kNoValue ? SG_OK : sg_fail(ctx, SG_ERR_HIP, "a reduction gave up waiting for its partial sums");
+  if (state[0] != kNoValue) return sg_fail(ctx, SG_ERR_HIP, "a reduction gave up waiting for its partial sums");
+  if (state[1] != kNoValue) return sg_fail(ctx, SG_ERR_HIP, "the preconditioner gave up waiting for edge values");
+  return SG_OK;
 }
 
 double host_dot(sg_ctx* ctx, const double* a, const double* b, int* rc) {
@@ -148,7 +153,8 @@ int precond_apply(sg_ctx* ctx, const double* v, double* z) {
     return SG_OK;
   }
   if (S->precond == 6 || S->precond == 7) {
-    SG_TRY(cilu_apply(nic, njc, ldi, nv, S->pc_width, S->precond == 7, S->cilu.p, v, z, S->transpose, ctx->stream),
+    SG_TRY(cilu_apply(nic, njc, ldi, nv, S->pc_width, S->precond == 7, S->cilu.p, v, z, S->transpose,
+                      ctx->wait_polls, ctx->stream),
            "cilu apply");
     return SG_OK;
   }
@@ -363,7 +369,7 @@ int fgmres_steps(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres
     }
     const double beta = total == 0 ? bnorm : std::sqrt(host_dot(ctx, V0, V0, &rc));
     if (rc) return rc;
-    if (std::isnan(beta) && (rc = reductions_ended(ctx))) return rc;
+    if (std::isnan(beta) && (rc = waits_ended(ctx))) return rc;
     if (beta == 0.0) { res = 0.0; break; }
     SG_TRY(axpby(0.0, V0, 1.0 / beta, V0, n, ctx->stream), "scale");
     std::fill(g.begin(), g.end(), 0.0);
@@ -387,7 +393,7 @@ int fgmres_steps(sg_ctx* ctx, double rtol, int maxit, int* iters, double* relres
       for (int i = 0; i <= j; ++i) hcol[i] = col[i];
       const double hn = col[j + 1];
       if (hn == 0.0 || std::any_of(col, col + j + 3, [](double v) { return std::isnan(v); }))
-        if ((rc = reductions_ended(ctx))) return rc;
+        if ((rc = waits_ended(ctx))) return rc;
       S->reorth_count += col[j + 2] == 1.0 ? 1 : 0;
       if (!std::isfinite(hn)) return sg_fail(ctx, SG_ERR_NAN, "non-finite Krylov vector");
       hcol[j + 1] = hn;

@@ -93,3 +93,31 @@ def test_linear_solve_after_a_wait_that_gave_up(eq):
     eq.ls_set_rhs(r2)
     got = eq.ls_solve()
     assert got[1:] == ref[1:] and np.array_equal(got[0], ref[0])
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+def test_preconditioner_after_a_wait_that_gave_up(eq, transpose):
+    q, _ = states(eq)
+    dt = eq.calc_dt(q, 20.0)
+    rng = np.random.default_rng(1)
+    v1, v2 = rng.standard_normal(q.shape), rng.standard_normal(q.shape)
+    eq.ls_preallocate(restart=4, precond=7, maxit=4, rtol=1e-6)
+    eq.ls_set_pc(1, 1.0, 32)
+    eq.ls_set_lhs(q, dt)
+    eq.ls_set_rhs(v1)
+    refs = [eq.ls_precond_apply(v, transpose=transpose) for v in (v1, v2)]
+
+    def apply(n):
+        z = eq.ls_precond_apply((v1, v2)[n], transpose=transpose)
+        nan, wrong = np.isnan(z), z != refs[n]
+        print("NaN", np.count_nonzero(nan), "wrong", np.count_nonzero(wrong & ~nan))
+        assert not (wrong & ~nan).any()
+        return nan.any()
+    set_polls(eq, 0)
+    assert apply(0)
+    set_polls(eq, -1)
+    assert apply(1) and apply(0)
+    with pytest.raises(lib.SgError):  # a solve does not take the NaN for the end of its iteration
+        eq.ls_solve()
+    eq.ls_set_lhs(q, dt)
+    assert not apply(0) and not apply(1)
