@@ -37,14 +37,14 @@ def oracle_blocks(case, q, wd):
 
 @pytest.mark.parametrize("cols,rows,sa,width", [
     (33, 3, True, 32),    # a chunk of one column, three rows
-    (23, 131, True, 32),  # groups of 11, 11 and 1 columns; the ring wraps
-    (11, 70, True, 32),   # one full group of a chunk whose others are absent
-    (24, 9, False, 24),   # two groups of 12
-    (30, 67, False, 32),  # nv = 4, last group not full, the ring wraps
-    (17, 66, False, 16),  # nv = 4: one group of 16, then one column
-    (6, 65, True, 32),    # the widths that two lanes a row allow: 6 columns, nv 5
+    (23, 131, True, 32),  # groups of 6, the last of 5; the ring wraps
+    (11, 70, True, 32),   # a group of 6 and one of 5 of a chunk whose others are absent
+    (24, 9, False, 24),   # three groups of 8
+    (30, 67, False, 32),  # nv = 4, groups of 8, the last of 6; the ring wraps
+    (17, 66, False, 16),  # nv = 4: two groups of 8, then one column
+    (6, 65, True, 32),    # one group of 6, nv 5
     (13, 12, True, 16),
-    (8, 64, False, 8),    # and 8, nv 4
+    (8, 64, False, 8),    # one group of 8, nv 4
     (25, 5, False, 32),
 ])
 @pytest.mark.parametrize("precond", [6, 7])
