@@ -51,9 +51,11 @@ __global__ __launch_bounds__(256) void forward_euler_kernel(DevGeom g, int nv, d
   }
 }
 
-int ensure_buffers(sg_ctx* ctx) {
+// The residual of forward Euler, or the two stage states of RK4.
+int ensure_buffers(sg_ctx* ctx, int scheme) {
   const size_t n = ctx->nsoa();
-  for (DevBuf* b : {&ctx->ex_a, &ctx->ex_b, &ctx->ex_r})
+  const bool euler = scheme == SG_SCHEME_FORWARD_EULER;
+  for (DevBuf* b : {euler ? &ctx->ex_r : &ctx->ex_a, euler ? &ctx->ex_r : &ctx->ex_b})
     if (b->n != n) SG_TRY(b->alloc(n), "explicit work buffers");
   return SG_OK;
 }
@@ -106,7 +108,7 @@ int sg_step_explicit_dev(sg_ctx* ctx, double* q_dev, int scheme, double cfl, dou
   if (!ctx || !q_dev) return SG_ERR_ARG;
   int rc;
   if ((rc = check_args(ctx, scheme, cfl))) return rc;
-  if ((rc = ensure_buffers(ctx))) return rc;
+  if ((rc = ensure_buffers(ctx, scheme))) return rc;
   if ((rc = enqueue_step(ctx, q_dev, scheme, cfl))) return rc;
   double h[10];
   SG_TRY(hipMemcpyAsync(h, ctx->l2.p, ctx->nvar * sizeof(double), hipMemcpyDeviceToHost, ctx->stream), "D2H");
@@ -123,7 +125,7 @@ int sg_solve_explicit(sg_ctx* ctx, double* q_aos, const sg_explicit_opts* o, sg_
   int rc;
   if ((rc = check_args(ctx, o->scheme, o->cfl))) return rc;
   if (o->iteration_max < 0) return sg_fail(ctx, SG_ERR_ARG, "iteration_max must be >= 0");
-  if ((rc = ensure_buffers(ctx))) return rc;
+  if ((rc = ensure_buffers(ctx, o->scheme))) return rc;
   const auto t0 = std::chrono::steady_clock::now();
   const int nv = ctx->nvar;
   const size_t ncell = ctx->ncell();

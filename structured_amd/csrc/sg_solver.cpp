@@ -45,7 +45,7 @@ using namespace sg;
 struct SolverState {
   int m = 0;                 // restart length
   size_t n = 0;              // vector length (nvar * plane)
-  DevBuf V, Z, blocks, fac, ilu, idt, dtv, rhs, x, tmp, jz, qop, seed, hdev, ydev, partial, gst, dbdiag, ones;
+  DevBuf V, Z, blocks, fac, ilu, idt, dtv, rhs, x, tmp, qop, seed, hdev, ydev, partial, gst, dbdiag, ones;
   DevBuf blocks_pc;          // preconditioner blocks when lhs_order > 0 (blocks keeps the exact J)
   DevBuf cilu;               // chunked line ILU(0) factors (precond 6)
   PinnedBuf hpin;            // a dot product, the Krylov coefficients going up
@@ -99,11 +99,11 @@ int ensure(sg_ctx* ctx, int restart) {
   const size_t nb = ctx->g.plane * NSLOT * nv * nv, nf = ctx->g.plane * 3 * nv * nv;
   if (S->V.alloc((size_t)(restart + 1) * n) || S->Z.alloc((size_t)restart * n) || S->blocks.alloc(nb) ||
       S->fac.alloc(nf) || S->ilu.alloc(nb) || S->gst.alloc(n) || S->dbdiag.alloc(n) || S->ones.alloc(ctx->g.plane) || S->idt.alloc(ctx->g.plane) || S->dtv.alloc(n) || S->rhs.alloc(n) || S->x.alloc(n) ||
-      S->tmp.alloc(n) || S->jz.alloc(n) || S->qop.alloc(n) || S->seed.alloc(n) || S->hdev.alloc(restart + 2) ||
+      S->tmp.alloc(n) || S->qop.alloc(n) || S->seed.alloc(n) || S->hdev.alloc(restart + 2) ||
       S->ydev.alloc(restart + 2) || S->partial.alloc(reduce_slots(restart + 2)) ||
       S->hpin.alloc((size_t)(restart + 2)) || S->hres.alloc(2 * (size_t)(restart + 3)))
     return sg_fail(ctx, SG_ERR_HIP, "solver allocation failed");
-  for (DevBuf* b : {&S->V, &S->Z, &S->blocks, &S->fac, &S->dtv, &S->rhs, &S->x, &S->tmp, &S->jz, &S->qop, &S->seed})
+  for (DevBuf* b : {&S->V, &S->Z, &S->blocks, &S->fac, &S->dtv, &S->rhs, &S->x, &S->tmp, &S->qop, &S->seed})
     if (hipMemset(b->p, 0, b->n * sizeof(double)) != hipSuccess) return sg_fail(ctx, SG_ERR_HIP, "memset");
   // seed stays zero and ones one: the directions of dR/dbeta
   const std::vector<double> one(ctx->g.plane, 1.0);
