@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <limits>
 
@@ -327,6 +328,28 @@ int compute_wall_distance(sg_ctx* ctx, const sg_bc* bcs, int nbc) {
   return SG_OK;
 }
 
+// Whether every CU of the device takes the stream's work, and there are enough for
+// 8 chunks of 8 column groups of the chunked ILU to be resident at once (they
+// are started in turn).  HSA_CU_MASK is below what the mask of a stream says.
+bool all_cus(hipStream_t s) {
+  for (const char* name : {"HSA_CU_MASK", "ROC_GLOBAL_CU_MASK"}) {
+    const char* v = std::getenv(name);
+    if (v && *v) return false;
+  }
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 64)
+    return false;
+  std::vector<uint32_t> mask((cus + 31) / 32, 0u);
+  if (hipExtStreamGetCUMask(s, (uint32_t)mask.size(), mask.data()) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  int on = 0;
+  for (uint32_t m : mask) on += __builtin_popcount(m);
+  return on >= cus;
+}
+
 int check_finite(sg_ctx* ctx, const double* l2) {
   for (int k = 0; k < ctx->nvar; ++k)
     if (!std::isfinite(l2[k])) return sg_fail(ctx, SG_ERR_NAN, "non-finite residual norm");
@@ -383,6 +406,7 @@ int sg_create(int ni, int nj, const double* xv, const double* yv, const sg_frees
     return code;
   };
   if (hipStreamCreate(&ctx->stream) != hipSuccess) return fail(SG_ERR_HIP);
+  ctx->all_cus = all_cus(ctx->stream);
   if ((rc = sg_noalloc_setup(ctx))) return fail(rc);
   // device geometry
   const int ldi = ((G.nic + 63) / 64) * 64, ldf = ((G.ni + 63) / 64) * 64;
@@ -569,6 +593,14 @@ int sg_residual_dev_async(sg_ctx* ctx, const double* q_dev, double* r_dev, doubl
                          ctx->stream, ctx->clo, ctx->nvar),
          "residual launch");
   return SG_OK;
+}
+
+// Not part of the interface: preconditioners 6 and 7 as on a device on which not
+// every CU takes part (few), from the next set_lhs on.  1 if every CU does.
+int sg_test_few_cus(sg_ctx* ctx, int few) {
+  if (!ctx) return SG_ERR_ARG;
+  ctx->all_cus = !few && all_cus(ctx->stream);
+  return ctx->all_cus ? 1 : 0;
 }
 
 // The bound of the kernels' waits for one another, in polls (negative: the

@@ -183,12 +183,11 @@ struct Lay {
     const int q = n / 4;
     return f < 4 * q ? (unsigned)((f / 4 * LN + lane) * 4 + (f & 3)) : (unsigned)(4 * q * LN + (f - 4 * q) * LN + lane);
   }
-  // words of one link (edge values, all rows), and of the links with their head
-  // (on whole lines)
+  // words of one link (edge values of one pass, all rows), of a pass's links, and
+  // of all of them with their head (on whole lines)
   __host__ __device__ static size_t link(int njc) { return (size_t)njc * GC * NV; }
-  static size_t links(int nchunk, int njc) {
-    return kSlotHead + ((size_t)nchunk * (NG - 1) * link(njc) + 15) / 16 * 16;
-  }
+  __host__ __device__ static size_t pass_links(int nchunk, int njc) { return (size_t)nchunk * (NG - 1) * link(njc); }
+  static size_t links(int nchunk, int njc) { return kSlotHead + (2 * pass_links(nchunk, njc) + 15) / 16 * 16; }
 };
 
 // Zeroes the records of M^-1 that the factorisation does not write, or writes
@@ -548,10 +547,15 @@ cilu_factor_kernel(int nic, int njc, int nlev, const double2* ops, float* rec) {
   }
 }
 
+// How far the waves of a work-group have got in a pass: steps solved,
+// right-hand-side rows loaded, edge rows received, rows taken out of the ring.
+struct Progress {
+  int step, loaded, edges, taken;
+};
 // LDS of one group's work-group: the solved values of the last kRing steps by
 // step, column and component (edge columns first; idle lanes store to the
 // column after the last), the right-hand sides of the steps to come, and how
-// far each wave has got.
+// far each wave has got in either pass.
 constexpr int kRing = 64;
 template <int NV, int W, bool NINE, int P>
 struct ApplyLds {
@@ -561,9 +565,8 @@ struct ApplyLds {
   double ring[kRing][NP + 1][NVP] __attribute__((aligned(16)));
   double x[kRing][La::ROWS + 1];  // the last place is always zero
   double tmp[La::GW + 1][8] __attribute__((aligned(16)));  // a row's halves at 0 and 4
-  // steps solved, right-hand-side rows loaded, edge rows received, rows taken
-  // out of the ring
-  int step, loaded, edges, taken;
+  Progress pass[2];
+  int stored;  // the first pass's stores are complete
 };
 __device__ __forceinline__ int lds_read(const int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -578,12 +581,12 @@ constexpr int kAll = 1 << 29;  // a count that never holds the solving wave up
 // The receiving wave of one pass: moves the edge rows the group before
 // publishes into the ring.  One poll reads as many rows as fit the wave; a
 // word is read as one 64-bit atomic and holds either a value or kNoValue, so
-// nothing has to be ordered between words.  The one that fills a link runs or has
-// run (sg_pass_order.hpp), so the wait ends.  One that gives up, after `most`
+// nothing has to be ordered between words.  The one that fills a link runs, has
+// run or will run (see the kernel), so the wait ends.  One that gives up, after `most`
 // polls without a new row, fills the state of the links' head (see SlotHead).
 template <int NV, int W, bool NINE, int P>
 __device__ void cilu_receive(unsigned long long* links, unsigned long long* in, int njc, int most,
-                             ApplyLds<NV, W, NINE, P>& sh) {
+                             ApplyLds<NV, W, NINE, P>& sh, Progress& pr) {
   using La = Lay<NV, W, NINE, P>;
   constexpr int EN = La::GCX * NV, RP = 64 / EN;
   const int lane = threadIdx.x & 63, rr = lane / EN, gi = lane % EN / NV, k = lane % NV;
@@ -591,7 +594,7 @@ __device__ void cilu_receive(unsigned long long* links, unsigned long long* in, 
   while (n < njc) {
     // edge column gi's row s belongs to step s + X - 2 (1 + gi); its place
     // holds a value that is read up to three steps after its own
-    const int row = n + rr, free = lds_read(&sh.step) + kRing - 8 - La::X;
+    const int row = n + rr, free = lds_read(&pr.step) + kRing - 8 - La::X;
     unsigned long long v = kNoValue;
     if (rr < RP && row < njc && row < free) v = slot_load(in + (size_t)row * EN + lane % EN);
     const unsigned long long missing = ~__ballot(v != kNoValue);
@@ -605,13 +608,13 @@ __device__ void cilu_receive(unsigned long long* links, unsigned long long* in, 
       sh.ring[(row + La::X - 2 * (1 + gi)) & (kRing - 1)][La::GCX - 1 - gi][k] = __longlong_as_double((long long)v);
     n += rows;
     lds_release();
-    if (lane == 0) lds_write(&sh.edges, n < njc ? n : kAll);
+    if (lane == 0) lds_write(&pr.edges, n < njc ? n : kAll);
   }
   if (n < njc) {  // never filled: every value that depends on it becomes NaN
     if (lane == 0) slots_lost(links);
     for (int e = lane; e < kRing * EN; e += 64) sh.ring[e / EN][e % EN / NV][e % NV] = __builtin_nan("");
     lds_release();
-    if (lane == 0) lds_write(&sh.edges, kAll);
+    if (lane == 0) lds_write(&pr.edges, kAll);
   }
 }
 
@@ -623,7 +626,7 @@ __device__ void cilu_receive(unsigned long long* links, unsigned long long* in, 
 // factorisation: values that came late may lie in the links.
 template <int NV, int W, bool NINE, int P, bool ASC>
 __device__ void cilu_store(double* z, int njc, int ldi, size_t plane, int col0, int wk, unsigned long long* out,
-                           const unsigned long long* links, ApplyLds<NV, W, NINE, P>& sh) {
+                           const unsigned long long* links, ApplyLds<NV, W, NINE, P>& sh, Progress& pr) {
   using La = Lay<NV, W, NINE, P>;
   constexpr int LAST = La::X + 2 * (La::GW - 1), RB = 4;
   const int lane = threadIdx.x & 63, k = lane % NV, c1 = lane / NV, c = ASC ? c1 : La::GW - 1 - c1;
@@ -632,7 +635,7 @@ __device__ void cilu_store(double* z, int njc, int ldi, size_t plane, int col0, 
   double* zl = z + (size_t)k * plane + col0 + (live ? c : 0);
   const bool lost = La::NG > 1 && slot_head(links).state != kNoValue;
   for (int n = 0; n < njc;) {
-    const int rows = min(min(lds_read(&sh.step) - LAST, njc) - n, RB);
+    const int rows = min(min(lds_read(&pr.step) - LAST, njc) - n, RB);
     if (rows <= 0) {
       __builtin_amdgcn_s_sleep(1);
       continue;
@@ -653,7 +656,7 @@ __device__ void cilu_store(double* z, int njc, int ldi, size_t plane, int col0, 
     }
     n += rows;
     lds_release();
-    if (lane == 0) lds_write(&sh.taken, n < njc ? n : kAll);
+    if (lane == 0) lds_write(&pr.taken, n < njc ? n : kAll);
   }
 }
 
@@ -664,7 +667,7 @@ __device__ void cilu_store(double* z, int njc, int ldi, size_t plane, int col0, 
 // L2 instead of memory (much further ahead, the groups of an XCD overflow it).
 template <int NV, int W, bool NINE, int P, bool ASC, bool DIAG>
 __device__ void cilu_load(const float* R, int njc, int ldi, size_t plane, int col0, int wk, const double* src,
-                          ApplyLds<NV, W, NINE, P>& sh) {
+                          ApplyLds<NV, W, NINE, P>& sh, Progress& pr) {
   using La = Lay<NV, W, NINE, P>;
   constexpr int RS = La::rs(DIAG ? La::n2 : La::n1), LB = 16, TAIL = 2 * (La::GW - 1);
   // a batch is fetched when the solving wave is at step s0 - (kRing - X - TAIL)
@@ -696,15 +699,15 @@ __device__ void cilu_load(const float* R, int njc, int ldi, size_t plane, int co
       for (int u = 0; u < LB; ++u) asm volatile("" ::"v"(touch[u]));
       fetch(s1 + LB, b ^ 1);
       // the last place this batch writes must have been read
-      while (lds_read(&sh.step) < La::X + s1 + LB - 1 + TAIL + 1 - kRing) __builtin_amdgcn_s_sleep(2);
+      while (lds_read(&pr.step) < La::X + s1 + LB - 1 + TAIL + 1 - kRing) __builtin_amdgcn_s_sleep(2);
 #pragma unroll
       for (int u = 0; u < LB; ++u)
         if (lane < La::ROWS) sh.x[(La::X + s1 + u + 2 * c1) & (kRing - 1)][lane] = live && s1 + u < njc ? v[b][u] : 0.0;
       lds_release();
-      if (lane == 0) lds_write(&sh.loaded, s1 + LB);
+      if (lane == 0) lds_write(&pr.loaded, s1 + LB);
     }
   }
-  if (lane == 0) lds_write(&sh.loaded, kAll);
+  if (lane == 0) lds_write(&pr.loaded, kAll);
 }
 
 
@@ -725,7 +728,7 @@ __device__ __forceinline__ double pair_sum(double v) {
 // neighbours is done by the other waves, and no step has a branch but the one
 // that waits for them.
 template <int NV, int W, bool NINE, bool DIAG>
-__device__ __forceinline__ void cilu_solve_pairs(const float* R, int njc, ApplyLds<NV, W, NINE, 2>& sh, bool up) {
+__device__ __forceinline__ void cilu_solve_pairs(const float* R, int njc, ApplyLds<NV, W, NINE, 2>& sh, Progress& pr, bool up) {
   using La = Lay<NV, W, NINE, 2>;
   using A = ApplyLds<NV, W, NINE, 2>;
   constexpr int N = DIAG ? La::n2 : La::n1, RS = La::rs(N), NQ = N / 4, NREM = N % 4, PD = La::pd(N), UN = La::UN, ND = La::ND;
@@ -770,8 +773,8 @@ __device__ __forceinline__ void cilu_solve_pairs(const float* R, int njc, ApplyL
     if (__builtin_expect(t < lim, 1)) return;
     do {
       // x is read one step early
-      const int a = lds_read(&sh.loaded) + La::X - 1, b = up ? lds_read(&sh.edges) + 1 : kAll;
-      const int c = lds_read(&sh.taken) + kRing + La::X;
+      const int a = lds_read(&pr.loaded) + La::X - 1, b = up ? lds_read(&pr.edges) + 1 : kAll;
+      const int c = lds_read(&pr.taken) + kRing + La::X;
       lim = __builtin_amdgcn_readfirstlane(min(min(a, b), c));
     } while (t >= lim);
     lds_acquire();
@@ -807,7 +810,6 @@ __device__ __forceinline__ void cilu_solve_pairs(const float* R, int njc, ApplyL
   for (int t0 = 0; t0 < T; t0 += UN) {
     rrec = block_of(t0);
     so = PD * RS * 4;
-    asm volatile("" : "+s"(so));  // a running scalar, not a constant per step
     const int r0 = t0 & (kRing - 1), r1 = (t0 + UN) & (kRing - 1);
     // cell of the column before that is ynext at the block's first step
     const double* y0 = sh.ring[h ? r0 : (r0 - 1) & (kRing - 1)][pos - 1];
@@ -841,7 +843,7 @@ __device__ __forceinline__ void cilu_solve_pairs(const float* R, int njc, ApplyL
       auto* cur = sh.ring[r0 + u];
       cur[wpos][k] = r;
       wave_order();
-      if (u & 1) lds_write(&sh.step, t + 1);
+      if (u & 1) lds_write(&pr.step, t + 1);
       if (u & 1) wait(t + 2);  // for the next two steps
       const double* yn = u == 0 ? y0 : sh.ring[r0 + u - 1 + h][pos - 1];
 #pragma unroll
@@ -862,7 +864,7 @@ __device__ __forceinline__ void cilu_solve_pairs(const float* R, int njc, ApplyL
 
 // The same with one lane a row, which takes both operands of either kind.
 template <int NV, int W, bool NINE, bool DIAG>
-__device__ __forceinline__ void cilu_solve_rows(const float* R, int njc, ApplyLds<NV, W, NINE, 1>& sh, bool up) {
+__device__ __forceinline__ void cilu_solve_rows(const float* R, int njc, ApplyLds<NV, W, NINE, 1>& sh, Progress& pr, bool up) {
   using La = Lay<NV, W, NINE, 1>;
   using A = ApplyLds<NV, W, NINE, 1>;
   constexpr int N = DIAG ? La::n2 : La::n1, RS = La::rs(N), NQ = N / 4, NREM = N % 4, PD = La::pd(N), UN = La::UN;
@@ -902,8 +904,8 @@ __device__ __forceinline__ void cilu_solve_rows(const float* R, int njc, ApplyLd
     if (__builtin_expect(t < lim, 1)) return;
     do {
       // x is read one step early
-      const int a = lds_read(&sh.loaded) + La::X - 1, b = up ? lds_read(&sh.edges) + 1 : kAll;
-      const int c = lds_read(&sh.taken) + kRing + La::X;
+      const int a = lds_read(&pr.loaded) + La::X - 1, b = up ? lds_read(&pr.edges) + 1 : kAll;
+      const int c = lds_read(&pr.taken) + kRing + La::X;
       lim = __builtin_amdgcn_readfirstlane(min(min(a, b), c));
     } while (t >= lim);
     lds_acquire();
@@ -946,7 +948,6 @@ __device__ __forceinline__ void cilu_solve_rows(const float* R, int njc, ApplyLd
   for (int t0 = 0; t0 < T; t0 += UN) {
     rrec = block_of(t0);
     so = PD * RS * 4;
-    asm volatile("" : "+s"(so));  // a running scalar, not a constant per step
     const int r0 = t0 & (kRing - 1), r1 = (t0 + UN) & (kRing - 1);
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
@@ -975,7 +976,7 @@ __device__ __forceinline__ void cilu_solve_rows(const float* R, int njc, ApplyLd
       auto* cur = sh.ring[r0 + u];
       cur[wpos][k] = r;
       wave_order();
-      if (u & 1) lds_write(&sh.step, t + 1);
+      if (u & 1) lds_write(&pr.step, t + 1);
       if (u & 1) wait(t + 2);  // for the next two steps
       double own2[NV], old[NV];
 #pragma unroll
@@ -997,19 +998,23 @@ __device__ __forceinline__ void cilu_solve_rows(const float* R, int njc, ApplyLd
 }
 
 template <int NV, int W, bool NINE, int P, bool DIAG>
-__device__ __forceinline__ void cilu_solve(const float* R, int njc, ApplyLds<NV, W, NINE, P>& sh, bool up) {
-  if constexpr (P == 2) cilu_solve_pairs<NV, W, NINE, DIAG>(R, njc, sh, up);
-  else cilu_solve_rows<NV, W, NINE, DIAG>(R, njc, sh, up);
+__device__ __forceinline__ void cilu_solve(const float* R, int njc, ApplyLds<NV, W, NINE, P>& sh, Progress& pr, bool up) {
+  if constexpr (P == 2) cilu_solve_pairs<NV, W, NINE, DIAG>(R, njc, sh, pr, up);
+  else cilu_solve_rows<NV, W, NINE, DIAG>(R, njc, sh, pr, up);
 }
 
-// One pass of z = (LU)^-1 b, or of (LU)^-T b when TR: the ascending one, or
-// the descending one, in place.  Wave 0 of a work-group solves one column
-// group, wave 1 loads and wave 2 stores for it, and wave 3 receives the edge
-// columns of the group before where a chunk has several.  A launch per pass:
-// with both in one, a group waited in the second for groups started after it,
-// which needs room for all groups of a chunk on its XCD.  The second launch
-// costs 2% of an apply at 1409x641 (450 us against 442), 1% of a Newton solve
-// at 97x65.
+// z = (LU)^-1 b, or (LU)^-T b when TR: the ascending and the descending pass, or
+// one of them.  Wave 0 of a work-group solves one column group, wave 1 loads and
+// wave 2 stores for it, and wave 3 receives the edge columns of the group before
+// where a chunk has several.  Work-groups are dealt to the XCDs round-robin by
+// index: the groups of a chunk sit on one XCD, consecutive in its order.
+//
+// Both passes in one launch: a group waits in the second for groups started after
+// it, so its XCD must have room for all groups of a chunk (at most 6; the chunks
+// before are complete and finish).  The host asks for that only where every CU
+// of the device takes part.  A launch per pass needs no room (see
+// sg_pass_order.hpp) and takes 1.5 to 2.5 us longer on small grids, 8 at 1409x641
+// (448 us).
 //
 // What bounds it: a step of the solving wave, some 57 instructions of one wave
 // and the LDS exchanges that link two steps, times njc + 2 W steps and a pass,
@@ -1017,54 +1022,76 @@ __device__ __forceinline__ void cilu_solve(const float* R, int njc, ApplyLds<NV,
 // a step (nv 4: 120-150), one lane 200-215 (155-185; with its records beyond
 // L2 290, as one CU takes about 18 bytes/ns from memory); with one work-group
 // of nv W threads per chunk and a barrier per level it was 600.  Precond 7,
-// W 32, M^-1 (M^-T alike), at first / one lane / two lanes (the first two of a
-// row with both passes in one launch): 97x65 nv 4 101 / 54 / 52 us, 97x257 nv 5
-// - / 156 / 136, 705x257 - / 160 / 143; 1409x641 (more groups than CUs with two
-// lanes) 966 / 448 / 576, the last with both passes in one launch.
-template <int NV, int W, bool NINE, int P, bool TR, bool ASC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void cilu_pass_kernel(
-    int nic, int njc, int ldi, int nchunk, const float* rec, unsigned long long* links, int most,
-    const double* src, double* z) {
+// W 32, M^-1 (M^-T alike), at first / one lane / two lanes: 97x65 nv 4 101 / 54
+// / 51 us, 97x257 nv 5 - / 156 / 135, 705x257 - / 160 / 141, 1409x641 966 / 442
+// / 576 (more groups than CUs).
+enum { kAscending, kDescending, kBoth };
+template <int NV, int W, bool NINE, int P, bool TR, int PASS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void cilu_apply_kernel(
+    int nic, int njc, int ldi, int nchunk, const float* rec, unsigned long long* links, int most, const double* b,
+    double* z) {
   using La = Lay<NV, W, NINE, P>;
-  // non-transposed: unit-lower L ascending, then D + U descending;
-  // transposed: (D + U)^T ascending, then unit-lower L^T descending
-  constexpr bool DIAG = TR == ASC;
-  constexpr int A = (TR ? 2 : 0) + (ASC ? 0 : 1);
+  constexpr bool UP = PASS != kDescending, DOWN = PASS != kAscending;
   __shared__ ApplyLds<NV, W, NINE, P> sh;
-  const PassGroup at = pass_group((int)blockIdx.x, La::NG, ASC);
+  const PassGroup at = pass_group((int)blockIdx.x, La::NG, UP);
   const int chunk = at.chunk, g = at.group;
   if (chunk >= nchunk) return;
   const int i0 = chunk * W, wk = min(W, nic - i0) - g * La::GW;  // columns from this group on
   if (wk <= 0) return;
-  const bool left = g > 0, right = wk > La::GW, from = ASC ? left : right, to = ASC ? right : left;
+  const bool left = g > 0, right = wk > La::GW;
   // values of steps not yet solved, and the place after an odd row's last
   // entry, meet zero factors: they need to be finite
   double* zero = &sh.ring[0][0][0];
   for (int e = threadIdx.x; e < (int)(sizeof(sh.ring) / sizeof(double)); e += blockDim.x) zero[e] = 0.0;
   for (int e = threadIdx.x; e < (int)(sizeof(sh.tmp) / sizeof(double)); e += blockDim.x) (&sh.tmp[0][0])[e] = 0.0;
-  if (threadIdx.x == 0) {
-    sh.step = sh.edges = sh.taken = 0;
-    sh.loaded = -La::X;  // not even the steps before the first row may start
-  }
+  if (threadIdx.x < 2)
+    sh.pass[threadIdx.x] = {0, -La::X, 0, 0};  // not even the steps before the first row may start
+  if (threadIdx.x == 0) sh.stored = 0;
   __syncthreads();
   const size_t plane = (size_t)njc * ldi, gr = (size_t)(chunk * La::NG + g) * La::nrec(njc);
-  const float* R = rec + La::array(A, nchunk, njc) + gr * La::rs(La::count(A));
+  const float* R1 = rec + La::array(TR ? 2 : 0, nchunk, njc) + gr * La::rs(TR ? La::n2 : La::n1);
+  const float* R2 = rec + La::array(TR ? 3 : 1, nchunk, njc) + gr * La::rs(TR ? La::n1 : La::n2);
   const int col0 = i0 + g * La::GW, wg = min(wk, La::GW);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // link l joins groups l and l + 1
+  Progress &up = sh.pass[0], &down = sh.pass[1];
+  // link l of a pass joins groups l and l + 1
   const size_t lw = La::link(njc);
-  unsigned long long* link = links + (size_t)chunk * (La::NG - 1) * lw;
-  unsigned long long *in = link + (ASC ? g - 1 : g) * lw, *out = link + (ASC ? g : g - 1) * lw;
+  unsigned long long* la = links + (size_t)chunk * (La::NG - 1) * lw;
+  unsigned long long* ld = la + La::pass_links(nchunk, njc);
+  // non-transposed: unit-lower L ascending, then D + U descending;
+  // transposed: (D + U)^T ascending, then unit-lower L^T descending
   if (wave == 0) {
-    cilu_solve<NV, W, NINE, P, DIAG>(R, njc, sh, from);
+    if (UP) cilu_solve<NV, W, NINE, P, TR>(R1, njc, sh, up, left);
+    if (DOWN) cilu_solve<NV, W, NINE, P, !TR>(R2, njc, sh, down, right);
   } else if (wave == 1) {
-    cilu_load<NV, W, NINE, P, ASC, DIAG>(R, njc, ldi, plane, col0, wg, src, sh);
+    if (UP) cilu_load<NV, W, NINE, P, true, TR>(R1, njc, ldi, plane, col0, wg, b, sh, up);
+    if (PASS == kBoth) {
+      // the second pass loads what the first stored, and reuses its LDS
+      while (!lds_read(&sh.stored) || lds_read(&up.step) < La::steps(njc)) __builtin_amdgcn_s_sleep(1);
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    }
+    if (DOWN) cilu_load<NV, W, NINE, P, false, !TR>(R2, njc, ldi, plane, col0, wg, z, sh, down);
   } else if (wave == 2) {
-    cilu_store<NV, W, NINE, P, ASC>(z, njc, ldi, plane, col0, wg, to ? out : nullptr, links, sh);
-  } else if (from) {
-    cilu_receive<NV, W, NINE, P>(links, in, njc, most, sh);
-    // empty for the next pass
-    for (size_t e = threadIdx.x & 63; e < lw; e += 64) slot_store(in + e, kNoValue);
+    if (UP) cilu_store<NV, W, NINE, P, true>(z, njc, ldi, plane, col0, wg, right ? la + g * lw : nullptr, links, sh, up);
+    if (PASS == kBoth) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      if ((threadIdx.x & 63) == 0) lds_write(&sh.stored, 1);
+    }
+    if (DOWN)
+      cilu_store<NV, W, NINE, P, false>(z, njc, ldi, plane, col0, wg, left ? ld + (g - 1) * lw : nullptr, links, sh, down);
+  } else {
+    if (UP && left) cilu_receive<NV, W, NINE, P>(links, la + (g - 1) * lw, njc, most, sh, up);
+    if (DOWN && right) {
+      // the first pass is done with the edge columns' places
+      if (PASS == kBoth)
+        while (lds_read(&up.step) < La::steps(njc)) __builtin_amdgcn_s_sleep(1);
+      cilu_receive<NV, W, NINE, P>(links, ld + g * lw, njc, most, sh, down);
+    }
+    // the links are empty for the next apply
+    for (size_t e = threadIdx.x & 63; e < lw; e += 64) {
+      if (UP && left) slot_store(la + (g - 1) * lw + e, kNoValue);
+      if (DOWN && right) slot_store(ld + g * lw + e, kNoValue);
+    }
   }
 }
 
@@ -1098,105 +1125,109 @@ static hipError_t cilu_factor_t(int nic, int njc, int ldi, const double* idt, co
 }
 
 template <int NV, int W, bool NINE, int P>
-static void cilu_apply_t(int nic, int njc, int ldi, double* store, const double* b, double* z, bool tr, int most,
-                         hipStream_t s) {
+static void cilu_apply_t(int nic, int njc, int ldi, double* store, const double* b, double* z, bool tr, bool apart,
+                         int most, hipStream_t s) {
   using La = Lay<NV, W, NINE, P>;
   const int nchunk = (nic + W - 1) / W;
   const float* rec = reinterpret_cast<const float*>(store + La::links(nchunk, njc));
   unsigned long long* links = reinterpret_cast<unsigned long long*>(store) + kSlotHead;
   const dim3 grid(pass_blocks(nchunk, La::NG)), block(La::NG > 1 ? 256 : 192);
-  auto pass = [&](auto kernel, const double* src) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, s, nic, njc, ldi, nchunk, rec, links, most, src, z);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, nic, njc, ldi, nchunk, rec, links, most, b, z);
   };
-  if (tr) {
-    pass(cilu_pass_kernel<NV, W, NINE, P, true, true>, b);
-    pass(cilu_pass_kernel<NV, W, NINE, P, true, false>, z);
-  } else {
-    pass(cilu_pass_kernel<NV, W, NINE, P, false, true>, b);
-    pass(cilu_pass_kernel<NV, W, NINE, P, false, false>, z);
+  if constexpr (P == 1) {
+    if (apart) {
+      launch(tr ? cilu_apply_kernel<NV, W, NINE, P, true, kAscending> : cilu_apply_kernel<NV, W, NINE, P, false, kAscending>);
+      launch(tr ? cilu_apply_kernel<NV, W, NINE, P, true, kDescending> : cilu_apply_kernel<NV, W, NINE, P, false, kDescending>);
+      return;
+    }
   }
+  launch(tr ? cilu_apply_kernel<NV, W, NINE, P, true, kBoth> : cilu_apply_kernel<NV, W, NINE, P, false, kBoth>);
 }
 
 bool cilu_width_ok(int w) { return w == 8 || w == 16 || w == 24 || w == 32; }
 
 // Lanes per row.  Two make a group's step cheaper, but its columns half as
 // many, so there are twice as many groups, and with more groups than CUs some
-// share one: 1409x641 (270) 576 us against 450.
+// share one: 1409x641 (264) 576 us against 442.  One with a launch per pass,
+// which is not where the time counts.
 template <int NV, int W, bool NINE>
-static int cilu_lanes(int nic) {
-  return (nic + W - 1) / W * Lay<NV, W, NINE, 2>::NG <= 256 ? 2 : 1;
+static int cilu_lanes(int nic, bool apart) {
+  return !apart && (nic + W - 1) / W * Lay<NV, W, NINE, 2>::NG <= 256 ? 2 : 1;
 }
 template <int NV, int W, bool NINE>
-static size_t cilu_size_w(int nic, int njc) {
-  return cilu_lanes<NV, W, NINE>(nic) == 2 ? cilu_size_t<NV, W, NINE, 2>(nic, njc) : cilu_size_t<NV, W, NINE, 1>(nic, njc);
+static size_t cilu_size_w(int nic, int njc, bool apart) {
+  return cilu_lanes<NV, W, NINE>(nic, apart) == 2 ? cilu_size_t<NV, W, NINE, 2>(nic, njc)
+                                                  : cilu_size_t<NV, W, NINE, 1>(nic, njc);
 }
 template <int NV, int W, bool NINE, class... T>
-static hipError_t cilu_factor_w(int nic, T... a) {
-  if (cilu_lanes<NV, W, NINE>(nic) == 2) return cilu_factor_t<NV, W, NINE, 2>(nic, a...);
+static hipError_t cilu_factor_w(bool apart, int nic, T... a) {
+  if (cilu_lanes<NV, W, NINE>(nic, apart) == 2) return cilu_factor_t<NV, W, NINE, 2>(nic, a...);
   return cilu_factor_t<NV, W, NINE, 1>(nic, a...);
 }
-template <int NV, int W, bool NINE, class... T>
-static void cilu_apply_w(int nic, T... a) {
-  if (cilu_lanes<NV, W, NINE>(nic) == 2) cilu_apply_t<NV, W, NINE, 2>(nic, a...);
-  else cilu_apply_t<NV, W, NINE, 1>(nic, a...);
+template <int NV, int W, bool NINE>
+static void cilu_apply_w(int nic, int njc, int ldi, double* store, const double* b, double* z, bool tr, bool apart,
+                         int most, hipStream_t s) {
+  if (cilu_lanes<NV, W, NINE>(nic, apart) == 2) cilu_apply_t<NV, W, NINE, 2>(nic, njc, ldi, store, b, z, tr, apart, most, s);
+  else cilu_apply_t<NV, W, NINE, 1>(nic, njc, ldi, store, b, z, tr, apart, most, s);
 }
 
 template <bool NINE>
-static hipError_t cilu_factor_n(int nic, int njc, int ldi, int nv, int w, const double* idt, const double* blocks,
-                                double* store, hipStream_t s) {
+static hipError_t cilu_factor_n(int nic, int njc, int ldi, int nv, int w, bool apart, const double* idt,
+                                const double* blocks, double* store, hipStream_t s) {
   if (nv == 5) {
-    if (w == 8) return cilu_factor_w<5, 8, NINE>(nic, njc, ldi, idt, blocks, store, s);
-    if (w == 16) return cilu_factor_w<5, 16, NINE>(nic, njc, ldi, idt, blocks, store, s);
-    if (w == 24) return cilu_factor_w<5, 24, NINE>(nic, njc, ldi, idt, blocks, store, s);
-    return cilu_factor_w<5, 32, NINE>(nic, njc, ldi, idt, blocks, store, s);
+    if (w == 8) return cilu_factor_w<5, 8, NINE>(apart, nic, njc, ldi, idt, blocks, store, s);
+    if (w == 16) return cilu_factor_w<5, 16, NINE>(apart, nic, njc, ldi, idt, blocks, store, s);
+    if (w == 24) return cilu_factor_w<5, 24, NINE>(apart, nic, njc, ldi, idt, blocks, store, s);
+    return cilu_factor_w<5, 32, NINE>(apart, nic, njc, ldi, idt, blocks, store, s);
   }
-  if (w == 8) return cilu_factor_w<4, 8, NINE>(nic, njc, ldi, idt, blocks, store, s);
-  if (w == 16) return cilu_factor_w<4, 16, NINE>(nic, njc, ldi, idt, blocks, store, s);
-  if (w == 24) return cilu_factor_w<4, 24, NINE>(nic, njc, ldi, idt, blocks, store, s);
-  return cilu_factor_w<4, 32, NINE>(nic, njc, ldi, idt, blocks, store, s);
+  if (w == 8) return cilu_factor_w<4, 8, NINE>(apart, nic, njc, ldi, idt, blocks, store, s);
+  if (w == 16) return cilu_factor_w<4, 16, NINE>(apart, nic, njc, ldi, idt, blocks, store, s);
+  if (w == 24) return cilu_factor_w<4, 24, NINE>(apart, nic, njc, ldi, idt, blocks, store, s);
+  return cilu_factor_w<4, 32, NINE>(apart, nic, njc, ldi, idt, blocks, store, s);
 }
 
 template <bool NINE>
 static void cilu_apply_n(int nic, int njc, int ldi, int nv, int w, double* store, const double* b, double* z,
-                         bool transpose, int most, hipStream_t s) {
+                         bool transpose, bool apart, int most, hipStream_t s) {
   if (nv == 5) {
-    if (w == 8) cilu_apply_w<5, 8, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
-    else if (w == 16) cilu_apply_w<5, 16, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
-    else if (w == 24) cilu_apply_w<5, 24, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
-    else cilu_apply_w<5, 32, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
+    if (w == 8) cilu_apply_w<5, 8, NINE>(nic, njc, ldi, store, b, z, transpose, apart, most, s);
+    else if (w == 16) cilu_apply_w<5, 16, NINE>(nic, njc, ldi, store, b, z, transpose, apart, most, s);
+    else if (w == 24) cilu_apply_w<5, 24, NINE>(nic, njc, ldi, store, b, z, transpose, apart, most, s);
+    else cilu_apply_w<5, 32, NINE>(nic, njc, ldi, store, b, z, transpose, apart, most, s);
   } else {
-    if (w == 8) cilu_apply_w<4, 8, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
-    else if (w == 16) cilu_apply_w<4, 16, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
-    else if (w == 24) cilu_apply_w<4, 24, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
-    else cilu_apply_w<4, 32, NINE>(nic, njc, ldi, store, b, z, transpose, most, s);
+    if (w == 8) cilu_apply_w<4, 8, NINE>(nic, njc, ldi, store, b, z, transpose, apart, most, s);
+    else if (w == 16) cilu_apply_w<4, 16, NINE>(nic, njc, ldi, store, b, z, transpose, apart, most, s);
+    else if (w == 24) cilu_apply_w<4, 24, NINE>(nic, njc, ldi, store, b, z, transpose, apart, most, s);
+    else cilu_apply_w<4, 32, NINE>(nic, njc, ldi, store, b, z, transpose, apart, most, s);
   }
 }
 
 template <bool NINE>
-static size_t cilu_size_n(int nic, int njc, int nv, int w) {
+static size_t cilu_size_n(int nic, int njc, int nv, int w, bool apart) {
   if (nv == 5)
-    return w == 8 ? cilu_size_w<5, 8, NINE>(nic, njc)
-                  : w == 16 ? cilu_size_w<5, 16, NINE>(nic, njc)
-                            : w == 24 ? cilu_size_w<5, 24, NINE>(nic, njc) : cilu_size_w<5, 32, NINE>(nic, njc);
-  return w == 8 ? cilu_size_w<4, 8, NINE>(nic, njc)
-                : w == 16 ? cilu_size_w<4, 16, NINE>(nic, njc)
-                          : w == 24 ? cilu_size_w<4, 24, NINE>(nic, njc) : cilu_size_w<4, 32, NINE>(nic, njc);
+    return w == 8 ? cilu_size_w<5, 8, NINE>(nic, njc, apart)
+                  : w == 16 ? cilu_size_w<5, 16, NINE>(nic, njc, apart)
+                            : w == 24 ? cilu_size_w<5, 24, NINE>(nic, njc, apart) : cilu_size_w<5, 32, NINE>(nic, njc, apart);
+  return w == 8 ? cilu_size_w<4, 8, NINE>(nic, njc, apart)
+                : w == 16 ? cilu_size_w<4, 16, NINE>(nic, njc, apart)
+                          : w == 24 ? cilu_size_w<4, 24, NINE>(nic, njc, apart) : cilu_size_w<4, 32, NINE>(nic, njc, apart);
 }
 
-size_t cilu_size(int nic, int njc, int nv, int w, bool nine) {
-  return nine ? cilu_size_n<true>(nic, njc, nv, w) : cilu_size_n<false>(nic, njc, nv, w);
+size_t cilu_size(int nic, int njc, int nv, int w, bool nine, bool apart) {
+  return nine ? cilu_size_n<true>(nic, njc, nv, w, apart) : cilu_size_n<false>(nic, njc, nv, w, apart);
 }
 
-hipError_t cilu_factor(int nic, int njc, int ldi, int nv, int w, bool nine, const double* idt, const double* blocks,
-                       double* store, hipStream_t s) {
-  return nine ? cilu_factor_n<true>(nic, njc, ldi, nv, w, idt, blocks, store, s)
-              : cilu_factor_n<false>(nic, njc, ldi, nv, w, idt, blocks, store, s);
+hipError_t cilu_factor(int nic, int njc, int ldi, int nv, int w, bool nine, bool apart, const double* idt,
+                       const double* blocks, double* store, hipStream_t s) {
+  return nine ? cilu_factor_n<true>(nic, njc, ldi, nv, w, apart, idt, blocks, store, s)
+              : cilu_factor_n<false>(nic, njc, ldi, nv, w, apart, idt, blocks, store, s);
 }
 
 hipError_t cilu_apply(int nic, int njc, int ldi, int nv, int w, bool nine, double* store, const double* b, double* z,
-                      bool transpose, int polls, hipStream_t s) {
-  if (nine) cilu_apply_n<true>(nic, njc, ldi, nv, w, store, b, z, transpose, polls, s);
-  else cilu_apply_n<false>(nic, njc, ldi, nv, w, store, b, z, transpose, polls, s);
+                      bool transpose, bool apart, int polls, hipStream_t s) {
+  if (nine) cilu_apply_n<true>(nic, njc, ldi, nv, w, store, b, z, transpose, apart, polls, s);
+  else cilu_apply_n<false>(nic, njc, ldi, nv, w, store, b, z, transpose, apart, polls, s);
   return hipGetLastError();
 }
 

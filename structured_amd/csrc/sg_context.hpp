@@ -108,6 +108,7 @@ struct sg_ctx {
   sg::DevBuf q, r, v, w;           // SoA work vectors (nvar * plane)
   sg::DevBuf partial, l2;  // slots of the norm's partial sums (empty between launches), the norms
   int wait_polls = sg::kWaitPolls;  // bound of the waits on slots
+  bool all_cus = false;             // every CU of the device takes work of the stream
   sg::DevBuf wall_cp, wall_cf, wall_f;
   sg::DevClosure clo;              // beta closure applied by every residual / J.v launch
   sg::DevBuf clo_params, clo_w2;   // MLP parameters (FP32) and W2 (BF16), raw storage

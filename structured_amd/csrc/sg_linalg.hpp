@@ -62,13 +62,15 @@ hipError_t lilu_apply(int nic, int njc, int ldi, int nv, const double* ilu, cons
 // is the storage in doubles that cilu_factor writes and cilu_apply reads: the
 // links between column groups with their SlotHead (empty between applies), the
 // FP32 factors in the order of M^-1 and of M^-T, and the factorisation's operands
-// gathered in level order.  polls bounds the apply's waits on the links
+// gathered in level order.  apart (the same in all three): the apply takes a
+// launch per pass, for a device on which not every CU takes part; polls bounds
+// the apply's waits on the links
 bool cilu_width_ok(int w);
-size_t cilu_size(int nic, int njc, int nv, int w, bool nine);
-hipError_t cilu_factor(int nic, int njc, int ldi, int nv, int w, bool nine, const double* idt, const double* blocks,
-                       double* rec, hipStream_t s);
+size_t cilu_size(int nic, int njc, int nv, int w, bool nine, bool apart);
+hipError_t cilu_factor(int nic, int njc, int ldi, int nv, int w, bool nine, bool apart, const double* idt,
+                       const double* blocks, double* rec, hipStream_t s);
 hipError_t cilu_apply(int nic, int njc, int ldi, int nv, int w, bool nine, double* store, const double* b, double* z,
-                      bool transpose, int polls, hipStream_t s);
+                      bool transpose, bool apart, int polls, hipStream_t s);
 // adjoint helpers: J^T psi from the blocks, or with idt psi idt - J^T psi
 hipError_t jt_gather(int nic, int njc, int ldi, int nv, const double* blocks, const double* psi, double* out,
                      hipStream_t s, const double* idt = nullptr);

@@ -51,6 +51,7 @@ struct SolverState {
   PinnedBuf hpin;            // a dot product, the Krylov coefficients going up
   PinnedBuf hres;            // results of two Arnoldi steps, written by the device
   int pc_width = 16;         // chunk width of precond 6
+  bool pc_apart = false;     // its passes take a launch each (as the factors were laid out)
   // have_lhs: the operator and preconditioner of the caller's last set_lhs are
   // in place.  Every call that changes the preconditioner settings or
   // overwrites the linearisation state (preallocate, set_pc, sg_solve, the
@@ -154,7 +155,7 @@ int precond_apply(sg_ctx* ctx, const double* v, double* z) {
   }
   if (S->precond == 6 || S->precond == 7) {
     SG_TRY(cilu_apply(nic, njc, ldi, nv, S->pc_width, S->precond == 7, S->cilu.p, v, z, S->transpose,
-                      ctx->wait_polls, ctx->stream),
+                      S->pc_apart, ctx->wait_polls, ctx->stream),
            "cilu apply");
     return SG_OK;
   }
@@ -242,9 +243,10 @@ int factor_preconditioner(sg_ctx* ctx, const double* idt_pc) {
     return SG_OK;
   }
   if (S->precond == 6 || S->precond == 7) {
-    const size_t need = cilu_size(nic, njc, nv, S->pc_width, S->precond == 7);
+    S->pc_apart = !ctx->all_cus;
+    const size_t need = cilu_size(nic, njc, nv, S->pc_width, S->precond == 7, S->pc_apart);
     if (S->cilu.n < need && S->cilu.alloc(need) != hipSuccess) return sg_fail(ctx, SG_ERR_HIP, "allocation failed");
-    SG_TRY(cilu_factor(nic, njc, ldi, nv, S->pc_width, S->precond == 7, pc_idt, blk, S->cilu.p, ctx->stream),
+    SG_TRY(cilu_factor(nic, njc, ldi, nv, S->pc_width, S->precond == 7, S->pc_apart, pc_idt, blk, S->cilu.p, ctx->stream),
            "cilu factor");
     return SG_OK;
   }

@@ -96,7 +96,9 @@ def test_linear_solve_after_a_wait_that_gave_up(eq):
 
 
 @pytest.mark.parametrize("transpose", [False, True])
-def test_preconditioner_after_a_wait_that_gave_up(eq, transpose):
+@pytest.mark.parametrize("few", [0, 1])  # a launch for both passes, a launch each
+def test_preconditioner_after_a_wait_that_gave_up(eq, transpose, few):
+    assert lib.load().sg_test_few_cus(eq.h, C.c_int(few)) == 1 - few
     q, _ = states(eq)
     dt = eq.calc_dt(q, 20.0)
     rng = np.random.default_rng(1)
