@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "sg_kernels.hpp"
 #include "sg_residual.hpp"
@@ -22,12 +23,15 @@ static bool wide_rows(const DevGeom& g) {
 // the most work-groups, and a work-group of 16 rows takes twice as long as one
 // of 8 (dual numbers 2.2 times: one of 16 rows or two of 8 fill the CU's
 // registers, and the one has nothing to run at its barriers).  Measured, 16
-// against 8 rows, SA residual: 67 / 75 us at 1409x641, 22 / 25 at 705x321,
-// equal at 545x385, 20.5 / 18 at 481x257, 15.7 / 14.7 at 449x225; J.v: 32 / 36
-// at 705x321, 32 / 30 at 545x385, 76 / 68 at 1001x501 (both sides while the
-// kernels still spilled, which cost either 4 to 8%).
-// With a coloured direction per z-layer the chip is full and the larger tile is
-// 4% faster (J^T psi at 385x193: 1.91 / 1.99 ms).
+// against 8 rows, states from memory, SA residual: 67.5 / 74.6 us at 1409x641,
+// 23.1 / 25.9 at 705x321, and where the rule takes 8: 58.1 / 61.4 at 1201x601,
+// 44.5 / 45.3 at 1001x501, 37.4 / 35.5 at 865x449, 22.6 / 23.0 at 545x385, 20.2 /
+// 18.1 at 481x257, 14.8 / 12.1 at 281x151; laminar 18.8 / 21.3 at 705x321, 18.4 /
+// 18.4 at 545x385.  J.v: 33.6 / 38.3 at 705x321, and 8: 123 / 118 at 1409x641,
+// 75.8 / 71.3 at 1001x501, 32.6 / 32.4 at 545x385.
+// Jacobian blocks (a coloured direction per z-layer) take 8 rows: 1,367 / 1,352 us
+// at 385x193, 403 / 347 at 193x97, 1,168 / 1,157 at 545x385 (45 directions), 9,207 /
+// 9,257 at 1001x501.
 template <class S>
 static int tile_rows(const DevGeom& g) {
   constexpr int kCUs = 256, kRatio = sizeof(S) == sizeof(double) ? 20 : 22;  // tenths
@@ -66,7 +70,9 @@ static void launch_cl(hipStream_t s, const DevGeom& g, const DevPhys& ph, const 
                       unsigned nz = 1) {
   const unsigned extra = no.slots ? 1 : 0;  // the work-group that sums the norms
   if (wide_rows(g)) launch_tiles<kTileSmall, size_t, S, SA>(extra, nz, s, g, ph, bc, fq, fo, beta_dot, clo, no);
-  else if (nz > 1 || tile_rows<S>(g) == kTileLarge)
+  else if constexpr (std::is_same_v<F, SeedField>)
+    launch_tiles<kTileSmall, unsigned, S, SA>(extra, nz, s, g, ph, bc, fq, fo, beta_dot, clo, no);
+  else if (tile_rows<S>(g) == kTileLarge)
     launch_tiles<kTileLarge, unsigned, S, SA>(extra, nz, s, g, ph, bc, fq, fo, beta_dot, clo, no);
   else launch_tiles<kTileSmall, unsigned, S, SA>(extra, nz, s, g, ph, bc, fq, fo, beta_dot, clo, no);
 }

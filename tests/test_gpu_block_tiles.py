@@ -1,5 +1,5 @@
 """Jacobian blocks from one launch over all coloured directions, on grids at the
-edges of the 31 x 15 tiles that launch takes: the exact blocks through J^T psi
+edges of 31 x 7 and 31 x 15 tiles: the exact blocks through J^T psi
 (dot products with the oracle's J.v), the first-order ones (3 x 3 colours) through
 the chunked ILU built from them, on the 3x3-box pattern and on the 13-point one,
 where the slots that no direction writes have to be zero."""
@@ -13,7 +13,7 @@ import precond_model as pm
 from structured_amd import cases, lib
 
 pytestmark = pytest.mark.gpu
-SIZES = [(31, 14), (31, 15), (32, 16), (62, 30), (63, 31)]
+SIZES = [(31, 14), (31, 15), (32, 16), (62, 21), (62, 30), (63, 31)]
 
 
 def make(cols, rows, sa):

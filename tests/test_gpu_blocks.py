@@ -1,6 +1,6 @@
-"""Jacobian blocks from one launch over all coloured directions, on small grids
-(of one to six 31 x 15 tiles): the exact blocks through J^T psi (the dot-product
-identity with J.v, and the oracle's J.v on unit vectors)."""
+"""Jacobian blocks from one launch over all coloured directions, on grids at
+the edges of the residual's 31 x 7 tiles: the exact blocks through J^T psi
+(the dot-product identity with J.v, and the oracle's J.v on unit vectors)."""
 import numpy as np
 import pytest
 
