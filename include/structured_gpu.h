@@ -195,14 +195,17 @@ int sg_jv_dev_async(sg_ctx* ctx, const double* q_dev, const double* v_dev, doubl
 int sg_jtv_dev(sg_ctx* ctx, const double* q_dev, const double* psi_dev, double* jtpsi_dev, double* dbeta_dev);
 /* Enqueue the residual (and, if l2_dev is not NULL, its per-equation L2 norm
  * ||R_k||_2 into l2_dev[0..nvar-1], device memory: exactly nvar doubles are
- * written) without synchronising. */
+ * written) without synchronising.  If the device stalls for seconds inside the
+ * launch the norms are NaN, and stay NaN until a call has returned norms to the
+ * host (sg_residual, sg_residual_dev, an explicit step, sg_solve). */
 int sg_residual_dev_async(sg_ctx* ctx, const double* q_dev, double* r_dev, double* l2_dev);
 /* sg_residual_dev_async without any device allocation, for callers that
  * cannot allocate (code under HIP graph capture, tight serving loops).  No
  * counterpart in the reference.  The norm scratch (per-tile partial sums)
  * lives in a static device array of each GPU, at most SG_NOALLOC_MAX_TILES
- * residual tiles of 31 x 7 cells (1.25 MiB, held until the process ends); a larger grid is SG_ERR_ARG.  Calls that overlap on one
- * GPU share that array and race: serialise them. */
+ * residual tiles of 31 x 7 cells (1.25 MiB, held until the process ends); a
+ * larger grid is SG_ERR_ARG.  Calls that overlap on one GPU share that array and
+ * race: serialise them. */
 #define SG_NOALLOC_MAX_TILES 16384
 int sg_residual_dev_async_noalloc(sg_ctx* ctx, const double* q_dev, double* r_dev, double* l2_dev);
 int sg_synchronize(sg_ctx* ctx);
@@ -439,7 +442,9 @@ int sg_mlp_loss_grad(sg_mlp* net, int n, const float* x, const float* t, float* 
 /* epochs of Adam over n samples (host arrays, copied to the device once) in
  * minibatches of `batch` rows drawn by a seeded shuffle per epoch (the last
  * partial minibatch is dropped when n > batch); loss_hist[epochs] receives
- * the mean minibatch loss of each epoch (may be NULL). */
+ * the mean minibatch loss of each epoch (may be NULL).  The network keeps the
+ * device memory of its largest training set so far (52 bytes a sample and 4 a
+ * minibatch) until it is destroyed. */
 int sg_mlp_train(sg_mlp* net, int n, const float* x, const float* t, int epochs, int batch, float lr,
                  unsigned long long seed, float* loss_hist);
 /* Closure of a context from the current parameters of a network. */

@@ -9,10 +9,10 @@
 //
 // The factorisation walks a chunk's levels L = j + 2 (i - i0) with one
 // work-group per chunk.  The apply cuts the chunk once more, into groups of
-// up to 6 (nv 5) or 8 (nv 4) columns, twice that on very wide grids, with one
-// solving wave each: a column depends on earlier columns only, so the groups
-// run as a pipeline, each on its own CU, and hand the solved values of their
-// edge columns on through memory.
+// up to 6 (nv 5) or 8 (nv 4) columns, twice that on very wide grids and where not
+// every CU of the device takes part, with one solving wave each: a column depends
+// on earlier columns only, so the groups run as a pipeline, each on its own CU,
+// and hand the solved values of their edge columns on through memory.
 //
 // Factors are stored in FP32 (the preconditioner only has to approximate
 // A^-1; FGMRES runs in FP64) in the order the solving waves read them, see

@@ -28,8 +28,8 @@
 // another and cost a third of the instructions that are not FP64; ghost cells
 // are evaluated once, by threads of their own.  With it, a finaliser that waits
 // on slots instead of counting arrivals, and metrics loaded just ahead of their
-// use so that nothing spills, SA at 545x385 24.0 -> 20.8 us, 1409x641 77 -> 62.5,
-// laminar 97x65 16.4 -> 9.0; J.v at 705x321 41.5 -> 32.6.
+// use so that nothing spills, SA at 545x385 24.0 -> 20.2 us, 1409x641 77 -> 61,
+// laminar 97x65 16.4 -> 9.2; J.v at 705x321 41.5 -> 32.4.
 #pragma once
 #include "sg_closure.hpp"
 #include "sg_device.hpp"
