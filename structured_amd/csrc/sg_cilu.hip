@@ -388,7 +388,8 @@ cilu_factor_kernel(int nic, int njc, int nlev, const double2* ops, float* rec) {
   const int c = cw < CW ? wave * CW + cw : W, cc = min(c, W - 1);
   double* mat = gj[cw < CW ? wave * CW + cw : Fa::NW * CW];
   const int nrec = La::nrec(njc);
-  // the record of cell (ci, jj) in array a, or the spare one
+  // the record of cell (ci, jj) in array a, or the spare one (where all lanes take
+  // the first place, so that they cost one store)
   auto record = [&](bool there, int a, int ci, int jj) {
     const int g = ci / La::GW, cl = ci % La::GW;
     const bool asc = a == 0 || a == 2;
@@ -496,7 +497,7 @@ cilu_factor_kernel(int nic, int njc, int nlev, const double2* ops, float* rec) {
     // wait for a load waits for all of them.
     float* const to0 = record(valid, 0, cc, j);
 #pragma unroll
-    for (int h = 0; h < P; ++h) put_record<La::n1, La::LN>(to0, lane_of(true, cc, r, h), r0[h]);
+    for (int h = 0; h < P; ++h) put_record<La::n1, La::LN>(to0, valid ? lane_of(true, cc, r, h) : 0, r0[h]);
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- inverse of the factored diagonal block
@@ -542,7 +543,7 @@ cilu_factor_kernel(int nic, int njc, int nlev, const double2* ops, float* rec) {
     }
     float* const to1 = record(valid, 1, cc, j);
 #pragma unroll
-    for (int h = 0; h < P; ++h) put_record<La::n2, La::LN>(to1, lane_of(false, cc, r, h), r1[h]);
+    for (int h = 0; h < P; ++h) put_record<La::n2, La::LN>(to1, valid ? lane_of(false, cc, r, h) : 0, r1[h]);
     lds_barrier();
   }
 }
